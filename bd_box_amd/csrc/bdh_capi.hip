@@ -375,7 +375,7 @@ int assemble_and_factor_launches(bdh_system* s, void* Abuf, const double4* pos2)
                      : launch_rpy_assemble<float>(s->pos, s->N, s->preDii, s->preDij, A, s->ld, s->st, pos2))
             return -1;
         REC_END(PH_ASSEMBLE);
-        if (chol_factor<float>(A, s->ld, s->n_pad, s->Lbuf, s->flags + 1, s->syrk_mode, s->st, s->rec)) return -1;
+        if (chol_factor<float>(A, s->ld, s->n, s->n_pad, s->Lbuf, s->flags + 1, s->syrk_mode, s->st, s->rec)) return -1;
     } else {
         double* A = (double*)M;
         REC_BEGIN(PH_ASSEMBLE);
@@ -383,7 +383,7 @@ int assemble_and_factor_launches(bdh_system* s, void* Abuf, const double4* pos2)
                      : launch_rpy_assemble<double>(s->pos, s->N, s->preDii, s->preDij, A, s->ld, s->st, pos2))
             return -1;
         REC_END(PH_ASSEMBLE);
-        if (chol_factor<double>(A, s->ld, s->n_pad, s->Lbuf, s->flags + 1, SYRK_F64, s->st, s->rec)) return -1;
+        if (chol_factor<double>(A, s->ld, s->n, s->n_pad, s->Lbuf, s->flags + 1, SYRK_F64, s->st, s->rec)) return -1;
     }
     if (M == s->A) s->have_L = true;
     return 0;
@@ -771,7 +771,7 @@ int dpotrf_impl(char uplo, double* A, int n, int ld, int* info, int syrk_mode)
         hipLaunchKernelGGL(full_to_lower_kernel<T>, grid, dim3(256), 0, st, d_full, (long long)n, n,
                            d_A, lda, up ? 1 : 0);
         rc = launch_set_identity_pad<T>(d_A, lda, n, n_pad, st);
-        if (!rc) rc = chol_factor<T>(d_A, lda, n_pad, d_Lbuf, d_status, syrk_mode, st);
+        if (!rc) rc = chol_factor<T>(d_A, lda, n, n_pad, d_Lbuf, d_status, syrk_mode, st);
         if (!rc) {
             hipLaunchKernelGGL(lower_to_full_kernel<T>, grid, dim3(256), 0, st, (const T*)d_A, lda, n,
                                d_full, (long long)n, 0);
@@ -1999,13 +1999,11 @@ struct bdh_batch {
     ForceParams fp{};
     Topology topo{};
     std::vector<BatchChain> hc;
-    std::vector<int> chol_blocks;   // workgroups of update launch k (host)
-    std::vector<int> tab;           // host copy of every prefix table
-    int left_max = -1;              // update schedule (batch_set_tiles)
-    int outer = 0;                  // outer panel width of every chain (batch_set_tiles)
+    int left_max = -1, outer = 256;   // settings of bdh_batch_set_tiles
     BatchPlan plan;
     BatchChain* d_ch = nullptr;
     int* d_tab = nullptr;           // every prefix table
+    FlowTask* d_tasks = nullptr;    // workgroups of the factorization
     double4* pos = nullptr;
     double* Q = nullptr;
     double2* LJ = nullptr;
@@ -2101,41 +2099,11 @@ int batch_factor(bdh_batch* b)
     return 0;
 }
 
-// Update schedule and outer panel width of every chain's factorization: chains with n_pad <=
-// left_max update left-looking inside each outer panel of `outer` columns, the others
-// right-looking (chol_step); left_max < 0 gives each chain the schedule a single system of
-// its size uses.  The update launches' prefix tables are rewritten, and the captured graphs,
-// whose grids they size, are dropped.
+// The settings of bdh_batch_set_tiles: recorded for bdh_batch_get_tiles.  The factorization is one
+// launch whose workgroups take whole tiles, so it has no panel schedule to choose.
 int batch_set_tiles(bdh_batch* b, int left_max, int outer)
 {
     BDH_CHECK(outer == 256 || outer == 512 || outer == 1024, "bdh_batch_set_tiles: outer width 256, 512 or 1024");
-    const int B = b->B, W = B + 1;
-    for (auto& h : b->hc) {
-        h.left = left_max < 0 ? chol_left_looking(h.n_pad) : h.n_pad <= left_max;
-        h.outer = outer;
-    }
-    for (int k = 0; k < b->plan.chol_steps; ++k) {
-        int* t = b->tab.data() + (size_t)(6 + k) * W;
-        long long acc = 0;
-        for (int c = 0; c < B; ++c) {
-            t[c] = (int)acc;
-            acc += chol_update_blocks(b->hc[c].n_pad, b->hc[c].left != 0, b->hc[c].outer, k);
-        }
-        BDH_CHECK(acc <= (long long)INT32_MAX, "bdh_batch_set_schedule: batch too large");
-        t[B] = (int)acc;
-        b->chol_blocks[k] = (int)acc;
-    }
-    BDH_HIP(hipStreamSynchronize(b->st));
-    BDH_HIP(hipMemcpy(b->d_tab, b->tab.data(), sizeof(int) * b->tab.size(), hipMemcpyHostToDevice));
-    BDH_HIP(hipMemcpy(b->d_ch, b->hc.data(), sizeof(BatchChain) * B, hipMemcpyHostToDevice));
-    if (b->cycle_exec) {
-        BDH_HIP(hipGraphExecDestroy(b->cycle_exec));
-        b->cycle_exec = nullptr;
-    }
-    if (b->factor_exec) {
-        BDH_HIP(hipGraphExecDestroy(b->factor_exec));
-        b->factor_exec = nullptr;
-    }
     b->left_max = left_max;
     b->outer = outer;
     return 0;
@@ -2368,8 +2336,6 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
     // layout
     b->hc.resize(B);
     long long bead = 0, mat = 0, lb = 0, xo = 0, pp = 0, pf = 0, pt = 0, bonds_tot = 0;
-    int max_steps = 0;
-    b->outer = chol_outer_default();
     for (int c = 0; c < B; ++c) {
         BDH_CHECK(N[c] > 0 && N[c] <= (1 << 20), "bdh_batch_create: chain size");
         BDH_CHECK(nbonds[c] >= 0 && (nbonds[c] == 0 || (bonds && bond_parms)), "bdh_batch_create: bonds");
@@ -2382,8 +2348,6 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
         h.fsplits = force_splits(h.N);
         h.tcols = trmv_col_blocks(h.n);
         h.ldx = h.n + (h.n & 1);
-        h.left = chol_left_looking(h.n_pad);
-        h.outer = chol_outer_default();
         h.mat = mat;
         h.lb = lb;
         h.xi_off = xo;
@@ -2398,7 +2362,6 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
         pf += (long long)h.fsplits * h.n;
         pt += (long long)h.tcols * TRMV_MAX_RHS * h.n;
         bonds_tot += nbonds[c];
-        max_steps = std::max(max_steps, chol_update_steps(h.n_pad));
     }
     BDH_CHECK(bead <= (1 << 26), "bdh_batch_create: too many beads");
     b->Ntot = (int)bead;
@@ -2406,11 +2369,10 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
     for (long long i = 0; i < bead; ++i)
         BDH_CHECK(coord[4 * i + 3] > 0.0, "bdh_batch_create: bead radius must be positive");
 
-    // prefix tables: asm, pair, force, trmv, rows, trsm, then max_steps chol tables
+    // prefix tables: asm, pair, force, trmv, rows
     const int W = B + 1;
-    const int ntab = 6 + max_steps;
+    const int ntab = 5;
     std::vector<int> tab((size_t)ntab * W, 0);
-    b->chol_blocks.assign(max_steps, 0);
     auto fill = [&](int t, auto count) -> int {
         long long acc = 0;
         for (int c = 0; c < B; ++c) {
@@ -2426,19 +2388,12 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
     b->plan.trmv_blocks = b->mixed ? fill(3, [](const BatchChain& h) { return trmv_blocks<float>(h.n); })
                                    : fill(3, [](const BatchChain& h) { return trmv_blocks<double>(h.n); });
     b->plan.rows_blocks = fill(4, [](const BatchChain& h) { return ceil_div(h.n, 64); });
-    b->plan.trsm_blocks = fill(5, [](const BatchChain& h) { return chol_trsm0_blocks(h.n_pad); });
-    for (int k = 0; k < max_steps; ++k)
-        b->chol_blocks[k] = fill(6 + k, [k](const BatchChain& h) { return chol_update_blocks(h.n_pad, h.left, h.outer, k); });
     BDH_CHECK(b->plan.asm_blocks >= 0 && b->plan.pair_blocks >= 0 && b->plan.force_blocks >= 0 &&
-              b->plan.trmv_blocks >= 0 && b->plan.rows_blocks >= 0 && b->plan.trsm_blocks >= 0,
-              "bdh_batch_create: batch too large");
-    for (int k = 0; k < max_steps; ++k)
-        BDH_CHECK(b->chol_blocks[k] >= 0, "bdh_batch_create: batch too large");
+              b->plan.trmv_blocks >= 0 && b->plan.rows_blocks >= 0, "bdh_batch_create: batch too large");
     if (dmalloc(&b->d_tab, sizeof(int) * tab.size())) return -1;
     BDH_HIP(hipMemcpy(b->d_tab, tab.data(), sizeof(int) * tab.size(), hipMemcpyHostToDevice));
     if (dmalloc(&b->d_ch, sizeof(BatchChain) * B)) return -1;
     BDH_HIP(hipMemcpy(b->d_ch, b->hc.data(), sizeof(BatchChain) * B, hipMemcpyHostToDevice));
-    b->tab = std::move(tab);
     b->plan.nch = B;
     b->plan.ch = b->d_ch;
     b->plan.asm_pre = b->d_tab;
@@ -2446,10 +2401,16 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
     b->plan.force_pre = b->d_tab + 2 * W;
     b->plan.trmv_pre = b->d_tab + 3 * W;
     b->plan.rows_pre = b->d_tab + 4 * W;
-    b->plan.trsm_pre = b->d_tab + 5 * W;
-    b->plan.chol_pre = b->d_tab + 6 * W;
-    b->plan.chol_steps = max_steps;
-    b->plan.chol_blocks = b->chol_blocks.data();
+    {
+        std::vector<int> orders;
+        for (const auto& h : b->hc) orders.push_back(h.n_pad);
+        const std::vector<FlowTask> tasks = chol_batch_tasks(orders);
+        BDH_CHECK(tasks.size() <= (size_t)INT32_MAX, "bdh_batch_create: batch too large");
+        if (dmalloc(&b->d_tasks, sizeof(FlowTask) * tasks.size())) return -1;
+        BDH_HIP(hipMemcpy(b->d_tasks, tasks.data(), sizeof(FlowTask) * tasks.size(), hipMemcpyHostToDevice));
+        b->plan.tasks = b->d_tasks;
+        b->plan.ntasks = (int)tasks.size();
+    }
 
     // forces (a single set of parameters; the pair-skip reach is the largest of any chain)
     ForceParams& fp = b->fp;
@@ -2585,7 +2546,7 @@ void bdh_batch_destroy(bdh_batch* b)
 {
     if (!b) return;
     if (b->st) (void)hipStreamSynchronize(b->st);
-    dfree(b->d_ch); dfree(b->d_tab);
+    dfree(b->d_ch); dfree(b->d_tab); dfree(b->d_tasks);
     dfree(b->pos); dfree(b->Q); dfree(b->LJ);
     dfree(b->conn_off); dfree(b->conn); dfree(b->bond_parm);
     dfree(b->F); dfree(b->Rf); dfree(b->RsB); dfree(b->xi); dfree(b->xi_user);

@@ -1,26 +1,17 @@
-// Blocked right-looking Cholesky D = L L^T and the triangular product L.x on gfx950.
+// Blocked Cholesky D = L L^T and the triangular product L.x on gfx950.
 //
 // Replaces the reference's my_dpotrf / my_dtrmv (src/myblas.c:45-118: LAPACK
 // dpotrf("U") + dtrmv("U","T"), or MAGMA spotrf_gpu('L') + cublasStrmv in the CUDA
 // build).  The factor is stored lower, column-major, in place of D; n is padded to a
 // multiple of PAD_TO with an identity block so every tile is whole.
 //
-// Per panel of CHOL_NB = 64 columns c0..c0+63:
-//   diagonal block  L_kk of the 64x64 block in FP64 (factor_diag64): the four wavefronts
-//                   own 16 columns each and run as a pipeline, each applying the earlier
-//                   columns' updates as they are published in LDS and then factoring its
-//                   own.  Stored in T into A and in FP64 into Lbuf.
-//   TRSM            L_ik = A_ik L_kk^{-T} for every row below, FP64 forward substitution,
-//                   four lanes per row (a quad exchanges each finished entry through DPP).
-//   trailing SYRK   A22 -= L21 L21^T over 128x128 lower tiles on MFMA:
-//                   T = float : v_mfma_f32_32x32x2_f32, FP32 accumulation
-//                   T = double: v_mfma_f64_16x16x4_f64
-//                   Workgroup 0 owns the tile holding the next panel's diagonal block; it
-//                   keeps that block in LDS and factors it right after its update, so the
-//                   next diagonal factorization overlaps the rest of the SYRK (lookahead
-//                   without a second stream).  Only panel 0 needs its own launch.
-// FP64 is used for the diagonal blocks and the panel solve in both precisions; in the FP32
-// variant the factor is rounded to FP32 when stored.
+// One launch factors a matrix, or all matrices of a batch: one workgroup per 128x128 tile,
+// left-looking (chol_flow_kernel).  The sums over earlier columns run on MFMA:
+//   T = float : v_mfma_f32_32x32x2_f32 (or split-bf16 v_mfma_f32_32x32x16_bf16), FP32 accumulation
+//   T = double: v_mfma_f64_16x16x4_f64
+// The 64x64 diagonal blocks are factored (factor_diag64) and the blocks below them solved
+// (flow_solve64) in FP64 in both precisions; in the FP32 variant the factor is rounded to FP32
+// when stored.
 #include <algorithm>
 
 #include "bdh_common.hpp"
@@ -30,8 +21,6 @@
 namespace bdh {
 
 constexpr int DG_LD = CHOL_NB + 1;   // row pitch (doubles) of the diagonal block in LDS
-constexpr int SY_TILE_C = 128;       // SYRK tile edge
-constexpr int TRSM_ROWS = 64;        // rows per TRSM workgroup (4 lanes per row)
 
 // Value of v held by lane `src` (uniform), through two v_readlane_b32.
 __device__ __forceinline__ double readlane_f64(double v, int src)
@@ -42,188 +31,225 @@ __device__ __forceinline__ double readlane_f64(double v, int src)
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// 1/sqrt(x): hardware estimate refined by two Newton steps y <- y (3 - x y^2) / 2.
+// 1/sqrt(x): hardware estimate (relative error about 2^-23) refined by one third-order step,
+// y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2, whose truncation (5/16 e^3) is below 2^-68.  Four
+// dependent operations where two Newton steps take eight; the diagonal factor's pivot chain
+// runs through it once per column.
 __device__ __forceinline__ double rsqrt_f64(double x)
 {
-    double y = __builtin_amdgcn_rsq(x);
-    y = y * (1.5 - 0.5 * x * y * y);
-    y = y * (1.5 - 0.5 * x * y * y);
-    return y;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = __builtin_fma(-(x * y), y, 1.0);
+    return __builtin_fma(__builtin_fma(e, 0.375, 0.5), y * e, y);
 }
 
 // Per diagonal block, the workspace Lb holds (FP64):
 //   Lb[0 .. 4095]      L_kk column-major, zeros above the diagonal
-//   Lb[4096 + 256 J]   inverse of its J-th 16x16 diagonal sub-block, column-major, J = 0..3
-constexpr int LB_STRIDE = CHOL_NB * CHOL_NB + 4 * 256;
+//   Lb[4096 + SINV J]  inverse of its J-th 16x16 diagonal sub-block, column-major with pitch
+//                      SINV_P (odd, so the factor's rows and the solve's columns of it both
+//                      spread over the LDS banks), J = 0..3
+// What lies above the diagonal of either is not part of the factor and is not read.
+constexpr int SINV_P = 17;
+constexpr int SINV = 16 * SINV_P;
+constexpr int LB_STRIDE = CHOL_NB * CHOL_NB + 4 * SINV;
 
-// Bounded wait (inside one workgroup) until the LDS counter reaches `need`; returns the
-// counter's value then, or -1 if it never did.  Every wavefront that publishes to the counter
-// runs concurrently with the waiting one, so the wait ends unless a wavefront faulted; the
-// bound keeps a defect from hanging the GPU.
-constexpr int LDS_SPIN = 1 << 22;
-__device__ __forceinline__ int wait_lds_count(int* cnt, int need)
+// One wavefront: columns cw .. cw + 15 of the 64x64 block, lane = row, p[u] = column cw + u with
+// every earlier group's update made; finished columns go to L (LDS, column-major; what a lane
+// above the diagonal holds is not part of the factor).
+// Per column t the pivot chain is: reciprocal square root, l_{t+1,t}, the next pivot
+// a_{t+1,t+1} - l_{t+1,t}^2.  Column t + 1 takes column t's update from a broadcast (v_readlane) of
+// its entry before it is scaled, so it does not wait for the LDS; the later ones take it one
+// column late from LDS broadcasts of the stored column, two at a time between the dependent
+// operations of the next pivot (fill), which are 12 cycles apart where an FP64 FMA issues in 4.
+// step(t): work of the caller's for the same gaps.
+// The inverse of the 16x16 diagonal sub-block is the solution of X L^T = I, i.e. what the column
+// steps make of 16 more rows that hold the identity: FIRST (cw = 0, every lane a row of the
+// block) carries them in y; the other groups hold them in lanes 0 .. 15 of p, whose rows lie
+// above the group's diagonal.
+template <bool FIRST, typename Step>
+__device__ __forceinline__ void factor_group16(double (&p)[16], double (&y)[16], double* __restrict__ L, int cw,
+                                               int lane, Step&& step)
 {
-    for (int it = 0; it < LDS_SPIN; ++it) {
-        const int v = __hip_atomic_load(cnt, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (v >= need) return v;
-        __builtin_amdgcn_s_sleep(1);
+    double piv = readlane_f64(p[0], cw);
+    double lprev = 0.0, yprev = 0.0, far[2][16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        const int c = cw + t;
+        double (&fp)[16] = far[(t + 1) & 1], (&fn)[16] = far[t & 1];
+        auto fill = [&](int u0, int u1) {
+#pragma unroll
+            for (int u = u0; u < u1; ++u)
+                if (t > 0 && u < 16) {
+                    p[u] = __builtin_fma(-lprev, fp[u], p[u]);
+                    if (FIRST) {
+                        y[u] = __builtin_fma(-yprev, fp[u], y[u]);
+                        // keeps the step here: left alone, all of y sinks behind the pivots
+                        asm volatile("" : "+v"(y[u]));
+                    }
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        const double q = __builtin_amdgcn_rsq(piv);
+        double a1 = 0.0, a2 = 0.0;
+        if (t < 15) a1 = readlane_f64(p[t], c + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const double m = piv * q;
+        step(t);
+        __builtin_amdgcn_sched_barrier(0);
+        const double e = __builtin_fma(-m, q, 1.0);
+        fill(t + 1, t + 3);
+        const double k = __builtin_fma(e, 0.375, 0.5), qe = q * e;
+        if (t < 15) a2 = readlane_f64(p[t + 1], c + 1);
+        fill(t + 3, t + 5);
+        const double rs = __builtin_fma(k, qe, q);
+        fill(t + 5, t + 7);
+        const double s1 = a1 * rs;   // l_{c+1, c}
+        const double l = p[t] * rs;
+        fill(t + 7, t + 9);
+        piv = __builtin_fma(-s1, s1, a2);
+        L[c * CHOL_NB + lane] = l;
+        // l_{cw+u, c}: LDS broadcasts of the column this wavefront has just stored (its own
+        // store, in order before these loads)
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = t + 2; u < 16; ++u) fn[u] = L[c * CHOL_NB + cw + u];
+        p[t] = l;
+        if (FIRST) y[t] *= rs;
+        if (t < 15) {
+            p[t + 1] = __builtin_fma(-l, s1, p[t + 1]);
+            if (FIRST) y[t + 1] = __builtin_fma(-y[t], s1, y[t + 1]);
+        }
+        fill(t + 9, 16);
+        lprev = l;
+        if (FIRST) yprev = y[t];
     }
-    return -1;
 }
 
 // In-place FP64 Cholesky of the 64x64 block held in LDS, called by all 256 threads.
 //   in : sD[r * DG_LD + c], lower part (r >= c) read
-//   out: the same memory as L[c * 64 + r] (column-major, pitch 64, zeros above the diagonal),
-//        the inverses of its four 16x16 diagonal sub-blocks after it (sD + 4096 + 256 J, the
-//        layout load_lkk leaves: sD is then sLT / sInv of the solve), and the same in Lb.
-//        sD must hold CHOL_NB * CHOL_NB + 4 * 256 doubles.
-// The four wavefronts form a pipeline over column groups: wavefront w owns columns
-// 16w .. 16w+15 (lane = row, one register per column).  It applies the rank-1 updates of the
-// 16w earlier columns as the wavefronts before it publish them (column in LDS, then an LDS
-// counter), then factors its own 16 columns one by one, publishing each.  So the pivot chain
-// runs through the wavefronts back to back and every update off it runs beside it.
-// Within a wavefront's own columns, pivot t+1 = a_{t+1,t+1} - (a_{t+1,t} / sqrt(d_t))^2 is
-// formed from two broadcasts (v_readlane) of the pre-update entries, issued before the
-// pivot's reciprocal square root is known; the rank-1 update of the later own columns reads
-// the scaled column back from LDS as broadcasts, and the same entries build the inverse of
-// the own 16x16 sub-block step by step, so it is complete with the last own column.
+//   out: the same memory in the layout of Lb (L[c * 64 + r], then the inverses of its four
+//        16x16 diagonal sub-blocks: sD is then sLT / sInv of the solve), and the same in Lb.
+//        sD must hold LB_STRIDE doubles.
+// Wavefront 0 factors the block alone, so no step of the chain waits for another wavefront; the
+// other three are free for work of the caller's (others(), called by each of them) until the
+// barrier at the end.  The block is taken in four groups of 16 columns: the group's columns on
+// the VALU (factor_group16), its update of the columns beyond on v_mfma_f64_16x16x4_f64.  The
+// trailing 16x16 tiles stay in MFMA accumulators from the start, transposed (accumulator r of
+// lane l: column 4 r + l/16 of the tile, row l%16), so the next group's tiles reach the
+// lane = row form with one conflict-free pass through the LDS columns they will be factored in.
+// What bounds it: the chain of 64 pivots, each about 80 cycles of dependent FP64 operations.
+// 64x64 block on an idle GPU: 11.2 us as a pipeline of the four wavefronts over the column
+// groups, 8.2 us as here.
 // A non-positive (or NaN) pivot records row c0 + j + 1 in *status (the first one wins) and the
 // factorization continues with NaN, as the reference's dpotrf reports INFO.
-// head(), tail(): work of the caller's for the wavefronts' idle stretches (wavefront w's own
-// columns begin only after the 16 w columns before them, and wavefront 0 waits from its last
-// column to the end): each wavefront runs head() once after its block entries are in
-// registers, before it takes the earlier columns, and tail() once after its own columns.
-template <typename Head, typename Tail>
+template <typename Others>
 __device__ __forceinline__ void factor_diag64(double* __restrict__ sD, int c0, int* __restrict__ status,
-                                              double* __restrict__ Lb, Head&& head, Tail&& tail)
+                                              Others&& others)
 {
-    __shared__ int s_done;   // columns published so far
-    __shared__ int s_bad;    // first non-positive pivot (64: none); -1: a wait timed out
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int cw = 16 * w;   // first own column
-    __syncthreads();   // the block in sD may have been written by one wavefront alone
-    double p[16];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __syncthreads();   // the block in sD may have been written by another wavefront
+    if (w == 0) {
+        const int lr = lane & 15, lq = lane >> 4;
+        double p[16], y[16];
+        doublex4 T[3][3];   // tile (i + 1, j + 1), j <= i, transposed
 #pragma unroll
-    for (int u = 0; u < 16; ++u) p[u] = (lane >= cw + u) ? sD[lane * DG_LD + cw + u] : 0.0;
-    if (tid == 0) {
-        s_done = 0;
-        s_bad = CHOL_NB;
-    }
-    __syncthreads();   // every block entry is in registers: sD is reused for L
-    head();
-    double* L = sD;
-    bool ok = true;
-    // updates by the earlier column groups, two columns at a time as they are published
-    // (cw is a multiple of 16, so a pair never straddles two groups)
-    int avail = 0;
-    for (int c = 0; c < cw; c += 2) {
-        if (avail < c + 2) {
-            avail = wait_lds_count(&s_done, c + 2);
-            if (avail < 0) {
-                ok = false;
-                break;
-            }
+        for (int u = 0; u < 16; ++u) {
+            p[u] = sD[lane * DG_LD + u];
+            y[u] = (u == lane) ? 1.0 : 0.0;
         }
-        // every LDS read of the pair is issued before its first use
-        const double x0 = L[c * CHOL_NB + lane], x1 = L[(c + 1) * CHOL_NB + lane];
-        const double2* b0 = reinterpret_cast<const double2*>(L + c * CHOL_NB + cw);
-        const double2* b1 = reinterpret_cast<const double2*>(L + (c + 1) * CHOL_NB + cw);
-        double2 v0[8], v1[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            v0[u] = b0[u];
-            v1[u] = b1[u];
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            p[2 * u] = __builtin_fma(-x1, v1[u].x, __builtin_fma(-x0, v0[u].x, p[2 * u]));
-            p[2 * u + 1] = __builtin_fma(-x1, v1[u].y, __builtin_fma(-x0, v0[u].y, p[2 * u + 1]));
-        }
-    }
-    int bad = CHOL_NB;
-    if (ok) {
-        // inverse of the own 16x16 diagonal sub-block, built beside the factorization: lane
-        // q < 16 solves L_ww y = e_q right-looking, step t taking column t's 1 / l_tt and the
-        // entries l_{cw+u, cw+t} the column update broadcasts anyway
-        double y[16];
+            for (int j = 0; j <= i; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) y[r] = (r == lane) ? 1.0 : 0.0;
-        double piv = readlane_f64(p[0], cw);
+                for (int r = 0; r < 4; ++r) T[i][j][r] = sD[(16 * i + 16 + lr) * DG_LD + 16 * j + 16 + 4 * r + lq];
+        __builtin_amdgcn_wave_barrier();   // the block is in registers: its memory is reused for L
+        double* L = sD;
+        double* sInv = sD + CHOL_NB * CHOL_NB;
+        double x[3][4];   // the last group's rows below, as MFMA operands
+        // the group's update of tile (i + 1, j + 1), its k-step s4
+        auto update = [&](int i, int j, int s4) { T[i][j] = mfma_f64_16x16x4(-x[j][s4], x[i][s4], T[i][j]); };
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            const int c = cw + t;
-            if (!(piv > 0.0) && bad == CHOL_NB) bad = c;
-            // the next pivot a_{c+1,c+1} - l_{c+1,c}^2 from the entries before this column's
-            // update (two broadcasts issued before the reciprocal square root is known)
-            double a1 = 0.0, a2 = 0.0;
-            if (t < 15) {
-                a1 = readlane_f64(p[t], c + 1);
-                a2 = readlane_f64(p[t + 1], c + 1);
+        for (int g = 0; g < 4; ++g) {
+            const int cw = 16 * g;
+            if (g == 0) {
+                factor_group16<true>(p, y, L, 0, lane, [](int) {});
+            } else {
+                // the previous group's update of the tiles beyond this one, a step per column
+                factor_group16<false>(p, y, L, cw, lane, [&](int t) {
+                    const int s4 = t & 3, q = t >> 2;
+                    if (g == 1 && q < 3) update(q == 0 ? 1 : 2, q == 2 ? 2 : 1, s4);
+                    if (g == 2 && q < 1) update(2, 2, s4);
+                });
             }
-            const double rs = rsqrt_f64(piv);
-            double nxt = 0.0;
-            if (t < 15) {
-                const double le = a1 * rs;   // l_{c+1, c}
-                nxt = __builtin_fma(-le, le, a2);
+            if (lane < 16) {
+#pragma unroll
+                for (int u = 0; u < 16; ++u) sInv[SINV * g + lane * SINV_P + u] = g == 0 ? y[u] : p[u];
             }
-            const double lp = p[t] * rs, ld = piv * rs;
-            double l = (lane == c) ? ld : lp;
-            l = (lane < c) ? 0.0 : l;
-            p[t] = l;
-            L[c * CHOL_NB + lane] = l;
-            y[t] *= rs;
-            if (t < 15) {
-                // l_{cw+u, c} of the later own columns: LDS broadcasts of the column this
-                // wavefront has just stored (its own stores, in order before these loads)
+            if (g < 3) {
+                // this group's update of the next group's tiles
+                const int cn = cw + 16;
+#pragma unroll
+                for (int i = g; i < 3; ++i)
+#pragma unroll
+                    for (int s4 = 0; s4 < 4; ++s4) x[i][s4] = L[(cw + 4 * s4 + lq) * CHOL_NB + 16 * i + 16 + lr];
+#pragma unroll
+                for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+                    for (int i = g; i < 3; ++i) update(i, g, s4);
+                // into the lane = row form through the LDS columns they will be factored in
+#pragma unroll
+                for (int i = g; i < 3; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) L[(cn + 4 * r + lq) * CHOL_NB + 16 * i + 16 + lr] = T[i][g][r];
                 __builtin_amdgcn_wave_barrier();
-                double lc[16];
+                // rows from the group's diagonal down; the identity in lanes 0 .. 15
 #pragma unroll
-                for (int u = t + 1; u < 16; ++u) lc[u] = L[c * CHOL_NB + cw + u];
-#pragma unroll
-                for (int u = t + 1; u < 16; ++u) p[u] = __builtin_fma(-l, lc[u], p[u]);
-#pragma unroll
-                for (int u = t + 1; u < 16; ++u) {
-                    y[u] = __builtin_fma(-lc[u], y[t], y[u]);
-                    // keeps the step here: left to the scheduler, the steps sink to the stores
-                    // at the end and every broadcast stays live until then
-                    asm volatile("" : "+v"(y[u]));
+                for (int u = 0; u < 16; ++u) {
+                    double v = L[(cn + u) * CHOL_NB + lane];
+                    asm volatile("" : "+v"(v));   // a select, not a branch around the load
+                    p[u] = (lane >= cn) ? v : (lane == u ? 1.0 : 0.0);
                 }
             }
-            // columns are published in pairs (the consumers take them in pairs)
-            if (t & 1) __hip_atomic_store(&s_done, c + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            piv = nxt;
         }
-        // own columns into Lb (zeros above the diagonal)
-#pragma unroll
-        for (int u = 0; u < 16; ++u) Lb[(cw + u) * CHOL_NB + lane] = (lane >= cw + u) ? p[u] : 0.0;
-        if (lane < 16) {
-            double* inv = Lb + CHOL_NB * CHOL_NB + 256 * w;
-            double* sinv = sD + CHOL_NB * CHOL_NB + 256 * w;   // the solve's sInv layout
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                inv[lane * 16 + r] = y[r];
-                sinv[lane * 16 + r] = y[r];
-            }
-        }
+        // a pivot that is not positive leaves NaN on the diagonal from its column on
+        const unsigned long long bad = __ballot(!(L[lane * CHOL_NB + lane] > 0.0));
+        if (bad && lane == 0) atomicCAS(status, 0, c0 + __builtin_ctzll(bad) + 1);
+    } else {
+        others();
     }
-    tail();
-    if (lane == 0) {
-        if (!ok) atomicExch(&s_bad, -1);
-        else if (bad < CHOL_NB) atomicMin(&s_bad, bad);
-    }
-    __syncthreads();   // L complete in LDS, every wavefront's Lb stores issued
-    if (tid == 0) {
-        if (s_bad < 0) atomicCAS(status, 0, -1);
-        else if (s_bad < CHOL_NB) atomicCAS(status, 0, c0 + s_bad + 1);
-    }
+    __syncthreads();   // L and the inverses complete in LDS
 }
 
-__device__ __forceinline__ void factor_diag64(double* __restrict__ sD, int c0, int* __restrict__ status,
-                                              double* __restrict__ Lb)
+__device__ __forceinline__ void factor_diag64(double* __restrict__ sD, int c0, int* __restrict__ status)
 {
-    factor_diag64(sD, c0, status, Lb, [] {}, [] {});
+    factor_diag64(sD, c0, status, [] {});
+}
+
+// Agent-scope store: written through to memory, so it is visible to every workgroup once it has
+// completed.
+__device__ __forceinline__ void st_agent(double* p, double v)
+{
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, v),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(float* p, float v)
+{
+    __hip_atomic_store(reinterpret_cast<unsigned*>(p), __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The factored block and its inverses from the LDS into Lb (the same layout), at agent scope.
+__device__ __forceinline__ void store_lkk(const double* __restrict__ sD, double* __restrict__ Lb)
+{
+    constexpr int NL = LB_STRIDE / 256;
+    double v[NL + 1];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) v[i] = sD[threadIdx.x + 256 * i];
+    if (threadIdx.x < LB_STRIDE % 256) v[NL] = sD[threadIdx.x + 256 * NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) st_agent(Lb + threadIdx.x + 256 * i, v[i]);
+    if (threadIdx.x < LB_STRIDE % 256) st_agent(Lb + threadIdx.x + 256 * NL, v[NL]);
 }
 
 // L (lower part) of the factored block, L[c * 64 + r] in LDS, into A, in T.
@@ -237,354 +263,25 @@ __device__ __forceinline__ void store_diag64(const double* __restrict__ L, T* __
     }
 }
 
-// Panel 0's diagonal block (later ones are factored inside the SYRK kernel).
-template <typename T>
-__device__ __forceinline__ void chol_diag_body(T* __restrict__ A, long long ld, int c0,
-                                               double* __restrict__ Lb, int* __restrict__ flags,
-                                               int nflags, int* __restrict__ status)
+// L_kk and its diagonal sub-block inverses (Lb, FP64) into LDS at sLT, in Lb's own layout.
+__device__ __forceinline__ void load_lkk(const double* __restrict__ Lb, double* __restrict__ sLT)
 {
-    __shared__ double sD[CHOL_NB * CHOL_NB + 4 * 256];
-    static_assert(CHOL_NB * CHOL_NB + 4 * 256 >= CHOL_NB * DG_LD, "diagonal block LDS");
-    for (int k = threadIdx.x; k < nflags; k += 256) flags[k] = 0;
-    double v[CHOL_NB * CHOL_NB / 256];
+    // all loads are issued before the LDS stores (which the compiler would otherwise order
+    // between them)
+    constexpr int NL = LB_STRIDE / 256;
+    double v[NL + 1];
 #pragma unroll
-    for (int i = 0; i < CHOL_NB * CHOL_NB / 256; ++i) {
-        const int e = threadIdx.x + 256 * i, r = e % CHOL_NB, c = e / CHOL_NB;
-        v[i] = (r >= c) ? (double)A[(long long)(c0 + c) * ld + c0 + r] : 0.0;
-    }
-#pragma unroll
-    for (int i = 0; i < CHOL_NB * CHOL_NB / 256; ++i) {
-        const int e = threadIdx.x + 256 * i, r = e % CHOL_NB, c = e / CHOL_NB;
-        sD[r * DG_LD + c] = v[i];
-    }
-    factor_diag64(sD, c0, status, Lb);   // begins with a barrier
-    store_diag64<T>(sD, A, ld, c0);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256)
-chol_diag_kernel(T* __restrict__ A, long long ld, int c0, double* __restrict__ Lb,
-                 int* __restrict__ flags, int nflags, int* __restrict__ status)
-{
-    chol_diag_body<T>(A, ld, c0, Lb, flags, nflags, status);
-}
-
-// Broadcast within each quad of lanes from quad lane Q (DPP quad_perm).
-template <int Q>
-__device__ __forceinline__ double quad_bcast_t(double v)
-{
-    constexpr int ctrl = Q | (Q << 2) | (Q << 4) | (Q << 6);
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)u, ctrl, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), ctrl, 0xF, 0xF, false);
-    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double quad_bcast(double v, int q)
-{
-    switch (q) {
-        case 0: return quad_bcast_t<0>(v);
-        case 1: return quad_bcast_t<1>(v);
-        case 2: return quad_bcast_t<2>(v);
-        default: return quad_bcast_t<3>(v);
-    }
-}
-
-// TRSM x L_kk^T = b for 16 rows (one wavefront), blocked by the four 16-column sub-blocks J
-// of the panel, on v_mfma_f64_16x16x4_f64:
-//   Y_J = B_J - sum_{K<J} X_K L_JK^T,   X_J = Y_J Linv_JJ^T
-// Y and X live in the MFMA result layout (accumulator r of lane l = row 4 r + l/16, column
-// l%16 of the 16x16 block); a finished block goes through LDS (pitch 17) to become an A
-// operand (lane l: row l%16, k = 4 s + l/16).  sLT[k * 64 + c] = L_kk[c][k];
-// sInv[256 J + c' * 16 + c] = Linv_JJ[c][c'].  All FP64.
-constexpr int SC_PITCH = 17;
-
-struct Trsm16 {
-    doublex4 y[4];   // B_J in, X_J out, result layout
-};
-
-template <typename T>
-__device__ __forceinline__ void trsm16_load(const T* __restrict__ A, long long ld, int t0, int g0,
-                                            int re, int lane, Trsm16& g)
-{
-    const int lr = lane & 15, lq = lane >> 4;
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-        const T* col = A + (long long)(t0 + 16 * J + lr) * ld;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = g0 + 4 * r + lq;
-            g.y[J][r] = (row < re) ? (double)col[row] : 0.0;
-        }
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void trsm16_solve_store(T* __restrict__ A, long long ld, int t0, int g0,
-                                                   int re, int lane, Trsm16& g,
-                                                   const double* __restrict__ sLT,
-                                                   const double* __restrict__ sInv,
-                                                   double* __restrict__ sc)
-{
-    const int lr = lane & 15, lq = lane >> 4;
-    double xa[4][4];   // A-operand form of the finished X_K: xa[K][s] = X_K[lr][4 s + lq]
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-        doublex4 yj = g.y[J];
-#pragma unroll
-        for (int K = 0; K < J; ++K)
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) {
-                const double b = sLT[(16 * K + 4 * s4 + lq) * CHOL_NB + 16 * J + lr];
-                yj = mfma_f64_16x16x4(-xa[K][s4], b, yj);
-            }
-        // Y_J into A-operand form
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sc[(4 * r + lq) * SC_PITCH + lr] = yj[r];
-        __builtin_amdgcn_wave_barrier();
-        double ya[4];
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) ya[s4] = sc[lr * SC_PITCH + 4 * s4 + lq];
-        __builtin_amdgcn_wave_barrier();
-        doublex4 xj = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4)
-            xj = mfma_f64_16x16x4(ya[s4], sInv[256 * J + (4 * s4 + lq) * 16 + lr], xj);
-        T* col = A + (long long)(t0 + 16 * J + lr) * ld;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = g0 + 4 * r + lq;
-            if (row < re) col[row] = (T)xj[r];
-        }
-        if (J < 3) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sc[(4 * r + lq) * SC_PITCH + lr] = xj[r];
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) xa[J][s4] = sc[lr * SC_PITCH + 4 * s4 + lq];
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-}
-
-// Two 16-row groups a and b of one wavefront solved together: the same L operands, two
-// independent MFMA chains interleaved (each hides the other's latency).  Rows of b at or
-// beyond re are neither loaded nor stored.
-template <typename T>
-__device__ __forceinline__ void trsm16x2_solve_store(T* __restrict__ A, long long ld, int t0, int ga0,
-                                                     int gb0, int re, int lane, Trsm16& ga, Trsm16& gb,
-                                                     const double* __restrict__ sLT,
-                                                     const double* __restrict__ sInv,
-                                                     double* __restrict__ sc)
-{
-    const int lr = lane & 15, lq = lane >> 4;
-    double xa[4][4], xb[4][4];
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-        doublex4 ya = ga.y[J], yb = gb.y[J];
-#pragma unroll
-        for (int K = 0; K < J; ++K)
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) {
-                const double b = sLT[(16 * K + 4 * s4 + lq) * CHOL_NB + 16 * J + lr];
-                ya = mfma_f64_16x16x4(-xa[K][s4], b, ya);
-                yb = mfma_f64_16x16x4(-xb[K][s4], b, yb);
-            }
-        double yaa[4], yba[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sc[(4 * r + lq) * SC_PITCH + lr] = ya[r];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) yaa[s4] = sc[lr * SC_PITCH + 4 * s4 + lq];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sc[(4 * r + lq) * SC_PITCH + lr] = yb[r];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) yba[s4] = sc[lr * SC_PITCH + 4 * s4 + lq];
-        __builtin_amdgcn_wave_barrier();
-        doublex4 xja = {0.0, 0.0, 0.0, 0.0}, xjb = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-            const double iv = sInv[256 * J + (4 * s4 + lq) * 16 + lr];
-            xja = mfma_f64_16x16x4(yaa[s4], iv, xja);
-            xjb = mfma_f64_16x16x4(yba[s4], iv, xjb);
-        }
-        T* col = A + (long long)(t0 + 16 * J + lr) * ld;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int rowa = ga0 + 4 * r + lq, rowb = gb0 + 4 * r + lq;
-            if (rowa < re) col[rowa] = (T)xja[r];
-            if (rowb < re) col[rowb] = (T)xjb[r];
-        }
-        if (J < 3) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sc[(4 * r + lq) * SC_PITCH + lr] = xja[r];
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) xa[J][s4] = sc[lr * SC_PITCH + 4 * s4 + lq];
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sc[(4 * r + lq) * SC_PITCH + lr] = xjb[r];
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) xb[J][s4] = sc[lr * SC_PITCH + 4 * s4 + lq];
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-}
-
-// L_kk and its diagonal sub-block inverses (Lb, FP64) into LDS.
-__device__ __forceinline__ void load_lkk(const double* __restrict__ Lb, double* __restrict__ sLT,
-                                         double* __restrict__ sInv)
-{
-    // Lb is column-major (Lb[k * CHOL_NB + c] = L_kk[c][k]), which is the sLT layout.  All
-    // loads are issued before the LDS stores (which the compiler would otherwise order
-    // between them).
-    constexpr int NL = CHOL_NB * CHOL_NB / 256, NI = 4;
-    double v[NL + NI];
-#pragma unroll
-    for (int i = 0; i < NL + NI; ++i) v[i] = Lb[threadIdx.x + 256 * i];
+    for (int i = 0; i < NL; ++i) v[i] = Lb[threadIdx.x + 256 * i];
+    if (threadIdx.x < LB_STRIDE % 256) v[NL] = Lb[threadIdx.x + 256 * NL];
 #pragma unroll
     for (int i = 0; i < NL; ++i) sLT[threadIdx.x + 256 * i] = v[i];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) sInv[threadIdx.x + 256 * i] = v[NL + i];
+    if (threadIdx.x < LB_STRIDE % 256) sLT[threadIdx.x + 256 * NL] = v[NL];
     __syncthreads();
 }
 
-// LDS of a TRSM workgroup: sLT, sInv, and 16 x SC_PITCH doubles per wavefront.
-constexpr int TRSM_LDS_DOUBLES = CHOL_NB * CHOL_NB + 4 * 256 + 4 * 16 * SC_PITCH;
-
-// Panel c0's TRSM as its own launch (panel 0 only; the others run inside the SYRK kernel):
-// 64 rows per workgroup, 16 per wavefront.
-template <typename T>
-__device__ __forceinline__ void chol_trsm_body(T* __restrict__ A, long long ld, int c0, int n_pad,
-                                               const double* __restrict__ Lb, int bid)
-{
-    __shared__ double smem[TRSM_LDS_DOUBLES];
-    double* sLT = smem;
-    double* sInv = sLT + CHOL_NB * CHOL_NB;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    double* sc = sInv + 4 * 256 + wave * 16 * SC_PITCH;
-    const int g0 = c0 + CHOL_NB + bid * TRSM_ROWS + 16 * wave;
-    Trsm16 g;
-    trsm16_load<T>(A, ld, c0, g0, n_pad, lane, g);
-    load_lkk(Lb, sLT, sInv);
-    if (g0 < n_pad) trsm16_solve_store<T>(A, ld, c0, g0, n_pad, lane, g, sLT, sInv, sc);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256)
-chol_trsm_kernel(T* __restrict__ A, long long ld, int c0, int n_pad, const double* __restrict__ Lb)
-{
-    chol_trsm_body<T>(A, ld, c0, n_pad, Lb, blockIdx.x);
-}
-
-// Flags of the diagonal blocks, after the FP64 blocks in the workspace: flag k is set once
-// block k's factor is in Lb (cleared by the panel-0 diagonal kernel of each factorization).
-__device__ __forceinline__ int* chol_flags(double* Lbuf, int n_pad)
-{
-    return reinterpret_cast<int*>(Lbuf + (long long)(n_pad / CHOL_NB) * LB_STRIDE);
-}
-
-// Bounded wait (about a second) for a flag set by another workgroup of the same grid.  The
-// polls are relaxed; one agent-scope acquire follows the flag (an acquiring poll would
-// invalidate this XCD's L2 at every iteration, under the feet of the other workgroups).
-constexpr int CHOL_SPIN = 1 << 20;
-// SLEEP: s_sleep units (64 cycles each) between polls; the bound on the polls scales with it.
-template <int SLEEP = 2>
-__device__ __forceinline__ bool wait_flag(int* flag)
-{
-    for (int it = 0; it < CHOL_SPIN * 2 / SLEEP; ++it) {
-        if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            return true;
-        }
-        __builtin_amdgcn_s_sleep(SLEEP);
-    }
-    return false;
-}
-
-// Tail of the SYRK kernels (tile column 0): the next panel's diagonal block was factored by
-// workgroup 0 (diag); every tile of column 0 then solves its own rows of that panel, 16 rows
-// per wavefront at a time.  The rows are loaded before the wait (this workgroup wrote
-// them), so the wait hides the loads.
-template <typename T>
-__device__ __forceinline__ void fused_trsm(T* __restrict__ A, long long ld, int t0, int ri0, int n_pad,
-                                           double* __restrict__ Lb_next, int* __restrict__ flag,
-                                           int* __restrict__ status, bool diag, unsigned char* smem,
-                                           const double* __restrict__ sD)
-{
-    double* sLT = reinterpret_cast<double*>(smem);
-    double* sInv = sLT + CHOL_NB * CHOL_NB;
-    __shared__ int s_ok;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double* sc = sInv + 4 * 256 + wave * 16 * SC_PITCH;
-    const int rb = max(ri0, t0 + CHOL_NB), re = min(n_pad, ri0 + SY_TILE_C);
-    const int g0 = rb + 16 * wave, g1 = g0 + 64;   // this wavefront's two 16-row groups
-    if (diag) {
-        // the FP64 block is in Lb (factor_diag64); the T copy in A is not read by this kernel
-        // each wavefront's Lb stores written back (release only: no L2 invalidation), then
-        // the flag
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __syncthreads();
-        if (tid == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        store_diag64<T>(sD, A, ld, t0);
-    }
-    // this workgroup's own C stores are read back below: workgroup scope suffices (no L2
-    // write-back / invalidation, which an agent-scope fence would cost every such workgroup)
-    __syncthreads();
-    Trsm16 x0, x1;
-    if (g0 < re) trsm16_load<T>(A, ld, t0, g0, re, lane, x0);
-    if (g1 < re) trsm16_load<T>(A, ld, t0, g1, re, lane, x1);
-    else x1 = Trsm16{};
-    if (tid == 0) {
-        if (diag) {
-            s_ok = 1;
-        } else {
-            s_ok = wait_flag(flag) ? 1 : 0;
-            if (!s_ok) atomicCAS(status, 0, -1);
-        }
-    }
-    __syncthreads();
-    if (!s_ok) return;
-    load_lkk(Lb_next, sLT, sInv);
-    if (g1 < re) trsm16x2_solve_store<T>(A, ld, t0, g0, g1, re, lane, x0, x1, sLT, sInv, sc);
-    else if (g0 < re) trsm16_solve_store<T>(A, ld, t0, g0, re, lane, x0, sLT, sInv, sc);
-}
-
-// Tile (ti, tj), ti >= tj, of a lower trapezoid with ni tile rows, enumerated column by
-// column (tile (0, 0) first).
-__device__ __forceinline__ void trap_tile(int x, int ni, int& ti, int& tj)
-{
-    int j = 0;
-    while (x >= ni - j) {
-        x -= ni - j;
-        ++j;
-    }
-    ti = j + x;
-    tj = j;
-}
-
-// ------------------------------------------------------------------ FP32 SYRK (MFMA)
-// Workgroup 256 = 4 waves in 2x2; tile 128x128; each wave 64x64 = 2x2 blocks of 32x32.
-//   SPLIT = false: v_mfma_f32_32x32x2_f32 on the FP32 operands.
-//   SPLIT = true : each FP32 operand x = hi + lo with hi = bf16(x), lo = bf16(x - hi)
-//                  (x - hi is exact in FP32), and a b = hi_a hi_b + hi_a lo_b + lo_a hi_b
-//                  on v_mfma_f32_32x32x16_bf16 with FP32 accumulation; the dropped lo_a lo_b
-//                  and the split residuals are below 2^-17 |a b|.
-constexpr int SY_TILE = SY_TILE_C;
-__device__ __forceinline__ int ceil_div_dev(int a, int b) { return (a + b - 1) / b; }
-constexpr int SY_KC32 = 32;
-constexpr int SY_KCH = 32;                 // k per stage of the split kernel
+// ------------------------------------------------------------------ MFMA pieces
+constexpr int SY_KCH = 32;                 // k per stage of the split products
 constexpr int SY_HP = SY_KCH / 2 + 4;      // row pitch of a split stage, in 32-bit words
-
-// LDS of the SYRK kernels: the operand stages, reused for the next diagonal block.
-constexpr int SY_SMEM_F32 = 2 * SY_KC32 * (SY_TILE + 4) * 4;
-constexpr int SY_SMEM_SPLIT = 4 * SY_TILE * SY_HP * 4;
-constexpr int SY_SMEM_MAX2 = SY_SMEM_SPLIT > SY_SMEM_F32 ? SY_SMEM_SPLIT : SY_SMEM_F32;
-constexpr int SY_SMEM = SY_SMEM_MAX2 > TRSM_LDS_DOUBLES * 8 ? SY_SMEM_MAX2 : TRSM_LDS_DOUBLES * 8;
-static_assert(SY_SMEM >= CHOL_NB * DG_LD * 8, "diagonal block does not fit the SYRK LDS");
-static_assert(SY_SMEM >= TRSM_LDS_DOUBLES * 8, "TRSM operands do not fit the SYRK LDS");
 
 // bf16 bits of x, round to nearest even (finite inputs)
 __device__ __forceinline__ unsigned bf16_bits(float x)
@@ -596,561 +293,6 @@ __device__ __forceinline__ void split_bf16(float x, unsigned& hi, unsigned& lo)
 {
     hi = bf16_bits(x);
     lo = bf16_bits(x - __builtin_bit_cast(float, hi << 16));
-}
-
-// acc += A[ri0 .. ri0+127, kb .. kb+K) A[rj0 .. rj0+127, kb .. kb+K)^T for one 128x128 tile on
-// MFMA (rows at or beyond n_pad read as zero).  Workgroup 256 = 4 waves in 2x2, each 64x64 =
-// 2x2 blocks of 32x32; acc[a][b] is the 32x32 block (a, b) of the wave in the MFMA result
-// layout.  The operand stages use smem (SY_SMEM bytes).
-template <bool SPLIT>
-__device__ __forceinline__ void tile_acc_f32(const float* __restrict__ A, long long ld, int kb, int K, int ri0,
-                                             int rj0, int n_pad, unsigned char* smem, floatx16 (&acc)[2][2])
-{
-    float (*sA)[SY_TILE + 4] = reinterpret_cast<float (*)[SY_TILE + 4]>(smem);
-    float (*sB)[SY_TILE + 4] = reinterpret_cast<float (*)[SY_TILE + 4]>(smem + SY_KC32 * (SY_TILE + 4) * 4);
-    // split stages: [0] A hi, [1] A lo, [2] B hi, [3] B lo; row-major (row, k pairs)
-    unsigned (*sH)[SY_TILE][SY_HP] = reinterpret_cast<unsigned (*)[SY_TILE][SY_HP]>(smem);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const int l32 = lane & 31, lh = lane >> 5;
-    if constexpr (SPLIT) {
-        // staging: thread t loads row t of the A rows (t < 128) or of the B rows, SY_KCH
-        // consecutive k (one coalesced load per k across the wave), splits, and writes
-        // k-contiguous hi / lo words
-        const bool isB = tid >= SY_TILE;
-        const int srow = isB ? rj0 + tid - SY_TILE : ri0 + tid;
-        const int lrow = tid & (SY_TILE - 1);
-        const bool live = srow < n_pad;
-        // the next chunk's loads are issued before this chunk's MFMAs (register double
-        // buffering: v is converted into LDS before it is refilled)
-        float v[SY_KCH];
-        {
-            const float* src = A + (long long)kb * ld + srow;
-#pragma unroll
-            for (int k = 0; k < SY_KCH; ++k) v[k] = live ? src[(long long)k * ld] : 0.f;
-        }
-        for (int k0 = 0; k0 < K; k0 += SY_KCH) {
-            __syncthreads();
-#pragma unroll
-            for (int k = 0; k < SY_KCH; k += 8) {
-                unsigned h[8], l[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) split_bf16(v[k + u], h[u], l[u]);
-                const uint4 hw = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16),
-                                            h[4] | (h[5] << 16), h[6] | (h[7] << 16));
-                const uint4 lw = make_uint4(l[0] | (l[1] << 16), l[2] | (l[3] << 16),
-                                            l[4] | (l[5] << 16), l[6] | (l[7] << 16));
-                *reinterpret_cast<uint4*>(&sH[isB ? 2 : 0][lrow][k / 2]) = hw;
-                *reinterpret_cast<uint4*>(&sH[isB ? 3 : 1][lrow][k / 2]) = lw;
-            }
-            __syncthreads();
-            if (k0 + SY_KCH < K) {
-                const float* src = A + (long long)(kb + k0 + SY_KCH) * ld + srow;
-#pragma unroll
-                for (int k = 0; k < SY_KCH; ++k) v[k] = live ? src[(long long)k * ld] : 0.f;
-            }
-#pragma unroll
-            for (int t = 0; t < SY_KCH / 16; ++t) {
-                const int w = 8 * t + 4 * lh;   // lane holds k = 16 t + 8 lh + 0..7
-                bf16x8 ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-                for (int a = 0; a < 2; ++a) {
-                    const int r = wr * 64 + a * 32 + l32;
-                    ah[a] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&sH[0][r][w]));
-                    al[a] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&sH[1][r][w]));
-                }
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    const int r = wc * 64 + b * 32 + l32;
-                    bh[b] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&sH[2][r][w]));
-                    bl[b] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&sH[3][r][w]));
-                }
-#pragma unroll
-                for (int a = 0; a < 2; ++a)
-#pragma unroll
-                    for (int b = 0; b < 2; ++b) {
-                        acc[a][b] = mfma_bf16_32x32x16(al[a], bh[b], acc[a][b]);
-                        acc[a][b] = mfma_bf16_32x32x16(ah[a], bl[b], acc[a][b]);
-                        acc[a][b] = mfma_bf16_32x32x16(ah[a], bh[b], acc[a][b]);
-                    }
-            }
-        }
-    } else {
-        // register double buffering: the next chunk's global loads are issued before this
-        // chunk's MFMAs (each thread: 4 float4 of the A rows and 4 of the B rows per chunk)
-        constexpr int NV = SY_KC32 * SY_TILE / 4 / 256;
-        float4 va[NV], vb[NV];
-        auto load_chunk = [&](int k0) {
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int idx = tid + 256 * i;
-                const int k = idx / (SY_TILE / 4);
-                const int r4 = (idx % (SY_TILE / 4)) * 4;
-                const float* col = A + (long long)(kb + k0 + k) * ld;
-                va[i] = (ri0 + r4 < n_pad) ? *reinterpret_cast<const float4*>(col + ri0 + r4) : make_float4(0.f, 0.f, 0.f, 0.f);
-                vb[i] = (rj0 + r4 < n_pad) ? *reinterpret_cast<const float4*>(col + rj0 + r4) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-        };
-        load_chunk(0);
-        for (int k0 = 0; k0 < K; k0 += SY_KC32) {
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int idx = tid + 256 * i;
-                const int k = idx / (SY_TILE / 4);
-                const int r4 = (idx % (SY_TILE / 4)) * 4;
-                *reinterpret_cast<float4*>(&sA[k][r4]) = va[i];
-                *reinterpret_cast<float4*>(&sB[k][r4]) = vb[i];
-            }
-            __syncthreads();
-            if (k0 + SY_KC32 < K) load_chunk(k0 + SY_KC32);
-#pragma unroll 4
-            for (int k = 0; k < SY_KC32; k += 2) {
-                float av[2], bv[2];
-#pragma unroll
-                for (int a = 0; a < 2; ++a) av[a] = sA[k + lh][wr * 64 + a * 32 + l32];
-#pragma unroll
-                for (int b = 0; b < 2; ++b) bv[b] = sB[k + lh][wc * 64 + b * 32 + l32];
-#pragma unroll
-                for (int a = 0; a < 2; ++a)
-#pragma unroll
-                    for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f32_32x32x2(av[a], bv[b], acc[a][b]);
-            }
-        }
-    }
-}
-
-// C -= acc for the tile (ri0, rj0): columns at or beyond t1 and rows at or beyond n_pad are
-// left alone.  With to_lds (wavefront 0 of the workgroup whose tile holds the next diagonal
-// block) the updated block goes to sD (row pitch DG_LD, FP64) instead of A.
-__device__ __forceinline__ void tile_epilogue_f32(float* __restrict__ A, long long ld, int ri0, int rj0, int t1,
-                                                  int n_pad, const floatx16 (&acc)[2][2], bool to_lds,
-                                                  double* __restrict__ sD)
-{
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const int l32 = lane & 31, lh = lane >> 5;
-    // C -= acc ; lane owns column l32 and rows 8*(r/4) + 4*lh + (0..3) of each 32x32 block.
-    // All 16 loads of C are issued before any store (the stores could alias them as far as
-    // the compiler knows, which would serialise every load behind the previous store).
-    float4 cv[2][2][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int col = rj0 + wc * 64 + b * 32 + l32;
-            const float* cp = A + (long long)col * ld;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = ri0 + wr * 64 + a * 32 + 8 * q + 4 * lh;
-                cv[a][b][q] = (col < t1 && row < n_pad) ? *reinterpret_cast<const float4*>(cp + row)
-                                                         : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-        }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int col = rj0 + wc * 64 + b * 32 + l32;
-            if (col >= t1) continue;
-            float* cp = A + (long long)col * ld;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = ri0 + wr * 64 + a * 32 + 8 * q + 4 * lh;
-                if (row >= n_pad) continue;
-                float4 c = cv[a][b][q];
-                c.x -= acc[a][b][4 * q + 0];
-                c.y -= acc[a][b][4 * q + 1];
-                c.z -= acc[a][b][4 * q + 2];
-                c.w -= acc[a][b][4 * q + 3];
-                if (to_lds) {
-                    const int lr = row - ri0, lc = col - rj0;
-                    sD[(lr + 0) * DG_LD + lc] = c.x;
-                    sD[(lr + 1) * DG_LD + lc] = c.y;
-                    sD[(lr + 2) * DG_LD + lc] = c.z;
-                    sD[(lr + 3) * DG_LD + lc] = c.w;
-                } else {
-                    *reinterpret_cast<float4*>(cp + row) = c;
-                }
-            }
-        }
-}
-
-// Three waves per SIMD: the accumulators live in VGPRs next to the fused TRSM's registers.
-template <bool SPLIT>
-__device__ __forceinline__ void syrk_f32_body(float* __restrict__ A, long long ld, int kb, int K, int t0,
-                                              int t1, int n_pad, double* __restrict__ Lb_next,
-                                              int* __restrict__ flag_next, int* __restrict__ status,
-                                              int bid)
-{
-    __shared__ __align__(16) unsigned char smem[SY_SMEM];
-    double* sD = reinterpret_cast<double*>(smem);
-    // workgroup 0 holds tile (0, 0), whose top-left 64x64 block (wave 0) is the next
-    // panel's diagonal block
-    const bool diag = bid == 0;
-    int ti, tj;
-    trap_tile(bid, ceil_div_dev(n_pad - t0, SY_TILE), ti, tj);
-    const int ri0 = t0 + ti * SY_TILE;
-    const int rj0 = t0 + tj * SY_TILE;
-    floatx16 acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-    tile_acc_f32<SPLIT>(A, ld, kb, K, ri0, rj0, n_pad, smem, acc);
-    if (diag) __syncthreads();   // operand stages are reused for the diagonal block
-    tile_epilogue_f32(A, ld, ri0, rj0, t1, n_pad, acc, diag && (threadIdx.x >> 6) == 0, sD);
-    // wavefront 0 wrote the whole diagonal block to LDS itself and starts factoring it while
-    // the other wavefronts finish their stores (the factor's first barrier joins them)
-    if (diag) factor_diag64(sD, t0, status, Lb_next);
-    if (tj == 0) fused_trsm<float>(A, ld, t0, ri0, n_pad, Lb_next, flag_next, status, diag, smem, sD);
-}
-
-template <bool SPLIT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8)))
-syrk_f32_kernel(float* __restrict__ A, long long ld, int kb, int K, int t0, int t1, int n_pad,
-                double* __restrict__ Lb_next, int* __restrict__ flag_next, int* __restrict__ status)
-{
-    syrk_f32_body<SPLIT>(A, ld, kb, K, t0, t1, n_pad, Lb_next, flag_next, status, blockIdx.x);
-}
-
-// ------------------------------------------------------------------ FP64 SYRK (MFMA)
-// Same tiling; each wave 64x64 = 4x4 blocks of 16x16 (v_mfma_f64_16x16x4_f64).  The f64
-// MFMA returns row 4*r + l/16 in accumulator r of lane l; feeding the A operand rows in the
-// order perm(m) = 4*(m%4) + m/4 makes accumulator r hold row 4*(l/16) + r instead, so each
-// lane owns 4 consecutive rows of one column (two 16-byte stores).
-constexpr int SY_KC64 = 16;
-
-// acc += A[ri0.., kb .. kb+K) A[rj0.., kb .. kb+K)^T for one 128x128 tile on FP64 MFMA:
-// each wave 64x64 = 4x4 blocks of 16x16, A-operand rows fed in the order perm(m) (above).
-__device__ __forceinline__ void tile_acc_f64(const double* __restrict__ A, long long ld, int kb, int K, int ri0,
-                                             int rj0, int n_pad, unsigned char* smem, doublex4 (&acc)[4][4])
-{
-    static_assert(2 * SY_KC64 * (SY_TILE + 2) * 8 <= SY_SMEM, "SYRK LDS");
-    double (*sA)[SY_TILE + 2] = reinterpret_cast<double (*)[SY_TILE + 2]>(smem);
-    double (*sB)[SY_TILE + 2] = reinterpret_cast<double (*)[SY_TILE + 2]>(smem + SY_KC64 * (SY_TILE + 2) * 8);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const int l16 = lane & 15, lq = lane >> 4;
-    const int prow = 4 * (l16 & 3) + (l16 >> 2);
-    for (int k0 = 0; k0 < K; k0 += SY_KC64) {
-        __syncthreads();
-        for (int idx = tid; idx < SY_KC64 * SY_TILE / 2; idx += 256) {
-            const int k = idx / (SY_TILE / 2);
-            const int r2 = (idx % (SY_TILE / 2)) * 2;
-            const double* col = A + (long long)(kb + k0 + k) * ld;
-            double2 va = make_double2(0.0, 0.0), vb = va;
-            if (ri0 + r2 < n_pad) va = *reinterpret_cast<const double2*>(col + ri0 + r2);
-            if (rj0 + r2 < n_pad) vb = *reinterpret_cast<const double2*>(col + rj0 + r2);
-            sA[k][r2] = va.x; sA[k][r2 + 1] = va.y;
-            sB[k][r2] = vb.x; sB[k][r2 + 1] = vb.y;
-        }
-        __syncthreads();
-#pragma unroll 2
-        for (int k = 0; k < SY_KC64; k += 4) {
-            double av[4], bv[4];
-#pragma unroll
-            for (int a = 0; a < 4; ++a) av[a] = sA[k + lq][wr * 64 + a * 16 + prow];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) bv[b] = sB[k + lq][wc * 64 + b * 16 + l16];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) acc[a][b] = mfma_f64_16x16x4(av[a], bv[b], acc[a][b]);
-        }
-    }
-}
-
-// C -= acc for the tile (ri0, rj0) (columns < t1, rows < n_pad), or into sD (to_lds).
-__device__ __forceinline__ void tile_epilogue_f64(double* __restrict__ A, long long ld, int ri0, int rj0, int t1,
-                                                  int n_pad, const doublex4 (&acc)[4][4], bool to_lds,
-                                                  double* __restrict__ sD)
-{
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const int l16 = lane & 15, lq = lane >> 4;
-    // lane owns column l16 and rows 4*lq + (0..3) of each 16x16 block; every load of C is
-    // issued before the stores
-    double2 cv[4][4][2];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int col = rj0 + wc * 64 + b * 16 + l16;
-            const int row = ri0 + wr * 64 + a * 16 + 4 * lq;
-            const double* cp = A + (long long)col * ld + row;
-            const bool in = col < t1 && row < n_pad;
-            cv[a][b][0] = in ? *reinterpret_cast<const double2*>(cp) : make_double2(0.0, 0.0);
-            cv[a][b][1] = in ? *reinterpret_cast<const double2*>(cp + 2) : make_double2(0.0, 0.0);
-        }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int col = rj0 + wc * 64 + b * 16 + l16;
-            const int row = ri0 + wr * 64 + a * 16 + 4 * lq;
-            if (col >= t1 || row >= n_pad) continue;
-            double* cp = A + (long long)col * ld + row;
-            double2 c0v = cv[a][b][0];
-            double2 c1v = cv[a][b][1];
-            c0v.x -= acc[a][b][0]; c0v.y -= acc[a][b][1];
-            c1v.x -= acc[a][b][2]; c1v.y -= acc[a][b][3];
-            if (to_lds) {
-                const int lr = row - ri0, lc = col - rj0;
-                sD[(lr + 0) * DG_LD + lc] = c0v.x;
-                sD[(lr + 1) * DG_LD + lc] = c0v.y;
-                sD[(lr + 2) * DG_LD + lc] = c1v.x;
-                sD[(lr + 3) * DG_LD + lc] = c1v.y;
-            } else {
-                *reinterpret_cast<double2*>(cp) = c0v;
-                *reinterpret_cast<double2*>(cp + 2) = c1v;
-            }
-        }
-}
-
-__device__ __forceinline__ void syrk_f64_body(double* __restrict__ A, long long ld, int kb, int K, int t0,
-                                              int t1, int n_pad, double* __restrict__ Lb_next,
-                                              int* __restrict__ flag_next, int* __restrict__ status,
-                                              int bid)
-{
-    __shared__ __align__(16) unsigned char smem[SY_SMEM];
-    double* sD = reinterpret_cast<double*>(smem);
-    const bool diag = bid == 0;
-    int ti, tj;
-    trap_tile(bid, ceil_div_dev(n_pad - t0, SY_TILE), ti, tj);
-    const int ri0 = t0 + ti * SY_TILE;
-    const int rj0 = t0 + tj * SY_TILE;
-    doublex4 acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[a][b][r] = 0.0;
-    tile_acc_f64(A, ld, kb, K, ri0, rj0, n_pad, smem, acc);
-    if (diag) __syncthreads();   // operand stages are reused for the diagonal block
-    tile_epilogue_f64(A, ld, ri0, rj0, t1, n_pad, acc, diag && (threadIdx.x >> 6) == 0, sD);
-    // wavefront 0 wrote the whole diagonal block to LDS itself and starts factoring it while
-    // the other wavefronts finish their stores (the factor's first barrier joins them)
-    if (diag) factor_diag64(sD, t0, status, Lb_next);
-    if (tj == 0) fused_trsm<double>(A, ld, t0, ri0, n_pad, Lb_next, flag_next, status, diag, smem, sD);
-}
-
-__global__ void __launch_bounds__(256)
-syrk_f64_kernel(double* __restrict__ A, long long ld, int kb, int K, int t0, int t1, int n_pad,
-                double* __restrict__ Lb_next, int* __restrict__ flag_next, int* __restrict__ status)
-{
-    syrk_f64_body(A, ld, kb, K, t0, t1, n_pad, Lb_next, flag_next, status, blockIdx.x);
-}
-
-// Two-level blocking: outer panels of CHOL_OUTER columns are factored panel by panel
-// (64 columns) with updates restricted to the outer panel; the trailing matrix beyond it is
-// updated once per outer panel with K = CHOL_OUTER, which divides its HBM traffic (read +
-// write of the trailing lower triangle) by CHOL_OUTER / 64.
-#ifndef CHOL_OUTER_COLS
-#define CHOL_OUTER_COLS 256
-#endif
-constexpr int CHOL_OUTER = CHOL_OUTER_COLS;
-static_assert(CHOL_OUTER % CHOL_NB == 0 && CHOL_OUTER >= CHOL_NB, "outer panel width");
-
-// Update launch k (k = 0, 1, ...) of an n_pad matrix, after panel k = columns 64 k ..:
-// inside an outer panel of `outer` columns, the update of the outer panel's later columns; at
-// the end of an outer panel, the whole outer panel's update of the trailing matrix.  Inside
-// the outer panel the schedule is either right-looking (panel k updates all of the outer
-// panel's later columns, K = 64) or left-looking (all of the outer panel's panels so far
-// update only the next panel's 64 columns, K = 64, 128, ...).  Every schedule and width
-// leaves the same factor up to rounding.  False once no columns are left.
-#ifndef CHOL_LEFT_MAX
-#define CHOL_LEFT_MAX 4096
-#endif
-__host__ __device__ inline bool chol_step(int n_pad, bool left, int outer, int k, int& kb, int& K, int& t0,
-                                          int& t1)
-{
-    const int c0 = k * CHOL_NB;
-    t0 = c0 + CHOL_NB;
-    if (t0 >= n_pad) return false;
-    const int P0 = c0 / outer * outer;
-    const int P1 = n_pad < P0 + outer ? n_pad : P0 + outer;
-    if (t0 < P1 && left) {
-        kb = P0;
-        K = c0 + CHOL_NB - P0;
-        t1 = t0 + CHOL_NB;
-    } else if (t0 < P1) {
-        kb = c0;
-        K = CHOL_NB;
-        t1 = P1;
-    } else {
-        kb = P0;
-        K = P1 - P0;
-        t1 = n_pad;
-    }
-    return true;
-}
-
-// The single-system schedule: left-looking for matrices up to CHOL_LEFT_MAX, whose launches
-// are bound by the HBM traffic of the updates, right-looking beyond, where the chain of
-// diagonal blocks bounds them and the longer left-looking update of the first tile would
-// lengthen it.
-bool chol_left_looking(int n_pad) { return n_pad <= CHOL_LEFT_MAX; }
-int chol_outer_default() { return CHOL_OUTER; }
-
-// Workgroups of an update launch: the lower-trapezoid tiles of rows t0..n_pad, columns
-// t0..t1.
-__host__ __device__ inline int update_tiles(int n_pad, int t0, int t1)
-{
-    const int ni = (n_pad - t0 + SY_TILE - 1) / SY_TILE;
-    const int nj = (t1 - t0 + SY_TILE - 1) / SY_TILE;
-    return nj * ni - nj * (nj - 1) / 2;
-}
-
-template <typename T>
-int launch_update(T* d_A, long long ld, int kb, int K, int t0, int t1, int n_pad, double* d_Lb_next,
-                  int* d_flag_next, int* d_status, int syrk_mode, hipStream_t st)
-{
-    const int ntiles = update_tiles(n_pad, t0, t1);
-    if constexpr (sizeof(T) == 4) {
-        if (syrk_mode == SYRK_BF16X3)
-            hipLaunchKernelGGL(syrk_f32_kernel<true>, dim3(ntiles), dim3(256), 0, st,
-                               reinterpret_cast<float*>(d_A), ld, kb, K, t0, t1, n_pad, d_Lb_next,
-                               d_flag_next, d_status);
-        else
-            hipLaunchKernelGGL(syrk_f32_kernel<false>, dim3(ntiles), dim3(256), 0, st,
-                               reinterpret_cast<float*>(d_A), ld, kb, K, t0, t1, n_pad, d_Lb_next,
-                               d_flag_next, d_status);
-    } else {
-        hipLaunchKernelGGL(syrk_f64_kernel, dim3(ntiles), dim3(256), 0, st,
-                           reinterpret_cast<double*>(d_A), ld, kb, K, t0, t1, n_pad, d_Lb_next,
-                           d_flag_next, d_status);
-    }
-    BDH_LAUNCH_CHECK();
-    return 0;
-}
-
-// ------------------------------------------------------------------ factorization by epochs
-// One launch per outer panel P (columns P0 .. P1, CHOL_OUTER wide) for the large single-system
-// matrices.  Each launch runs three things side by side, which the per-panel launches above
-// run one after another:
-//   the panel factorization of P (its 64-column panels k: diagonal block, triangular solve of
-//   the rows below, right-looking update of P's later columns), on the row strips of P;
-//   the lookahead: the next outer panel's columns (P1 .. Q1) receive the previous outer
-//   panel's update and then each panel k's as soon as its rows are solved, so they are final
-//   when the launch ends and the next launch starts its diagonal block at once;
-//   the previous outer panel's update of every column beyond Q1.
-// Invariant at the start of epoch P: columns P0 .. P1 carry the updates of every column below
-// P0; columns beyond P1 those of every column below P0 - CHOL_OUTER.
-// Roles by workgroup index (the chain's workgroups have the lowest indices, so they are
-// dispatched first and all resident; every wait is for a lower index):
-//   b < R            row strip s = b (rows P0 + 128 s ..); for each panel k of P, in order:
-//                    the diagonal block if it lies in the strip (flag D_k) or a wait for D_k;
-//                    the solve of the strip's rows below block k (flag T_k,strip); panel k's
-//                    update of the strip's rows of P's later columns (right-looking, the next
-//                    diagonal block first; see epoch_strip), after the flags T_k of the strips
-//                    that hold those columns' rows.
-//   R <= b < R + NL  a 128 x 128 tile of the lookahead columns: K = CHOL_OUTER from the previous
-//                    outer panel, then K = 64 from each panel k after T_k of its two strips,
-//                    accumulated in registers and applied to C once.
-//   later b          a tile beyond Q1: the previous outer panel's update (K = CHOL_OUTER).
-struct EpochArgs {
-    int P0, P1, Q1;   // this outer panel, the end of the lookahead columns
-    int prevP0;       // the previous outer panel's first column (< 0 in the first epoch)
-    int R, NL, NB;    // row strips, lookahead tiles, bulk tiles
-};
-
-
-// Flags of the epoch schedule, after the diagonal-block flags in the workspace: T_k,g for
-// panel k and global row strip g (rows 128 g ..), n_pad / 64 x n_pad / 128 of them.
-__device__ __forceinline__ int* epoch_tflags(double* Lbuf, int n_pad)
-{
-    return chol_flags(Lbuf, n_pad) + n_pad / CHOL_NB;
-}
-
-// The epoch schedule's solve flags sit one per 128-byte line, so the tiles that poll one of
-// them do not share a line with the flags the diagonal chain sets and reads.
-constexpr int FLAG_STRIDE = 32;
-__device__ __forceinline__ int* tflag(int* tflags, int k, int g, int gstrips)
-{
-    return tflags + ((long long)k * gstrips + g) * FLAG_STRIDE;
-}
-
-// The workgroup's stores so far made visible at agent scope, then *flag set.
-__device__ __forceinline__ void publish_flag(int* flag)
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// All threads: wait until *flag is set (thread 0 polls, bounded); false after a timeout, which
-// is reported through status.
-template <int SLEEP = 2>
-__device__ __forceinline__ bool wg_wait_flag(int* flag, int* status)
-{
-    __shared__ int s_flag_ok;
-    if (threadIdx.x == 0) {
-        s_flag_ok = wait_flag<SLEEP>(flag) ? 1 : 0;
-        if (!s_flag_ok) atomicCAS(status, 0, -1);
-    }
-    __syncthreads();
-    return s_flag_ok != 0;
-}
-
-// All threads: wait until *f1 and *f2 are set (thread 0 polls both relaxed, then acquires once:
-// each agent-scope acquire invalidates this XCD's L2, which the tiles around share).
-template <int SLEEP = 2>
-__device__ __forceinline__ bool wg_wait_flags2(int* f1, int* f2, int* status)
-{
-    __shared__ int s_flags_ok;
-    if (threadIdx.x == 0) {
-        int ok = 0;
-        for (int it = 0; it < CHOL_SPIN * 2 / SLEEP; ++it) {
-            if (__hip_atomic_load(f1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 &&
-                __hip_atomic_load(f2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                ok = 1;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(SLEEP);
-        }
-        s_flags_ok = ok;
-        if (!ok) atomicCAS(status, 0, -1);
-    }
-    __syncthreads();
-    return s_flags_ok != 0;
-}
-
-// C[ri0.., rj0..] -= A[ri0.., kb .. kb+K) A[rj0.., kb .. kb+K)^T for one 128 x 128 tile
-// (columns < t1, rows < n_pad).
-template <typename T, bool SPLIT>
-__device__ __forceinline__ void epoch_tile_update(T* __restrict__ A, long long ld, int kb, int K, int ri0,
-                                                  int rj0, int t1, int n_pad, unsigned char* smem)
-{
-    if constexpr (sizeof(T) == 4) {
-        floatx16 acc[2][2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-        tile_acc_f32<SPLIT>(A, ld, kb, K, ri0, rj0, n_pad, smem, acc);
-        tile_epilogue_f32(A, ld, ri0, rj0, t1, n_pad, acc, false, nullptr);
-    } else {
-        doublex4 acc[4][4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[a][b][r] = 0.0;
-        tile_acc_f64(A, ld, kb, K, ri0, rj0, n_pad, smem, acc);
-        tile_epilogue_f64(A, ld, ri0, rj0, t1, n_pad, acc, false, nullptr);
-    }
 }
 
 // acc[q] = sum_k A[ra + i][kb + k] A[ca + 32 q + j][kb + k] over NQ 32 x 32 quadrants side by side
@@ -1251,473 +393,793 @@ __device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long
     }
 }
 
-// A[ra + i][ca + j] - acc of a quadrant, into dst[i * pitch + j] (LDS, FP64) or back into A
-// (dst null).
-__device__ __forceinline__ void quad_sub(float* __restrict__ A, long long ld, int ra, int ca, const floatx16& acc,
-                                         double* __restrict__ dst, int pitch)
-{
-    const int lane = threadIdx.x & 63, l32 = lane & 31, lh = lane >> 5;
-    float v[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = 8 * (r >> 2) + 4 * lh + (r & 3);
-        v[r] = A[(long long)(ca + l32) * ld + ra + row] - acc[r];
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = 8 * (r >> 2) + 4 * lh + (r & 3);
-        if (dst) dst[row * pitch + l32] = (double)v[r];
-        else A[(long long)(ca + l32) * ld + ra + row] = v[r];
-    }
-}
+// ------------------------------------------------------------------ factorization as one launch
+// The whole factorization of one matrix, or of every matrix of a batch, is one launch of one
+// workgroup per 128x128 tile of the lower triangle, left-looking: the workgroup of tile (i, j)
+// accumulates sum_k L_ik L_jk^T over the tile columns k < j as they are published, then finishes
+// its tile and publishes it.
+//   i > j  (flow_tile)  z = A_ij - sum, solved with L_jj and stored: the rows 128 i .. of panel j.
+//   i = j  (flow_diag)  z factored: the two 64x64 diagonal blocks and the block below the first.
+// Workgroups take the tiles column by column in the order of their index, so every tile a
+// workgroup waits for belongs to a lower index: it is finished or resident, and the waits end
+// whatever the number of resident workgroups.  The waits are bounded anyway (flow_wait).
+// What bounds it: for small matrices the chain diagonal block -> solve of the next block row ->
+// its update -> next diagonal block; for large ones MFMA issue of the accumulation, which no
+// longer reads and writes C once per outer panel and whose operands are shared in L2.  The chain
+// overlaps with everything else, since the workgroups of the following tile columns are
+// resident and accumulate what is already published.
+// Measured against one launch per 256-column outer panel (n_pad >= 1024) or per 64-column panel
+// (below), right-looking: n = 768 FP64 640 -> 220 us, n = 1353 FP32 720 -> 333 us, n = 3072 FP64
+// 1900 -> 925 us, n = 9000 FP32 5.95 -> 3.98 ms, FP64 11.3 -> 7.5 ms; the batch of 256 chains of
+// 64 .. 1024 beads FP32 6.9 -> 5.7 ms.
+//
+// Visibility across XCDs, whose L2 caches are not coherent within a launch: what other
+// workgroups read is stored at agent scope (write-through), the flag that announces it is set
+// after those stores have completed, and it lies in memory that no workgroup reads before that
+// flag -- the operand copy of tile (i, k) is the mirrored tile (k, i) of the upper triangle, which
+// holds no part of the factor; the diagonal blocks are in the workspace.  So no cache holds an
+// older copy of such a line, plain loads after the flag see the stored values, and no L2
+// invalidation is needed (an acquire per tile was measured to halve the rate of the tiles).
+// A tile's own entries (D before, L after) are read and written by its workgroup alone.
+//   operand copy: L(128 i + r, 128 k + c) at A[(128 i + c) ld + 128 k + r], r, c < 128, k < i.
 
-__device__ __forceinline__ void quad_sub(double* __restrict__ A, long long ld, int ra, int ca,
-                                         const doublex4 (&acc)[2][2], double* __restrict__ dst, int pitch)
-{
-    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
-    double v[2][2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                v[i][j][r] = A[(long long)(ca + 16 * j + l16) * ld + ra + 16 * i + 4 * r + lq] - acc[i][j][r];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 16 * i + 4 * r + lq, col = 16 * j + l16;
-                if (dst) dst[row * pitch + col] = v[i][j][r];
-                else A[(long long)(ca + col) * ld + ra + row] = v[i][j][r];
-            }
-}
+// Workspace per tile column j (doubles): diagonal block 2 j (LB_STRIDE), L21 (64 x 64, column c
+// at 64 c), diagonal block 2 j + 1; after all of them the flags, one per 128-byte line:
+//   dprog[j]  1: diagonal block 2 j and L21 are published, 2: diagonal block 2 j + 1 also
+//   rdy[i]    64-column panels of tile row i published so far
+constexpr int FLOW_T = 128;
+constexpr int FLOW_COL = 2 * LB_STRIDE + CHOL_NB * CHOL_NB;
+constexpr int FLAG_STRIDE = 32;
 
-template <typename T, int NQ>
-struct QuadAcc;
-template <int NQ>
-struct QuadAcc<float, NQ> {
-    floatx16 v[NQ];
-};
-template <int NQ>
-struct QuadAcc<double, NQ> {
-    doublex4 v[NQ][2][2];
-};
-
-// sD[r * DG_LD + c] = A[c1 + r][c1 + c] - sum_k A[c1 + r][kb + k] A[c1 + c][kb + k] for the 64 x 64
-// diagonal block at c1 (the strict upper 32 x 32 quadrant is not written; the factor reads only
-// r >= c), on MFMA in T: three wavefronts take the quadrants (0, 0), (1, 0), (1, 1).
 template <typename T>
-__device__ __forceinline__ void diag_block_update(T* __restrict__ A, long long ld, int c1, int kb, int K,
-                                                  double* __restrict__ sD)
+struct FlowMat {
+    T* A;
+    long long ld;
+    int n, nt;   // order (without the identity padding), tile rows
+    double* ws;
+    int* status;
+    __device__ int* dprog(int j) const { return flags() + j * FLAG_STRIDE; }
+    __device__ int* rdy(int i) const { return flags() + (nt + i) * FLAG_STRIDE; }
+    __device__ int* flags() const { return reinterpret_cast<int*>(ws + (long long)nt * FLOW_COL); }
+    // first element of column k (k < 128 x) of the operand copy of tile row x: rows r = 0 .. 127
+    __device__ const T* opnd(int x, int k) const
+    {
+        return A + (long long)(FLOW_T * x + (k & (FLOW_T - 1))) * ld + (k & ~(FLOW_T - 1));
+    }
+    __device__ T* tile(int i, int j) const { return A + (long long)FLOW_T * j * ld + FLOW_T * i; }
+};
+
+// All threads: this workgroup's agent-scope stores have completed, then *flag = v.
+__device__ __forceinline__ void flow_publish(int* flag, int v)
 {
-    const int wave = threadIdx.x >> 6;
-    if (wave == 3) return;
-    const int qr = wave == 0 ? 0 : 1, qc = wave == 2 ? 1 : 0;
-    QuadAcc<T, 1> acc;
-    quad_acc<1>(A, ld, c1 + 32 * qr, c1 + 32 * qc, kb, K, acc.v);
-    quad_sub(A, ld, c1 + 32 * qr, c1 + 32 * qc, acc.v[0], sD + 32 * qr * DG_LD + 32 * qc, DG_LD);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// One wavefront: A[ra + i][ca + j] -= sum_k A[ra + i][kb + k] A[ca + j][kb + k] over the
-// 32 x 32 NQ quadrants at rows ra .., columns ca, ca + 32, ...
-template <typename T, int NQ>
-__device__ __forceinline__ void wave_quads_update(T* __restrict__ A, long long ld, int ra, int ca, int kb, int K)
+// Each wavefront: wait until *flag >= need, return the value seen.  After FLOW_TIMEOUT (100 MHz
+// ticks: 10 s), or once another wait has timed out, it reports -1 through status and returns
+// need: the factorization then ends with wrong values and that status instead of hanging.
+constexpr long long FLOW_TIMEOUT = 1000000000ll;
+__device__ __forceinline__ int flow_wait(int* flag, int need, int* status)
 {
-    QuadAcc<T, NQ> acc;
-    quad_acc<NQ>(A, ld, ra, ca, kb, K, acc.v);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) quad_sub(A, ld, ra, ca + 32 * q, acc.v[q], nullptr, 0);
-}
-
-// A[rb + i][cb + j] -= sum_k A[rb + i][kb + k] A[cb + j][kb + k] for the rows rb .. rb + 32 W
-// of the 64 columns cb .. (the block lies below the diagonal): wavefront W0 + w, w < W, takes
-// rows rb + 32 w .. with both column quadrants.
-template <typename T, int W, int W0 = 0>
-__device__ __forceinline__ void block_update64(T* __restrict__ A, long long ld, int rb, int cb, int kb, int K)
-{
-    const int wave = (threadIdx.x >> 6) - W0;
-    if (wave < 0 || wave >= W) return;
-    const int ra = rb + 32 * wave;
-    QuadAcc<T, 2> acc;
-    quad_acc<2>(A, ld, ra, cb, kb, K, acc.v);
-    quad_sub(A, ld, ra, cb, acc.v[0], nullptr, 0);
-    quad_sub(A, ld, ra, cb + 32, acc.v[1], nullptr, 0);
-}
-
-// Row strip s of outer panel P (see above), right-looking: after solving its rows of panel k
-// the strip applies panel k to its rows of the later columns of P.  The diagonal chain comes
-// first and stays in LDS.  A strip holding the next two diagonal blocks kA (rows r0 ..) and
-// kB = kA + 1:
-//   panel kA - 1: only block kA's update (64 x 64, K = 64) is made, into LDS; the strip's lower
-//                 block row (rows r0 + 64 ..) keeps panel kA - 1 pending;
-//   block kA:     factor, publish D_kA, then the pending panel's update of block (kB, kA)
-//                 (64 x 64, into A), the solve of rows r0 + 64 .. with L_kA, and block kB's
-//                 update with panels kA - 1 and kA (K = 128) into LDS;
-//   block kB:     factor, publish D_kB.
-// Only the epoch's first block is read from A.
-template <typename T, bool SPLIT>
-__device__ __forceinline__ void epoch_strip(T* __restrict__ A, long long ld, int n_pad, double* __restrict__ Lbuf,
-                                            int* __restrict__ status, const EpochArgs& e, int s,
-                                            unsigned char* smem)
-{
-    int* dflags = chol_flags(Lbuf, n_pad);
-    int* tflags = epoch_tflags(Lbuf, n_pad);
-    const int gstrips = n_pad / SY_TILE;
-    const int r0 = e.P0 + SY_TILE * s, r1 = min(r0 + SY_TILE, n_pad);
-    const int g = r0 / SY_TILE;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double* sD = reinterpret_cast<double*>(smem);
-    double* sLT = sD;
-    double* sInv = sLT + CHOL_NB * CHOL_NB;
-    double* sc = sInv + 4 * 256 + wave * 16 * SC_PITCH;
-    bool block_in_lds = false;   // sD holds the next diagonal block, fully updated
-    int pend = -1;   // first column of panel kA - 1 while it is pending on the lower block row
-    int kdef = -1;   // first column of panel kA - 2 while it is deferred on block kB
-    for (int c0 = e.P0; c0 < e.P1 && c0 < r1; c0 += CHOL_NB) {
-        const int k = c0 / CHOL_NB;
-        double* Lb = Lbuf + (long long)k * LB_STRIDE;
-        const bool diag = c0 >= r0;   // block k lies in this strip
-        int rs = r0;                  // first row of the strip solved with panel k
-        if (diag) {
-            if (!block_in_lds) {
-                // the epoch's first block: it carries every update (earlier launches'); all 16
-                // loads of a thread are issued before its LDS stores
-                __syncthreads();
-                T v[CHOL_NB * CHOL_NB / 256];
-#pragma unroll
-                for (int i = 0; i < CHOL_NB * CHOL_NB / 256; ++i) {
-                    const int e2 = tid + 256 * i, r = e2 % CHOL_NB, c = e2 / CHOL_NB;
-                    v[i] = A[(long long)(c0 + c) * ld + c0 + r];
-                }
-#pragma unroll
-                for (int i = 0; i < CHOL_NB * CHOL_NB / 256; ++i) {
-                    const int e2 = tid + 256 * i, r = e2 % CHOL_NB, c = e2 / CHOL_NB;
-                    sD[r * DG_LD + c] = (r >= c) ? (double)v[i] : 0.0;
-                }
-            }
-            rs = c0 + CHOL_NB;
-            // Made in the factor's idle stretches (the operand rows were solved by this
-            // workgroup, behind a barrier): the pending panel on block (kB, kA), which the solve
-            // below reads (wavefront 3, before its columns), and the deferred and pending panels
-            // on block kB, so that its update after the solve takes panel kA alone (quadrants
-            // (1, 0), (1, 1) by wavefront 2 before its columns, (0, 0) by wavefront 0 after).
-            // In FP64 (slower MFMA, shorter idle stretches to fill) only block (kB, kA) is made
-            // there, by wavefronts 2 and 3, and block kB takes its panels after the solve.
-            const bool lower = pend >= 0 && rs < r1;
-            const int klo = kdef >= 0 ? kdef : pend, kK = lower ? pend + CHOL_NB - klo : 0;
-            factor_diag64(sD, c0, status, Lb,
-                [&] {
-                    if (!lower) return;
-                    if constexpr (sizeof(T) == 4) {
-                        if (wave == 3) {
-                            wave_quads_update<T, 2>(A, ld, rs, c0, pend, CHOL_NB);
-                            wave_quads_update<T, 2>(A, ld, rs + 32, c0, pend, CHOL_NB);
-                        } else if (wave == 2) {
-                            wave_quads_update<T, 2>(A, ld, rs + 32, rs, klo, kK);
-                        }
-                    } else {
-                        block_update64<T, 2, 2>(A, ld, rs, c0, pend, CHOL_NB);
-                    }
-                },
-                [&] {
-                    if constexpr (sizeof(T) == 4)
-                        if (lower && wave == 0) wave_quads_update<T, 1>(A, ld, rs, rs, klo, kK);
-                });                              // begins with a barrier; leaves sLT / sInv
-            publish_flag(dflags + k);            // Lb (the stores of store_diag64 are not read here)
-            store_diag64<T>(sD, A, ld, c0);
-        }
-        block_in_lds = false;
-        if (rs < r1) {
-            // rows rs .. r1 of panel k, two 16-row groups per wavefront; the rows carry every
-            // update once this workgroup's stores to them are done (a barrier), and are loaded
-            // before the wait for D_k
-            __syncthreads();
-            const int g0 = rs + 16 * wave, g1 = g0 + 64;
-            Trsm16 x0, x1;
-            if (g0 < r1) trsm16_load<T>(A, ld, c0, g0, r1, lane, x0);
-            if (g1 < r1) trsm16_load<T>(A, ld, c0, g1, r1, lane, x1);
-            else x1 = Trsm16{};
-            if (!diag) {
-                if (!wg_wait_flag(dflags + k, status)) return;   // a barrier: smem is free
-                load_lkk(Lb, sLT, sInv);    // ends with a barrier
-            }
-            if (g1 < r1) trsm16x2_solve_store<T>(A, ld, c0, g0, g1, r1, lane, x0, x1, sLT, sInv, sc);
-            else if (g0 < r1) trsm16_solve_store<T>(A, ld, c0, g0, r1, lane, x0, sLT, sInv, sc);
-        }
-        publish_flag(tflag(tflags, k, g, gstrips));
-        // panel k on the strip's rows of columns cb .. ce of P
-        const int cb = c0 + CHOL_NB, ce = min(e.P1, r1);
-        if (cb >= ce) continue;
-        if (diag) {
-            // block kA was factored: below the strip's diagonal the later columns hold block kB
-            // alone, which takes panel kA into LDS (FP32: the earlier panels came in the
-            // factor; FP64: with the pending panel, contiguous)
-            __syncthreads();   // the solve's stores done; smem is free
-            const int kb = sizeof(T) == 4 || pend < 0 ? c0 : pend;
-            diag_block_update<T>(A, ld, cb, kb, cb - kb, sD);
-            block_in_lds = true;
-            pend = -1;
-            kdef = -1;
-        } else if (cb == r0) {
-            // the next panel is block kA: its update (the strip's own rows of panel k) into LDS,
-            // the lower block row's left pending
-            __syncthreads();
-            diag_block_update<T>(A, ld, cb, c0, CHOL_NB, sD);
-            block_in_lds = true;
-            pend = c0;
-        } else {
-            // on a strip holding diagonal blocks, FP32 leaves block kB's columns to its
-            // factor's idle stretches (kdef)
-            const int cu = sizeof(T) == 4 && r0 < e.P1 ? min(ce, r0 + CHOL_NB) : ce;
-            if (cu < ce) kdef = c0;
-            if constexpr (sizeof(T) == 4) {
-                // tiles of up to 128 columns (LDS-staged, faster in FP32 than the pieces below),
-                // after the flags T_k of the strips holding rows cb .. cu
-                for (int gg = cb / SY_TILE; gg <= (cu - 1) / SY_TILE; ++gg)
-                    if (gg != g && !wg_wait_flag(tflag(tflags, k, gg, gstrips), status)) return;
-                for (int rj0 = cb; rj0 < cu; rj0 += SY_TILE) {
-                    __syncthreads();   // smem is free (the solve's operands, the previous tile's stages)
-                    floatx16 acc[2][2];
-#pragma unroll
-                    for (int a2 = 0; a2 < 2; ++a2)
-#pragma unroll
-                        for (int b2 = 0; b2 < 2; ++b2)
-#pragma unroll
-                            for (int r = 0; r < 16; ++r) acc[a2][b2][r] = 0.f;
-                    tile_acc_f32<SPLIT>(A, ld, c0, CHOL_NB, r0, rj0, n_pad, smem, acc);
-                    tile_epilogue_f32(A, ld, r0, rj0, cu, n_pad, acc, false, nullptr);
-                }
-            } else {
-                // 64-column pieces in column order (the next panel's first), each after the
-                // flag T_k of the strip holding its rows; a piece on the strip's own diagonal
-                // blocks takes only the rows from its diagonal down
-                __syncthreads();   // the solve's stores done
-                for (int j = cb; j < cu; j += CHOL_NB) {
-                    const int gg = j / SY_TILE;
-                    if (gg != g && !wg_wait_flag(tflag(tflags, k, gg, gstrips), status)) return;
-                    if (j < r0) block_update64<T, 4>(A, ld, r0, j, c0, CHOL_NB);
-                    else if (j == r0) block_update64<T, 4>(A, ld, j, j, c0, CHOL_NB);
-                    else block_update64<T, 2>(A, ld, j, j, c0, CHOL_NB);
-                }
+    int v = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v < need) {
+        const long long t0 = wall_clock64();
+        for (int it = 1;; ++it) {
+            __builtin_amdgcn_s_sleep(1);
+            v = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (v >= need) break;
+            if ((it & 255) == 0 && (wall_clock64() - t0 > FLOW_TIMEOUT ||
+                                    __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < 0)) {
+                if ((threadIdx.x & 63) == 0) atomicCAS(status, 0, -1);
+                v = need;
+                break;
             }
         }
     }
+    // the loads that follow stay behind the flag
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return __builtin_amdgcn_readfirstlane(v);
 }
 
-// Lookahead tile x (rows from P1, columns P1 .. Q1).
-template <typename T, bool SPLIT>
-__device__ __forceinline__ void epoch_lookahead(T* __restrict__ A, long long ld, int n_pad,
-                                                double* __restrict__ Lbuf, int* __restrict__ status,
-                                                const EpochArgs& e, int x, unsigned char* smem)
-{
-    int* tflags = epoch_tflags(Lbuf, n_pad);
-    const int gstrips = n_pad / SY_TILE;
-    int ti, tj;
-    trap_tile(x, ceil_div_dev(n_pad - e.P1, SY_TILE), ti, tj);
-    const int ri0 = e.P1 + SY_TILE * ti, rj0 = e.P1 + SY_TILE * tj;
-    const int gi = ri0 / SY_TILE, gj = rj0 / SY_TILE;
-    if constexpr (sizeof(T) == 4) {
-        floatx16 acc[2][2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-        if (e.prevP0 >= 0) tile_acc_f32<SPLIT>(A, ld, e.prevP0, e.P0 - e.prevP0, ri0, rj0, n_pad, smem, acc);
-        for (int c0 = e.P0; c0 < e.P1; c0 += CHOL_NB) {
-            const int k = c0 / CHOL_NB;
-            if (!wg_wait_flags2<16>(tflag(tflags, k, gi, gstrips), tflag(tflags, k, gj, gstrips), status)) return;
-            tile_acc_f32<SPLIT>(A, ld, c0, CHOL_NB, ri0, rj0, n_pad, smem, acc);
-        }
-        tile_epilogue_f32(A, ld, ri0, rj0, e.Q1, n_pad, acc, false, nullptr);
-    } else {
-        doublex4 acc[4][4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[a][b][r] = 0.0;
-        if (e.prevP0 >= 0) tile_acc_f64(A, ld, e.prevP0, e.P0 - e.prevP0, ri0, rj0, n_pad, smem, acc);
-        for (int c0 = e.P0; c0 < e.P1; c0 += CHOL_NB) {
-            const int k = c0 / CHOL_NB;
-            if (!wg_wait_flags2<16>(tflag(tflags, k, gi, gstrips), tflag(tflags, k, gj, gstrips), status)) return;
-            tile_acc_f64(A, ld, c0, CHOL_NB, ri0, rj0, n_pad, smem, acc);
-        }
-        tile_epilogue_f64(A, ld, ri0, rj0, e.Q1, n_pad, acc, false, nullptr);
+// Panels known to be published in two tile rows (the same row twice for a diagonal tile).
+struct FlowReady {
+    int *fi, *fj, *status;
+    int ri = 0, rj = 0;
+    __device__ bool poll(int need)
+    {
+        if (ri < need) ri = __builtin_amdgcn_readfirstlane(__hip_atomic_load(fi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (rj < need) rj = fj == fi ? ri : __builtin_amdgcn_readfirstlane(__hip_atomic_load(fj, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        const bool ok = ri >= need && rj >= need;
+        if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        return ok;
     }
-}
-
-// Tile (ti, tj), ti >= tj, of the lower triangle of an ni x ni tile matrix at position x of an
-// order that walks 8 x 8 super-tiles (column-major over the super-tiles, column-major inside
-// an off-diagonal one, trap_tile's order inside a diagonal one).
-__device__ __forceinline__ void super_tile(int x, int ni, int& ti, int& tj)
-{
-    constexpr int S = 8;
-    const int ns = (ni + S - 1) / S;
-    for (int SJ = 0; SJ < ns; ++SJ) {
-        const int c0 = S * SJ, mc = min(S, ni - c0);
-        const int dc = mc * (mc + 1) / 2;
-        if (x < dc) {
-            trap_tile(x, mc, ti, tj);
-            ti += c0;
-            tj += c0;
-            return;
-        }
-        x -= dc;
-        const int below = (ni - c0 - mc) * mc;   // the off-diagonal super-tiles of this column
-        if (x < below) {
-            const int blk = x / (S * mc), rem = x - blk * S * mc;
-            const int r0 = c0 + S * (blk + 1), mr = min(S, ni - r0);
-            ti = r0 + rem % mr;
-            tj = c0 + rem / mr;
-            return;
-        }
-        x -= below;
+    __device__ void wait(int need)
+    {
+        if (ri < need) ri = flow_wait(fi, need, status);
+        if (rj < need) rj = fj == fi ? ri : flow_wait(fj, need, status);
     }
-    ti = tj = 0;
-}
+};
 
-template <typename T, bool SPLIT>
-__device__ __forceinline__ void chol_epoch_body(T* __restrict__ A, long long ld, int n_pad,
-                                                double* __restrict__ Lbuf, int* __restrict__ status,
-                                                EpochArgs e)
-{
-    __shared__ __align__(16) unsigned char smem[SY_SMEM];
-    const int b = blockIdx.x;
-    if (b < e.R) {
-        epoch_strip<T, SPLIT>(A, ld, n_pad, Lbuf, status, e, b, smem);
-    } else if (b < e.R + e.NL) {
-        epoch_lookahead<T, SPLIT>(A, ld, n_pad, Lbuf, status, e, b - e.R, smem);
-    } else {
-        // workgroups b, b + 8, ... run on one XCD: give each XCD a contiguous run of the
-        // super-tile order, so the tiles it runs at a time share their operand row blocks in
-        // its L2
-        const int xb = b - e.R - e.NL;
-        const int c = xb & 7, q = e.NB >> 3, r = e.NB & 7;
-        int ti, tj;
-        super_tile(c * q + min(c, r) + (xb >> 3), ceil_div_dev(n_pad - e.Q1, SY_TILE), ti, tj);
-        epoch_tile_update<T, SPLIT>(A, ld, e.prevP0, e.P0 - e.prevP0, e.Q1 + SY_TILE * ti, e.Q1 + SY_TILE * tj,
-                                    n_pad, n_pad, smem);
-    }
-}
+constexpr int FLOW_KC32 = 32, FLOW_KC64 = 16;        // columns per LDS stage
+constexpr int FLOW_P32 = FLOW_T + 4, FLOW_P64 = FLOW_T + 2;   // row pitch of a stage
+constexpr int FLOW_SMEM = (LB_STRIDE + CHOL_NB * CHOL_NB) * 8;
+static_assert(2 * 2 * FLOW_KC32 * FLOW_P32 * 4 <= FLOW_SMEM && 2 * 2 * FLOW_KC64 * FLOW_P64 * 8 <= FLOW_SMEM &&
+              4 * FLOW_T * SY_HP * 4 <= FLOW_SMEM && CHOL_NB * DG_LD <= LB_STRIDE, "LDS of the factorization");
 
-// Two waves per SIMD: the row strips hold the diagonal factor's, the solve's and the tile
-// update's registers in one kernel.
+// The accumulated sums of a tile, per wavefront w rows 32 w .. 32 w + 31 of tile row i and all
+// 128 columns, transposed (the MFMA row index runs over the tile's columns): FP32 four 32x32 blocks,
+// FP64 8 x 2 16x16 blocks.  FP32 keeps C - sum in m and adds a partial sum of at most FLOW_FLUSH
+// columns to it at a time, so a partial sum's rounding is relative to that part alone (the
+// rounding of a C updated once per 256 columns); FP64 accumulates on -C.
+constexpr int FLOW_FLUSH = 256;
+template <typename T>
+struct FlowAcc;
+template <>
+struct FlowAcc<float> {
+    floatx16 m[4], a[4];
+};
+template <>
+struct FlowAcc<double> {
+    doublex4 a[8][2];
+};
+
+// Sums over the K columns 0 .. K - 1 (K a multiple of 128) of tile (i, j) into acc.
 template <bool SPLIT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
-chol_epoch_f32_kernel(float* __restrict__ A, long long ld, int n_pad, double* __restrict__ Lbuf,
-                      int* __restrict__ status, EpochArgs e)
+__device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, int j, int K, FlowReady& rd,
+                                                unsigned char* smem, FlowAcc<float>& acc)
 {
-    chol_epoch_body<float, SPLIT>(A, ld, n_pad, Lbuf, status, e);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const float* C = M.tile(i, j) + 32 * w + l32;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            acc.m[q][r] = C[(long long)(32 * q + 8 * (r >> 2) + 4 * lh + (r & 3)) * M.ld];
+            acc.a[q][r] = 0.f;
+        }
+    const int nc = K / FLOW_KC32;
+    if (nc == 0) return;
+    auto flush = [&] {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc.m[q][r] -= acc.a[q][r];
+                acc.a[q][r] = 0.f;
+            }
+    };
+    auto need = [](int c) { return c * FLOW_KC32 / CHOL_NB + 1; };
+    if constexpr (SPLIT) {
+        // [0] hi, [1] lo of tile row j; [2] hi, [3] lo of tile row i; row-major (row, k pairs)
+        unsigned (*sH)[FLOW_T][SY_HP] = reinterpret_cast<unsigned (*)[FLOW_T][SY_HP]>(smem);
+        const bool isI = tid >= FLOW_T;
+        const int lrow = tid & (FLOW_T - 1);
+        float v[FLOW_KC32];
+        auto load = [&](int c) {
+            const float* src = M.opnd(isI ? i : j, c * FLOW_KC32) + lrow;
+#pragma unroll
+            for (int k = 0; k < FLOW_KC32; ++k) v[k] = src[(long long)k * M.ld];
+        };
+        rd.wait(need(0));
+        load(0);
+        for (int c = 0; c < nc; ++c) {
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < FLOW_KC32; k += 8) {
+                unsigned h[8], l[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) split_bf16(v[k + u], h[u], l[u]);
+                *reinterpret_cast<uint4*>(&sH[isI ? 2 : 0][lrow][k / 2]) =
+                    make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
+                *reinterpret_cast<uint4*>(&sH[isI ? 3 : 1][lrow][k / 2]) =
+                    make_uint4(l[0] | (l[1] << 16), l[2] | (l[3] << 16), l[4] | (l[5] << 16), l[6] | (l[7] << 16));
+            }
+            __syncthreads();
+            const bool more = c + 1 < nc;
+            const bool pre = more && rd.poll(need(c + 1));
+            if (pre) load(c + 1);
+#pragma unroll
+            for (int t = 0; t < FLOW_KC32 / 16; ++t) {
+                const int x = 8 * t + 4 * lh;   // lane holds k = 16 t + 8 lh + 0..7
+                const bf16x8 bh = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&sH[2][32 * w + l32][x]));
+                const bf16x8 bl = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&sH[3][32 * w + l32][x]));
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const bf16x8 ah = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&sH[0][32 * q + l32][x]));
+                    const bf16x8 al = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&sH[1][32 * q + l32][x]));
+                    acc.a[q] = mfma_bf16_32x32x16(al, bh, acc.a[q]);
+                    acc.a[q] = mfma_bf16_32x32x16(ah, bl, acc.a[q]);
+                    acc.a[q] = mfma_bf16_32x32x16(ah, bh, acc.a[q]);
+                }
+            }
+            if (more && !pre) {
+                rd.wait(need(c + 1));
+                load(c + 1);
+            }
+            if ((c + 1) % (FLOW_FLUSH / FLOW_KC32) == 0 || !more) flush();
+        }
+        __syncthreads();
+    } else {
+        float (*st)[2][FLOW_KC32][FLOW_P32] = reinterpret_cast<float (*)[2][FLOW_KC32][FLOW_P32]>(smem);
+        constexpr int NV = FLOW_KC32 * FLOW_T / 4 / 256;
+        float4 vj[NV], vi[NV];
+        auto load = [&](int c) {
+            const float *pj = M.opnd(j, c * FLOW_KC32), *pi = M.opnd(i, c * FLOW_KC32);
+#pragma unroll
+            for (int u = 0; u < NV; ++u) {
+                const int idx = tid + 256 * u, k = idx / (FLOW_T / 4), r = (idx % (FLOW_T / 4)) * 4;
+                vj[u] = *reinterpret_cast<const float4*>(pj + (long long)k * M.ld + r);
+                vi[u] = *reinterpret_cast<const float4*>(pi + (long long)k * M.ld + r);
+            }
+        };
+        auto store = [&](int b) {
+#pragma unroll
+            for (int u = 0; u < NV; ++u) {
+                const int idx = tid + 256 * u, k = idx / (FLOW_T / 4), r = (idx % (FLOW_T / 4)) * 4;
+                *reinterpret_cast<float4*>(&st[b][0][k][r]) = vj[u];
+                *reinterpret_cast<float4*>(&st[b][1][k][r]) = vi[u];
+            }
+        };
+        rd.wait(need(0));
+        load(0);
+        store(0);
+        __syncthreads();
+        for (int c = 0; c < nc; ++c) {
+            const bool more = c + 1 < nc;
+            const bool pre = more && rd.poll(need(c + 1));
+            if (pre) load(c + 1);
+            float (*sj)[FLOW_P32] = st[c & 1][0], (*si)[FLOW_P32] = st[c & 1][1];
+#pragma unroll 4
+            for (int k = 0; k < FLOW_KC32; k += 2) {
+                const float b = si[k + lh][32 * w + l32];
+                float a[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) a[q] = sj[k + lh][32 * q + l32];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc.a[q] = mfma_f32_32x32x2(a[q], b, acc.a[q]);
+            }
+            if (more) {
+                if (!pre) {
+                    rd.wait(need(c + 1));
+                    load(c + 1);
+                }
+                store((c + 1) & 1);
+            }
+            if ((c + 1) % (FLOW_FLUSH / FLOW_KC32) == 0 || !more) flush();
+            __syncthreads();
+        }
+    }
 }
 
-__global__ void __launch_bounds__(256)
-chol_epoch_f64_kernel(double* __restrict__ A, long long ld, int n_pad, double* __restrict__ Lbuf,
-                      int* __restrict__ status, EpochArgs e)
+template <bool SPLIT>
+__device__ __forceinline__ void flow_accumulate(const FlowMat<double>& M, int i, int j, int K, FlowReady& rd,
+                                                unsigned char* smem, FlowAcc<double>& acc)
 {
-    chol_epoch_body<double, false>(A, ld, n_pad, Lbuf, status, e);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lq = lane >> 4;
+    const double* C = M.tile(i, j) + 32 * w + lr;
+#pragma unroll
+    for (int J = 0; J < 8; ++J)
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc.a[J][g][r] = -C[(long long)(16 * J + 4 * r + lq) * M.ld + 16 * g];
+    const int nc = K / FLOW_KC64;
+    if (nc == 0) return;
+    auto need = [](int c) { return c * FLOW_KC64 / CHOL_NB + 1; };
+    double (*st)[2][FLOW_KC64][FLOW_P64] = reinterpret_cast<double (*)[2][FLOW_KC64][FLOW_P64]>(smem);
+    constexpr int NV = FLOW_KC64 * FLOW_T / 2 / 256;
+    double2 vj[NV], vi[NV];
+    auto load = [&](int c) {
+        const double *pj = M.opnd(j, c * FLOW_KC64), *pi = M.opnd(i, c * FLOW_KC64);
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const int idx = tid + 256 * u, k = idx / (FLOW_T / 2), r = (idx % (FLOW_T / 2)) * 2;
+            vj[u] = *reinterpret_cast<const double2*>(pj + (long long)k * M.ld + r);
+            vi[u] = *reinterpret_cast<const double2*>(pi + (long long)k * M.ld + r);
+        }
+    };
+    auto store = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const int idx = tid + 256 * u, k = idx / (FLOW_T / 2), r = (idx % (FLOW_T / 2)) * 2;
+            *reinterpret_cast<double2*>(&st[b][0][k][r]) = vj[u];
+            *reinterpret_cast<double2*>(&st[b][1][k][r]) = vi[u];
+        }
+    };
+    rd.wait(need(0));
+    load(0);
+    store(0);
+    __syncthreads();
+    for (int c = 0; c < nc; ++c) {
+        const bool more = c + 1 < nc;
+        const bool pre = more && rd.poll(need(c + 1));
+        if (pre) load(c + 1);
+        double (*sj)[FLOW_P64] = st[c & 1][0], (*si)[FLOW_P64] = st[c & 1][1];
+#pragma unroll
+        for (int k = 0; k < FLOW_KC64; k += 4) {
+            double a[8], b[2];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) b[g] = si[k + lq][32 * w + 16 * g + lr];
+#pragma unroll
+            for (int J = 0; J < 8; ++J) a[J] = sj[k + lq][16 * J + lr];
+#pragma unroll
+            for (int J = 0; J < 8; ++J)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) acc.a[J][g] = mfma_f64_16x16x4(a[J], b[g], acc.a[J][g]);
+        }
+        if (more) {
+            if (!pre) {
+                rd.wait(need(c + 1));
+                load(c + 1);
+            }
+            store((c + 1) & 1);
+        }
+        __syncthreads();
+    }
 }
 
-// Clears the diagonal-block and solve flags of one factorization (a kernel rather than a
-// memset node, so a captured factorization replays it correctly).
-__global__ void chol_epoch_clear_kernel(int* __restrict__ flags, int count)
+// z = sum - C in FP64, z[J][g][r] = column 16 J + 4 r + l/16, row 16 g + l%16 of the wavefront's 32
+// rows.  FP32: through the wavefront's own part of the LDS at sc (2048 floats).
+__device__ __forceinline__ void flow_negated(const FlowAcc<double>& acc, float*, doublex4 (&z)[8][2])
+{
+#pragma unroll
+    for (int J = 0; J < 8; ++J)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) z[J][g] = acc.a[J][g];
+}
+__device__ __forceinline__ void flow_negated(const FlowAcc<float>& acc, float* __restrict__ sc, doublex4 (&z)[8][2])
+{
+    const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4, l32 = lane & 31, lh = lane >> 5;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                sc[(32 * q + 8 * (r >> 2) + 4 * lh + (r & 3)) * 32 + l32] = acc.m[2 * h + q][r];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int J = 0; J < 4; ++J)
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) z[4 * h + J][g][r] = -(double)sc[(16 * J + 4 * r + lq) * 32 + 16 * g + lr];
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// X L_kk^T = -z for G groups of 16 rows on one wavefront, X over z: transposed, X_J^T = -Linv_J
+// (z_J^T + sum_K L_JK X_K^T), so a finished block's accumulators (column 4 r + l/16, row l%16) are
+// the next product's operands as they are (k = 4 s + l/16 of row l%16), and only L comes from the
+// LDS.  sLT[k * 64 + c] = L_kk[c][k]; sInv[SINV J + c' * SINV_P + c] = Linv_JJ[c][c'].
+template <int G, int Z>
+__device__ __forceinline__ void flow_solve64(doublex4 (&z)[Z][G], int J0, const double* __restrict__ sLT,
+                                             const double* __restrict__ sInv)
+{
+    const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
+#pragma unroll
+    for (int J = 0; J < 4; ++J) {
+#pragma unroll
+        for (int K = 0; K < J; ++K)
+#pragma unroll
+            for (int s4 = 0; s4 < 4; ++s4) {
+                const double a = sLT[(16 * K + 4 * s4 + lq) * CHOL_NB + 16 * J + lr];
+#pragma unroll
+                for (int g = 0; g < G; ++g) z[J0 + J][g] = mfma_f64_16x16x4(a, z[J0 + K][g][s4], z[J0 + J][g]);
+            }
+        doublex4 x[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) x[g] = doublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) {
+            const double a = sInv[SINV * J + (4 * s4 + lq) * SINV_P + lr];
+#pragma unroll
+            for (int g = 0; g < G; ++g) x[g] = mfma_f64_16x16x4(a, z[J0 + J][g][s4], x[g]);
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) z[J0 + J][g] = -x[g];
+    }
+}
+
+// Blocks J0 .. J0 + 3 of z (X) into the tile (i, j) and its operand copy.
+template <typename T>
+__device__ __forceinline__ void flow_store(const FlowMat<T>& M, int i, int j, int J0, const doublex4 (&z)[8][2])
+{
+    const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
+    const int row = 32 * (threadIdx.x >> 6) + lr;
+    T* o = const_cast<T*>(M.opnd(i, FLOW_T * j)) + row;   // columns of tile column j: ld apart, as in the tile
+    T* t = M.tile(i, j) + row;
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const long long col = (long long)(16 * (J0 + J) + 4 * r + lq) * M.ld;
+#pragma unroll
+            for (int g = 0; g < 2; ++g) st_agent(o + col + 16 * g, (T)z[J0 + J][g][r]);
+        }
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const long long col = (long long)(16 * (J0 + J) + 4 * r + lq) * M.ld;
+#pragma unroll
+            for (int g = 0; g < 2; ++g) t[col + 16 * g] = (T)z[J0 + J][g][r];
+        }
+}
+
+template <typename T, bool SPLIT>
+__device__ __forceinline__ void flow_tile(const FlowMat<T>& M, int i, int j, unsigned char* smem)
+{
+    double* s0 = reinterpret_cast<double*>(smem);   // diagonal block
+    double* s1 = s0 + LB_STRIDE;                    // L21
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    doublex4 z[8][2];
+    {
+        FlowAcc<T> acc;
+        FlowReady rd{M.rdy(i), M.rdy(j), M.status};
+        flow_accumulate<SPLIT>(M, i, j, FLOW_T * j, rd, smem, acc);   // ends with a barrier
+        flow_negated(acc, reinterpret_cast<float*>(s1) + 2048 * (tid >> 6), z);
+    }
+    const double* ws = M.ws + (long long)j * FLOW_COL;
+    int have = flow_wait(M.dprog(j), 1, M.status);
+    __syncthreads();   // s1 is free
+    {
+        constexpr int N1 = CHOL_NB * CHOL_NB / 256;
+        double v[N1];
+#pragma unroll
+        for (int u = 0; u < N1; ++u) v[u] = ws[LB_STRIDE + tid + 256 * u];
+        load_lkk(ws, s0);   // ends with a barrier
+#pragma unroll
+        for (int u = 0; u < N1; ++u) s1[tid + 256 * u] = v[u];
+    }
+    flow_solve64<2>(z, 0, s0, s0 + CHOL_NB * CHOL_NB);
+    flow_store<T>(M, i, j, 0, z);
+    flow_publish(M.rdy(i), 2 * j + 1);   // a barrier: s1 is complete, s0 free
+    // z_2 += L21 X_1^T
+#pragma unroll
+    for (int K = 0; K < 4; ++K)
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+            for (int J = 0; J < 4; ++J) {
+                const double a = s1[(16 * K + 4 * s4 + lq) * CHOL_NB + 16 * J + lr];
+#pragma unroll
+                for (int g = 0; g < 2; ++g) z[4 + J][g] = mfma_f64_16x16x4(a, z[K][g][s4], z[4 + J][g]);
+            }
+    if (have < 2) flow_wait(M.dprog(j), 2, M.status);
+    load_lkk(ws + LB_STRIDE + CHOL_NB * CHOL_NB, s0);
+    flow_solve64<2>(z, 4, s0, s0 + CHOL_NB * CHOL_NB);
+    flow_store<T>(M, i, j, 4, z);
+    flow_publish(M.rdy(i), 2 * j + 2);
+}
+
+// One 32x32 block of a diagonal tile on one wavefront, transposed as in FlowAcc: columns 32 mb ..,
+// rows 32 nb .. of the tile.
+template <typename T>
+struct FlowQuad;
+template <>
+struct FlowQuad<float> {
+    floatx16 m, a;
+    __device__ void init(const float* t, long long ld, int mb, int nb, int lane)
+    {
+        const float* C = t + 32 * nb + (lane & 31);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            m[r] = C[(long long)(32 * mb + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * ld];
+            a[r] = 0.f;
+        }
+    }
+    __device__ void flush()
+    {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            m[r] -= a[r];
+            a[r] = 0.f;
+        }
+    }
+    // rows k0 .. of s (pitch P): the k-th holds column k of the 128 (or 64) rows
+    template <int KC, typename S>
+    __device__ void mac(const S* s, int P, int mb, int nb, int lane)
+    {
+        const int l32 = lane & 31, lh = lane >> 5;
+#pragma unroll 8
+        for (int k = 0; k < KC; k += 2)
+            a = mfma_f32_32x32x2((float)s[(k + lh) * P + 32 * mb + l32], (float)s[(k + lh) * P + 32 * nb + l32], a);
+    }
+    // K = 64 columns straight from memory
+    __device__ void mac_global(const float* p, long long ld, int mb, int nb)
+    {
+        floatx16 t[1];
+        quad_acc<1>(p, ld, 32 * mb, 32 * nb, 0, CHOL_NB, t);
+        a += t[0];
+    }
+    template <typename F>
+    __device__ void each(int lane, F&& f)
+    {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) f(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), lane & 31, (double)(m[r] - a[r]));
+    }
+};
+template <>
+struct FlowQuad<double> {
+    doublex4 a[2][2];
+    __device__ void init(const double* t, long long ld, int mb, int nb, int lane)
+    {
+        const double* C = t + 32 * nb + (lane & 15);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    a[x][y][r] = -C[(long long)(32 * mb + 16 * x + 4 * r + (lane >> 4)) * ld + 16 * y];
+    }
+    __device__ void flush() {}
+    template <int KC, typename S>
+    __device__ void mac(const S* s, int P, int mb, int nb, int lane)
+    {
+        const int lr = lane & 15, lq = lane >> 4;
+#pragma unroll 4
+        for (int k = 0; k < KC; k += 4) {
+            double u[2], v[2];
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                u[x] = s[(k + lq) * P + 32 * mb + 16 * x + lr];
+                v[x] = s[(k + lq) * P + 32 * nb + 16 * x + lr];
+            }
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) a[x][y] = mfma_f64_16x16x4(u[x], v[y], a[x][y]);
+        }
+    }
+    __device__ void mac_global(const double* p, long long ld, int mb, int nb)
+    {
+        doublex4 t[1][2][2];
+        quad_acc<1>(p, ld, 32 * mb, 32 * nb, 0, CHOL_NB, t);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) a[x][y] += t[0][x][y];
+    }
+    template <typename F>
+    __device__ void each(int lane, F&& f)
+    {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) f(16 * x + 4 * r + (lane >> 4), 16 * y + (lane & 15), -a[x][y][r]);
+    }
+};
+
+// Diagonal tile j.  Its ten 32x32 blocks of the lower triangle lie on the wavefronts as (column
+// block, row block)
+//   wavefront 0: (0,0)           1: (0,1) (0,2) (2,2)    2: (1,1) (0,3) (2,3)    3: (1,2) (1,3) (3,3)
+// so that the update that precedes each diagonal block's factor, the last step of the chain, is
+// one block per wavefront: the last 64 columns are applied to the first diagonal block from the
+// LDS, to the others by wavefronts 1 .. 3 while wavefront 0 factors it.
+template <typename T>
+__device__ __forceinline__ void flow_diag(const FlowMat<T>& M, int j, unsigned char* smem)
+{
+    constexpr int KC = sizeof(T) == 4 ? FLOW_KC32 : FLOW_KC64;
+    constexpr int P = sizeof(T) == 4 ? FLOW_P32 : FLOW_P64;
+    constexpr int V = 16 / sizeof(T);   // entries of one 16-byte access
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    double* s0 = reinterpret_cast<double*>(smem);
+    double* s1 = s0 + LB_STRIDE;
+    double* ws = M.ws + (long long)j * FLOW_COL;
+    T* tl = M.tile(j, j);
+    const int c0 = FLOW_T * j;
+    const bool second = c0 + CHOL_NB < M.n;   // else the second block is identity padding
+    const int m0 = w == 2 || w == 3 ? 1 : 0, n0 = w == 0 ? 0 : (w == 3 ? 2 : 1);
+    const int m1 = w == 3 ? 1 : 0, n1 = w == 1 ? 2 : 3;
+    const int m2 = w == 3 ? 3 : 2, n2 = w == 1 ? 2 : 3;
+    FlowQuad<T> q0, q1, q2;
+    q0.init(tl, M.ld, m0, n0, lane);
+    if (w) {
+        q1.init(tl, M.ld, m1, n1, lane);
+        q2.init(tl, M.ld, m2, n2, lane);
+    }
+    if (j > 0) {
+        FlowReady rd{M.rdy(j), M.rdy(j), M.status};
+        const int nc = (FLOW_T * j - CHOL_NB) / KC;
+        auto need = [](int c) { return c * KC / CHOL_NB + 1; };
+        T (*st)[KC][P] = reinterpret_cast<T (*)[KC][P]>(smem);
+        constexpr int NV = KC * FLOW_T / V / 256;
+        typedef T vec __attribute__((ext_vector_type(V)));
+        vec v[NV];
+        auto load = [&](int c) {
+            const T* p = M.opnd(j, c * KC);
+#pragma unroll
+            for (int u = 0; u < NV; ++u) {
+                const int idx = tid + 256 * u, k = idx / (FLOW_T / V), r = (idx % (FLOW_T / V)) * V;
+                v[u] = *reinterpret_cast<const vec*>(p + (long long)k * M.ld + r);
+            }
+        };
+        auto store = [&](int b) {
+#pragma unroll
+            for (int u = 0; u < NV; ++u) {
+                const int idx = tid + 256 * u, k = idx / (FLOW_T / V), r = (idx % (FLOW_T / V)) * V;
+                *reinterpret_cast<vec*>(&st[b][k][r]) = v[u];
+            }
+        };
+        rd.wait(need(0));
+        load(0);
+        store(0);
+        __syncthreads();
+        for (int c = 0; c < nc; ++c) {
+            const bool more = c + 1 < nc;
+            const bool pre = more && rd.poll(need(c + 1));
+            if (pre) load(c + 1);
+            const T* s = &st[c & 1][0][0];
+            q0.template mac<KC>(s, P, m0, n0, lane);
+            if (w) {
+                q1.template mac<KC>(s, P, m1, n1, lane);
+                q2.template mac<KC>(s, P, m2, n2, lane);
+            }
+            if (more) {
+                if (!pre) {
+                    rd.wait(need(c + 1));
+                    load(c + 1);
+                }
+                store((c + 1) & 1);
+            }
+            if ((c + 1) % (FLOW_FLUSH / KC) == 0 || !more) {
+                q0.flush();
+                if (w) {
+                    q1.flush();
+                    q2.flush();
+                }
+            }
+            __syncthreads();
+        }
+        // the last 64 columns of rows 0 .. 63 through s1
+        rd.wait(2 * j);
+        constexpr int NL = CHOL_NB * CHOL_NB / V / 256;
+        vec x[NL];
+        const T* p = M.opnd(j, FLOW_T * j - CHOL_NB);
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int idx = tid + 256 * u, k = idx / (CHOL_NB / V), r = (idx % (CHOL_NB / V)) * V;
+            x[u] = *reinterpret_cast<const vec*>(p + (long long)k * M.ld + r);
+        }
+        T* sl = reinterpret_cast<T*>(s1);
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+            const int idx = tid + 256 * u, k = idx / (CHOL_NB / V), r = (idx % (CHOL_NB / V)) * V;
+            *reinterpret_cast<vec*>(sl + k * CHOL_NB + r) = x[u];
+        }
+        __syncthreads();
+        if (w < 3) q0.template mac<CHOL_NB>(sl, CHOL_NB, m0, n0, lane);
+    }
+    auto to_block = [&](FlowQuad<T>& q, int mb, int nb) {
+        q.each(lane, [&](int c, int r, double v) { s0[(32 * nb + r) * DG_LD + 32 * mb + c] = v; });
+    };
+    auto to_lower = [&](FlowQuad<T>& q, int mb, int nb) {
+        q.each(lane, [&](int c, int r, double v) { s1[(32 * mb + c) * CHOL_NB + 32 * (nb - 2) + r] = v; });
+    };
+    if (w < 3) to_block(q0, m0, n0);
+    factor_diag64(s0, c0, M.status, [&] {   // begins with a barrier
+        if (!second) return;
+        if (j > 0) {
+            const T* p = M.opnd(j, FLOW_T * j - CHOL_NB);
+            if (w == 3) q0.mac_global(p, M.ld, m0, n0);
+            q1.mac_global(p, M.ld, m1, n1);
+            q2.mac_global(p, M.ld, m2, n2);
+        }
+        if (w == 3) to_lower(q0, m0, n0);
+        to_lower(q1, m1, n1);
+    });
+    store_lkk(s0, ws);
+    if (!second) {
+        store_diag64<T>(s0, tl, M.ld, 0);
+        return;
+    }
+    // L21: 16 rows per wavefront
+    doublex4 z[4][1];
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[J][0][r] = -s1[(16 * J + 4 * r + lq) * CHOL_NB + 16 * w + lr];
+    flow_solve64<1>(z, 0, s0, s0 + CHOL_NB * CHOL_NB);
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = 16 * J + 4 * r + lq, row = 16 * w + lr;
+            s1[c * CHOL_NB + row] = z[J][0][r];
+            st_agent(ws + LB_STRIDE + c * CHOL_NB + row, z[J][0][r]);
+            tl[(long long)c * M.ld + CHOL_NB + row] = (T)z[J][0][r];
+        }
+    __syncthreads();   // L21 in s1; s0 is free
+    if (w) {
+        q2.flush();
+        q2.template mac<CHOL_NB>(s1, CHOL_NB, m2 - 2, n2 - 2, lane);
+        to_block(q2, m2 - 2, n2 - 2);
+    }
+    flow_publish(M.dprog(j), 1);
+    factor_diag64(s0, c0 + CHOL_NB, M.status, [&] {
+        // L11 into the tile
+        for (int e = tid - 64; e < CHOL_NB * CHOL_NB; e += 192) {
+            const int r = e % CHOL_NB, c = e / CHOL_NB;
+            if (r >= c) tl[(long long)c * M.ld + r] = (T)ws[e];
+        }
+    });
+    store_lkk(s0, ws + LB_STRIDE + CHOL_NB * CHOL_NB);
+    flow_publish(M.dprog(j), 2);
+    store_diag64<T>(s0, tl, M.ld, CHOL_NB);
+}
+
+template <typename T, bool SPLIT>
+__device__ __forceinline__ void flow_body(const FlowMat<T>& M, int i, int j)
+{
+    __shared__ __align__(16) unsigned char smem[FLOW_SMEM];
+    if (i == j) flow_diag<T>(M, j, smem);
+    else flow_tile<T, SPLIT>(M, i, j, smem);
+}
+
+template <typename T, bool SPLIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+chol_flow_kernel(FlowMat<T> M)
+{
+    // tile column by column
+    int x = blockIdx.x, j = 0;
+    while (x >= M.nt - j) {
+        x -= M.nt - j;
+        ++j;
+    }
+    flow_body<T, SPLIT>(M, j + x, j);
+}
+
+__global__ void chol_flow_clear_kernel(int* __restrict__ flags, int count)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) flags[i] = 0;
 }
 
-// Matrices at least this large factor by epochs; smaller ones (one or two outer panels, where
-// nothing is left to overlap) by the per-panel launches.
-#ifndef CHOL_EPOCH_MIN
-#define CHOL_EPOCH_MIN 1024
-#endif
-
+// d_status: 0, or the 1-based row of the first non-positive pivot; -1 after a timed-out wait.
 template <typename T>
-int chol_factor_epochs(T* d_A, long long ld, int n_pad, double* d_Lbuf, int* d_status, int syrk_mode,
-                       hipStream_t st, PhaseRecorder* rec)
-{
-    const int nblk = n_pad / CHOL_NB, gstrips = n_pad / SY_TILE;
-    int* d_flags = reinterpret_cast<int*>(d_Lbuf + (long long)nblk * LB_STRIDE);
-    const int nflags = nblk + nblk * gstrips * FLAG_STRIDE;
-    if (rec) rec->begin(PH_PANEL, st);
-    hipLaunchKernelGGL(chol_epoch_clear_kernel, dim3(ceil_div(nflags, 256)), dim3(256), 0, st, d_flags, nflags);
-    BDH_LAUNCH_CHECK();
-    if (rec) rec->end(PH_PANEL, st);
-    for (int P0 = 0; P0 < n_pad; P0 += CHOL_OUTER) {
-        EpochArgs e;
-        e.P0 = P0;
-        e.P1 = std::min(P0 + CHOL_OUTER, n_pad);
-        e.Q1 = std::min(e.P1 + CHOL_OUTER, n_pad);
-        e.prevP0 = P0 - CHOL_OUTER;
-        e.R = (n_pad - P0) / SY_TILE;
-        e.NL = e.Q1 > e.P1 ? update_tiles(n_pad, e.P1, e.Q1) : 0;
-        e.NB = (e.prevP0 >= 0 && e.Q1 < n_pad) ? update_tiles(n_pad, e.Q1, n_pad) : 0;
-        const dim3 grid(e.R + e.NL + e.NB);
-        if (rec) rec->begin(PH_SYRK, st);
-        if constexpr (sizeof(T) == 4) {
-            if (syrk_mode == SYRK_BF16X3)
-                hipLaunchKernelGGL(chol_epoch_f32_kernel<true>, grid, dim3(256), 0, st, reinterpret_cast<float*>(d_A),
-                                   ld, n_pad, d_Lbuf, d_status, e);
-            else
-                hipLaunchKernelGGL(chol_epoch_f32_kernel<false>, grid, dim3(256), 0, st, reinterpret_cast<float*>(d_A),
-                                   ld, n_pad, d_Lbuf, d_status, e);
-        } else {
-            hipLaunchKernelGGL(chol_epoch_f64_kernel, grid, dim3(256), 0, st, reinterpret_cast<double*>(d_A), ld,
-                               n_pad, d_Lbuf, d_status, e);
-        }
-        BDH_LAUNCH_CHECK();
-        if (rec) rec->end(PH_SYRK, st);
-    }
-    return 0;
-}
-
-// Matrices of CHOL_EPOCH_MIN and more factor by epochs (above).  Smaller ones: one launch per
-// panel, the update kernel of panel k also factoring diagonal block k + 1 (workgroup 0) and
-// solving panel k + 1 (its tile column 0, after workgroup 0's flag).
-template <typename T>
-int chol_factor(T* d_A, long long ld, int n_pad, double* d_Lbuf, int* d_status, int syrk_mode,
+int chol_factor(T* d_A, long long ld, int n, int n_pad, double* d_Lbuf, int* d_status, int syrk_mode,
                 hipStream_t st, PhaseRecorder* rec)
 {
-    BDH_CHECK(n_pad % PAD_TO == 0, "chol_factor: n_pad must be a multiple of 128");
+    BDH_CHECK(n_pad % PAD_TO == 0 && n <= n_pad && n > n_pad - PAD_TO, "chol_factor: n_pad must be n rounded up to 128");
     BDH_CHECK(ld >= n_pad && ld % 4 == 0, "chol_factor: bad leading dimension");
     BDH_CHECK(syrk_mode != SYRK_BF16X3 || sizeof(T) == 4, "chol_factor: split SYRK needs FP32 storage");
-    if (n_pad >= CHOL_EPOCH_MIN) return chol_factor_epochs<T>(d_A, ld, n_pad, d_Lbuf, d_status, syrk_mode, st, rec);
-    constexpr long long LB = LB_STRIDE;
-    const int nblk = n_pad / CHOL_NB;
-    int* d_flags = reinterpret_cast<int*>(d_Lbuf + nblk * LB);
+    const int nt = n_pad / FLOW_T;
+    FlowMat<T> M{d_A, ld, n, nt, d_Lbuf, d_status};
+    int* d_flags = reinterpret_cast<int*>(d_Lbuf + (long long)nt * FLOW_COL);
+    const int nflags = 2 * nt * FLAG_STRIDE;
     if (rec) rec->begin(PH_PANEL, st);
-    hipLaunchKernelGGL(chol_diag_kernel<T>, dim3(1), dim3(256), 0, st, d_A, ld, 0, d_Lbuf, d_flags,
-                       nblk, d_status);
+    hipLaunchKernelGGL(chol_flow_clear_kernel, dim3(ceil_div(nflags, 256)), dim3(256), 0, st, d_flags, nflags);
     BDH_LAUNCH_CHECK();
-    if (n_pad > CHOL_NB) {
-        hipLaunchKernelGGL(chol_trsm_kernel<T>, dim3(ceil_div(n_pad - CHOL_NB, TRSM_ROWS)), dim3(256),
-                           0, st, d_A, ld, 0, n_pad, (const double*)d_Lbuf);
-        BDH_LAUNCH_CHECK();
-    }
     if (rec) rec->end(PH_PANEL, st);
-    int kb, K, t0, t1;
-    const bool left = chol_left_looking(n_pad);
-    for (int k = 0; chol_step(n_pad, left, CHOL_OUTER, k, kb, K, t0, t1); ++k) {
-        if (rec) rec->begin(PH_SYRK, st);
-        const int rc = launch_update<T>(d_A, ld, kb, K, t0, t1, n_pad, d_Lbuf + (k + 1) * LB,
-                                        d_flags + k + 1, d_status, syrk_mode, st);
-        if (rc) return rc;
-        if (rec) rec->end(PH_SYRK, st);
+    if (rec) rec->begin(PH_SYRK, st);
+    const dim3 grid(nt * (nt + 1) / 2);
+    if constexpr (sizeof(T) == 4) {
+        if (syrk_mode == SYRK_BF16X3)
+            hipLaunchKernelGGL((chol_flow_kernel<T, true>), grid, dim3(256), 0, st, M);
+        else
+            hipLaunchKernelGGL((chol_flow_kernel<T, false>), grid, dim3(256), 0, st, M);
+    } else {
+        hipLaunchKernelGGL((chol_flow_kernel<T, false>), grid, dim3(256), 0, st, M);
     }
+    BDH_LAUNCH_CHECK();
+    if (rec) rec->end(PH_SYRK, st);
     return 0;
 }
 
 size_t chol_lbuf_doubles(int n_pad)
 {
-    const size_t nblk = n_pad / CHOL_NB, gstrips = n_pad / SY_TILE;
-    // FP64 blocks with inverses, then the int flags: one per diagonal block, then (epochs
-    // only) the solve flags, one per panel and row strip, each on its own 128-byte line
-    if (n_pad < CHOL_EPOCH_MIN) return nblk * LB_STRIDE + (nblk + 1) / 2;
-    return nblk * LB_STRIDE + (nblk + nblk * gstrips * FLAG_STRIDE + 1) / 2;
+    const size_t nt = n_pad / FLOW_T;
+    return nt * FLOW_COL + 2 * nt * FLAG_STRIDE / 2;
 }
 
 // ------------------------------------------------------------------ Y = L X (partials)
@@ -1855,28 +1317,6 @@ int launch_trmv_partials(const T* d_L, long long ld, int n, const double* d_X, l
 int trmv_blk_cols() { return TRMV_COLS; }
 
 // ------------------------------------------------------------------ batches of matrices
-// Launch k of every chain's factorization runs as one grid: workgroup x maps to its chain
-// through the prefix table of launch k and then does exactly what workgroup
-// x - prefix[c] of the chain's own launch k does (chol_factor), on the chain's matrix,
-// workspace, flags and status.  A chain's diagonal workgroup (local index 0) has the lowest
-// index of the chain's workgroups, so it is dispatched before any workgroup that waits for
-// its flag, as in the single-matrix launch.  Chains whose factorization has fewer launches
-// drop out of the later grids.
-int chol_update_steps(int n_pad)
-{
-    int kb, K, t0, t1, k = 0;
-    while (chol_step(n_pad, true, CHOL_OUTER, k, kb, K, t0, t1)) ++k;
-    return k;
-}
-
-int chol_update_blocks(int n_pad, bool left, int outer, int k)
-{
-    int kb, K, t0, t1;
-    return chol_step(n_pad, left, outer, k, kb, K, t0, t1) ? update_tiles(n_pad, t0, t1) : 0;
-}
-
-int chol_trsm0_blocks(int n_pad) { return n_pad > CHOL_NB ? ceil_div(n_pad - CHOL_NB, TRSM_ROWS) : 0; }
-
 template <typename T>
 int trmv_blocks(int n)
 {
@@ -1884,52 +1324,47 @@ int trmv_blocks(int n)
     return ceil_div(n, ROWS) * trmv_col_blocks(n);
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256)
-chol_diag_batch_kernel(T* __restrict__ A, double* __restrict__ Lbuf, const BatchChain* __restrict__ ch,
-                       int* __restrict__ status)
+// The tiles of every chain's matrix in one launch.  Key of a tile (i, j) of a matrix of nt tile
+// rows: nt - j, the tile columns left on its chain of diagonal blocks; larger keys first, so the
+// chains with the most columns left start first and all end together.  Among equal keys the
+// diagonal tiles, then the tiles below them (the next on their chains), then the rest.  A tile
+// waits for tiles of larger keys and for its own diagonal tile only, all of lower index.
+std::vector<FlowTask> chol_batch_tasks(const std::vector<int>& n_pad)
 {
-    const int c = blockIdx.x;
-    const BatchChain b = ch[c];
-    double* Lb = Lbuf + b.lb;
-    chol_diag_body<T>(A + b.mat, b.n_pad, 0, Lb, chol_flags(Lb, b.n_pad), b.n_pad / CHOL_NB, status + c);
+    std::vector<FlowTask> t;
+    int key = 0;
+    for (int np : n_pad) key = std::max(key, np / FLOW_T);
+    for (; key > 0; --key)
+        for (int d = 0; d < 3; ++d)
+            for (size_t c = 0; c < n_pad.size(); ++c) {
+                const int nt = n_pad[c] / FLOW_T, j = nt - key;
+                if (j < 0) continue;
+                const int i0 = j + d, i1 = d < 2 ? std::min(nt, i0 + 1) : nt;
+                for (int i = i0; i < i1; ++i) t.push_back(FlowTask{(int)c, (short)i, (short)j});
+            }
+    return t;
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256)
-chol_trsm_batch_kernel(T* __restrict__ A, const double* __restrict__ Lbuf,
-                       const BatchChain* __restrict__ ch, const int* __restrict__ prefix, int nch)
+__device__ __forceinline__ FlowMat<T> flow_mat(T* A, double* Lbuf, const BatchChain& b, int* status)
 {
-    const int c = batch_find(prefix, nch, blockIdx.x);
-    const BatchChain b = ch[c];
-    chol_trsm_body<T>(A + b.mat, b.n_pad, 0, b.n_pad, Lbuf + b.lb, blockIdx.x - prefix[c]);
+    return FlowMat<T>{A + b.mat, b.n_pad, b.n, b.n_pad / FLOW_T, Lbuf + b.lb, status};
 }
 
-template <bool SPLIT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8)))
-syrk_f32_batch_kernel(float* __restrict__ A, double* __restrict__ Lbuf, const BatchChain* __restrict__ ch,
-                      const int* __restrict__ prefix, int nch, int k, int* __restrict__ status)
+template <typename T, bool SPLIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+chol_flow_batch_kernel(T* __restrict__ A, double* __restrict__ Lbuf, const BatchChain* __restrict__ ch,
+                       const FlowTask* __restrict__ tasks, int* __restrict__ status)
 {
-    const int c = batch_find(prefix, nch, blockIdx.x);
-    const BatchChain b = ch[c];
-    int kb, K, t0, t1;
-    chol_step(b.n_pad, b.left != 0, b.outer, k, kb, K, t0, t1);
-    double* Lb = Lbuf + b.lb;
-    syrk_f32_body<SPLIT>(A + b.mat, b.n_pad, kb, K, t0, t1, b.n_pad, Lb + (long long)(k + 1) * LB_STRIDE,
-                         chol_flags(Lb, b.n_pad) + k + 1, status + c, blockIdx.x - prefix[c]);
+    const FlowTask t = tasks[blockIdx.x];
+    flow_body<T, SPLIT>(flow_mat(A, Lbuf, ch[t.c], status + t.c), t.i, t.j);
 }
 
-__global__ void __launch_bounds__(256)
-syrk_f64_batch_kernel(double* __restrict__ A, double* __restrict__ Lbuf, const BatchChain* __restrict__ ch,
-                      const int* __restrict__ prefix, int nch, int k, int* __restrict__ status)
+template <typename T>
+__global__ void chol_flow_clear_batch_kernel(double* __restrict__ Lbuf, const BatchChain* __restrict__ ch)
 {
-    const int c = batch_find(prefix, nch, blockIdx.x);
-    const BatchChain b = ch[c];
-    int kb, K, t0, t1;
-    chol_step(b.n_pad, b.left != 0, b.outer, k, kb, K, t0, t1);
-    double* Lb = Lbuf + b.lb;
-    syrk_f64_body(A + b.mat, b.n_pad, kb, K, t0, t1, b.n_pad, Lb + (long long)(k + 1) * LB_STRIDE,
-                  chol_flags(Lb, b.n_pad) + k + 1, status + c, blockIdx.x - prefix[c]);
+    const FlowMat<T> M = flow_mat((T*)nullptr, Lbuf, ch[blockIdx.x], nullptr);
+    for (int x = threadIdx.x; x < 2 * M.nt * FLAG_STRIDE; x += blockDim.x) M.flags()[x] = 0;
 }
 
 template <typename T>
@@ -1939,34 +1374,19 @@ int chol_factor_batch(T* d_A, double* d_Lbuf, const BatchPlan& plan, int* d_stat
     BDH_CHECK(syrk_mode != SYRK_BF16X3 || sizeof(T) == 4, "chol_factor_batch: split SYRK needs FP32 storage");
     BDH_CHECK(sizeof(T) == 8 || syrk_mode != SYRK_F64, "chol_factor_batch: FP32 storage needs an FP32 SYRK");
     if (rec) rec->begin(PH_PANEL, st);
-    hipLaunchKernelGGL(chol_diag_batch_kernel<T>, dim3(plan.nch), dim3(256), 0, st, d_A, d_Lbuf, plan.ch,
-                       d_status);
+    hipLaunchKernelGGL(chol_flow_clear_batch_kernel<T>, dim3(plan.nch), dim3(256), 0, st, d_Lbuf, plan.ch);
     BDH_LAUNCH_CHECK();
-    if (plan.trsm_blocks > 0) {
-        hipLaunchKernelGGL(chol_trsm_batch_kernel<T>, dim3(plan.trsm_blocks), dim3(256), 0, st, d_A,
-                           (const double*)d_Lbuf, plan.ch, plan.trsm_pre, plan.nch);
-        BDH_LAUNCH_CHECK();
-    }
     if (rec) rec->end(PH_PANEL, st);
-    for (int k = 0; k < plan.chol_steps; ++k) {
-        const int blocks = plan.chol_blocks[k];
-        if (blocks == 0) continue;
-        const int* pre = plan.chol_pre + (long long)k * (plan.nch + 1);
-        if (rec) rec->begin(PH_SYRK, st);
-        if constexpr (sizeof(T) == 4) {
-            if (syrk_mode == SYRK_BF16X3)
-                hipLaunchKernelGGL(syrk_f32_batch_kernel<true>, dim3(blocks), dim3(256), 0, st,
-                                   reinterpret_cast<float*>(d_A), d_Lbuf, plan.ch, pre, plan.nch, k, d_status);
-            else
-                hipLaunchKernelGGL(syrk_f32_batch_kernel<false>, dim3(blocks), dim3(256), 0, st,
-                                   reinterpret_cast<float*>(d_A), d_Lbuf, plan.ch, pre, plan.nch, k, d_status);
-        } else {
-            hipLaunchKernelGGL(syrk_f64_batch_kernel, dim3(blocks), dim3(256), 0, st,
-                               reinterpret_cast<double*>(d_A), d_Lbuf, plan.ch, pre, plan.nch, k, d_status);
-        }
-        BDH_LAUNCH_CHECK();
-        if (rec) rec->end(PH_SYRK, st);
-    }
+    if (rec) rec->begin(PH_SYRK, st);
+    const dim3 grid(plan.ntasks);
+    if (sizeof(T) == 4 && syrk_mode == SYRK_BF16X3)
+        hipLaunchKernelGGL((chol_flow_batch_kernel<T, sizeof(T) == 4>), grid, dim3(256), 0, st, d_A, d_Lbuf, plan.ch,
+                           plan.tasks, d_status);
+    else
+        hipLaunchKernelGGL((chol_flow_batch_kernel<T, false>), grid, dim3(256), 0, st, d_A, d_Lbuf, plan.ch,
+                           plan.tasks, d_status);
+    BDH_LAUNCH_CHECK();
+    if (rec) rec->end(PH_SYRK, st);
     return 0;
 }
 
@@ -2013,8 +1433,8 @@ template int launch_trmv_batch<double>(const double*, const double*, long long, 
 template int trmv_blocks<float>(int);
 template int trmv_blocks<double>(int);
 
-template int chol_factor<float>(float*, long long, int, double*, int*, int, hipStream_t, PhaseRecorder*);
-template int chol_factor<double>(double*, long long, int, double*, int*, int, hipStream_t, PhaseRecorder*);
+template int chol_factor<float>(float*, long long, int, int, double*, int*, int, hipStream_t, PhaseRecorder*);
+template int chol_factor<double>(double*, long long, int, int, double*, int*, int, hipStream_t, PhaseRecorder*);
 template int launch_trmv_partials<float>(const float*, long long, int, const double*, long long, int, double*, hipStream_t);
 template int launch_trmv_partials<double>(const double*, long long, int, const double*, long long, int, double*, hipStream_t);
 

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 namespace bdh {
 
@@ -23,13 +24,10 @@ struct PhaseRecorder {
 // (ld = n_pad) at A + mat, FP64 factor workspace at Lbuf + lb, its Gaussians at xi + xi_off
 // (rows of ldx), and partial-sum rows at pp (pair sums: psplits rows), pf (forces: fsplits
 // rows) and pt (L.x: tcols x 16 rows).  Every per-chain launch shape is the one the
-// single-system launchers use, so a chain's arithmetic is the same as on its own, as long as
-// `left` (the update schedule of its factorization, chol_left_looking) and `outer` (its outer
-// panel width) are the ones the single system picks for its n_pad.
+// single-system launchers use, so a chain's arithmetic is the same as on its own.
 struct BatchChain {
     int N, n, n_pad, bead0;
     int psplits, fsplits, tcols, ldx;
-    int left, outer;
     long long mat, lb, xi_off, pp, pf, pt;
 };
 
@@ -46,17 +44,21 @@ __device__ __forceinline__ int batch_find(const int* __restrict__ prefix, int nc
     return lo;
 }
 
+// One workgroup of the batch's factorization: tile (i, j) of chain c's lower triangle.
+struct FlowTask {
+    int c;
+    short i, j;
+};
+
 // Prefix tables (nch + 1 ints on the device) and workgroup totals of one batch's launches.
 struct BatchPlan {
     int nch = 0;
     const BatchChain* ch = nullptr;
     const int *asm_pre = nullptr, *pair_pre = nullptr, *force_pre = nullptr, *trmv_pre = nullptr;
-    const int *rows_pre = nullptr, *diag_pre = nullptr, *trsm_pre = nullptr;
-    int asm_blocks = 0, pair_blocks = 0, force_blocks = 0, trmv_blocks = 0, rows_blocks = 0,
-        trsm_blocks = 0;
-    const int* chol_pre = nullptr;   // steps x (nch + 1): launch k of every chain's factorization
-    int chol_steps = 0;
-    const int* chol_blocks = nullptr;   // host: workgroups of launch k
+    const int *rows_pre = nullptr;
+    int asm_blocks = 0, pair_blocks = 0, force_blocks = 0, trmv_blocks = 0, rows_blocks = 0;
+    const FlowTask* tasks = nullptr;   // the factorization's workgroups in index order
+    int ntasks = 0;
 };
 
 // ---- random stream (bdh_rng.hip)
@@ -111,10 +113,11 @@ int launch_tea_close(const double4* d_pos, const double* d_xi, const double* d_F
 constexpr int CHOL_NB = 64;   // panel width
 constexpr int PAD_TO = 128;   // n is padded to a multiple of this with an identity block
 enum SyrkMode { SYRK_F32 = 0, SYRK_F64 = 1, SYRK_BF16X3 = 2 };
-// d_Lbuf: chol_lbuf_doubles(n_pad) doubles of workspace (FP64 diagonal blocks).
+// d_Lbuf: chol_lbuf_doubles(n_pad) doubles of workspace (FP64 diagonal blocks, flags).  The tiles
+// above the diagonal tiles of A are overwritten (operand copies of the factor).
 size_t chol_lbuf_doubles(int n_pad);
 template <typename T>
-int chol_factor(T* d_A, long long ld, int n_pad, double* d_Lbuf, int* d_status, int syrk_mode,
+int chol_factor(T* d_A, long long ld, int n, int n_pad, double* d_Lbuf, int* d_status, int syrk_mode,
                 hipStream_t st, PhaseRecorder* rec = nullptr);
 int trmv_col_blocks(int n);
 // Y = L X for m <= TRMV_MAX_RHS right-hand sides X[k * ldx + c]; partials P[cb][k][n].
@@ -123,15 +126,11 @@ template <typename T>
 int launch_trmv_partials(const T* d_L, long long ld, int n, const double* d_X, long long ldx, int m,
                          double* d_P, hipStream_t st);
 int trmv_blk_cols();   // columns per partial of the L.x kernel
-// Per-chain workgroup counts of the batched launches (host).
-int chol_update_steps(int n_pad);                 // update launches of one factorization
-bool chol_left_looking(int n_pad);                // the single-system update schedule
-int chol_outer_default();                         // the single-system outer panel width
-int chol_update_blocks(int n_pad, bool left, int outer, int k);   // workgroups of launch k (0 when none)
-int chol_trsm0_blocks(int n_pad);                 // panel-0 solve workgroups
+// Workgroups of the factorization of a batch with the given padded orders, in index order.
+std::vector<FlowTask> chol_batch_tasks(const std::vector<int>& n_pad);
 template <typename T>
 int trmv_blocks(int n);                           // row x column blocks of the L.x partials
-// Factorization of every chain's matrix, launch k of all chains together.
+// Factorization of every chain's matrix in one launch.
 template <typename T>
 int chol_factor_batch(T* d_A, double* d_Lbuf, const BatchPlan& plan, int* d_status, int syrk_mode,
                       hipStream_t st, PhaseRecorder* rec = nullptr);

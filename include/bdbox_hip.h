@@ -303,27 +303,21 @@ int bdh_batch_phase_timing(bdh_batch* batch, int enable);
 int bdh_batch_phase_times(bdh_batch* batch, double* ms, long long* counts);
 
 /* Update schedule of the batch's factorizations (no counterpart in the reference, whose
- * CPU path calls LAPACK dpotrf).  Inside each 256-column outer panel, a chain whose padded
- * size n_pad is at most left_max updates left-looking (every panel of the outer panel so
- * far updates the next 64 columns); the others update right-looking (each panel updates all
- * later columns of the outer panel).  left_max < 0 (the default) gives every chain the
- * schedule a single system of its size uses: left-looking up to n_pad 4096, so chain c's
- * trajectory is then bitwise the single system's.  Schedules differ in rounding only. */
+ * CPU path calls LAPACK dpotrf).  The factorization of all chains is one launch of one
+ * workgroup per 128x128 tile and has a single schedule, so every left_max gives the same
+ * launches and the same results; the value is kept for bdh_batch_get_schedule. */
 int bdh_batch_set_schedule(bdh_batch* batch, int left_max);
 int bdh_batch_get_schedule(bdh_batch* batch, int* left_max);
-/* Tile-schedule autotuner (no counterpart in the reference): times the refactor of every
- * chain (assembly + factorization, graph replays, fastest of `reps`) under each candidate
- * left_max -- 0, then up to BDH_TUNE_MAX - 1 of the batch's padded sizes, the largest
- * included -- and keeps the fastest.  cand / ms (BDH_TUNE_MAX entries each, may be NULL)
- * receive the candidates and their times, *ncand their count, *best the choice.  Call it
- * before the first step; the first step then refactors as usual. */
+/* Times the refactor of every chain (assembly + factorization, graph replays, fastest of
+ * `reps`) under each candidate left_max -- 0, then up to BDH_TUNE_MAX - 1 of the batch's padded
+ * sizes, the largest included -- and keeps the fastest.  cand / ms (BDH_TUNE_MAX entries each,
+ * may be NULL) receive the candidates and their times, *ncand their count, *best the choice.
+ * Call it before the first step; the first step then refactors as usual. */
 #define BDH_TUNE_MAX 8
 int bdh_batch_autotune(bdh_batch* batch, int reps, int* cand, double* ms, int* ncand, int* best);
 
-/* Tile shape of the batch's factorizations (no counterpart in the reference): the update
- * schedule as in bdh_batch_set_schedule, and the width of the outer panels (256, 512 or
- * 1024 columns) within which panels of 64 columns update, before the trailing matrix is
- * updated with the whole outer panel.  Widths and schedules differ in rounding only. */
+/* bdh_batch_set_schedule with an outer panel width (256, 512 or 1024; other widths are an
+ * error), kept for bdh_batch_get_tiles; neither changes the launches. */
 int bdh_batch_set_tiles(bdh_batch* batch, int left_max, int outer);
 int bdh_batch_get_tiles(bdh_batch* batch, int* left_max, int* outer);
 /* bdh_batch_autotune over tile shapes: every schedule candidate of bdh_batch_autotune under

@@ -1,0 +1,58 @@
+"""The one-launch Cholesky factorization at the edges of its tiles: orders on either side of the
+64-column diagonal blocks and 128x128 tiles, every precision, against LAPACK, and the INFO of a
+non-positive pivot in every 16-column group and block position."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 2, 15, 17, 63, 64, 65, 127, 128, 129, 191, 193, 255, 257, 385, 641]
+
+
+@pytest.fixture(scope="module")
+def api():
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from bd_box_amd import system
+    return system
+
+
+def _matrix(n):
+    """SPD with 3 on the diagonal and 1 / (2 + 0.1 d^2) off it, plus a ripple."""
+    d = np.arange(n)[:, None] - np.arange(n)[None, :]
+    return np.where(d == 0, 3.0, 1.0 / (2.0 + 0.1 * d * d)) + 0.01 * np.cos(d * 1.7)
+
+
+@pytest.mark.parametrize("n", EDGES)
+def test_factor_edges_vs_lapack(api, n):
+    """FP64: entries within n eps |a| of LAPACK's, taken 8 times for the two orders of summation.
+    FP32 storage: each entry of L is rounded to 2^-24, so |L L^T - A| <= 2 2^-24 a_max, taken 4
+    times for the accumulation; split-bf16 products drop terms below 2^-17 |l l'|."""
+    A = _matrix(n)
+    ref = np.linalg.cholesky(A)
+    print(f"factor n={n}", flush=True)
+    L, info = api.dpotrf(A, "L", api.FP64)
+    assert info == 0
+    assert np.abs(np.tril(L) - ref).max() <= 8 * max(n, 16) * 2.0 ** -53 * 3.0
+    for prec, tol in ((api.MIXED, 4 * 2 * 2.0 ** -24 * 3.02), (api.MIXED_SPLIT, 4 * 2.0 ** -17 * 3.02)):
+        L, info = api.dpotrf(A, "L", prec)
+        assert info == 0
+        L = np.tril(L)
+        assert np.abs(L @ L.T - A).max() <= tol, prec
+
+
+@pytest.mark.parametrize("row", [0, 1, 15, 16, 47, 63, 64, 79, 127, 128, 191, 192, 299])
+def test_factor_reports_first_bad_pivot(api, row):
+    """LAPACK's INFO: the 1-based row of the first non-positive pivot."""
+    A = _matrix(300)
+    A[row, row] = -1.0
+    if row + 5 < 300:
+        A[row + 5, row + 5] = -2.0
+    print(f"bad pivot row={row}", flush=True)
+    for prec in (api.FP64, api.MIXED):
+        from bd_box_amd import _lib
+        import ctypes as C
+        M = np.asfortranarray(A).copy(order="F")
+        rc = _lib.load().bdh_dpotrf(b"L", M.ctypes.data_as(C.POINTER(C.c_double)), 300, 300, prec)
+        assert rc == row + 1, (prec, rc)
