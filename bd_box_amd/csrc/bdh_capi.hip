@@ -429,7 +429,7 @@ int tea_parts(bdh_system* s, const double* X, double dt, double* Rf_out, const d
         jobs.job[nj++] = ReduceJob{s->Px, s->Feff, s->n, s->msplits, 0, 1.0};
         jobs.job[nj++] = ReduceJob{s->Pc, s->Cs, s->n, s->msplits, 0, 1.0};
         if (launch_reduce_partials(jobs, nj, s->n, s->st)) return -1;
-        if (launch_tea_close(s->pos_s, s->X_s, s->Feff, s->Cs, s->Pe, pair_eparts(N), N, s->preDii, dt, s->bt,
+        if (launch_tea_close(s->pos_s, s->X_s, s->Feff, s->Cs, s->Pe, pair_eparts(N, s->ewald), N, s->preDii, dt, s->bt,
                              s->Rs_s, s->st))
             return -1;
         hipLaunchKernelGGL(pair_order_scatter_kernel, g, b, 0, s->st, (const int*)s->perm, N,
@@ -444,7 +444,7 @@ int tea_parts(bdh_system* s, const double* X, double dt, double* Rf_out, const d
     jobs.job[nj++] = ReduceJob{s->Px, s->Feff, s->n, s->msplits, 0, 1.0};
     jobs.job[nj++] = ReduceJob{s->Pc, s->Cs, s->n, s->msplits, 0, 1.0};
     if (launch_reduce_partials(jobs, nj, s->n, s->st)) return -1;
-    return launch_tea_close(s->pos, X, s->Feff, s->Cs, s->Pe, pair_eparts(s->N), s->N, s->preDii, dt, s->bt,
+    return launch_tea_close(s->pos, X, s->Feff, s->Cs, s->Pe, pair_eparts(s->N, s->ewald), s->N, s->preDii, dt, s->bt,
                             s->Rs, s->st);
 }
 
@@ -1016,7 +1016,7 @@ static int create_impl(const bdh_config* cfg, int N, const double* coord, const 
     if (s->tea) {
         if (dmalloc(&s->Px, sizeof(double) * s->n * s->msplits)) return -1;
         if (dmalloc(&s->Pc, sizeof(double) * s->n * s->msplits)) return -1;
-        if (dmalloc(&s->Pe, sizeof(double) * pair_eparts(N))) return -1;
+        if (dmalloc(&s->Pe, sizeof(double) * pair_eparts(N, s->ewald))) return -1;
         if (dmalloc(&s->Feff, sizeof(double) * s->n)) return -1;
         if (dmalloc(&s->Cs, sizeof(double) * s->n)) return -1;
         if (dmalloc(&s->bt, sizeof(double) * 2)) return -1;
@@ -2383,7 +2383,7 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
         return acc <= (long long)INT32_MAX ? (int)acc : -1;
     };
     b->plan.asm_blocks = fill(0, [](const BatchChain& h) { return rpy_blocks(h.N); });
-    b->plan.pair_blocks = fill(1, [](const BatchChain& h) { return pair_eparts(h.N); });
+    b->plan.pair_blocks = fill(1, [](const BatchChain& h) { return pair_eparts(h.N, false); });
     b->plan.force_blocks = fill(2, [](const BatchChain& h) { return force_blocks(h.N); });
     b->plan.trmv_blocks = b->mixed ? fill(3, [](const BatchChain& h) { return trmv_blocks<float>(h.n); })
                                    : fill(3, [](const BatchChain& h) { return trmv_blocks<double>(h.n); });

@@ -89,8 +89,8 @@ int launch_rpy_assemble_batch(const double4* d_pos, double preDii, double preDij
 // ---- pair sums, Ewald, TEA (bdh_pairs.hip)
 int ewald_upload(double box, int R, int method, double alpha_smith, double alpha_scale, int R_real,
                  int R_recip, double r_cut);
-int pair_splits(int N, bool ewald);   // row partials per bead: one per 64-bead tile
-int pair_eparts(int N);                // eps partials of the TEA sums: one per tile pair
+int pair_splits(int N, bool ewald);   // row partials per bead
+int pair_eparts(int N, bool ewald);   // workgroups and eps partials (TEA) of the pair sums
 // d_pos2 (TEA only): the sums of the mean tensor (D(pos2) + D(pos)) / 2 (the IG-T corrector).
 template <typename T>
 int launch_pair_sums(const double4* d_pos, const double* d_F, const double* d_xi, int N,
@@ -104,7 +104,7 @@ int launch_pair_sums_batch(const double4* d_pos, const double* d_F, double preDi
 template <typename T>
 int launch_ewald_assemble(const double4* d_pos, int N, double preDii, double preDij, T* d_A,
                           long long ld, hipStream_t st, const double4* d_pos2 = nullptr);
-// S = pair_eparts(N) eps partials in d_Pe
+// S = pair_eparts eps partials in d_Pe
 int launch_tea_close(const double4* d_pos, const double* d_xi, const double* d_Feff,
                      const double* d_C, const double* d_Pe, int S, int N, double preDii, double dt,
                      double* d_bt, double* d_Rs, hipStream_t st);

@@ -26,9 +26,8 @@ namespace bdh {
 
 // ------------------------------------------------------------------ Ewald tables
 __constant__ EwaldTables c_ew;
-__constant__ double4 c_recip[EW_MAXV];
-__constant__ double c_recip_z[EW_MAXV];
-__constant__ double c_recip_w[EW_MAXV];
+__constant__ RecipClass c_recip[EW_MAXV];
+__constant__ ImageCoef c_img = IMAGE_COEF;
 
 // Method of the tables last uploaded (the launchers pick the matching instantiation; every
 // launch is preceded by an upload check for the calling system).
@@ -43,11 +42,7 @@ int ewald_upload(double box, int R, int method, double alpha_smith, double alpha
     if (!ext) R_real = R_recip = R;
     BDH_CHECK(method == EW_BEENAKKER || !ext, "Ewald: a split of its own only for the Beenakker sums");
     BDH_CHECK(R_real >= 0 && R_real <= 5 && R_recip >= 0 && R_recip <= 5, "Ewald split: radii 0..5");
-    R = R_real > R_recip ? R_real : R_recip;
     EwaldTables t{};
-    int nv = 0;
-    std::vector<double4> rec;
-    std::vector<double> recz, recw;
     t.method = method;
     t.box = box;
     t.inv_L = 1.0 / box;
@@ -60,29 +55,28 @@ int ewald_upload(double box, int R, int method, double alpha_smith, double alpha
     t.alpha2 = t.alpha * t.alpha;
     t.alpha3 = t.alpha * t.alpha2;
     t.inv_alpha2 = 1.0 / t.alpha2;
-    t.preQ = t.inv_L * t.inv_L * t.inv_L;
+    t.phase = 2.0 * PI_F / M_PI * t.inv_L;
     t.preO = 0.75 * t.inv_L;
     t.self_a = -6.0 * t.alpha / SQRTPI;
     t.self_b = 40.0 * t.alpha3 / (3.0 * SQRTPI);
+    const double inv_L3 = t.inv_L * t.inv_L * t.inv_L;
     // M_PI_ALPHA_SQ = -M_PIF * M_PIF / alpha2 with the product of the float pis in float
     // (diff_tensor.c:557)
     const float pif = 3.14159265358979323846f;
     const float mpp = -pif * pif;
     const double m_pi_alpha_sq = (double)mpp / t.alpha2;
-    if (method == EW_BEENAKKER) {
-        // the half sphere (h, f, g) > 0 lexicographically, |.|^2 <= R_recip^2, h then f then g
-        // ascending (beenakker_block's loop order), each vector standing for itself and its
-        // negative (2 G)
-        const int rk = R_recip * R_recip;
-        bool any = false;
-        for (int h = 0; h * h <= rk; ++h) {
-            const int nf = (int)std::sqrt((double)(rk - h * h));
-            for (int f = (h == 0 ? 0 : -nf); f <= nf; ++f) {
-                const int ng = (int)std::sqrt((double)(rk - h * h - f * f));
-                for (int g = (h == 0 && f == 0 ? 1 : -ng); g <= ng; ++g) {
-                    ++nv;
-                    const double s = (double)(h * h + f * f + g * g);
-                    const double nrm = std::sqrt(s);
+    // one class per (h, f, g) >= 0 but (0, 0, 0), |.|^2 <= R_recip^2, h then f then g ascending
+    const int rk = R_recip * R_recip;
+    std::vector<RecipClass> rec;
+    bool any = false;
+    for (int h = 0; h <= R_recip; ++h)
+        for (int f = 0; f <= R_recip; ++f)
+            for (int g = 0; g <= R_recip; ++g) {
+                const int sq = h * h + f * f + g * g;
+                if (sq == 0 || sq > rk) continue;
+                const double s = (double)sq, nrm = std::sqrt(s), members = (h ? 2 : 1) * (f ? 2 : 1) * (g ? 2 : 1);
+                RecipClass k{};
+                if (method == EW_BEENAKKER) {
                     // The reference forms k = 2 pi (h, f, g) in box units (diff_tensor.c:372-376)
                     // against alpha and sigma in A, so its reciprocal terms underflow to zero for
                     // any box of more than a few A; the extension takes k = 2 pi (h, f, g) / L,
@@ -91,57 +85,38 @@ int ewald_upload(double box, int R, int method, double alpha_smith, double alpha
                     const double six_pi = ext ? 6.0 * M_PI : 6.0 * PI_F;
                     const double G = (1.0 + (t.inv_alpha2 * k2 / 4.0) * (1.0 + t.inv_alpha2 * k2 / 2.0)) *
                                      (six_pi * std::exp(-t.inv_alpha2 * k2 / 4.0) / k2);
-                    any = any || G != 0.0;
-                    rec.push_back(make_double4(2.0 * G, k2 / 3.0, h / nrm, f / nrm));
-                    recz.push_back(g / nrm);
-                    recw.push_back(0.0);
+                    k.u0 = members * inv_L3 * G;
+                    k.u1 = -k.u0 * (k2 / 3.0);
+                    k.w0 = -k.u0;
+                    k.w1 = -k.u1;
+                } else {
+                    // diff_tensor.c:199-225
+                    const double ex = std::exp(m_pi_alpha_sq * s);
+                    k.u0 = members * t.preO * (2.0 * ex / ((double)pif * s));
+                    k.w0 = k.u0 * (-1.0 + m_pi_alpha_sq * s);
+                    k.w1 = members * 0.5 * inv_L3 * (4.0 * (double)pif * ex);
                 }
+                any = any || k.u0 != 0.0 || k.w1 != 0.0;
+                const double e[3] = {h / nrm, f / nrm, g / nrm};
+                k.e[0] = e[0] * e[0];
+                k.e[1] = e[1] * e[1];
+                k.e[2] = e[2] * e[2];
+                k.e[3] = e[0] * e[1];
+                k.e[4] = e[0] * e[2];
+                k.e[5] = e[1] * e[2];
+                rec.push_back(k);
             }
-        }
-        t.RR_recip = rk;
-        t.nrecip = any ? nv : 0;
-    } else {
-        const int rr = R * R;
-        for (int h = -R; h <= R; ++h) {
-            const int nf = (int)std::sqrt((double)(rr - h * h));
-            for (int f = -nf; f <= nf; ++f) {
-                const int ng = (int)std::sqrt((double)(rr - h * h - f * f));
-                for (int g = -ng; g <= ng; ++g) {
-                    ++nv;
-                    const double s = (double)(h * h + f * f + g * g);
-                    if (s == 0.0) {
-                        rec.push_back(make_double4(0, 0, 0, 0));
-                        recz.push_back(0.0);
-                        recw.push_back(0.0);
-                        continue;
-                    }
-                    // diff_tensor.c:199-225; e = (h, f, g) / |.| as get_ev2_norms forms it
-                    const double nrm = std::sqrt(s);
-                    const double inv = 1.0 / nrm;
-                    const double ex = h * inv, ey = f * inv, ez = g * inv;
-                    const double G1 = 2.0 * std::exp(m_pi_alpha_sq * s) / ((double)pif * s);
-                    rec.push_back(make_double4(G1, -1.0 + m_pi_alpha_sq * s, ex, ey));
-                    recz.push_back(ez);
-                    recw.push_back(4.0 * (double)pif * std::exp(m_pi_alpha_sq * s));
-                }
-            }
-        }
-    }
-    t.nv = nv;
-    t.R = R;
+    t.RR_recip = rk;
+    t.nrecip = any ? (int)rec.size() : 0;
     t.RR_real = R_real * R_real;
     t.min_image = ext ? 1 : 0;
     BDH_CHECK(r_cut <= 0.0 || ext, "Ewald: a real-space cutoff only for the extension split");
     t.rc2 = r_cut > 0.0 ? r_cut * r_cut : 1e300;
-    BDH_CHECK(t.nv <= EW_MAXV, "Ewald table overflow");
+    BDH_CHECK((int)rec.size() <= EW_MAXV, "Ewald table overflow");
     BDH_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_ew), &t, sizeof(t)));
-    if (!rec.empty()) {
-        BDH_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_recip), rec.data(), sizeof(double4) * rec.size()));
-        BDH_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_recip_z), recz.data(), sizeof(double) * recz.size()));
-        BDH_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_recip_w), recw.data(), sizeof(double) * recw.size()));
-    }
+    if (!rec.empty()) BDH_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_recip), rec.data(), sizeof(RecipClass) * rec.size()));
     g_uploaded_method = method;
-    return t.nv;
+    return (int)rec.size();
 }
 
 // ------------------------------------------------------------------ blocks
@@ -212,17 +187,34 @@ __device__ __forceinline__ Blk6 pair_block(const double4& pi, const double4& pj,
 // every row is written exactly once, so the partials need no clearing.  The eps sums of
 // the workgroup (each unordered pair i != j counted twice, as from both rows) are reduced
 // into Pe[b].
+// With S > 1 a tile pair's shifts are dealt out to S workgroups (workgroup b takes tile pair b / S
+// and every S-th group of four shifts from 4 (b % S) on), whose sums land in splits of their own,
+// S J + b % S and S I + b % S.
 constexpr int PS_TILE = 64;
+constexpr int PS_MAX_SUB = PS_TILE / 4;   // then every wavefront has one shift
 
-int pair_splits(int N, bool) { return ceil_div(N, PS_TILE); }
-int pair_eparts(int N) { const int t = ceil_div(N, PS_TILE); return t * (t + 1) / 2; }
+// Workgroups per tile pair: with Ewald blocks a shift takes a wavefront 10 us and more, so the tile
+// pairs of a small system are split until there are PS_WORKGROUPS workgroups, two per CU
+// (N = 343 FP64 Smith: 21 workgroups 223 us, 336 24 us; N = 1100 FP64 Beenakker: 171 workgroups
+// 201 us, 684 130 us, 1368 130 us and twice the partial rows).  A free-space shift takes less than
+// the few hundred ns a workgroup spends on its LDS sums: no split.
+constexpr int PS_WORKGROUPS = 512;
+static int pair_sub(int N, bool ewald)
+{
+    const int t = ceil_div(N, PS_TILE);
+    int S = 1;
+    while (ewald && S < PS_MAX_SUB && (long long)S * t * (t + 1) / 2 < PS_WORKGROUPS) S *= 2;
+    return S;
+}
+int pair_splits(int N, bool ewald) { return ceil_div(N, PS_TILE) * pair_sub(N, ewald); }
+int pair_eparts(int N, bool ewald) { const int t = ceil_div(N, PS_TILE); return t * (t + 1) / 2 * pair_sub(N, ewald); }
 
 template <typename T, int EW, bool TEA, bool MEAN = false>
 __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, const double* __restrict__ F,
                                                const double* __restrict__ xi, int N, double preDii,
                                                double preDij, double dt, double* __restrict__ Pf,
                                                double* __restrict__ Px, double* __restrict__ Pc,
-                                               double* __restrict__ Pe, int b,
+                                               double* __restrict__ Pe, int wg, int S,
                                                const double4* __restrict__ pos2 = nullptr)
 {
     constexpr int NV = TEA ? 10 : 3;
@@ -233,6 +225,7 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
     __shared__ double s_col[4][NV][PS_TILE];
     __shared__ double s_row[4][NV][PS_TILE];
     const int t = threadIdx.x, w = threadIdx.y, tid = w * PS_TILE + t;
+    const int b = wg / S, sub = wg - b * S;
     int J = (int)((sqrt(8.0 * b + 1.0) - 1.0) * 0.5);
     while (J * (J + 1) / 2 > b) --J;
     while ((J + 1) * (J + 2) / 2 <= b) ++J;
@@ -274,7 +267,7 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
     double acc[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) acc[v] = 0.0;
-    for (int sh = w; sh < PS_TILE; sh += 4) {
+    for (int sh = w + 4 * sub; sh < PS_TILE; sh += 4 * S) {
         const int jl = (t + sh) & (PS_TILE - 1);
         if (!iv || j0 + jl >= N) continue;
         const bool self = diag && sh == 0;
@@ -332,7 +325,7 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
     __syncthreads();
 #define sum4(a, v) (((a)[0][v][t] + (a)[1][v][t]) + ((a)[2][v][t] + (a)[3][v][t]))
     if (w == 0 && iv) {
-        const long long o = (long long)J * 3 * N + 3 * i;
+        const long long o = (long long)(J * S + sub) * 3 * N + 3 * i;
 #pragma unroll
         for (int k = 0; k < 3; ++k) Pf[o + k] = sum4(s_row, k);
         if constexpr (TEA) {
@@ -344,7 +337,7 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
         }
     }
     if (w == 1 && !diag && j0 + t < N) {
-        const long long o = (long long)I * 3 * N + 3 * (j0 + t);
+        const long long o = (long long)(I * S + sub) * 3 * N + 3 * (j0 + t);
 #pragma unroll
         for (int k = 0; k < 3; ++k) Pf[o + k] = sum4(s_col, k);
         if constexpr (TEA) {
@@ -360,20 +353,20 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
             double e = sum4(s_row, 9);
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
-            if (t == 0) Pe[b] = diag ? e : 2.0 * e;
+            if (t == 0) Pe[wg] = diag ? e : 2.0 * e;
         }
     }
 #undef sum4
 }
 
 template <typename T, int EW, bool TEA, bool MEAN = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8)))
 pair_sums_kernel(const double4* __restrict__ pos, const double* __restrict__ F,
                  const double* __restrict__ xi, int N, double preDii, double preDij, double dt,
                  double* __restrict__ Pf, double* __restrict__ Px, double* __restrict__ Pc,
-                 double* __restrict__ Pe, const double4* __restrict__ pos2)
+                 double* __restrict__ Pe, int S, const double4* __restrict__ pos2)
 {
-    pair_sums_body<T, EW, TEA, MEAN>(pos, F, xi, N, preDii, preDij, dt, Pf, Px, Pc, Pe, blockIdx.x, pos2);
+    pair_sums_body<T, EW, TEA, MEAN>(pos, F, xi, N, preDii, preDij, dt, Pf, Px, Pc, Pe, blockIdx.x, S, pos2);
 }
 
 // Free-space D.F of every chain of a batch: workgroup x of chain c is the chain's tile pair x.
@@ -386,7 +379,7 @@ pair_sums_batch_kernel(const double4* __restrict__ pos, const double* __restrict
     const int c = batch_find(prefix, nch, blockIdx.x);
     const BatchChain bc = ch[c];
     pair_sums_body<T, 0, false>(pos + bc.bead0, F + 3LL * bc.bead0, nullptr, bc.N, preDii, preDij, 0.0,
-                                Pp + bc.pp, nullptr, nullptr, nullptr, blockIdx.x - prefix[c]);
+                                Pp + bc.pp, nullptr, nullptr, nullptr, blockIdx.x - prefix[c], 1);
 }
 
 template <typename T>
@@ -407,14 +400,15 @@ int launch_pair_sums(const double4* d_pos, const double* d_F, const double* d_xi
 {
     BDH_CHECK(splits == pair_splits(N, ewald), "launch_pair_sums: split count");
     BDH_CHECK(!d_pos2 || tea, "launch_pair_sums: the mean tensor only for TEA sums");
-    const dim3 grid(pair_eparts(N)), blk(PS_TILE, 4);
+    const int S = pair_sub(N, ewald);
+    const dim3 grid(pair_eparts(N, ewald)), blk(PS_TILE, 4);
     const int ew = ewald ? (g_uploaded_method == EW_SMITH ? 2 : 1) : 0;
 #define PS_LAUNCH(E, TE)                                                                          \
     hipLaunchKernelGGL((pair_sums_kernel<T, E, TE>), grid, blk, 0, st, d_pos, d_F, d_xi, N, preDii, \
-                       preDij, dt, d_Pf, d_Px, d_Pc, d_Pe, (const double4*)nullptr)
+                       preDij, dt, d_Pf, d_Px, d_Pc, d_Pe, S, (const double4*)nullptr)
 #define PS_MEAN(E)                                                                                 \
     hipLaunchKernelGGL((pair_sums_kernel<T, E, true, true>), grid, blk, 0, st, d_pos, d_F, d_xi, N, \
-                       preDii, preDij, dt, d_Pf, d_Px, d_Pc, d_Pe, d_pos2)
+                       preDii, preDij, dt, d_Pf, d_Px, d_Pc, d_Pe, S, d_pos2)
     if (d_pos2) {
         if (ew == 1) PS_MEAN(1);
         else if (ew == 2) PS_MEAN(2);
@@ -462,40 +456,36 @@ int launch_single_block(const double4* d_pos, int i, int j, int ew, double preDi
 
 // ------------------------------------------------------------------ Ewald assembly
 // Lower triangle of the Beenakker-Ewald D (rows of i, columns of j, i >= j), the same
-// tiling as the free-space assembly: (64 row beads) x (16 column beads) per workgroup.
+// (64 row beads) x (4 column beads) per workgroup, one block per thread: a block is hundreds to
+// thousands of operations, so what counts is to have a wavefront for every SIMD (N = 343: 516
+// workgroups; with four blocks per thread and 132 workgroups 59 us FP64 Smith, so 26 us).
 // With pos2, the mean of the blocks at pos and pos2 (the IG-T tensor).  EW as pair_block.
 template <typename T, int EW>
 __global__ void __launch_bounds__(256)
 ewald_assemble_kernel(const double4* __restrict__ pos, const double4* __restrict__ pos2, int N,
                       double preDii, double preDij, T* __restrict__ A, long long ld)
 {
-    const int i0 = blockIdx.x * 64, j0 = blockIdx.y * 16;
-    if (j0 > i0 + 63) return;
-    const int i = i0 + threadIdx.x;
-    if (i >= N) return;
+    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+    if (i >= N || j > i) return;
     const double4 pi = pos[i];
-    for (int q = 0; q < 4; ++q) {
-        const int j = j0 + threadIdx.y * 4 + q;
-        if (j >= N || j > i) continue;
-        Blk6 B = pair_block<T, EW>(pi, pos[j], i == j, preDii, preDij);
-        if (pos2 && i != j) {
-            const double4 qi = pos2[i], qj = pos2[j];
-            const Blk6 B2 = pair_block<T, EW>(qi, qj, false, preDii, preDij);
-            B.xx = (B.xx + B2.xx) / 2; B.yy = (B.yy + B2.yy) / 2; B.zz = (B.zz + B2.zz) / 2;
-            B.xy = (B.xy + B2.xy) / 2; B.xz = (B.xz + B2.xz) / 2; B.yz = (B.yz + B2.yz) / 2;
-        }
-        T* c0 = A + (long long)(3 * j) * ld + 3 * i;
-        c0[0] = (T)B.xx; c0[1] = (T)B.xy; c0[2] = (T)B.xz;
-        c0[ld] = (T)B.xy; c0[ld + 1] = (T)B.yy; c0[ld + 2] = (T)B.yz;
-        c0[2 * ld] = (T)B.xz; c0[2 * ld + 1] = (T)B.yz; c0[2 * ld + 2] = (T)B.zz;
+    Blk6 B = pair_block<T, EW>(pi, pos[j], i == j, preDii, preDij);
+    if (pos2 && i != j) {
+        const double4 qi = pos2[i], qj = pos2[j];
+        const Blk6 B2 = pair_block<T, EW>(qi, qj, false, preDii, preDij);
+        B.xx = (B.xx + B2.xx) / 2; B.yy = (B.yy + B2.yy) / 2; B.zz = (B.zz + B2.zz) / 2;
+        B.xy = (B.xy + B2.xy) / 2; B.xz = (B.xz + B2.xz) / 2; B.yz = (B.yz + B2.yz) / 2;
     }
+    T* c0 = A + (long long)(3 * j) * ld + 3 * i;
+    c0[0] = (T)B.xx; c0[1] = (T)B.xy; c0[2] = (T)B.xz;
+    c0[ld] = (T)B.xy; c0[ld + 1] = (T)B.yy; c0[ld + 2] = (T)B.yz;
+    c0[2 * ld] = (T)B.xz; c0[2 * ld + 1] = (T)B.yz; c0[2 * ld + 2] = (T)B.zz;
 }
 
 template <typename T>
 int launch_ewald_assemble(const double4* d_pos, int N, double preDii, double preDij, T* d_A,
                           long long ld, hipStream_t st, const double4* d_pos2)
 {
-    dim3 grid(ceil_div(N, 64), ceil_div(N, 16));
+    dim3 grid(ceil_div(N, 64), ceil_div(N, 4));
     if (g_uploaded_method == EW_SMITH)
         hipLaunchKernelGGL((ewald_assemble_kernel<T, 2>), grid, dim3(64, 4), 0, st, d_pos, d_pos2, N,
                            preDii, preDij, d_A, ld);
