@@ -43,6 +43,34 @@ __global__ void diag_mobility_kernel(const double4* __restrict__ pos, const doub
     if (Rs) Rs[r] = xi[r] * sqrt(dii * 2.0 * dt);
 }
 
+// diag_mobility_kernel and em_update_kernel (without a flow field) in one launch: entry r moves
+// component r % 3 of bead r / 3.  Rf and Rs are rounded as stored before they meet the
+// coordinate, so all three are bitwise those of the two launches.
+__global__ void free_move_kernel(double* __restrict__ pos, const double* __restrict__ F,
+                                 const double* __restrict__ xi, int N, double preDii, double dt, double rf_scale,
+                                 double* __restrict__ Rf, double* __restrict__ Rs, int pbc, double box)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= 3 * N) return;
+    double* q = pos + 4LL * (r / 3);
+    const double dii = preDii / q[3];
+    double rf, rs;
+    {
+#pragma clang fp contract(off)
+        rf = rf_scale * dii * F[r];
+        rs = xi[r] * sqrt(dii * 2.0 * dt);
+    }
+    Rf[r] = rf;
+    Rs[r] = rs;
+    q += r % 3;
+    double x = (rf + rs) + *q;
+    if (pbc) {
+        const double inv = 1.0 / box;
+        x -= box * floor(x * inv + 0.5);
+    }
+    *q = x;
+}
+
 // The TEA pair sums of a large periodic system over beads in a space-filling-curve order
 // perm: pos_s[i] = pos[perm[i]] (pos2 alike), F_s and X_s the 3-vectors alike.  A 64-bead tile
 // is then a compact region, and a wavefront evaluates few real-space images beyond those its
@@ -262,11 +290,13 @@ int alloc_cells(bdh_system* s)
 {
     if (s->cl.grid) return 0;
     if (dmalloc(&s->cl.grid, cell_grid_bytes())) return -1;
-    if (dmalloc(&s->cl.key, sizeof(int) * s->N)) return -1;
+    if (dmalloc(&s->cl.key, sizeof(int) * 4 * ceil_div(s->N, 4))) return -1;
     if (dmalloc(&s->cl.count, sizeof(int) * CELL_MAX)) return -1;
     if (dmalloc(&s->cl.fill, sizeof(int) * CELL_MAX)) return -1;
     if (dmalloc(&s->cl.start, sizeof(int) * (CELL_MAX + 1))) return -1;
+    if (dmalloc(&s->cl.list, sizeof(int) * s->N)) return -1;
     if (dmalloc(&s->cl.sorted, sizeof(int) * s->N)) return -1;
+    if (dmalloc(&s->cl.pos, sizeof(double4) * s->N)) return -1;
     return 0;
 }
 
@@ -515,10 +545,17 @@ int one_step(bdh_system* s, const double* xi_dev, const double* Rs_dev, double d
         REC_END(PH_MOVE);
     } else {
         REC_BEGIN(PH_MOVE);
-        hipLaunchKernelGGL(diag_mobility_kernel, dim3(ceil_div(s->n, 256)), dim3(256), 0, s->st,
-                           s->pos, s->F, xi_dev, s->N, s->preDii, dt, rf_scale, s->Rf, s->Rs);
-        BDH_LAUNCH_CHECK();
-        if (launch_em_update(s->pos, s->N, s->Rf, s->Rs, c.bc == 1, c.box, s->st, &fl)) return -1;
+        if (s->flow) {
+            hipLaunchKernelGGL(diag_mobility_kernel, dim3(ceil_div(s->n, 256)), dim3(256), 0, s->st,
+                               s->pos, s->F, xi_dev, s->N, s->preDii, dt, rf_scale, s->Rf, s->Rs);
+            BDH_LAUNCH_CHECK();
+            if (launch_em_update(s->pos, s->N, s->Rf, s->Rs, c.bc == 1, c.box, s->st, &fl)) return -1;
+        } else {
+            hipLaunchKernelGGL(free_move_kernel, dim3(ceil_div(s->n, 256)), dim3(256), 0, s->st,
+                               reinterpret_cast<double*>(s->pos), (const double*)s->F, xi_dev, s->N, s->preDii, dt,
+                               rf_scale, s->Rf, s->Rs, c.bc == 1, c.box);
+            BDH_LAUNCH_CHECK();
+        }
         REC_END(PH_MOVE);
     }
     if (compute_forces_dev(s)) return -1;
@@ -857,7 +894,7 @@ void bdh_destroy(bdh_system* s)
     dfree(s->Rf_s); dfree(s->Rs_s); dfree(s->rng); dfree(s->rng_off); dfree(s->rng_cnt); dfree(s->gwork); dfree(s->flags);
     dfree(s->Px); dfree(s->Pc); dfree(s->Pe); dfree(s->Feff); dfree(s->Cs); dfree(s->bt);
     dfree(s->cl.grid); dfree(s->cl.key); dfree(s->cl.count); dfree(s->cl.fill);
-    dfree(s->cl.start); dfree(s->cl.sorted);
+    dfree(s->cl.start); dfree(s->cl.list); dfree(s->cl.sorted); dfree(s->cl.pos);
     if (s->factor_exec) (void)hipGraphExecDestroy(s->factor_exec);
     dfree(s->adj);
     dfree(s->fcache);

@@ -181,7 +181,9 @@ struct CellList {
     int* count;     // CELL_MAX
     int* fill;      // CELL_MAX
     int* start;     // CELL_MAX + 1
+    int* list;      // N: bead indices grouped by cell (scratch of the build)
     int* sorted;    // N: bead indices grouped by cell, ascending within a cell
+    double4* pos;   // N: their positions
 };
 size_t cell_grid_bytes();
 int launch_cell_build(const double4* d_pos, int N, double cutoff, int pbc, double box,
