@@ -409,9 +409,11 @@ __device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long
 // overlaps with everything else, since the workgroups of the following tile columns are
 // resident and accumulate what is already published.
 // Measured against one launch per 256-column outer panel (n_pad >= 1024) or per 64-column panel
-// (below), right-looking: n = 768 FP64 640 -> 220 us, n = 1353 FP32 720 -> 333 us, n = 3072 FP64
-// 1900 -> 925 us, n = 9000 FP32 5.95 -> 3.98 ms, FP64 11.3 -> 7.5 ms; the batch of 256 chains of
-// 64 .. 1024 beads FP32 6.9 -> 5.7 ms.
+// (below), right-looking: n = 768 FP64 640 -> 210 us, n = 1353 FP32 720 -> 331 us, n = 3072 FP64
+// 1900 -> 856 us, n = 9000 FP32 5.95 -> 2.81 ms, FP64 11.3 -> 5.0 ms; the batch of 256 chains of
+// 64 .. 1024 beads FP32 6.9 -> 4.4 ms.  Beside another tile on its CU a tile takes 13.4 us for 128
+// columns in FP32 and 28.7 in FP64, MFMA issue at its peak; the rest at n = 9000 is the chain (31
+// us per tile column FP32, 36 FP64) and tiles that become resident too late to have caught up.
 //
 // Visibility across XCDs, whose L2 caches are not coherent within a launch: what other
 // workgroups read is stored at agent scope (write-through), the flag that announces it is set
@@ -438,6 +440,7 @@ struct FlowMat {
     int n, nt;   // order (without the identity padding), tile rows
     double* ws;
     int* status;
+    int* quiet;  // FLOW_CUS counters (FlowQuiet), or null
     __device__ int* dprog(int j) const { return flags() + j * FLAG_STRIDE; }
     __device__ int* rdy(int i) const { return flags() + (nt + i) * FLAG_STRIDE; }
     __device__ int* flags() const { return reinterpret_cast<int*>(ws + (long long)nt * FLOW_COL); }
@@ -483,6 +486,39 @@ __device__ __forceinline__ int flow_wait(int* flag, int need, int* status)
     return __builtin_amdgcn_readfirstlane(v);
 }
 
+// The chain's steps are a serial FP64 chain on one wavefront and short MFMA solves.  Beside the
+// MFMAs of another workgroup on the same CU, none of which can be interrupted, a diagonal block
+// takes 20 .. 27 us instead of 10 and a solve 9 instead of 6, and the whole factorization waits.  So
+// the workgroups of tiles (j, j) and (j + 1, j) count themselves on their CU's counter while they
+// take those steps, and a workgroup further below the diagonal pauses its accumulation, between
+// two stages, while its CU's counter is not zero.  A workgroup counts itself only once what it
+// still waits for comes from workgroups that are past their accumulation (or none is left to wait
+// for), so a paused one is never waited for.
+// Only where workgroups share CUs, that is with more tiles than the chip's 256 CUs (us without /
+// with, FP32 and FP64): n = 3072 737 / 735, 861 / 856; 4500 1175 / 1103, 1413 / 1318; 6000 1606 /
+// 1467, 2111 / 1917; 9000 3087 / 2808, 5092 / 5009.
+constexpr int FLOW_CUS = 2048;
+constexpr int QUIET_TILES = 256;
+struct FlowQuiet {
+    int* q;
+    __device__ explicit FlowQuiet(int* quiet)
+    {
+        // HW_ID bits 8 .. 15: CU and shader array of the XCD; XCC_ID: the XCD
+        q = quiet ? quiet + ((__builtin_amdgcn_s_getreg(20 | (2 << 11)) << 8) | __builtin_amdgcn_s_getreg(4 | (8 << 6) | (7 << 11)))
+                  : nullptr;
+    }
+    __device__ void add(int v)
+    {
+        if (q && threadIdx.x == 0) __hip_atomic_fetch_add(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ int busy() const { return q ? __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0; }
+    __device__ void pause() const
+    {
+        const long long t0 = wall_clock64();
+        while (busy() && wall_clock64() - t0 < FLOW_TIMEOUT) __builtin_amdgcn_s_sleep(8);
+    }
+};
+
 // Panels known to be published in two tile rows (the same row twice for a diagonal tile).
 struct FlowReady {
     int *fi, *fj, *status;
@@ -525,10 +561,14 @@ struct FlowAcc<double> {
     doublex4 a[8][2];
 };
 
-// Sums over the K columns 0 .. K - 1 (K a multiple of 128) of tile (i, j) into acc.
+// Sums over the K columns 0 .. K - 1 (K a multiple of 128) of tile (i, j) into acc.  The next
+// stage's columns are in registers while this one's are multiplied (ext_vector_type elements: an
+// array of HIP's own vector class, loaded under a condition, went through scratch memory and each
+// load was waited for at once), and the LDS reads of a product are issued before the MFMAs of the
+// one before: 22.6 -> 13.4 us per 128 columns FP32, 46.5 -> 28.7 FP64.
 template <bool SPLIT>
 __device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, int j, int K, FlowReady& rd,
-                                                unsigned char* smem, FlowAcc<float>& acc)
+                                                const FlowQuiet& quiet, unsigned char* smem, FlowAcc<float>& acc)
 {
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -581,6 +621,7 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, 
             __syncthreads();
             const bool more = c + 1 < nc;
             const bool pre = more && rd.poll(need(c + 1));
+            const int busy = quiet.busy();
             if (pre) load(c + 1);
 #pragma unroll
             for (int t = 0; t < FLOW_KC32 / 16; ++t) {
@@ -596,6 +637,7 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, 
                     acc.a[q] = mfma_bf16_32x32x16(ah, bh, acc.a[q]);
                 }
             }
+            if (busy) quiet.pause();
             if (more && !pre) {
                 rd.wait(need(c + 1));
                 load(c + 1);
@@ -606,22 +648,22 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, 
     } else {
         float (*st)[2][FLOW_KC32][FLOW_P32] = reinterpret_cast<float (*)[2][FLOW_KC32][FLOW_P32]>(smem);
         constexpr int NV = FLOW_KC32 * FLOW_T / 4 / 256;
-        float4 vj[NV], vi[NV];
+        floatx4 vj[NV], vi[NV];
         auto load = [&](int c) {
             const float *pj = M.opnd(j, c * FLOW_KC32), *pi = M.opnd(i, c * FLOW_KC32);
 #pragma unroll
             for (int u = 0; u < NV; ++u) {
                 const int idx = tid + 256 * u, k = idx / (FLOW_T / 4), r = (idx % (FLOW_T / 4)) * 4;
-                vj[u] = *reinterpret_cast<const float4*>(pj + (long long)k * M.ld + r);
-                vi[u] = *reinterpret_cast<const float4*>(pi + (long long)k * M.ld + r);
+                vj[u] = *reinterpret_cast<const floatx4*>(pj + (long long)k * M.ld + r);
+                vi[u] = *reinterpret_cast<const floatx4*>(pi + (long long)k * M.ld + r);
             }
         };
         auto store = [&](int b) {
 #pragma unroll
             for (int u = 0; u < NV; ++u) {
                 const int idx = tid + 256 * u, k = idx / (FLOW_T / 4), r = (idx % (FLOW_T / 4)) * 4;
-                *reinterpret_cast<float4*>(&st[b][0][k][r]) = vj[u];
-                *reinterpret_cast<float4*>(&st[b][1][k][r]) = vi[u];
+                *reinterpret_cast<floatx4*>(&st[b][0][k][r]) = vj[u];
+                *reinterpret_cast<floatx4*>(&st[b][1][k][r]) = vi[u];
             }
         };
         rd.wait(need(0));
@@ -631,17 +673,24 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, 
         for (int c = 0; c < nc; ++c) {
             const bool more = c + 1 < nc;
             const bool pre = more && rd.poll(need(c + 1));
+            const int busy = quiet.busy();
             if (pre) load(c + 1);
             float (*sj)[FLOW_P32] = st[c & 1][0], (*si)[FLOW_P32] = st[c & 1][1];
-#pragma unroll 4
-            for (int k = 0; k < FLOW_KC32; k += 2) {
-                const float b = si[k + lh][32 * w + l32];
-                float a[4];
+            float a[2][4], b[2];
+            auto fetch = [&](int s) {
+                b[s & 1] = si[2 * s + lh][32 * w + l32];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) a[q] = sj[k + lh][32 * q + l32];
+                for (int q = 0; q < 4; ++q) a[s & 1][q] = sj[2 * s + lh][32 * q + l32];
+            };
+            fetch(0);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc.a[q] = mfma_f32_32x32x2(a[q], b, acc.a[q]);
+            for (int s = 0; s < FLOW_KC32 / 2; ++s) {
+                if (s + 1 < FLOW_KC32 / 2) fetch(s + 1);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc.a[q] = mfma_f32_32x32x2(a[s & 1][q], b[s & 1], acc.a[q]);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if (busy) quiet.pause();
             if (more) {
                 if (!pre) {
                     rd.wait(need(c + 1));
@@ -657,7 +706,7 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, 
 
 template <bool SPLIT>
 __device__ __forceinline__ void flow_accumulate(const FlowMat<double>& M, int i, int j, int K, FlowReady& rd,
-                                                unsigned char* smem, FlowAcc<double>& acc)
+                                                const FlowQuiet& quiet, unsigned char* smem, FlowAcc<double>& acc)
 {
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -674,22 +723,22 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<double>& M, int i,
     auto need = [](int c) { return c * FLOW_KC64 / CHOL_NB + 1; };
     double (*st)[2][FLOW_KC64][FLOW_P64] = reinterpret_cast<double (*)[2][FLOW_KC64][FLOW_P64]>(smem);
     constexpr int NV = FLOW_KC64 * FLOW_T / 2 / 256;
-    double2 vj[NV], vi[NV];
+    doublex2 vj[NV], vi[NV];
     auto load = [&](int c) {
         const double *pj = M.opnd(j, c * FLOW_KC64), *pi = M.opnd(i, c * FLOW_KC64);
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
             const int idx = tid + 256 * u, k = idx / (FLOW_T / 2), r = (idx % (FLOW_T / 2)) * 2;
-            vj[u] = *reinterpret_cast<const double2*>(pj + (long long)k * M.ld + r);
-            vi[u] = *reinterpret_cast<const double2*>(pi + (long long)k * M.ld + r);
+            vj[u] = *reinterpret_cast<const doublex2*>(pj + (long long)k * M.ld + r);
+            vi[u] = *reinterpret_cast<const doublex2*>(pi + (long long)k * M.ld + r);
         }
     };
     auto store = [&](int b) {
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
             const int idx = tid + 256 * u, k = idx / (FLOW_T / 2), r = (idx % (FLOW_T / 2)) * 2;
-            *reinterpret_cast<double2*>(&st[b][0][k][r]) = vj[u];
-            *reinterpret_cast<double2*>(&st[b][1][k][r]) = vi[u];
+            *reinterpret_cast<doublex2*>(&st[b][0][k][r]) = vj[u];
+            *reinterpret_cast<doublex2*>(&st[b][1][k][r]) = vi[u];
         }
     };
     rd.wait(need(0));
@@ -699,20 +748,28 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<double>& M, int i,
     for (int c = 0; c < nc; ++c) {
         const bool more = c + 1 < nc;
         const bool pre = more && rd.poll(need(c + 1));
+        const int busy = quiet.busy();
         if (pre) load(c + 1);
         double (*sj)[FLOW_P64] = st[c & 1][0], (*si)[FLOW_P64] = st[c & 1][1];
+        double a[2][8], b[2][2];
+        auto fetch = [&](int s) {
+            const int k = 4 * s + lq;
 #pragma unroll
-        for (int k = 0; k < FLOW_KC64; k += 4) {
-            double a[8], b[2];
+            for (int g = 0; g < 2; ++g) b[s & 1][g] = si[k][32 * w + 16 * g + lr];
 #pragma unroll
-            for (int g = 0; g < 2; ++g) b[g] = si[k + lq][32 * w + 16 * g + lr];
+            for (int J = 0; J < 8; ++J) a[s & 1][J] = sj[k][16 * J + lr];
+        };
+        fetch(0);
 #pragma unroll
-            for (int J = 0; J < 8; ++J) a[J] = sj[k + lq][16 * J + lr];
+        for (int s = 0; s < FLOW_KC64 / 4; ++s) {
+            if (s + 1 < FLOW_KC64 / 4) fetch(s + 1);
 #pragma unroll
             for (int J = 0; J < 8; ++J)
 #pragma unroll
-                for (int g = 0; g < 2; ++g) acc.a[J][g] = mfma_f64_16x16x4(a[J], b[g], acc.a[J][g]);
+                for (int g = 0; g < 2; ++g) acc.a[J][g] = mfma_f64_16x16x4(a[s & 1][J], b[s & 1][g], acc.a[J][g]);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        if (busy) quiet.pause();
         if (more) {
             if (!pre) {
                 rd.wait(need(c + 1));
@@ -820,10 +877,12 @@ __device__ __forceinline__ void flow_tile(const FlowMat<T>& M, int i, int j, uns
     double* s1 = s0 + LB_STRIDE;                    // L21
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
     doublex4 z[8][2];
+    FlowQuiet quiet(i == j + 1 ? M.quiet : nullptr);
     {
         FlowAcc<T> acc;
         FlowReady rd{M.rdy(i), M.rdy(j), M.status};
-        flow_accumulate<SPLIT>(M, i, j, FLOW_T * j, rd, smem, acc);   // ends with a barrier
+        flow_accumulate<SPLIT>(M, i, j, FLOW_T * j, rd, FlowQuiet(i == j + 1 ? nullptr : M.quiet), smem, acc);   // ends with a barrier
+        quiet.add(1);   // all of row j is published: tile (j, j) is past its accumulation or about to be
         flow_negated(acc, reinterpret_cast<float*>(s1) + 2048 * (tid >> 6), z);
     }
     const double* ws = M.ws + (long long)j * FLOW_COL;
@@ -857,6 +916,7 @@ __device__ __forceinline__ void flow_tile(const FlowMat<T>& M, int i, int j, uns
     flow_solve64<2>(z, 4, s0, s0 + CHOL_NB * CHOL_NB);
     flow_store<T>(M, i, j, 4, z);
     flow_publish(M.rdy(i), 2 * j + 2);
+    quiet.add(-1);
 }
 
 // One 32x32 block of a diagonal tile on one wavefront, transposed as in FlowAcc: columns 32 mb ..,
@@ -983,6 +1043,7 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T>& M, int j, unsigned c
     const int m0 = w == 2 || w == 3 ? 1 : 0, n0 = w == 0 ? 0 : (w == 3 ? 2 : 1);
     const int m1 = w == 3 ? 1 : 0, n1 = w == 1 ? 2 : 3;
     const int m2 = w == 3 ? 3 : 2, n2 = w == 1 ? 2 : 3;
+    FlowQuiet quiet(M.quiet);
     FlowQuad<T> q0, q1, q2;
     q0.init(tl, M.ld, m0, n0, lane);
     if (w) {
@@ -1043,6 +1104,7 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T>& M, int j, unsigned c
             __syncthreads();
         }
         // the last 64 columns of rows 0 .. 63 through s1
+        quiet.add(1);   // tile (j, j - 1) has published its first panel
         rd.wait(2 * j);
         constexpr int NL = CHOL_NB * CHOL_NB / V / 256;
         vec x[NL];
@@ -1082,6 +1144,7 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T>& M, int j, unsigned c
     store_lkk(s0, ws);
     if (!second) {
         store_diag64<T>(s0, tl, M.ld, 0);
+        if (j > 0) quiet.add(-1);
         return;
     }
     // L21: 16 rows per wavefront
@@ -1116,6 +1179,7 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T>& M, int j, unsigned c
     });
     store_lkk(s0, ws + LB_STRIDE + CHOL_NB * CHOL_NB);
     flow_publish(M.dprog(j), 2);
+    if (j > 0) quiet.add(-1);
     store_diag64<T>(s0, tl, M.ld, CHOL_NB);
 }
 
@@ -1154,15 +1218,18 @@ int chol_factor(T* d_A, long long ld, int n, int n_pad, double* d_Lbuf, int* d_s
     BDH_CHECK(ld >= n_pad && ld % 4 == 0, "chol_factor: bad leading dimension");
     BDH_CHECK(syrk_mode != SYRK_BF16X3 || sizeof(T) == 4, "chol_factor: split SYRK needs FP32 storage");
     const int nt = n_pad / FLOW_T;
-    FlowMat<T> M{d_A, ld, n, nt, d_Lbuf, d_status};
     int* d_flags = reinterpret_cast<int*>(d_Lbuf + (long long)nt * FLOW_COL);
-    const int nflags = 2 * nt * FLAG_STRIDE;
+    int nflags = 2 * nt * FLAG_STRIDE;
+    const int tiles = nt * (nt + 1) / 2;
+    const bool shared = tiles > QUIET_TILES;
+    FlowMat<T> M{d_A, ld, n, nt, d_Lbuf, d_status, shared ? d_flags + nflags : nullptr};
+    if (shared) nflags += FLOW_CUS;
     if (rec) rec->begin(PH_PANEL, st);
     hipLaunchKernelGGL(chol_flow_clear_kernel, dim3(ceil_div(nflags, 256)), dim3(256), 0, st, d_flags, nflags);
     BDH_LAUNCH_CHECK();
     if (rec) rec->end(PH_PANEL, st);
     if (rec) rec->begin(PH_SYRK, st);
-    const dim3 grid(nt * (nt + 1) / 2);
+    const dim3 grid(tiles);
     if constexpr (sizeof(T) == 4) {
         if (syrk_mode == SYRK_BF16X3)
             hipLaunchKernelGGL((chol_flow_kernel<T, true>), grid, dim3(256), 0, st, M);
@@ -1179,7 +1246,7 @@ int chol_factor(T* d_A, long long ld, int n, int n_pad, double* d_Lbuf, int* d_s
 size_t chol_lbuf_doubles(int n_pad)
 {
     const size_t nt = n_pad / FLOW_T;
-    return nt * FLOW_COL + 2 * nt * FLAG_STRIDE / 2;
+    return nt * FLOW_COL + (2 * nt * FLAG_STRIDE + FLOW_CUS) / 2;
 }
 
 // ------------------------------------------------------------------ Y = L X (partials)
@@ -1348,7 +1415,7 @@ std::vector<FlowTask> chol_batch_tasks(const std::vector<int>& n_pad)
 template <typename T>
 __device__ __forceinline__ FlowMat<T> flow_mat(T* A, double* Lbuf, const BatchChain& b, int* status)
 {
-    return FlowMat<T>{A + b.mat, b.n_pad, b.n, b.n_pad / FLOW_T, Lbuf + b.lb, status};
+    return FlowMat<T>{A + b.mat, b.n_pad, b.n, b.n_pad / FLOW_T, Lbuf + b.lb, status, nullptr};
 }
 
 template <typename T, bool SPLIT>

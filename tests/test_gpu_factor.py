@@ -42,6 +42,20 @@ def test_factor_edges_vs_lapack(api, n):
         assert np.abs(L @ L.T - A).max() <= tol, prec
 
 
+@pytest.mark.parametrize("n", [2816, 2817, 4225])
+def test_factor_shared_cus(api, n):
+    """253, 276 and 595 tiles: one workgroup a CU, a few CUs with two, more workgroups than are
+    resident.  FP64 and split as above; FP32 adds one rounding of a partial sum per 256 columns."""
+    A = _matrix(n)
+    print(f"factor n={n}", flush=True)
+    for prec, tol in ((api.FP64, 8 * n * 2.0 ** -53 * 3.02), (api.MIXED, (4 + n / 256) * 2 * 2.0 ** -24 * 3.02),
+                      (api.MIXED_SPLIT, 4 * 2.0 ** -17 * 3.02)):
+        L, info = api.dpotrf(A, "L", prec)
+        assert info == 0
+        L = np.tril(L)
+        assert np.abs(L @ L.T - A).max() <= tol, prec
+
+
 @pytest.mark.parametrize("row", [0, 1, 15, 16, 47, 63, 64, 79, 127, 128, 191, 192, 299])
 def test_factor_reports_first_bad_pivot(api, row):
     """LAPACK's INFO: the 1-based row of the first non-positive pivot."""
