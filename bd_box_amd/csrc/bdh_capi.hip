@@ -304,22 +304,23 @@ int compute_forces_dev(bdh_system* s, bool energies = false)
 {
     REC_BEGIN(PH_FORCES);
     int rc = 0;
+    double* PE = energies ? s->PE : nullptr;
     if (s->cells) {
         if (launch_cell_build(s->pos, s->N, s->cell_cut, s->fp.pbc, s->fp.box, s->cl, s->st))
             return -1;
         rc = s->mixed ? launch_forces_cells<float>(s->pos, s->Q, s->LJ, s->N, s->topo, s->fp, s->cl,
-                                                   s->F, s->PE, s->flags, s->st)
+                                                   s->F, PE, s->flags, s->st)
                       : launch_forces_cells<double>(s->pos, s->Q, s->LJ, s->N, s->topo, s->fp, s->cl,
-                                                    s->F, s->PE, s->flags, s->st);
+                                                    s->F, PE, s->flags, s->st);
         if (!rc && energies) rc = launch_energy_reduce(s->PE, s->fblocks, s->E, s->st);
         REC_END(PH_FORCES);
         return rc;
     }
     if (s->mixed) {
-        if (launch_forces<float>(s->pos, s->Q, s->LJ, s->N, s->topo, s->fp, s->PF, s->PE,
+        if (launch_forces<float>(s->pos, s->Q, s->LJ, s->N, s->topo, s->fp, s->PF, PE,
                                  s->flags, s->fsplits, s->st)) return -1;
     } else {
-        if (launch_forces<double>(s->pos, s->Q, s->LJ, s->N, s->topo, s->fp, s->PF, s->PE,
+        if (launch_forces<double>(s->pos, s->Q, s->LJ, s->N, s->topo, s->fp, s->PF, PE,
                                   s->flags, s->fsplits, s->st)) return -1;
     }
     ReduceJobs jobs{};

@@ -484,7 +484,7 @@ forces_cells_kernel(const double4* __restrict__ pos, const double* __restrict__ 
                 if (r2 <= fp.far_r2)
                     pair_term<T>(dx, dy, dz, r2, qi, Q[j], lji, LJ[j], bonded(topo, nb0, nb1, j), fp, a);
             });
-        if (sub == CELL_LANES - 1) e_b = bond_terms(pos, i, pi, topo, fp, a);
+        if (sub == CELL_LANES - 1) e_b = bond_terms(pos, i, pi, topo, fp, a, PE != nullptr);
     }
 #pragma unroll
     for (int w = CELL_LANES / 2; w > 0; w >>= 1) {
@@ -507,7 +507,7 @@ forces_cells_kernel(const double4* __restrict__ pos, const double* __restrict__ 
         s_e[2][slot] = e_b;
     }
     __syncthreads();
-    if (threadIdx.x < 3) {
+    if (PE && threadIdx.x < 3) {
         double s = 0;
         for (int k = 0; k < CF_THREADS / CELL_LANES; ++k) s += s_e[threadIdx.x][k];
         PE[3 * blockIdx.x + threadIdx.x] = 0.5 * s;

@@ -14,6 +14,8 @@
 // of the column beads per workgroup, full row sums with every pair evaluated from both
 // sides.  Pair arithmetic runs in T (float in the mixed-precision step), separations and
 // accumulation in FP64.
+#include <type_traits>
+
 #include "bdh_common.hpp"
 #include "bdh_kernels.hpp"
 #include "bdh_pairterm.hpp"
@@ -23,6 +25,13 @@ namespace bdh {
 constexpr int FR_ROWS = 64;
 constexpr int FR_CHUNK = 256;
 
+struct RowsShared {
+    double4 pos[FR_CHUNK];
+    double q[FR_CHUNK];
+    double2 lj[FR_CHUNK];
+    double red[6][4][FR_ROWS];
+};
+
 // Workgroup (bx, by): row beads 64 bx .., column split by; PE (when given) receives the
 // workgroup's energies at 3 pe_idx.
 template <typename T>
@@ -30,12 +39,13 @@ __device__ __forceinline__ void forces_body(const double4* __restrict__ pos, con
                                             const double2* __restrict__ LJ, int N, const Topology& topo,
                                             const ForceParams& fp, int cols_per_split,
                                             double* __restrict__ PF, double* __restrict__ PE,
-                                            int* __restrict__ flags, int bx, int by, int pe_idx)
+                                            int* __restrict__ flags, int bx, int by, int pe_idx,
+                                            RowsShared& sh)
 {
-    __shared__ double4 s_pos[FR_CHUNK];
-    __shared__ double s_q[FR_CHUNK];
-    __shared__ double2 s_lj[FR_CHUNK];
-    __shared__ double s_red[6][4][FR_ROWS];
+    auto& s_pos = sh.pos;
+    auto& s_q = sh.q;
+    auto& s_lj = sh.lj;
+    auto& s_red = sh.red;
     const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * FR_ROWS + tx;
     const int i = bx * FR_ROWS + tx;
     const int jb = by * cols_per_split;
@@ -67,7 +77,7 @@ __device__ __forceinline__ void forces_body(const double4* __restrict__ pos, con
     }
     // bonds (only in the first column split, so each bond end is added once)
     double e_b = 0.0;
-    if (i < N && by == 0 && ty == 0) e_b = bond_terms(pos, i, pi, topo, fp, a);
+    if (i < N && by == 0 && ty == 0) e_b = bond_terms(pos, i, pi, topo, fp, a, PE != nullptr);
     s_red[0][ty][tx] = a.fx;
     s_red[1][ty][tx] = a.fy;
     s_red[2][ty][tx] = a.fz;
@@ -97,22 +107,48 @@ constexpr int FT_TILE = 64;
 constexpr int FT_MAX_N = 16384;   // tile-pair partials: 3N x ceil(N / 64) doubles
 
 // Tile pair b = J (J + 1) / 2 + I of the upper triangle of 64-bead tiles.  Lane t owns row
-// bead I*64 + t; wave w takes the shifts s = w, w + 4, ... and pairs row t with column bead
-// (t + s) mod 64 of tile J, so the column beads of one shift are distinct within a wave and
-// its column sums go to the wave's own LDS rows.  Diagonal tiles (I = J) visit every ordered
-// pair and keep row sums only; their workgroup also adds every row bead's bond terms.
-template <typename T>
+// bead I*64 + t; group g of FT_GROUPS takes the shifts s = g, g + FT_GROUPS, ... and pairs row t
+// with column bead (t + s) mod 64 of tile J, so the column beads of one shift are distinct within
+// a wave and a wave's column sums go to its own LDS rows.  Diagonal tiles (I = J) visit every
+// ordered pair and keep row sums only; their workgroup also adds every row bead's bond terms, bond
+// k on wavefront k mod 4.  W wavefronts take FT_GROUPS / W groups each, one after the other; the groups'
+// sums meet in one binary tree, so the forces do not depend on W.
+// Partners in tile J are known from a bit mask made once: looking them up in the topology for
+// every pair cost a chain of global loads per shift.  A first pass over the separations finds the
+// shifts that have a pair in reach anywhere in the wavefront; most tile pairs of a large system
+// have none and end there.
+// Bound by the serial pair terms of the tile pairs near the diagonal where N is small, by VALU
+// issue where it is large.  One wavefront's 16 shifts with the partner look-up, five divisions and
+// the bond energies' logarithms: N = 256 FP64 21.5 us; now 8.7, the batch of 256 chains 102 -> 80.
+constexpr int FT_GROUPS = 16;
+constexpr int FT_BATCH_W = 4;   // a batch fills the chip
+
+template <int W>
+struct TilesShared {
+    double4 pos[FT_TILE];
+    double q[FT_TILE];
+    double2 lj[FT_TILE];
+    double col[W][3][FT_TILE];
+    double row[W][3][FT_TILE];
+    double bond[4][3][FT_TILE];
+    double e[W][3];
+};
+
+template <typename T, int W>
 __device__ __forceinline__ void forces_tiles_body(const double4* __restrict__ pos, const double* __restrict__ Q,
                                                   const double2* __restrict__ LJ, int N, const Topology& topo,
                                                   const ForceParams& fp, double* __restrict__ PF,
                                                   double* __restrict__ PE, int* __restrict__ flags, int b,
-                                                  int pe_idx)
+                                                  int pe_idx, TilesShared<W>& sm)
 {
-    __shared__ double4 s_pos[FT_TILE];
-    __shared__ double s_q[FT_TILE];
-    __shared__ double2 s_lj[FT_TILE];
-    __shared__ double s_col[4][3][FT_TILE];
-    __shared__ double s_row[4][6][FT_TILE];
+    auto& s_pos = sm.pos;
+    auto& s_q = sm.q;
+    auto& s_lj = sm.lj;
+    auto& s_col = sm.col;
+    auto& s_row = sm.row;
+    auto& s_bond = sm.bond;
+    auto& s_e = sm.e;
+    static_assert(FT_GROUPS == 16 && (W == 4 || W == 8 || W == 16), "groups are summed by a binary tree");
     const int t = threadIdx.x, w = threadIdx.y, tid = w * FT_TILE + t;
     int J = (int)((sqrt(8.0 * b + 1.0) - 1.0) * 0.5);
     while (J * (J + 1) / 2 > b) --J;
@@ -127,82 +163,137 @@ __device__ __forceinline__ void forces_tiles_body(const double4* __restrict__ po
         s_q[tid] = ok ? Q[j] : 0.0;
         s_lj[tid] = ok ? LJ[j] : make_double2(0, 0);
     }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) s_col[w][k][t] = 0.0;
     const bool iv = i < N;
     const double4 pi = iv ? pos[i] : make_double4(0, 0, 0, 1);
     const double qi = iv ? Q[i] : 0.0;
     const double2 lji = iv ? LJ[i] : make_double2(0, 0);
-    const int nb0 = (iv && fp.use_conn) ? topo.conn_off[i] : 0;
-    const int nb1 = (iv && fp.use_conn) ? topo.conn_off[i + 1] : 0;
+    double e[3] = {0.0, 0.0, 0.0}, one[6], two[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int rep = 0;
     __syncthreads();
-    PairAcc a{0, 0, 0, 0, 0, 0};
-    for (int sh = w; sh < FT_TILE; sh += 4) {
+    // shift 16 y + x of group g(x) near anywhere in the wavefront: bit y + 4 x
+    constexpr int PER = FT_TILE / FT_GROUPS, GW = FT_GROUPS / W;
+    unsigned near = 0;
+#pragma unroll 2
+    for (int u = 0; u < GW * PER; ++u) {
+        const int sh = w * GW + u / PER + FT_GROUPS * (u % PER);
         const int jl = (t + sh) & (FT_TILE - 1);
-        const int j = j0 + jl;
-        if (!iv || j >= N || (diag && sh == 0)) continue;
         double dx = s_pos[jl].x - pi.x, dy = s_pos[jl].y - pi.y, dz = s_pos[jl].z - pi.z;
-        const double r2 = pair_r2(dx, dy, dz, fp.pbc, fp.box);
-        if (r2 > fp.far_r2) continue;
-        PairAcc p{0, 0, 0, 0, 0, 0};
-        pair_term<T>(dx, dy, dz, r2, qi, s_q[jl], lji, s_lj[jl], bonded(topo, nb0, nb1, j), fp, p);
-        a.fx += p.fx;
-        a.fy += p.fy;
-        a.fz += p.fz;
-        a.e_lj += p.e_lj;
-        a.e_c += p.e_c;
-        a.rep |= p.rep;
-        if (!diag) {
-            s_col[w][0][jl] -= p.fx;
-            s_col[w][1][jl] -= p.fy;
-            s_col[w][2][jl] -= p.fz;
+        const bool far = !iv || j0 + jl >= N || (diag && sh == 0) || pair_r2(dx, dy, dz, fp.pbc, fp.box) > fp.far_r2;
+        if (__ballot(!far)) near |= 1u << u;
+    }
+    unsigned long long partners = 0;
+    if (near && iv && fp.use_conn)
+        for (int k = topo.conn_off[i]; k < topo.conn_off[i + 1]; ++k) {
+            const int jl = topo.conn[k] - j0;
+            if (jl >= 0 && jl < FT_TILE) partners |= 1ull << jl;
+        }
+#pragma unroll 1
+    for (int x = 0; x < (near ? GW : 0); ++x) {
+        const int g = w * GW + x;
+        const bool any = (near >> (PER * x)) & ((1 << PER) - 1);
+        PairAcc a{0, 0, 0, 0, 0, 0};
+        if (any) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) s_col[w][k][t] = 0.0;
+#pragma unroll 1
+            for (int y = 0; y < PER; ++y) {
+                if (!((near >> (PER * x + y)) & 1)) continue;
+                const int sh = g + FT_GROUPS * y;
+                const int jl = (t + sh) & (FT_TILE - 1);
+                if (!iv || j0 + jl >= N || (diag && sh == 0)) continue;
+                double dx = s_pos[jl].x - pi.x, dy = s_pos[jl].y - pi.y, dz = s_pos[jl].z - pi.z;
+                const double r2 = pair_r2(dx, dy, dz, fp.pbc, fp.box);
+                if (r2 > fp.far_r2) continue;
+                PairAcc p{0, 0, 0, 0, 0, 0};
+                pair_term<T>(dx, dy, dz, r2, qi, s_q[jl], lji, s_lj[jl], (partners >> jl) & 1, fp, p, PE != nullptr);
+                a.fx += p.fx;
+                a.fy += p.fy;
+                a.fz += p.fz;
+                e[0] += p.e_lj;
+                e[1] += p.e_c;
+                rep |= p.rep;
+                if (!diag) {
+                    s_col[w][0][jl] -= p.fx;
+                    s_col[w][1][jl] -= p.fy;
+                    s_col[w][2][jl] -= p.fz;
+                }
+            }
+        }
+        double v[6] = {a.fx, a.fy, a.fz, 0.0, 0.0, 0.0};
+        if (any)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) v[3 + k] = s_col[w][k][t];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            one[k] = x & 1 ? one[k] + v[k] : v[k];
+            if (W == 16 || x == 1) two[k] = one[k];
+            else if (x == 3) two[k] += one[k];
         }
     }
-    double e_b = 0.0;
-    if (iv && diag && w == 0) e_b = bond_terms(pos, i, pi, topo, fp, a);
-    s_row[w][0][t] = a.fx;
-    s_row[w][1][t] = a.fy;
-    s_row[w][2][t] = a.fz;
-    s_row[w][3][t] = a.e_lj;
-    s_row[w][4][t] = a.e_c;
-    s_row[w][5][t] = e_b;
+    if (diag && w < 4) {
+        PairAcc a{0, 0, 0, 0, 0, 0};
+        if (iv) e[2] = bond_terms(pos, i, pi, topo, fp, a, PE != nullptr, w, 4);
+        rep |= a.rep;
+        s_bond[w][0][t] = a.fx;
+        s_bond[w][1][t] = a.fy;
+        s_bond[w][2][t] = a.fz;
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        s_row[w][k][t] = two[k];
+        s_col[w][k][t] = two[3 + k];
+    }
+    if (PE) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) e[k] += __shfl_xor(e[k], off);
+            if (t == 0) s_e[w][k] = e[k];
+        }
+    }
     __syncthreads();
-#define FT_SUM4(arr, v) ((((arr)[0][v][t] + (arr)[1][v][t]) + (arr)[2][v][t]) + (arr)[3][v][t])
+    auto sum = [&](const double (*s)[3][FT_TILE], int k) {
+        double v[4];
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const int q = y * (W / 4);
+            if constexpr (W == 4) v[y] = s[q][k][t];
+            else if constexpr (W == 8) v[y] = s[q][k][t] + s[q + 1][k][t];
+            else v[y] = (s[q][k][t] + s[q + 1][k][t]) + (s[q + 2][k][t] + s[q + 3][k][t]);
+        }
+        return (v[0] + v[1]) + (v[2] + v[3]);
+    };
     if (w == 0 && iv) {
         double* out = PF + (long long)J * 3 * N + 3 * i;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) out[k] = FT_SUM4(s_row, k);
+        for (int k = 0; k < 3; ++k) {
+            out[k] = sum(s_row, k);
+            if (diag) out[k] += (s_bond[0][k][t] + s_bond[1][k][t]) + (s_bond[2][k][t] + s_bond[3][k][t]);
+        }
     }
     if (w == 1 && !diag && j0 + t < N) {
         double* out = PF + (long long)I * 3 * N + 3 * (j0 + t);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) out[k] = FT_SUM4(s_col, k);
+        for (int k = 0; k < 3; ++k) out[k] = sum(s_col, k);
     }
-    if (PE && w == 2) {
+    if (PE && w == 2 && t < 3) {
         // pairs of a diagonal tile are seen from both ends; bonds from both of theirs
-        double e[3] = {FT_SUM4(s_row, 3), FT_SUM4(s_row, 4), FT_SUM4(s_row, 5)};
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) e[k] += __shfl_xor(e[k], off);
-        if (t == 0) {
-            PE[3 * pe_idx] = diag ? 0.5 * e[0] : e[0];
-            PE[3 * pe_idx + 1] = diag ? 0.5 * e[1] : e[1];
-            PE[3 * pe_idx + 2] = 0.5 * e[2];
-        }
+        double v = 0.0;
+        for (int y = 0; y < W; ++y) v += s_e[y][t];
+        PE[3 * pe_idx + t] = diag || t == 2 ? 0.5 * v : v;
     }
-#undef FT_SUM4
-    if (a.rep && fp.check_overlap) atomicOr(flags, 1);
-    if (a.rep & 2) atomicOr(flags, 2);
+    if (rep && fp.check_overlap) atomicOr(flags, 1);
+    if (rep & 2) atomicOr(flags, 2);
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256)
+template <typename T, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 && sizeof(T) == 4 ? 5 : 4)))
 forces_tiles_kernel(const double4* __restrict__ pos, const double* __restrict__ Q,
                     const double2* __restrict__ LJ, int N, Topology topo, ForceParams fp,
                     double* __restrict__ PF, double* __restrict__ PE, int* __restrict__ flags)
 {
-    forces_tiles_body<T>(pos, Q, LJ, N, topo, fp, PF, PE, flags, blockIdx.x, blockIdx.x);
+    __shared__ TilesShared<W> sm;
+    forces_tiles_body<T, W>(pos, Q, LJ, N, topo, fp, PF, PE, flags, blockIdx.x, blockIdx.x, sm);
 }
 
 template <typename T>
@@ -212,20 +303,22 @@ forces_kernel(const double4* __restrict__ pos, const double* __restrict__ Q,
               int cols_per_split, double* __restrict__ PF, double* __restrict__ PE,
               int* __restrict__ flags)
 {
+    __shared__ RowsShared sm;
     forces_body<T>(pos, Q, LJ, N, topo, fp, cols_per_split, PF, PE, flags, blockIdx.x, blockIdx.y,
-                   blockIdx.y * gridDim.x + blockIdx.x);
+                   blockIdx.y * gridDim.x + blockIdx.x, sm);
 }
 
 // Every chain of a batch: workgroup x of chain c is (x % gx, x / gx) of the chain's own grid
 // (gx row blocks, fsplits column splits).  The bond tables of chain c start at entry
 // bead0 + c of the concatenated CSR offsets (N + 1 per chain) and name chain-local beads.
 template <typename T>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(64 * FT_BATCH_W) __attribute__((amdgpu_waves_per_eu(4)))
 forces_batch_kernel(const double4* __restrict__ pos, const double* __restrict__ Q,
                     const double2* __restrict__ LJ, Topology topo, ForceParams fp,
                     const BatchChain* __restrict__ ch, const int* __restrict__ prefix, int nch,
                     double* __restrict__ Pf, int* __restrict__ flags)
 {
+    __shared__ union { TilesShared<FT_BATCH_W> tiles; RowsShared rows; } sm;
     const int c = batch_find(prefix, nch, blockIdx.x);
     const BatchChain b = ch[c];
     const int x = blockIdx.x - prefix[c];
@@ -233,12 +326,12 @@ forces_batch_kernel(const double4* __restrict__ pos, const double* __restrict__ 
     t.conn_off += b.bead0 + c;
     t.bond_off += b.bead0 + c;
     if (b.N <= FT_MAX_N) {
-        forces_tiles_body<T>(pos + b.bead0, Q + b.bead0, LJ + b.bead0, b.N, t, fp, Pf + b.pf, nullptr, flags,
-                             x, 0);
+        forces_tiles_body<T, FT_BATCH_W>(pos + b.bead0, Q + b.bead0, LJ + b.bead0, b.N, t, fp, Pf + b.pf, nullptr, flags,
+                             x, 0, sm.tiles);
     } else {
         const int gx = (b.N + FR_ROWS - 1) / FR_ROWS;
         forces_body<T>(pos + b.bead0, Q + b.bead0, LJ + b.bead0, b.N, t, fp, (b.N + b.fsplits - 1) / b.fsplits,
-                       Pf + b.pf, nullptr, flags, x % gx, x / gx, 0);
+                       Pf + b.pf, nullptr, flags, x % gx, x / gx, 0, sm.rows);
     }
 }
 
@@ -247,7 +340,7 @@ int launch_forces_batch(const double4* d_pos, const double* d_Q, const double2* 
                         const Topology& topo, const ForceParams& fp, const BatchPlan& plan,
                         double* d_Pf, int* d_flags, hipStream_t st)
 {
-    hipLaunchKernelGGL(forces_batch_kernel<T>, dim3(plan.force_blocks), dim3(FR_ROWS, 4), 0, st, d_pos,
+    hipLaunchKernelGGL(forces_batch_kernel<T>, dim3(plan.force_blocks), dim3(FR_ROWS, FT_BATCH_W), 0, st, d_pos,
                        d_Q, d_LJ, topo, fp, plan.ch, plan.force_pre, plan.nch, d_Pf, d_flags);
     BDH_LAUNCH_CHECK();
     return 0;
@@ -279,8 +372,21 @@ int launch_forces(const double4* d_pos, const double* d_Q, const double2* d_LJ, 
 {
     if (N <= FT_MAX_N) {
         BDH_CHECK(splits == ceil_div(N, FT_TILE), "forces: tile-pair partials expect one split per tile");
-        hipLaunchKernelGGL(forces_tiles_kernel<T>, dim3(force_blocks(N)), dim3(FT_TILE, 4), 0, st, d_pos, d_Q,
-                           d_LJ, N, topo, fp, d_PF, d_PE, d_flags);
+        // Few tile pairs: the time is one workgroup's serial shifts, so more wavefronts take them;
+        // many: the chip is full and wide workgroups only add prologues.  A step without
+        // hydrodynamics, us, W = 4 / 8 / 16, FP32 and FP64: N = 1000 (136 pairs) 23.5 / 16.3 / 16.1,
+        // 24.2 / 18.0 / 17.2; 1500 (300) 23.9 / 17.1 / 16.6, 24.5 / 18.5 / 18.0; 2000 (528) 23.8 / 17.8
+        // / 19.9, 24.6 / 19.1 / 20.6; 3000 (1128) 26.9 / 24.0 / 27.1, 28.8 / 25.6 / 27.3; 5000 (3160)
+        // 36.6 / 38.1 / 47.3, 38.9 / 39.8 / 46.5; 10000 74.3 / 95.2 / 138, 81.1 / 96.2 / 132.
+        const int blocks = force_blocks(N);
+        auto launch = [&](auto w) {
+            constexpr int W = decltype(w)::value;
+            hipLaunchKernelGGL((forces_tiles_kernel<T, W>), dim3(blocks), dim3(FT_TILE, W), 0, st, d_pos, d_Q,
+                               d_LJ, N, topo, fp, d_PF, d_PE, d_flags);
+        };
+        if (blocks <= 320) launch(std::integral_constant<int, 16>{});
+        else if (blocks <= 2048) launch(std::integral_constant<int, 8>{});
+        else launch(std::integral_constant<int, 4>{});
         BDH_LAUNCH_CHECK();
         return 0;
     }

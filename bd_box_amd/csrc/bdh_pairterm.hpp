@@ -22,38 +22,53 @@ struct PairAcc {
     int rep;            // bit 0: overlap, bit 1: overstretched bond
 };
 
+// 1 / r and, in FP64, 1 / r again: equal for T = double; from T = float one Newton step, so
+// that the force's direction keeps the FP64 separation's precision.
+__device__ __forceinline__ double wide_inverse(double, double inv) { return inv; }
+__device__ __forceinline__ double wide_inverse(float r, float inv)
+{
+    const double y = (double)inv;
+    return fma(y, fma(-(double)r, y, 1.0), y);
+}
+
 // Pair (i, j) seen from i: d = r_j - r_i (minimum image applied), r2d = |d|^2 from pair_r2.
+// One root and one division a pair (five divisions in the formulas as written); the cutoffs
+// and the overlap compare with the root itself.  Energies only where asked for.
 template <typename T>
 __device__ __forceinline__ void pair_term(double dx, double dy, double dz, double r2d, double qi,
                                           double qj, double2 lji, double2 ljj, bool conn,
-                                          const ForceParams& fp, PairAcc& a)
+                                          const ForceParams& fp, PairAcc& a, bool energy = true)
 {
     const T gam = (T)fp.gam, kap = (T)fp.kappa_c, alj = (T)fp.alpha_lj, lj6 = (T)fp.lj_6_term;
     const T r2 = (T)r2d;
     const T r = sqrt(r2);
+    const T inv = (T)1 / r;
     const T sig = (T)(lji.x + ljj.x);
     T F = 0;
     int ov = 0;
     if (fp.elec && r <= (T)fp.cutoff_c && (!conn || fp.bond_c_scale != 0.0)) {
-        const T ex = exp(-kap * r);
-        T f = gam * (T)qi * (T)qj * ((T)1 + kap * r) * ex / r2;
-        T en = gam * (T)qi * (T)qj * ex / r;
-        if (conn) { f *= (T)fp.bond_c_scale; en *= (T)fp.bond_c_scale; }
-        F += f;
-        a.e_c += (double)en;
+        T en = gam * (T)qi * (T)qj * exp(-kap * r) * inv;
+        if (conn) en *= (T)fp.bond_c_scale;
+        F += en * ((T)1 + kap * r) * inv;
+        if (energy) a.e_c += (double)en;
     }
     const T lj_cut = fp.cutoff_lj > 0.0 ? (T)fp.cutoff_lj : (T)1.122462f * sig;
     if (fp.alpha_lj != 0.0 && r <= lj_cut) {
         if (!conn || fp.bond_lj_scale != 0.0) {
-            const T eps = (T)sqrt(lji.y * ljj.y);
-            T s6 = sig / r;
+            // equal depths: the root of a square is exact
+            const T eps = (T)(lji.y == ljj.y ? fabs(lji.y) : sqrt(lji.y * ljj.y));
+            T s6 = sig * inv;
+            if (r > (T)0) s6 = fma(fma(-s6, r, sig), inv, s6);   // sig / r to its last place: s6^6 follows
             s6 *= s6;
             s6 *= s6 * s6;
-            T f = alj * eps * (T)6 * (s6 * ((T)2 * s6 - lj6)) / r;
-            T en = alj * eps * (s6 * (s6 - lj6));
-            if (conn) { f *= (T)fp.bond_lj_scale; en *= (T)fp.bond_lj_scale; }
+            T f = alj * eps * (T)6 * (s6 * ((T)2 * s6 - lj6)) * inv;
+            if (conn) f *= (T)fp.bond_lj_scale;
             F += f;
-            a.e_lj += (double)en;
+            if (energy) {
+                T en = alj * eps * (s6 * (s6 - lj6));
+                if (conn) en *= (T)fp.bond_lj_scale;
+                a.e_lj += (double)en;
+            }
             ov = (sig > r) || !isfinite(f);
         } else {
             ov = sig * sig > r2;
@@ -63,7 +78,7 @@ __device__ __forceinline__ void pair_term(double dx, double dy, double dz, doubl
     }
     a.rep |= ov;
     // force on i: -e_ij F with e_ij = (r_j - r_i)/r
-    const double s = (double)F / (double)r;
+    const double s = (double)F * wide_inverse(r, inv);
     a.fx -= dx * s;
     a.fy -= dy * s;
     a.fz -= dz * s;
@@ -76,13 +91,15 @@ __device__ __forceinline__ bool bonded(const Topology& topo, int nb0, int nb1, i
     return conn;
 }
 
-// All bonds of bead i (both ends carry each bond), returns the bond energy seen from i.
+// Every stride-th bond of bead i from the first-th (both ends carry each bond); returns, when
+// energies are asked for, the bond energy seen from i.
 __device__ __forceinline__ double bond_terms(const double4* __restrict__ pos, int i, double4 pi,
                                              const Topology& topo, const ForceParams& fp,
-                                             PairAcc& a)
+                                             PairAcc& a, bool energy, int first = 0, int stride = 1)
 {
     double e_b = 0.0;
-    for (int b = topo.bond_off[i]; b < topo.bond_off[i + 1]; ++b) {
+    const int end = topo.bond_off[i + 1];
+    for (int b = topo.bond_off[i] + first; b < end; b += stride) {
         const int p = topo.bond_p[b];
         const double r0 = topo.bond_parm[3 * b], rmax = topo.bond_parm[3 * b + 1];
         const double H = topo.bond_parm[3 * b + 2];
@@ -91,11 +108,13 @@ __device__ __forceinline__ double bond_terms(const double4* __restrict__ pos, in
         const double r = sqrt(r2);
         if (!(r < rmax)) a.rep |= 2;  // overstretched bond: fatal in the reference
         const double Ff = H * (r0 - r) / (1.0 - r2 / (rmax * rmax));
-        a.fx -= Ff * dx / r;
-        a.fy -= Ff * dy / r;
-        a.fz -= Ff * dz / r;
-        e_b += -0.5 * H * (rmax * rmax * log((rmax * rmax - r2) / (rmax * rmax - r0 * r0)) +
-                           r0 * rmax * log((rmax + r) * (rmax - r0) / ((rmax - r) * (rmax + r0))));
+        const double s = Ff / r;
+        a.fx -= s * dx;
+        a.fy -= s * dy;
+        a.fz -= s * dz;
+        if (energy)
+            e_b += -0.5 * H * (rmax * rmax * log((rmax * rmax - r2) / (rmax * rmax - r0 * r0)) +
+                               r0 * rmax * log((rmax + r) * (rmax - r0) / ((rmax - r) * (rmax + r0))));
     }
     return e_b;
 }
