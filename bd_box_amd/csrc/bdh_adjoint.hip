@@ -12,17 +12,24 @@
 //
 // H is the Hessian of the potential energy (dF/dr = -H), Phi the lower triangle with the
 // diagonal halved (derivative of the Cholesky factor, Murray 2016).  With a = L^T g,
-// Phi(L^T Lbar) = s Phi(a xi^T), so S comes from two triangular solves with n right-hand
-// sides: Y1 = L^-T (s Phi(a xi^T)), Y2 = L^-T Y1^T = S^T.
+// Phi(L^T Lbar) = s Phi(a xi^T), and the contraction needs only
 //
-// Kernels (FP64; the two solves are the O(n^3) part):
+//   Z = S + S^T = L^-T B L^-1,   B = s (Phi(a xi^T) + Phi(a xi^T)^T):  B_ij = s a_max(i,j) xi_min(i,j)
+//
+// B is a rank-one matrix on either side of its diagonal, so with M = L^-1 the product G^T =
+// L^-T B costs two running sums along each column of M:
+//   G(j, r) = s (xi_j sum_{i >= j} M_ir a_i + a_j sum_{r <= i < j} M_ir xi_i),   j >= r
+// and Z(r, c) = sum_{j >= c} G(j, r) M(j, c) for r <= c, the only half a symmetric Z needs.  The
+// inverse and that product are n^3 / 3 operations each; the two triangular solves with n
+// right-hand sides that give S as written are n^3 each.
+//
+// Kernels (FP64; the inverse and the product are the O(n^3) part):
 //   adj_lt_g_kernel         a = L^T g
-//   adj_diag_inv_kernel     inverses of L's 64 x 64 diagonal blocks
-//   adj_rhs_kernel, adj_trsm_super_kernel, adj_trsm_update_kernel
-//                           L^T X = B blocked by 64 rows, four block rows per step (their
-//                           triangle, then one K = 256 update of the rows above), B =
-//                           s Phi(a xi^T) or Y1^T
-//   adj_symmetrize_kernel   Z = Y2 + Y2^T
+//   adj_diag_inv_kernel     64 x 64 diagonal blocks of M
+//   adj_mul_kernel          M from its diagonal blocks, doubling their size: [A 0; C D]^-1 has
+//                           -D^-1 (C A^-1) below the diagonal; and Z's upper triangle
+//   adj_semi_kernel         G
+//   adj_mirror_kernel       Z from its upper triangle
 //   adj_contract_kernel     grad_r <U, D(r)> over the RPY blocks (diff_tensor.c:45-92), column splits
 //   adj_hvp_pairs_kernel,   g + contraction - c H y  (pair and bond Hessians, the forward
 //   adj_hvp_finish_kernel   pass's cutoffs and bonded-partner scaling; bond.c:43-85)
@@ -53,279 +60,264 @@ adj_lt_g_kernel(const double* __restrict__ L, long long ld, int n, const double*
     if (threadIdx.x == 0) a[i] = s_red[0];
 }
 
-// ---- L^T X = B for np right-hand sides (np = the padded order: L's padding is an identity
-// block, so the padded rows and columns of X stay zero), blocked by 64 rows from the last
-// block up: X_J <- L_JJ^-T X_J, then X_I -= L_JI^T X_J for every I < J.  X is column-major
-// (ld np), solved in place after the right-hand sides are written into it.
 constexpr int ADJ_NB = 64;
-constexpr int ADJ_SUPER = 4;   // block rows of L^T X = B per triangular launch / update K
 
-// mode 0: X(i, q) = s a_i xi_q (i > q), s a_q xi_q / 2 (i = q), 0 (i < q or beyond n)
-// mode 1: X = Y^T (64 x 64 tiles through LDS)
-__global__ void __launch_bounds__(256)
-adj_rhs_kernel(int mode, int np, int n, const double* __restrict__ a, const double* __restrict__ xi,
-               double s, const double* __restrict__ Y, double* __restrict__ X)
-{
-    __shared__ double t[ADJ_NB][ADJ_NB + 1];
-    const int i0 = blockIdx.x * ADJ_NB, q0 = blockIdx.y * ADJ_NB;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    if (mode == 0) {
-        for (int qq = ty; qq < ADJ_NB; qq += 4) {
-            const int i = i0 + tx, q = q0 + qq;
-            double v = 0.0;
-            if (i < n && q < n) v = i > q ? s * a[i] * xi[q] : (i == q ? 0.5 * s * a[i] * xi[q] : 0.0);
-            X[(long long)q * np + i] = v;
-        }
-        return;
-    }
-    // X(i, q) = Y(q, i): read the tile of Y with rows q0.., columns i0.. (column-major)
-#pragma unroll
-    for (int u = 0; u < ADJ_NB / 4; ++u) t[ty + 4 * u][tx] = Y[(long long)(i0 + ty + 4 * u) * np + q0 + tx];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < ADJ_NB / 4; ++u) X[(long long)(q0 + ty + 4 * u) * np + i0 + tx] = t[tx][ty + 4 * u];
-}
-
-// P = sA^T sB for 64 x 64 LDS tiles (sA[k][i], sB[k][q], k < 64) on v_mfma_f64_16x16x4_f64:
-// wavefront w owns the 32 x 32 quarter (rows 32 (w / 2), columns 32 (w % 2)) as 2 x 2 blocks;
-// accumulator r of lane l holds row 4 r + l / 16, column l % 16 of its block.
-__device__ __forceinline__ void tile_tn_mfma_acc(const double (*sA)[ADJ_NB + 1],
-                                                 const double (*sB)[ADJ_NB + 1], doublex4 acc[2][2])
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = 32 * (wave >> 1), c0 = 32 * (wave & 1);
-    const int lr = lane & 15, lk = lane >> 4;
-#pragma unroll 4
-    for (int k = 0; k < ADJ_NB; k += 4) {
-        double av[2], bv[2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a) av[a] = sA[k + lk][r0 + 16 * a + lr];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) bv[b] = sB[k + lk][c0 + 16 * b + lr];
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f64_16x16x4(av[a], bv[b], acc[a][b]);
-    }
-}
-
-__device__ __forceinline__ void tile_tn_mfma(const double (*sA)[ADJ_NB + 1], const double (*sB)[ADJ_NB + 1],
-                                             doublex4 acc[2][2])
-{
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = doublex4{0.0, 0.0, 0.0, 0.0};
-    tile_tn_mfma_acc(sA, sB, acc);
-}
-
-// A 64 x 64 tile of a column-major matrix (column c at P + c ld, rows contiguous) through
-// registers: every thread's 16 loads are issued before any of them is stored to LDS, as
-// sT[k][c] = P(k, c).
-struct TileRegs {
-    double v[16];
-};
-__device__ __forceinline__ void tile_load(const double* __restrict__ P, long long ld, TileRegs& t)
-{
-    const int k = threadIdx.x & 63, c = threadIdx.x >> 6;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) t.v[u] = P[(long long)(c + 4 * u) * ld + k];
-}
-__device__ __forceinline__ void tile_to_lds(const TileRegs& t, double (*sT)[ADJ_NB + 1])
-{
-    const int k = threadIdx.x & 63, c = threadIdx.x >> 6;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) sT[k][c + 4 * u] = t.v[u];
-}
-
-// sT[i][q] = P(i, q) from tile_tn_mfma's accumulators.
-__device__ __forceinline__ void tile_store_lds(double (*sT)[ADJ_NB + 1], const doublex4 acc[2][2])
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = 32 * (wave >> 1), c0 = 32 * (wave & 1);
-    const int lr = lane & 15, lk = lane >> 4;
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sT[r0 + 16 * a + lk + 4 * r][c0 + 16 * b + lr] = acc[a][b][r];
-}
-
-// X(i0 + i, q0 + q) = P(i, q) (sub = false) or -= P(i, q) (sub = true) from tile_tn_mfma's
-// accumulators.
-__device__ __forceinline__ void tile_store(double* __restrict__ X, int np, int i0, int q0,
-                                           const doublex4 acc[2][2], bool sub)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = 32 * (wave >> 1), c0 = 32 * (wave & 1);
-    const int lr = lane & 15, lk = lane >> 4;
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            double* xc = X + (long long)(q0 + c0 + 16 * b + lr) * np + i0 + r0 + 16 * a + lk;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (sub) xc[4 * r] -= acc[a][b][r];
-                else xc[4 * r] = acc[a][b][r];
-            }
-        }
-}
-
-// Inverses of the 64 x 64 diagonal blocks of L (workgroup J, thread c: column c of
-// L_JJ^-1 by forward substitution), column-major into Minv + 4096 J.
+// Column c of the inverse of the 64 x 64 diagonal block J of L by forward substitution
+// (workgroup J, thread c), zeros above the diagonal included, into the diagonal block of M.
 __global__ void __launch_bounds__(64)
-adj_diag_inv_kernel(const double* __restrict__ L, long long ld, double* __restrict__ Minv)
+adj_diag_inv_kernel(const double* __restrict__ L, long long ld, int np, double* __restrict__ M)
 {
     __shared__ double sL[ADJ_NB][ADJ_NB + 1];   // sL[i][k] = L(64 J + i, 64 J + k)
+    __shared__ double s_inv[ADJ_NB];
     const int j0 = blockIdx.x * ADJ_NB, c = threadIdx.x;
 #pragma unroll 16
     for (int k = 0; k < ADJ_NB; ++k) sL[c][k] = L[(long long)(j0 + k) * ld + j0 + c];
+    s_inv[c] = 1.0 / sL[c][c];
     __syncthreads();
     double m[ADJ_NB];
 #pragma unroll
     for (int i = 0; i < ADJ_NB; ++i) {
-        double b = (i == c) ? 1.0 : 0.0;
+        double b[2] = {(i == c) ? 1.0 : 0.0, 0.0};
 #pragma unroll
-        for (int k = 0; k < i; ++k) b -= sL[i][k] * m[k];
-        m[i] = (i >= c) ? b / sL[i][i] : 0.0;
+        for (int k = 0; k < i; ++k) b[k & 1] -= sL[i][k] * m[k];
+        m[i] = (i >= c) ? (b[0] + b[1]) * s_inv[i] : 0.0;
     }
-    double* out = Minv + (long long)blockIdx.x * ADJ_NB * ADJ_NB + (long long)c * ADJ_NB;
+    double* out = M + (long long)(j0 + c) * np + j0;
 #pragma unroll
     for (int i = 0; i < ADJ_NB; ++i) out[i] = m[i];
 }
 
-// Block rows Jlo..Jhi (at most ADJ_SUPER) of L^T X = B for one ADJ_SC-column tile of X
-// (workgroup = column tile), the rows below Jhi already applied.  The tile's rows of these
-// block rows stay in LDS: for J = Jhi down to Jlo, X_J <- M_J^T X_J (M_J = L_JJ^-1), then
-// X_I -= L_JI^T X_J for Jlo <= I < J.  The A operands come in that fixed order (M_J, then the
-// L_JI), each loaded into registers while the previous one is multiplied.  Wavefront w owns
-// rows 16 w.. of every 64 x ADJ_SC product (two 16 x 16 blocks on v_mfma_f64_16x16x4_f64).
-constexpr int ADJ_SC = 32;
+// One 64 x 64 tile of a product per workgroup, over the 64-blocks k0 .. k1 - 1 of its inner
+// index, in stages of 32: FP64 MFMA, wavefront w the 32 x 32 quarter (rows 32 (w / 2), columns
+// 32 (w % 2)), the next stage in registers while the current one is multiplied from LDS.
+// All matrices are column-major.  An operand whose tile index runs along memory lies in LDS as
+// [k][tile index], one whose k does as [tile index][k], both with pitches that leave the operand
+// reads without bank conflicts.
+//   MUL_T  T(i, q) = sum_k L(i, k) M(k, q), k in the first of two blocks of sb 64-blocks, q there,
+//          i in the second
+//   MUL_M  M(i, q) = -sum_k M(i, k) T(k, q), k in the second block
+//   MUL_Z  Z(r, c) = sum_j G(j, r) M(j, c), r <= c
+// Tiles with the longest sums come first.  Bound by MFMA issue in the large levels and MUL_Z and
+// by one tile's length in the small ones: n = 3072 the inverse 0.44 ms in 12 launches, Z 0.20 ms (48
+// TFLOP/s), against 2.25 ms for the two triangular solves they replace.
+enum { MUL_T, MUL_M, MUL_Z };
+constexpr int ADJ_KC = 32, ADJ_PN = ADJ_NB + 16, ADJ_PT = ADJ_KC + 2;
 
-__global__ void __launch_bounds__(256)
-adj_trsm_super_kernel(const double* __restrict__ L, long long ld, const double* __restrict__ Minv, int np,
-                      int Jlo, int Jhi, double* __restrict__ X)
+template <int MODE>
+__global__ void __launch_bounds__(256, 2)
+adj_mul_kernel(const double* A, long long lda, const double* B, int np, int sb, double* C)
 {
-    __shared__ double sX[ADJ_SUPER][ADJ_NB][ADJ_SC + 1];   // sX[j][k][q] = X(64 (Jlo + j) + k, q0 + q)
-    __shared__ double sA[2][ADJ_NB][ADJ_NB + 1];          // sA[.][k][i] = A(k, i)
-    const int q0 = blockIdx.x * ADJ_SC;
-    const int nbr = Jhi - Jlo + 1;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lr = lane & 15, lk = lane >> 4;
-    const int tk = threadIdx.x & 63, tc = threadIdx.x >> 6;   // loads: row tk, columns tc + 4 u
-    TileRegs ta;
-    tile_load(Minv + (long long)Jhi * ADJ_NB * ADJ_NB, ADJ_NB, ta);
-#pragma unroll
-    for (int j = 0; j < ADJ_SUPER; ++j) {
-        if (j < nbr) {
-            const double* src = X + (long long)q0 * np + (long long)(Jlo + j) * ADJ_NB + tk;
-            double v[ADJ_SC / 4];
-#pragma unroll
-            for (int u = 0; u < ADJ_SC / 4; ++u) v[u] = src[(long long)(tc + 4 * u) * np];
-#pragma unroll
-            for (int u = 0; u < ADJ_SC / 4; ++u) sX[j][tk][tc + 4 * u] = v[u];
+    constexpr bool AN = MODE != MUL_Z;   // A's tile index runs along memory
+    constexpr int ASZ = AN ? ADJ_KC * ADJ_PN : ADJ_NB * ADJ_PT, BSZ = ADJ_NB * ADJ_PT;
+    __shared__ __align__(16) double smem[2 * (ASZ + BSZ)];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nb = np / ADJ_NB;
+    int i, q, k0, k1;   // 64-blocks
+    if constexpr (MODE == MUL_Z) {
+        int c = (int)((sqrt(8.0 * blockIdx.x + 1.0) - 1.0) * 0.5);
+        while (c * (c + 1) / 2 > (int)blockIdx.x) --c;
+        while ((c + 1) * (c + 2) / 2 <= (int)blockIdx.x) ++c;
+        q = c;
+        i = blockIdx.x - c * (c + 1) / 2;
+        k0 = c;
+        k1 = nb;
+    } else {
+        const int base = 2 * sb * (blockIdx.x / (sb * sb)), e = blockIdx.x % (sb * sb);
+        if (MODE == MUL_T) {
+            i = base + sb + e % sb;
+            q = base + e / sb;
+            k0 = q;
+            k1 = base + sb;
+        } else {
+            i = base + 2 * sb - 1 - e / sb;
+            q = base + e % sb;
+            k0 = base + sb;
+            k1 = i + 1;
         }
+        if (i >= nb) return;
     }
-    int step = 0;
-    for (int J = Jhi; J >= Jlo; --J) {
-        const int j = J - Jlo;
-        for (int I = J; I >= Jlo; --I, ++step) {
-            const int buf = step & 1;
-            tile_to_lds(ta, sA[buf]);
-            __syncthreads();   // sA[buf] and the last writes of sX are visible
-            // the next A operand: L_J,I-1, else M_J-1
-            const int nJ = I > Jlo ? J : J - 1, nI = I > Jlo ? I - 1 : J - 1;
-            if (nJ >= Jlo) {
-                if (nI == nJ) tile_load(Minv + (long long)nJ * ADJ_NB * ADJ_NB, ADJ_NB, ta);
-                else tile_load(L + (long long)nI * ADJ_NB * ld + (long long)nJ * ADJ_NB, ld, ta);
-            }
-            doublex4 acc[2] = {doublex4{0.0, 0.0, 0.0, 0.0}, doublex4{0.0, 0.0, 0.0, 0.0}};
-#pragma unroll 4
-            for (int k = 0; k < ADJ_NB; k += 4) {
-                const double av = sA[buf][k + lk][16 * wave + lr];
+    const double* a0 = AN ? A + (long long)i * ADJ_NB : A + (long long)i * ADJ_NB * lda;
+    const double* b0 = B + (long long)q * ADJ_NB * np;
+    doublex2 va[4], vb[4];
+    const int nr = (tid & 31) * 2, nk = tid >> 5;    // [k][tile index]: two rows of columns nk + 8 u
+    const int tk = (tid & 15) * 2, tc = tid >> 4;    // [tile index][k]: two k of tile columns tc + 16 u
+    auto load = [&](int k) {
 #pragma unroll
-                for (int b = 0; b < 2; ++b) acc[b] = mfma_f64_16x16x4(av, sX[j][k + lk][16 * b + lr], acc[b]);
-            }
-            if (I == J) {
-                __syncthreads();   // every wavefront is done reading X_J
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) sX[j][16 * wave + lk + 4 * r][16 * b + lr] = acc[b][r];
-            } else {
-                const int i = I - Jlo;
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) sX[i][16 * wave + lk + 4 * r][16 * b + lr] -= acc[b][r];
-            }
+        for (int u = 0; u < 4; ++u) {
+            va[u] = *reinterpret_cast<const doublex2*>(AN ? a0 + (long long)(k + nk + 8 * u) * lda + nr
+                                                          : a0 + (long long)(tc + 16 * u) * lda + k + tk);
+            vb[u] = *reinterpret_cast<const doublex2*>(b0 + (long long)(tc + 16 * u) * np + k + tk);
         }
-    }
-    __syncthreads();
+    };
+    auto store = [&](int buf) {
+        double* sa = smem + buf * (ASZ + BSZ);
+        double* sb_ = sa + ASZ;
 #pragma unroll
-    for (int j = 0; j < ADJ_SUPER; ++j) {
-        if (j < nbr) {
-            double* dst = X + (long long)q0 * np + (long long)(Jlo + j) * ADJ_NB + tk;
-#pragma unroll
-            for (int u = 0; u < ADJ_SC / 4; ++u) dst[(long long)(tc + 4 * u) * np] = sX[j][tk][tc + 4 * u];
+        for (int u = 0; u < 4; ++u) {
+            *reinterpret_cast<doublex2*>(AN ? sa + (nk + 8 * u) * ADJ_PN + nr : sa + (tc + 16 * u) * ADJ_PT + tk) = va[u];
+            *reinterpret_cast<doublex2*>(sb_ + (tc + 16 * u) * ADJ_PT + tk) = vb[u];
         }
-    }
-}
-
-// X_I -= sum_{kk < kb} L_{J+kk,I}^T X_{J+kk}: workgroup (I, column tile), K = 64 kb on MFMA,
-// the next 64-row slice of both operands loaded while the current one is multiplied.
-__global__ void __launch_bounds__(256)
-adj_trsm_update_kernel(const double* __restrict__ L, long long ld, int np, int J, int kb,
-                       double* __restrict__ X)
-{
-    __shared__ double sA[ADJ_NB][ADJ_NB + 1];   // sA[k][i] = L(64 (J + kk) + k, 64 I + i)
-    __shared__ double sB[ADJ_NB][ADJ_NB + 1];   // sB[k][q] = X(64 (J + kk) + k, q0 + q)
-    const int I = blockIdx.x, q0 = blockIdx.y * ADJ_NB;
-    const int i0 = I * ADJ_NB;
-    const double* La = L + (long long)i0 * ld;
-    const double* Xq = X + (long long)q0 * np;
-    doublex4 acc[2][2];
+    };
+    const int r0 = 32 * (wave >> 1), c0 = 32 * (wave & 1), lr = lane & 15, lk = lane >> 4;
+    doublex4 acc[2][2];   // transposed: accumulator r of lane l is column 4 r + l / 16, row l % 16
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = doublex4{0.0, 0.0, 0.0, 0.0};
-    TileRegs ta, tb;
-    tile_load(La + J * ADJ_NB, ld, ta);
-    tile_load(Xq + J * ADJ_NB, np, tb);
-    for (int kk = 0; kk < kb; ++kk) {
-        if (kk) __syncthreads();   // the previous slice's products are done with sA and sB
-        tile_to_lds(ta, sA);
-        tile_to_lds(tb, sB);
+        for (int y = 0; y < 2; ++y) acc[x][y] = doublex4{0.0, 0.0, 0.0, 0.0};
+    const int kb = k0 * ADJ_NB, ke = k1 * ADJ_NB;
+    load(kb);
+    store(0);
+    for (int k = kb, buf = 0; k < ke; k += ADJ_KC, buf ^= 1) {
         __syncthreads();
-        if (kk + 1 < kb) {
-            const int j1 = (J + kk + 1) * ADJ_NB;
-            tile_load(La + j1, ld, ta);
-            tile_load(Xq + j1, np, tb);
+        const bool more = k + ADJ_KC < ke;
+        if (more) load(k + ADJ_KC);
+        const double* sa = smem + buf * (ASZ + BSZ);
+        const double* sb_ = sa + ASZ;
+        double av[2][2], bv[2][2];
+        auto fetch = [&](int s) {
+            const int kk = 4 * s + lk;
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                av[s & 1][x] = AN ? sa[kk * ADJ_PN + r0 + 16 * x + lr] : sa[(r0 + 16 * x + lr) * ADJ_PT + kk];
+                bv[s & 1][x] = sb_[(c0 + 16 * x + lr) * ADJ_PT + kk];
+            }
+        };
+        fetch(0);
+#pragma unroll
+        for (int s = 0; s < ADJ_KC / 4; ++s) {
+            if (s + 1 < ADJ_KC / 4) fetch(s + 1);
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) acc[x][y] = mfma_f64_16x16x4(bv[s & 1][x], av[s & 1][y], acc[x][y]);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        tile_tn_mfma_acc(sA, sB, acc);
+        if (more) store(buf ^ 1);
     }
-    tile_store(X, np, i0, q0, acc, true);
+    double* out = C + ((long long)q * ADJ_NB + c0 + lk) * np + i * ADJ_NB + r0 + lr;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+                out[(long long)(16 * x + 4 * r) * np + 16 * y] = MODE == MUL_M ? -acc[x][y][r] : acc[x][y][r];
 }
 
-// Z = Y + Y^T (np x np, column-major; 64 x 64 tiles through LDS), so that the contraction
+// Column r of G (workgroup r) from the start of r's 64-block, zero above the diagonal.  Thread t
+// takes rows 4 t .. 4 t + 3 of each 1024 of a span of 4096; sums of a wavefront by lane shifts, of
+// the workgroup through LDS.  Bound by reading M's and writing G's lower triangle: n = 3072 45 us.
+constexpr int SEMI_SPAN = 4096, SEMI_SPANS = 64;
+
+__global__ void __launch_bounds__(256)
+adj_semi_kernel(int np, int n, const double* __restrict__ M, const double* __restrict__ a,
+                const double* __restrict__ xi, double s, double* __restrict__ G)
+{
+    __shared__ double s_w[2][4][4];
+    __shared__ double s_span[SEMI_SPANS];   // sums of M_ir a_i over the spans
+    const int r = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int jb = r & ~(ADJ_NB - 1);
+    const double* m = M + (long long)r * np;
+    double* g = G + (long long)r * np;
+    const int spans = (np - jb + SEMI_SPAN - 1) / SEMI_SPAN;
+    if (spans > 1) {
+        for (int p = 0; p < spans; ++p) {
+            double v = 0.0;
+            for (int j = jb + p * SEMI_SPAN + t, e = min(n, jb + (p + 1) * SEMI_SPAN); j < e; j += 256)
+                if (j >= r) v += m[j] * a[j];
+#pragma unroll
+            for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w);
+            if (lane == 0) s_w[0][0][wave] = v;
+            __syncthreads();
+            if (t == 0) s_span[p] = (s_w[0][0][0] + s_w[0][0][1]) + (s_w[0][0][2] + s_w[0][0][3]);
+            __syncthreads();
+        }
+    }
+    double before = 0.0;   // sum of M_ir xi_i over the spans before
+    for (int p = 0; p < spans; ++p) {
+        double after = 0.0;
+        for (int x = spans - 1; x > p; --x) after += s_span[x];
+        double va[4][4], vx[4][4], sa[4], sx[4], ca[4], cx[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = jb + p * SEMI_SPAN + 1024 * u + 4 * t;
+            doublex2 v[2] = {{0.0, 0.0}, {0.0, 0.0}};
+            if (j < np) {
+                v[0] = *reinterpret_cast<const doublex2*>(m + j);
+                v[1] = *reinterpret_cast<const doublex2*>(m + j + 2);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool in = j + e >= r && j + e < n;
+                va[u][e] = in ? v[e >> 1][e & 1] * a[j + e] : 0.0;
+                vx[u][e] = in ? v[e >> 1][e & 1] * xi[j + e] : 0.0;
+            }
+            sa[u] = ca[u] = (va[u][0] + va[u][1]) + (va[u][2] + va[u][3]);
+            sx[u] = cx[u] = (vx[u][0] + vx[u][1]) + (vx[u][2] + vx[u][3]);
+        }
+#pragma unroll
+        for (int w = 1; w < 64; w <<= 1)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const double da = __shfl_down(ca[u], w), dx = __shfl_up(cx[u], w);
+                if (lane + w < 64) ca[u] += da;
+                if (lane >= w) cx[u] += dx;
+            }
+        __syncthreads();   // s_w is free
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (lane == 0) s_w[0][u][wave] = ca[u];
+            if (lane == 63) s_w[1][u][wave] = cx[u];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            double oa = after, ox = before;   // outside this wavefront's part
+            for (int x = 15; x > 4 * u + wave; --x) oa += s_w[0][x >> 2][x & 3];
+            for (int x = 0; x < 4 * u + wave; ++x) ox += s_w[1][x >> 2][x & 3];
+            oa += ca[u] - sa[u];
+            ox += cx[u] - sx[u];
+            const int j = jb + p * SEMI_SPAN + 1024 * u + 4 * t;
+            double o[4];
+#pragma unroll
+            for (int e = 3; e >= 0; --e) {
+                oa += va[u][e];
+                o[e] = oa;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool in = j + e >= r && j + e < n;
+                o[e] = in ? s * (xi[j + e] * o[e] + a[j + e] * ox) : 0.0;
+                ox += vx[u][e];
+            }
+            if (j < np) {
+                *reinterpret_cast<doublex2*>(g + j) = doublex2{o[0], o[1]};
+                *reinterpret_cast<doublex2*>(g + j + 2) = doublex2{o[2], o[3]};
+            }
+        }
+        for (int x = 0; x < 16; ++x) before += s_w[1][x >> 2][x & 3];
+    }
+}
+
+// Z (np x np) from its upper triangle in Y; 64 x 64 tiles through LDS, so that the contraction
 // reads one coalesced matrix.
 __global__ void __launch_bounds__(256)
-adj_symmetrize_kernel(int np, const double* __restrict__ Y, double* __restrict__ Z)
+adj_mirror_kernel(int np, const double* __restrict__ Y, double* __restrict__ Z)
 {
     __shared__ double t[ADJ_NB][ADJ_NB + 1];
     const int i0 = blockIdx.x * ADJ_NB, q0 = blockIdx.y * ADJ_NB;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    // t[ii][tx] = Y(q0 + tx, i0 + ii) = Y^T(i0 + ii, q0 + tx)
+    const bool upper = i0 < q0;
+    // t[c][x]: the tile itself (upper) or its mirror image (rows q0 .., columns i0 ..)
+    const double* src = upper ? Y + (long long)q0 * np + i0 : Y + (long long)i0 * np + q0;
 #pragma unroll
-    for (int u = 0; u < ADJ_NB / 4; ++u) t[ty + 4 * u][tx] = Y[(long long)(i0 + ty + 4 * u) * np + q0 + tx];
+    for (int u = 0; u < ADJ_NB / 4; ++u) t[ty + 4 * u][tx] = src[(long long)(ty + 4 * u) * np + tx];
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < ADJ_NB / 4; ++u) {
         const int qq = ty + 4 * u;
-        const long long e = (long long)(q0 + qq) * np + i0 + tx;
-        Z[e] = Y[e] + t[tx][qq];
+        const bool direct = upper || (i0 == q0 && tx <= qq);   // on the diagonal tile both are the same tile
+        Z[(long long)(q0 + qq) * np + i0 + tx] = direct ? t[qq][tx] : t[tx][qq];
     }
 }
 
@@ -347,7 +339,7 @@ __device__ __forceinline__ void rpy_fg(double r, double ai, double aj, double pr
 }
 
 // Term of pair (k, j) of out_k = sum_{j != k} grad_d <W_kj, B(d)> at d = r_k - r_j, with
-// W_kj = c (g_k F_j^T + F_k g_j^T) + Z(3k.., 3j..),  Z = Y2 + Y2^T  (W = 2 U_kj).
+// W_kj = c (g_k F_j^T + F_k g_j^T) + Z(3k.., 3j..)  (W = 2 U_kj).
 __device__ __forceinline__ void contract_pair(const double4& pk, const double4& pj, int k, int j,
                                               double preDii, double preDij, const double* __restrict__ Z,
                                               long long ldz, const double* gk, const double* Fk,
@@ -562,42 +554,42 @@ int launch_adj_lt_g(const double* d_L, long long ld, int n, const double* d_g, d
     return 0;
 }
 
-int launch_adj_diag_inverses(const double* d_L, long long ld, int np, double* d_Minv, hipStream_t st)
+int launch_adj_inverse(const double* d_L, long long ld, int np, double* d_M, double* d_T, hipStream_t st)
 {
-    BDH_CHECK(np % ADJ_NB == 0 && ld >= np, "adjoint solve: padded order");
-    hipLaunchKernelGGL(adj_diag_inv_kernel, dim3(np / ADJ_NB), dim3(ADJ_NB), 0, st, d_L, ld, d_Minv);
-    BDH_LAUNCH_CHECK();
-    return 0;
-}
-
-int launch_adj_upper_solve(const double* d_L, long long ld, int np, int n, int mode, const double* d_a,
-                           const double* d_xi, double s, const double* d_B, const double* d_Minv,
-                           double* d_X, hipStream_t st)
-{
-    BDH_CHECK(np % ADJ_NB == 0 && ld >= np, "adjoint solve: padded order");
+    BDH_CHECK(np % ADJ_NB == 0 && ld >= np && ld % 2 == 0, "adjoint inverse: padded order");
     const int nb = np / ADJ_NB;
-    hipLaunchKernelGGL(adj_rhs_kernel, dim3(nb, nb), dim3(256), 0, st, mode, np, n, d_a, d_xi, s, d_B, d_X);
+    hipLaunchKernelGGL(adj_diag_inv_kernel, dim3(nb), dim3(ADJ_NB), 0, st, d_L, ld, np, d_M);
     BDH_LAUNCH_CHECK();
-    // ADJ_SUPER block rows at a time: their own triangle in one launch (a workgroup per column
-    // tile), then every block row above them in one update launch with K = 64 ADJ_SUPER
-    for (int Jhi = nb - 1; Jhi >= 0; Jhi -= ADJ_SUPER) {
-        const int Jlo = std::max(0, Jhi - ADJ_SUPER + 1);
-        hipLaunchKernelGGL(adj_trsm_super_kernel, dim3(np / ADJ_SC), dim3(256), 0, st, d_L, ld, d_Minv, np, Jlo,
-                           Jhi, d_X);
+    for (int sb = 1; sb < nb; sb *= 2) {
+        const int pairs = (nb + sb - 1) / (2 * sb);   // those with a second block, perhaps a short one
+        const dim3 grid((unsigned)(pairs * sb * sb));
+        hipLaunchKernelGGL(adj_mul_kernel<MUL_T>, grid, dim3(256), 0, st, d_L, ld, (const double*)d_M, np, sb, d_T);
         BDH_LAUNCH_CHECK();
-        if (Jlo > 0) {
-            hipLaunchKernelGGL(adj_trsm_update_kernel, dim3(Jlo, nb), dim3(256), 0, st, d_L, ld, np, Jlo,
-                               Jhi - Jlo + 1, d_X);
-            BDH_LAUNCH_CHECK();
-        }
+        hipLaunchKernelGGL(adj_mul_kernel<MUL_M>, grid, dim3(256), 0, st, (const double*)d_M, (long long)np,
+                           (const double*)d_T, np, sb, d_M);
+        BDH_LAUNCH_CHECK();
     }
     return 0;
 }
 
-int launch_adj_symmetrize(int np, const double* d_Y, double* d_Z, hipStream_t st)
+int launch_adj_noise_part(int np, int n, const double* d_M, const double* d_a, const double* d_xi, double s,
+                          double* d_G, hipStream_t st)
+{
+    BDH_CHECK(np % ADJ_NB == 0 && np <= SEMI_SPAN * SEMI_SPANS, "adjoint: padded order");
+    const int nb = np / ADJ_NB;
+    hipLaunchKernelGGL(adj_semi_kernel, dim3(np), dim3(256), 0, st, np, n, d_M, d_a, d_xi, s, d_G);
+    BDH_LAUNCH_CHECK();
+    // Z's upper triangle into G's storage: its diagonal tiles are G's own, read by no other
+    hipLaunchKernelGGL(adj_mul_kernel<MUL_Z>, dim3(nb * (nb + 1) / 2), dim3(256), 0, st, (const double*)d_G,
+                       (long long)np, d_M, np, 0, d_G);
+    BDH_LAUNCH_CHECK();
+    return 0;
+}
+
+int launch_adj_mirror(int np, const double* d_Y, double* d_Z, hipStream_t st)
 {
     BDH_CHECK(np % ADJ_NB == 0, "adjoint: padded order");
-    hipLaunchKernelGGL(adj_symmetrize_kernel, dim3(np / ADJ_NB, np / ADJ_NB), dim3(256), 0, st, np, d_Y, d_Z);
+    hipLaunchKernelGGL(adj_mirror_kernel, dim3(np / ADJ_NB, np / ADJ_NB), dim3(256), 0, st, np, d_Y, d_Z);
     BDH_LAUNCH_CHECK();
     return 0;
 }

@@ -1675,10 +1675,9 @@ static int step_vjp_impl(bdh_system* s, int slot, const double* coord, const dou
     BDH_HIP(hipSetDevice(s->device));
     const int n = s->n, np = s->n_pad;
     const size_t nn = (size_t)np * np;
-    const size_t ninv = (size_t)(np / 64) * 4096;
     // mixed precision: room for the FP32 factor promoted to FP64 after the vectors
     const size_t nL = s->mixed ? nn : 0;
-    if (!s->adj && dmalloc(&s->adj, sizeof(double) * (2 * nn + 7 * (size_t)n + ninv + nL))) return -1;
+    if (!s->adj && dmalloc(&s->adj, sizeof(double) * (2 * nn + 6 * (size_t)n + nL))) return -1;
     double* Y1 = s->adj;
     double* Y2 = Y1 + nn;
     double* xi_d = Y2 + nn;
@@ -1687,8 +1686,7 @@ static int step_vjp_impl(bdh_system* s, int slot, const double* coord, const dou
     double* Dg = a_d + n;
     double* ctr = Dg + n;
     double* out = ctr + n;
-    double* Minv = out + n;
-    double* Lp = Minv + ninv;   // mixed: the factor in FP64
+    double* Lp = out + n;   // mixed: the factor in FP64
     // the forward step's state at coord: forces and the factor of D
     BDH_HIP(hipMemcpyAsync(s->pos, coord, sizeof(double) * 4 * s->N, hipMemcpyHostToDevice, s->st));
     if (compute_forces_dev(s)) return -1;
@@ -1712,14 +1710,13 @@ static int step_vjp_impl(bdh_system* s, int slot, const double* coord, const dou
         if (launch_adj_promote((const float*)s->A, (long long)nn, Lp, s->st)) return -1;
         L = Lp;
     }
-    // S^T = L^-T (L^-T s Phi(a xi^T))^T, a = L^T g
+    // Z = L^-T s (Phi(a xi^T) + Phi(a xi^T)^T) L^-1, a = L^T g: the inverse in Y1, the upper
+    // triangle of Z in Y2, then all of Z in Y1; Y2's storage then holds the contraction's partial
+    // sums (at most 64 x n doubles <= n_pad^2)
     if (launch_adj_lt_g(L, s->ld, n, g_d, a_d, s->st)) return -1;
-    if (launch_adj_diag_inverses(L, s->ld, np, Minv, s->st)) return -1;
-    if (launch_adj_upper_solve(L, s->ld, np, n, 0, a_d, xi_d, sq, nullptr, Minv, Y1, s->st)) return -1;
-    if (launch_adj_upper_solve(L, s->ld, np, n, 1, nullptr, nullptr, 0.0, Y1, Minv, Y2, s->st)) return -1;
-    // Z = Y2 + Y2^T into Y1's storage (Y1 is no longer needed); Y2's storage then holds the
-    // contraction's partial sums (at most 64 x n doubles <= n_pad^2)
-    if (launch_adj_symmetrize(np, Y2, Y1, s->st)) return -1;
+    if (launch_adj_inverse(L, s->ld, np, Y1, Y2, s->st)) return -1;
+    if (launch_adj_noise_part(np, n, Y1, a_d, xi_d, sq, Y2, s->st)) return -1;
+    if (launch_adj_mirror(np, Y2, Y1, s->st)) return -1;
     if (launch_adj_contract(s->pos, s->N, s->preDii, s->preDij, Y1, np, g_d, s->F, c, Y2, ctr, s->st))
         return -1;
     // D g from blocks on the fly, then g + contraction - c H (D g)

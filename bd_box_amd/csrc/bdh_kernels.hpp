@@ -240,22 +240,22 @@ int launch_em_update(double4* d_pos, int N, const double* d_Rf, const double* d_
 
 // ---- reverse-mode derivative of an FP64 step (bdh_adjoint.hip)
 int launch_adj_lt_g(const double* d_L, long long ld, int n, const double* d_g, double* d_a, hipStream_t st);
-// L^T X = B for n right-hand sides: mode 0 B = s Phi(a xi^T), mode 1 B = Y^T (d_B = Y)
-// (np = padded order, a multiple of 64; X and B are np x np column-major)
-// inverses of the 64 x 64 diagonal blocks (np / 64 x 4096 doubles)
-int launch_adj_diag_inverses(const double* d_L, long long ld, int np, double* d_Minv, hipStream_t st);
+// M = L^-1 (lower triangle, block diagonal's zeros included; np = the padded order, a multiple of
+// 64; column-major, ld np); d_T: np x np scratch
+int launch_adj_inverse(const double* d_L, long long ld, int np, double* d_M, double* d_T, hipStream_t st);
+// Z = M^T s (Phi(a xi^T) + its transpose) M, upper triangle, into d_G's storage (np x np)
+int launch_adj_noise_part(int np, int n, const double* d_M, const double* d_a, const double* d_xi, double s,
+                          double* d_G, hipStream_t st);
+// Z from its upper triangle in Y
+int launch_adj_mirror(int np, const double* d_Y, double* d_Z, hipStream_t st);
 // Ld[e] = A[e] for e < count (an FP32 factor promoted to FP64; count a multiple of 4)
 int launch_adj_promote(const float* d_A, long long count, double* d_Ld, hipStream_t st);
-int launch_adj_upper_solve(const double* d_L, long long ld, int np, int n, int mode, const double* d_a,
-                           const double* d_xi, double s, const double* d_B, const double* d_Minv,
-                           double* d_X, hipStream_t st);
-int launch_adj_symmetrize(int np, const double* d_Y, double* d_Z, hipStream_t st);
-// d_Y2 = Z = Y2 + Y2^T (ld ldy).  The column splits' partial sums go to d_part
+// d_Z (ld ldz).  The column splits' partial sums go to d_part
 // (adj_contract_splits(N) rows of 3N doubles) and are summed in split order into d_out.
 constexpr int ADJ_CONTRACT_MAX_SPLITS = 64;
 int adj_contract_splits(int N);
-int launch_adj_contract(const double4* d_pos, int N, double preDii, double preDij, const double* d_Y2,
-                        long long ldy, const double* d_g, const double* d_F, double c, double* d_part,
+int launch_adj_contract(const double4* d_pos, int N, double preDii, double preDij, const double* d_Z,
+                        long long ldz, const double* d_g, const double* d_F, double c, double* d_part,
                         double* d_out, hipStream_t st);
 // d_part: adj_contract_splits(N) rows of 3N doubles for the pair partials.
 int launch_adj_hvp(const double4* d_pos, const double* d_Q, const double2* d_LJ, int N,
