@@ -409,8 +409,8 @@ __device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long
 // overlaps with everything else, since the workgroups of the following tile columns are
 // resident and accumulate what is already published.
 // Measured against one launch per 256-column outer panel (n_pad >= 1024) or per 64-column panel
-// (below), right-looking: n = 768 FP64 640 -> 210 us, n = 1353 FP32 720 -> 331 us, n = 3072 FP64
-// 1900 -> 856 us, n = 9000 FP32 5.95 -> 2.81 ms, FP64 11.3 -> 5.0 ms; the batch of 256 chains of
+// (below), right-looking: n = 768 FP64 640 -> 205 us, n = 1353 FP32 720 -> 331 us, n = 3072 FP64
+// 1900 -> 840 us, n = 9000 FP32 5.95 -> 2.81 ms, FP64 11.3 -> 5.0 ms; the batch of 256 chains of
 // 64 .. 1024 beads FP32 6.9 -> 4.4 ms.  Beside another tile on its CU a tile takes 13.4 us for 128
 // columns in FP32 and 28.7 in FP64, MFMA issue at its peak; the rest at n = 9000 is the chain (31
 // us per tile column FP32, 36 FP64) and tiles that become resident too late to have caught up.
@@ -844,7 +844,9 @@ __device__ __forceinline__ void flow_solve64(doublex4 (&z)[Z][G], int J0, const 
     }
 }
 
-// Blocks J0 .. J0 + 3 of z (X) into the tile (i, j) and its operand copy.
+// Blocks J0 .. J0 + 3 of z (X): their operand copy, published as panel 2 j + J0 / 4 of tile row i,
+// then the tile (i, j) itself, which nobody waits for (stored before the flag it cost the chain
+// 0.4 us a panel in FP64).
 template <typename T>
 __device__ __forceinline__ void flow_store(const FlowMat<T>& M, int i, int j, int J0, const doublex4 (&z)[8][2])
 {
@@ -860,6 +862,7 @@ __device__ __forceinline__ void flow_store(const FlowMat<T>& M, int i, int j, in
 #pragma unroll
             for (int g = 0; g < 2; ++g) st_agent(o + col + 16 * g, (T)z[J0 + J][g][r]);
         }
+    flow_publish(M.rdy(i), 2 * j + J0 / 4 + 1);
 #pragma unroll
     for (int J = 0; J < 4; ++J)
 #pragma unroll
@@ -898,8 +901,7 @@ __device__ __forceinline__ void flow_tile(const FlowMat<T>& M, int i, int j, uns
         for (int u = 0; u < N1; ++u) s1[tid + 256 * u] = v[u];
     }
     flow_solve64<2>(z, 0, s0, s0 + CHOL_NB * CHOL_NB);
-    flow_store<T>(M, i, j, 0, z);
-    flow_publish(M.rdy(i), 2 * j + 1);   // a barrier: s1 is complete, s0 free
+    flow_store<T>(M, i, j, 0, z);   // with a barrier: s1 is complete, s0 free
     // z_2 += L21 X_1^T
 #pragma unroll
     for (int K = 0; K < 4; ++K)
@@ -915,7 +917,6 @@ __device__ __forceinline__ void flow_tile(const FlowMat<T>& M, int i, int j, uns
     load_lkk(ws + LB_STRIDE + CHOL_NB * CHOL_NB, s0);
     flow_solve64<2>(z, 4, s0, s0 + CHOL_NB * CHOL_NB);
     flow_store<T>(M, i, j, 4, z);
-    flow_publish(M.rdy(i), 2 * j + 2);
     quiet.add(-1);
 }
 
