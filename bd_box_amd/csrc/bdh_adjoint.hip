@@ -70,11 +70,13 @@ adj_diag_inv_kernel(const double* __restrict__ L, long long ld, int np, double* 
     __shared__ double sL[ADJ_NB][ADJ_NB + 1];   // sL[i][k] = L(64 J + i, 64 J + k)
     __shared__ double s_inv[ADJ_NB];
     const int j0 = blockIdx.x * ADJ_NB, c = threadIdx.x;
-#pragma unroll 16
-    for (int k = 0; k < ADJ_NB; ++k) sL[c][k] = L[(long long)(j0 + k) * ld + j0 + c];
+    double m[ADJ_NB];
+#pragma unroll
+    for (int k = 0; k < ADJ_NB; ++k) m[k] = L[(long long)(j0 + k) * ld + j0 + c];
+#pragma unroll
+    for (int k = 0; k < ADJ_NB; ++k) sL[c][k] = m[k];
     s_inv[c] = 1.0 / sL[c][c];
     __syncthreads();
-    double m[ADJ_NB];
 #pragma unroll
     for (int i = 0; i < ADJ_NB; ++i) {
         double b[2] = {(i == c) ? 1.0 : 0.0, 0.0};
@@ -88,8 +90,10 @@ adj_diag_inv_kernel(const double* __restrict__ L, long long ld, int np, double* 
 }
 
 // One 64 x 64 tile of a product per workgroup, over the 64-blocks k0 .. k1 - 1 of its inner
-// index, in stages of 32: FP64 MFMA, wavefront w the 32 x 32 quarter (rows 32 (w / 2), columns
-// 32 (w % 2)), the next stage in registers while the current one is multiplied from LDS.
+// index, in stages of 32: FP64 MFMA, wavefront w the 32 x 16 part at rows 32 (w % 2), columns
+// 16 (w / 2), the next two stages in registers while the current one is multiplied from LDS.
+// Eight wavefronts, so that one alone on a SIMD does not wait for the LDS between its MFMAs where
+// tiles are fewer than CUs.
 // All matrices are column-major.  An operand whose tile index runs along memory lies in LDS as
 // [k][tile index], one whose k does as [tile index][k], both with pitches that leave the operand
 // reads without bank conflicts.
@@ -98,14 +102,15 @@ adj_diag_inv_kernel(const double* __restrict__ L, long long ld, int np, double* 
 //   MUL_M  M(i, q) = -sum_k M(i, k) T(k, q), k in the second block
 //   MUL_Z  Z(r, c) = sum_j G(j, r) M(j, c), r <= c
 // Tiles with the longest sums come first.  Bound by MFMA issue in the large levels and MUL_Z and
-// by one tile's length in the small ones: n = 3072 the inverse 0.44 ms in 12 launches, Z 0.20 ms (48
-// TFLOP/s), against 2.25 ms for the two triangular solves they replace.
+// by one tile's length in the small ones: n = 3072 the inverse 0.36 ms in 12 launches, Z 0.19 ms (51
+// TFLOP/s), against 2.25 ms for the two triangular solves they replace; with four wavefronts 0.44
+// and 0.20 ms.
 enum { MUL_T, MUL_M, MUL_Z };
 constexpr int ADJ_KC = 32, ADJ_PN = ADJ_NB + 16, ADJ_PT = ADJ_KC + 2;
 
 template <int MODE>
-__global__ void __launch_bounds__(256, 2)
-adj_mul_kernel(const double* A, long long lda, const double* B, int np, int sb, double* C)
+__global__ void __launch_bounds__(512, 4)
+adj_mul_kernel(const double* A, long long lda, const double* B, int np, int sb, int last, double* C)
 {
     constexpr bool AN = MODE != MUL_Z;   // A's tile index runs along memory
     constexpr int ASZ = AN ? ADJ_KC * ADJ_PN : ADJ_NB * ADJ_PT, BSZ = ADJ_NB * ADJ_PT;
@@ -122,98 +127,97 @@ adj_mul_kernel(const double* A, long long lda, const double* B, int np, int sb, 
         k0 = c;
         k1 = nb;
     } else {
-        const int base = 2 * sb * (blockIdx.x / (sb * sb)), e = blockIdx.x % (sb * sb);
+        // `last` is the number of block rows of the last pair's second block
+        const int pair = min((int)blockIdx.x / (sb * sb), ((int)gridDim.x - sb * last) / (sb * sb));
+        const int e = blockIdx.x - pair * sb * sb, base = 2 * sb * pair;
+        const int rows = base + 2 * sb <= nb ? sb : last;
         if (MODE == MUL_T) {
-            i = base + sb + e % sb;
-            q = base + e / sb;
+            i = base + sb + e % rows;
+            q = base + e / rows;
             k0 = q;
             k1 = base + sb;
         } else {
-            i = base + 2 * sb - 1 - e / sb;
+            i = base + sb + rows - 1 - e / sb;
             q = base + e % sb;
             k0 = base + sb;
             k1 = i + 1;
         }
-        if (i >= nb) return;
     }
     const double* a0 = AN ? A + (long long)i * ADJ_NB : A + (long long)i * ADJ_NB * lda;
     const double* b0 = B + (long long)q * ADJ_NB * np;
-    doublex2 va[4], vb[4];
-    const int nr = (tid & 31) * 2, nk = tid >> 5;    // [k][tile index]: two rows of columns nk + 8 u
-    const int tk = (tid & 15) * 2, tc = tid >> 4;    // [tile index][k]: two k of tile columns tc + 16 u
-    auto load = [&](int k) {
+    doublex2 va[2][2], vb[2][2];
+    const int nr = (tid & 31) * 2, nk = tid >> 5;    // [k][tile index]: two rows of columns nk + 16 u
+    const int tk = (tid & 15) * 2, tc = tid >> 4;    // [tile index][k]: two k of tile columns tc + 32 u
+    auto load = [&](int k, int h) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            va[u] = *reinterpret_cast<const doublex2*>(AN ? a0 + (long long)(k + nk + 8 * u) * lda + nr
-                                                          : a0 + (long long)(tc + 16 * u) * lda + k + tk);
-            vb[u] = *reinterpret_cast<const doublex2*>(b0 + (long long)(tc + 16 * u) * np + k + tk);
+        for (int u = 0; u < 2; ++u) {
+            va[h][u] = *reinterpret_cast<const doublex2*>(AN ? a0 + (long long)(k + nk + 16 * u) * lda + nr
+                                                          : a0 + (long long)(tc + 32 * u) * lda + k + tk);
+            vb[h][u] = *reinterpret_cast<const doublex2*>(b0 + (long long)(tc + 32 * u) * np + k + tk);
         }
     };
-    auto store = [&](int buf) {
+    auto store = [&](int buf, int h) {
         double* sa = smem + buf * (ASZ + BSZ);
         double* sb_ = sa + ASZ;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            *reinterpret_cast<doublex2*>(AN ? sa + (nk + 8 * u) * ADJ_PN + nr : sa + (tc + 16 * u) * ADJ_PT + tk) = va[u];
-            *reinterpret_cast<doublex2*>(sb_ + (tc + 16 * u) * ADJ_PT + tk) = vb[u];
+        for (int u = 0; u < 2; ++u) {
+            *reinterpret_cast<doublex2*>(AN ? sa + (nk + 16 * u) * ADJ_PN + nr : sa + (tc + 32 * u) * ADJ_PT + tk) = va[h][u];
+            *reinterpret_cast<doublex2*>(sb_ + (tc + 32 * u) * ADJ_PT + tk) = vb[h][u];
         }
     };
-    const int r0 = 32 * (wave >> 1), c0 = 32 * (wave & 1), lr = lane & 15, lk = lane >> 4;
-    doublex4 acc[2][2];   // transposed: accumulator r of lane l is column 4 r + l / 16, row l % 16
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = doublex4{0.0, 0.0, 0.0, 0.0};
+    const int r0 = 32 * (wave & 1), c0 = 16 * (wave >> 1), lr = lane & 15, lk = lane >> 4;
+    doublex4 acc[2] = {doublex4{0.0, 0.0, 0.0, 0.0}, doublex4{0.0, 0.0, 0.0, 0.0}};
+    // transposed: accumulator r of lane l is column 4 r + l / 16, row l % 16
     const int kb = k0 * ADJ_NB, ke = k1 * ADJ_NB;
-    load(kb);
-    store(0);
-    for (int k = kb, buf = 0; k < ke; k += ADJ_KC, buf ^= 1) {
+    auto stage = [&](int k, int buf) {   // stage k is in LDS half buf, the next in registers buf ^ 1, two on to buf
         __syncthreads();
-        const bool more = k + ADJ_KC < ke;
-        if (more) load(k + ADJ_KC);
+        if (k + 2 * ADJ_KC < ke) load(k + 2 * ADJ_KC, buf);
         const double* sa = smem + buf * (ASZ + BSZ);
         const double* sb_ = sa + ASZ;
-        double av[2][2], bv[2][2];
+        double av[2][2], bv[2];
         auto fetch = [&](int s) {
             const int kk = 4 * s + lk;
+            bv[s & 1] = sb_[(c0 + lr) * ADJ_PT + kk];
 #pragma unroll
-            for (int x = 0; x < 2; ++x) {
+            for (int x = 0; x < 2; ++x)
                 av[s & 1][x] = AN ? sa[kk * ADJ_PN + r0 + 16 * x + lr] : sa[(r0 + 16 * x + lr) * ADJ_PT + kk];
-                bv[s & 1][x] = sb_[(c0 + 16 * x + lr) * ADJ_PT + kk];
-            }
         };
         fetch(0);
 #pragma unroll
         for (int s = 0; s < ADJ_KC / 4; ++s) {
             if (s + 1 < ADJ_KC / 4) fetch(s + 1);
 #pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y) acc[x][y] = mfma_f64_16x16x4(bv[s & 1][x], av[s & 1][y], acc[x][y]);
+            for (int x = 0; x < 2; ++x) acc[x] = mfma_f64_16x16x4(bv[s & 1], av[s & 1][x], acc[x]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (more) store(buf ^ 1);
+        if (k + ADJ_KC < ke) store(buf ^ 1, buf ^ 1);
+    };
+    static_assert(ADJ_NB % (2 * ADJ_KC) == 0, "whole pairs of stages");
+    load(kb, 0);
+    load(kb + ADJ_KC, 1);
+    store(0, 0);
+    for (int k = kb; k < ke; k += 2 * ADJ_KC) {
+        stage(k, 0);
+        stage(k + ADJ_KC, 1);
     }
     double* out = C + ((long long)q * ADJ_NB + c0 + lk) * np + i * ADJ_NB + r0 + lr;
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int y = 0; y < 2; ++y)
-                out[(long long)(16 * x + 4 * r) * np + 16 * y] = MODE == MUL_M ? -acc[x][y][r] : acc[x][y][r];
+        for (int x = 0; x < 2; ++x) out[(long long)4 * r * np + 16 * x] = MODE == MUL_M ? -acc[x][r] : acc[x][r];
 }
 
 // Column r of G (workgroup r) from the start of r's 64-block, zero above the diagonal.  Thread t
 // takes rows 4 t .. 4 t + 3 of each 1024 of a span of 4096; sums of a wavefront by lane shifts, of
-// the workgroup through LDS.  Bound by reading M's and writing G's lower triangle: n = 3072 45 us.
+// the workgroup through LDS.  Bound by reading M's and writing G's lower triangle: n = 3072 39 us.
 constexpr int SEMI_SPAN = 4096, SEMI_SPANS = 64;
 
 __global__ void __launch_bounds__(256)
 adj_semi_kernel(int np, int n, const double* __restrict__ M, const double* __restrict__ a,
                 const double* __restrict__ xi, double s, double* __restrict__ G)
 {
-    __shared__ double s_w[2][4][4];
+    __shared__ double s_w[2][16];      // wavefront w's part u of the span at 4 u + w
+    __shared__ double s_off[2][16];    // sums of M_ir a_i after, of M_ir xi_i before each part
     __shared__ double s_span[SEMI_SPANS];   // sums of M_ir a_i over the spans
     const int r = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int jb = r & ~(ADJ_NB - 1);
@@ -227,9 +231,9 @@ adj_semi_kernel(int np, int n, const double* __restrict__ M, const double* __res
                 if (j >= r) v += m[j] * a[j];
 #pragma unroll
             for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w);
-            if (lane == 0) s_w[0][0][wave] = v;
+            if (lane == 0) s_w[0][wave] = v;
             __syncthreads();
-            if (t == 0) s_span[p] = (s_w[0][0][0] + s_w[0][0][1]) + (s_w[0][0][2] + s_w[0][0][3]);
+            if (t == 0) s_span[p] = (s_w[0][0] + s_w[0][1]) + (s_w[0][2] + s_w[0][3]);
             __syncthreads();
         }
     }
@@ -266,17 +270,24 @@ adj_semi_kernel(int np, int n, const double* __restrict__ M, const double* __res
         __syncthreads();   // s_w is free
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            if (lane == 0) s_w[0][u][wave] = ca[u];
-            if (lane == 63) s_w[1][u][wave] = cx[u];
+            if (lane == 0) s_w[0][4 * u + wave] = ca[u];
+            if (lane == 63) s_w[1][4 * u + wave] = cx[u];
+        }
+        __syncthreads();
+        if (t < 16) {
+            double v = after;
+            for (int x = 15; x > t; --x) v += s_w[0][x];
+            s_off[0][t] = v;
+        } else if (t >= 64 && t < 80) {
+            double v = before;
+            for (int x = 0; x < t - 64; ++x) v += s_w[1][x];
+            s_off[1][t - 64] = v;
         }
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            double oa = after, ox = before;   // outside this wavefront's part
-            for (int x = 15; x > 4 * u + wave; --x) oa += s_w[0][x >> 2][x & 3];
-            for (int x = 0; x < 4 * u + wave; ++x) ox += s_w[1][x >> 2][x & 3];
-            oa += ca[u] - sa[u];
-            ox += cx[u] - sx[u];
+            double oa = s_off[0][4 * u + wave] + (ca[u] - sa[u]);
+            double ox = s_off[1][4 * u + wave] + (cx[u] - sx[u]);
             const int j = jb + p * SEMI_SPAN + 1024 * u + 4 * t;
             double o[4];
 #pragma unroll
@@ -295,7 +306,7 @@ adj_semi_kernel(int np, int n, const double* __restrict__ M, const double* __res
                 *reinterpret_cast<doublex2*>(g + j + 2) = doublex2{o[2], o[3]};
             }
         }
-        for (int x = 0; x < 16; ++x) before += s_w[1][x >> 2][x & 3];
+        before = s_off[1][15] + s_w[1][15];
     }
 }
 
@@ -499,6 +510,7 @@ adj_hvp_finish_kernel(const double4* __restrict__ pos, int N, Topology topo, con
     const double4 pk = pos[k];
     const double yk[3] = {y[3 * k], y[3 * k + 1], y[3 * k + 2]};
     double acc[3] = {0.0, 0.0, 0.0};
+#pragma unroll 8
     for (int sp = 0; sp < S; ++sp) {
 #pragma unroll
         for (int u = 0; u < 3; ++u) acc[u] += P[(long long)sp * 3 * N + 3 * k + u];
@@ -562,11 +574,13 @@ int launch_adj_inverse(const double* d_L, long long ld, int np, double* d_M, dou
     BDH_LAUNCH_CHECK();
     for (int sb = 1; sb < nb; sb *= 2) {
         const int pairs = (nb + sb - 1) / (2 * sb);   // those with a second block, perhaps a short one
-        const dim3 grid((unsigned)(pairs * sb * sb));
-        hipLaunchKernelGGL(adj_mul_kernel<MUL_T>, grid, dim3(256), 0, st, d_L, ld, (const double*)d_M, np, sb, d_T);
+        const int last = std::min(sb, nb - (2 * pairs - 1) * sb);
+        const dim3 grid((unsigned)((pairs - 1) * sb * sb + sb * last));
+        hipLaunchKernelGGL(adj_mul_kernel<MUL_T>, grid, dim3(512), 0, st, d_L, ld, (const double*)d_M, np, sb, last,
+                           d_T);
         BDH_LAUNCH_CHECK();
-        hipLaunchKernelGGL(adj_mul_kernel<MUL_M>, grid, dim3(256), 0, st, (const double*)d_M, (long long)np,
-                           (const double*)d_T, np, sb, d_M);
+        hipLaunchKernelGGL(adj_mul_kernel<MUL_M>, grid, dim3(512), 0, st, (const double*)d_M, (long long)np,
+                           (const double*)d_T, np, sb, last, d_M);
         BDH_LAUNCH_CHECK();
     }
     return 0;
@@ -580,8 +594,8 @@ int launch_adj_noise_part(int np, int n, const double* d_M, const double* d_a, c
     hipLaunchKernelGGL(adj_semi_kernel, dim3(np), dim3(256), 0, st, np, n, d_M, d_a, d_xi, s, d_G);
     BDH_LAUNCH_CHECK();
     // Z's upper triangle into G's storage: its diagonal tiles are G's own, read by no other
-    hipLaunchKernelGGL(adj_mul_kernel<MUL_Z>, dim3(nb * (nb + 1) / 2), dim3(256), 0, st, (const double*)d_G,
-                       (long long)np, d_M, np, 0, d_G);
+    hipLaunchKernelGGL(adj_mul_kernel<MUL_Z>, dim3(nb * (nb + 1) / 2), dim3(512), 0, st, (const double*)d_G,
+                       (long long)np, d_M, np, 0, 0, d_G);
     BDH_LAUNCH_CHECK();
     return 0;
 }
@@ -624,7 +638,7 @@ int launch_adj_hvp(const double4* d_pos, const double* d_Q, const double2* d_LJ,
     hipLaunchKernelGGL(adj_hvp_pairs_kernel, dim3(ceil_div(N, 64), S), dim3(256), 0, st, d_pos, d_Q, d_LJ,
                        N, topo, fp, d_y, js, d_part);
     BDH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(adj_hvp_finish_kernel, dim3(ceil_div(N, 256)), dim3(256), 0, st, d_pos, N, topo, d_y,
+    hipLaunchKernelGGL(adj_hvp_finish_kernel, dim3(ceil_div(N, 64)), dim3(64), 0, st, d_pos, N, topo, d_y,
                        (const double*)d_part, S, d_contract, d_g, c, d_out);
     BDH_LAUNCH_CHECK();
     return 0;
@@ -718,6 +732,7 @@ adj_param_finish_kernel(const double4* __restrict__ pos, const double2* __restri
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= N) return;
     double acc[3] = {0.0, 0.0, 0.0};
+#pragma unroll 8
     for (int sp = 0; sp < S; ++sp) {
 #pragma unroll
         for (int u = 0; u < 3; ++u) acc[u] += P[(long long)sp * 3 * N + u * N + k];
@@ -750,7 +765,7 @@ int launch_adj_params(const double4* d_pos, const double* d_Q, const double2* d_
     hipLaunchKernelGGL(adj_param_pairs_kernel, dim3(ceil_div(N, 64), S), dim3(256), 0, st, d_pos, d_Q, d_LJ,
                        N, topo, fp, d_y, js, d_part);
     BDH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(adj_param_finish_kernel, dim3(ceil_div(N, 256)), dim3(256), 0, st, d_pos, d_LJ, N, topo,
+    hipLaunchKernelGGL(adj_param_finish_kernel, dim3(ceil_div(N, 64)), dim3(64), 0, st, d_pos, d_LJ, N, topo,
                        d_bond_id, d_y, (const double*)d_part, S, c, d_eps_bar, d_R_bar, d_Q_bar, d_H_bar);
     BDH_LAUNCH_CHECK();
     return 0;
