@@ -124,10 +124,48 @@ template <typename T>
 __device__ __forceinline__ T rsqrt_p(T x);
 template <>
 __device__ __forceinline__ float rsqrt_p<float>(float x) { return __frsqrt_rn(x); }
+// hardware estimate (relative error about 2^-23) and one third-order step: a third of the
+// instructions of a root and a division, to the same place
 template <>
-__device__ __forceinline__ double rsqrt_p<double>(double x) { return 1.0 / sqrt(x); }
+__device__ __forceinline__ double rsqrt_p<double>(double x)
+{
+    const double q = __builtin_amdgcn_rsq(x), e = fma(-(x * q), q, 1.0);
+    return fma(fma(e, 0.375, 0.5), q * e, q);
+}
 
-// Free-space RPY block for separation d = r_i - r_j (diff_tensor.c:45-92), or the diagonal.
+// Free-space RPY block d I + o e e^T for separation r_i - r_j (diff_tensor.c:45-92).
+template <typename T>
+struct FreePair {
+    T d, o, ex, ey, ez;
+};
+template <typename T>
+__device__ __forceinline__ FreePair<T> free_pair(double dx, double dy, double dz, double ai, double aj,
+                                                 double preDii, double preDij)
+{
+    const T x = (T)dx, y = (T)dy, z = (T)dz, ta = (T)ai, tb = (T)aj;
+    const T r2 = x * x + y * y + z * z;
+    const T inv_r = rsqrt_p<T>(r2);
+    const T r = r2 * inv_r;
+    FreePair<T> f;
+    f.ex = x * inv_r;
+    f.ey = y * inv_r;
+    f.ez = z * inv_r;
+    if (r < ta + tb) {
+        const T sig = (T)0.5 * (ta + tb);
+        const T pre = (T)preDii / sig;
+        const T c = (T)(3.0 / 32.0) * r / sig;
+        f.d = pre * ((T)1 - (T)3 * c);
+        f.o = pre * c;
+    } else {
+        const T pre = (T)preDij * inv_r;
+        const T s = (ta * ta + tb * tb) * inv_r * inv_r;
+        f.d = pre * ((T)1 + s * (T)(1.0 / 3.0));
+        f.o = pre * ((T)1 - s);
+    }
+    return f;
+}
+
+// The block itself, or the diagonal.
 template <typename T>
 __device__ __forceinline__ Blk6 free_block(double dx, double dy, double dz, double ai, double aj,
                                            bool self, double preDii, double preDij)
@@ -136,26 +174,10 @@ __device__ __forceinline__ Blk6 free_block(double dx, double dy, double dz, doub
         const double dii = preDii / ai;
         return Blk6{dii, dii, dii, 0.0, 0.0, 0.0};
     }
-    const T x = (T)dx, y = (T)dy, z = (T)dz, ta = (T)ai, tb = (T)aj;
-    const T r2 = x * x + y * y + z * z;
-    const T inv_r = rsqrt_p<T>(r2);
-    const T r = r2 * inv_r;
-    const T ex = x * inv_r, ey = y * inv_r, ez = z * inv_r;
-    T d, o;
-    if (r < ta + tb) {
-        const T sig = (T)0.5 * (ta + tb);
-        const T pre = (T)preDii / sig;
-        const T c = (T)(3.0 / 32.0) * r / sig;
-        d = pre * ((T)1 - (T)3 * c);
-        o = pre * c;
-    } else {
-        const T pre = (T)preDij * inv_r;
-        const T s = (ta * ta + tb * tb) * inv_r * inv_r;
-        d = pre * ((T)1 + s * (T)(1.0 / 3.0));
-        o = pre * ((T)1 - s);
-    }
-    return Blk6{(double)(d + o * ex * ex), (double)(d + o * ey * ey), (double)(d + o * ez * ez),
-                (double)(o * ex * ey), (double)(o * ex * ez), (double)(o * ey * ez)};
+    const FreePair<T> f = free_pair<T>(dx, dy, dz, ai, aj, preDii, preDij);
+    return Blk6{(double)(f.d + f.o * f.ex * f.ex), (double)(f.d + f.o * f.ey * f.ey),
+                (double)(f.d + f.o * f.ez * f.ez), (double)(f.o * f.ex * f.ey), (double)(f.o * f.ex * f.ez),
+                (double)(f.o * f.ey * f.ez)};
 }
 
 // EW: 0 free space, 1 Beenakker-Ewald, 2 Smith-Ewald
@@ -199,6 +221,13 @@ constexpr int PS_MAX_SUB = PS_TILE / 4;   // then every wavefront has one shift
 // 201 us, 684 130 us, 1368 130 us and twice the partial rows).  A free-space shift takes less than
 // the few hundred ns a workgroup spends on its LDS sums: no split.
 constexpr int PS_WORKGROUPS = 512;
+
+// Free-space TEA sums of up to TEA_WIDE tile pairs (two per CU) on eight wavefronts instead of four:
+// the time there is one wavefront's shifts one after the other.  A TEA step, us, 4 / 8 / 16
+// wavefronts, FP64: N = 256 36.0 / 32.5 / 35.7, 1000 37.9 / 34.4 / 37.0, 1777 (406 pairs) 47.9 / 44.8
+// / 48.0, 2500 (820) 62.3 / 63.4 / 72.6, 4000 95.6 / 100 / 121; FP32 alike.
+constexpr int TEA_W = 8;
+constexpr unsigned TEA_WIDE = 512;
 static int pair_sub(int N, bool ewald)
 {
     const int t = ceil_div(N, PS_TILE);
@@ -209,7 +238,7 @@ static int pair_sub(int N, bool ewald)
 int pair_splits(int N, bool ewald) { return ceil_div(N, PS_TILE) * pair_sub(N, ewald); }
 int pair_eparts(int N, bool ewald) { const int t = ceil_div(N, PS_TILE); return t * (t + 1) / 2 * pair_sub(N, ewald); }
 
-template <typename T, int EW, bool TEA, bool MEAN = false>
+template <typename T, int EW, bool TEA, bool MEAN = false, int W = 4>
 __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, const double* __restrict__ F,
                                                const double* __restrict__ xi, int N, double preDii,
                                                double preDij, double dt, double* __restrict__ Pf,
@@ -222,8 +251,7 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
     __shared__ double4 s_pos2[MEAN ? PS_TILE : 1];
     __shared__ double s_f[3 * PS_TILE];
     __shared__ double s_x[TEA ? 3 * PS_TILE : 1];
-    __shared__ double s_col[4][NV][PS_TILE];
-    __shared__ double s_row[4][NV][PS_TILE];
+    __shared__ double s_sum[W][NV][PS_TILE];   // column sums, then row sums
     const int t = threadIdx.x, w = threadIdx.y, tid = w * PS_TILE + t;
     const int b = wg / S, sub = wg - b * S;
     int J = (int)((sqrt(8.0 * b + 1.0) - 1.0) * 0.5);
@@ -247,7 +275,7 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
         }
     }
 #pragma unroll
-    for (int v = 0; v < NV; ++v) s_col[w][v][t] = 0.0;
+    for (int v = 0; v < NV; ++v) s_sum[w][v][t] = 0.0;
     const bool iv = i < N;
     const double4 pi = iv ? pos[i] : make_double4(0, 0, 0, 1);
     double4 pi2 = pi;
@@ -267,11 +295,36 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
     double acc[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) acc[v] = 0.0;
-    for (int sh = w + 4 * sub; sh < PS_TILE; sh += 4 * S) {
+    for (int sh = w + W * sub; sh < PS_TILE; sh += W * S) {
         const int jl = (t + sh) & (PS_TILE - 1);
         if (!iv || j0 + jl >= N) continue;
         const bool self = diag && sh == 0;
         const double4 pj = s_pos[jl];
+        if constexpr (EW == 0 && !TEA && !MEAN) {
+            // the two products alone: d F + o e (e . F), without the block's six entries
+            double d = preDii / pi.w, o = 0.0, e0 = 0.0, e1 = 0.0, e2 = 0.0;
+            if (!self) {
+                const FreePair<T> f = free_pair<T>(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z, pi.w, pj.w, preDii, preDij);
+                d = (double)f.d;
+                o = (double)f.o;
+                e0 = (double)f.ex;
+                e1 = (double)f.ey;
+                e2 = (double)f.ez;
+            }
+            const double fx = s_f[3 * jl], fy = s_f[3 * jl + 1], fz = s_f[3 * jl + 2];
+            const double sj = o * (e0 * fx + e1 * fy + e2 * fz);
+            acc[0] += d * fx + sj * e0;
+            acc[1] += d * fy + sj * e1;
+            acc[2] += d * fz + sj * e2;
+            if (!diag) {
+                const double si = o * (e0 * Fi[0] + e1 * Fi[1] + e2 * Fi[2]);
+                double* c = &s_sum[w][0][jl];
+                c[0] += d * Fi[0] + si * e0;
+                c[PS_TILE] += d * Fi[1] + si * e1;
+                c[2 * PS_TILE] += d * Fi[2] + si * e2;
+            }
+            continue;
+        }
         Blk6 B = pair_block<T, EW>(pi, pj, self, preDii, preDij);
         if constexpr (MEAN) {
             const Blk6 B2 = pair_block<T, EW>(pi2, s_pos2[jl], self, preDii, preDij);
@@ -305,7 +358,7 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
             }
         }
         if (!diag) {
-            double* c = &s_col[w][0][jl];
+            double* c = &s_sum[w][0][jl];
             c[0] += B.xx * Fi[0] + B.xy * Fi[1] + B.xz * Fi[2];
             c[PS_TILE] += B.xy * Fi[0] + B.yy * Fi[1] + B.yz * Fi[2];
             c[2 * PS_TILE] += B.xz * Fi[0] + B.yz * Fi[1] + B.zz * Fi[2];
@@ -320,53 +373,45 @@ __device__ __forceinline__ void pair_sums_body(const double4* __restrict__ pos, 
             }
         }
     }
+    // value v of the W wavefronts summed by wavefront v mod W; v / 3 names the output, 9 is eps
+    auto sum = [&](int v) {
+        double p[W];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) s_row[w][v][t] = acc[v];
+        for (int x = 0; x < W; ++x) p[x] = s_sum[x][v][t];
+#pragma unroll
+        for (int h = 1; h < W; h *= 2)
+#pragma unroll
+            for (int x = 0; x < W; x += 2 * h) p[x] += p[x + h];
+        return p[0];
+    };
+    auto put = [&](int v, long long o) { (v < 3 ? Pf : v < 6 ? Px : Pc)[o + v % 3] = sum(v); };
     __syncthreads();
-#define sum4(a, v) (((a)[0][v][t] + (a)[1][v][t]) + ((a)[2][v][t] + (a)[3][v][t]))
-    if (w == 0 && iv) {
-        const long long o = (long long)(J * S + sub) * 3 * N + 3 * i;
+    if (!diag && j0 + t < N)
+        for (int v = w; v < (TEA ? 9 : 3); v += W) put(v, (long long)(I * S + sub) * 3 * N + 3 * (j0 + t));
+    __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 3; ++k) Pf[o + k] = sum4(s_row, k);
-        if constexpr (TEA) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                Px[o + k] = sum4(s_row, 3 + k);
-                Pc[o + k] = sum4(s_row, 6 + k);
-            }
-        }
-    }
-    if (w == 1 && !diag && j0 + t < N) {
-        const long long o = (long long)(I * S + sub) * 3 * N + 3 * (j0 + t);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) Pf[o + k] = sum4(s_col, k);
-        if constexpr (TEA) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                Px[o + k] = sum4(s_col, 3 + k);
-                Pc[o + k] = sum4(s_col, 6 + k);
-            }
-        }
-    }
+    for (int v = 0; v < NV; ++v) s_sum[w][v][t] = acc[v];
+    __syncthreads();
+    if (iv)
+        for (int v = w; v < (TEA ? 9 : 3); v += W) put(v, (long long)(J * S + sub) * 3 * N + 3 * i);
     if constexpr (TEA) {
-        if (w == 2) {
-            double e = sum4(s_row, 9);
+        if (w == W - 1) {
+            double e = sum(9);
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
             if (t == 0) Pe[wg] = diag ? e : 2.0 * e;
         }
     }
-#undef sum4
 }
 
-template <typename T, int EW, bool TEA, bool MEAN = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8)))
+template <typename T, int EW, bool TEA, bool MEAN = false, int W = 4>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ? 3 : 4, 8)))
 pair_sums_kernel(const double4* __restrict__ pos, const double* __restrict__ F,
                  const double* __restrict__ xi, int N, double preDii, double preDij, double dt,
                  double* __restrict__ Pf, double* __restrict__ Px, double* __restrict__ Pc,
                  double* __restrict__ Pe, int S, const double4* __restrict__ pos2)
 {
-    pair_sums_body<T, EW, TEA, MEAN>(pos, F, xi, N, preDii, preDij, dt, Pf, Px, Pc, Pe, blockIdx.x, S, pos2);
+    pair_sums_body<T, EW, TEA, MEAN, W>(pos, F, xi, N, preDii, preDij, dt, Pf, Px, Pc, Pe, blockIdx.x, S, pos2);
 }
 
 // Free-space D.F of every chain of a batch: workgroup x of chain c is the chain's tile pair x.
@@ -409,6 +454,14 @@ int launch_pair_sums(const double4* d_pos, const double* d_F, const double* d_xi
 #define PS_MEAN(E)                                                                                 \
     hipLaunchKernelGGL((pair_sums_kernel<T, E, true, true>), grid, blk, 0, st, d_pos, d_F, d_xi, N, \
                        preDii, preDij, dt, d_Pf, d_Px, d_Pc, d_Pe, S, d_pos2)
+#define PS_TEA()                                                                                   \
+    do {                                                                                           \
+        if (grid.x <= TEA_WIDE)                                                                    \
+            hipLaunchKernelGGL((pair_sums_kernel<T, 0, true, false, TEA_W>), grid, dim3(PS_TILE, TEA_W), 0, st, d_pos, \
+                               d_F, d_xi, N, preDii, preDij, dt, d_Pf, d_Px, d_Pc, d_Pe, S,        \
+                               (const double4*)nullptr);                                           \
+        else PS_LAUNCH(0, true);                                                                   \
+    } while (0)
     if (d_pos2) {
         if (ew == 1) PS_MEAN(1);
         else if (ew == 2) PS_MEAN(2);
@@ -418,10 +471,11 @@ int launch_pair_sums(const double4* d_pos, const double* d_F, const double* d_xi
     } else if (ew == 2) {
         if (tea) PS_LAUNCH(2, true); else PS_LAUNCH(2, false);
     } else {
-        if (tea) PS_LAUNCH(0, true); else PS_LAUNCH(0, false);
+        if (tea) PS_TEA(); else PS_LAUNCH(0, false);
     }
 #undef PS_LAUNCH
 #undef PS_MEAN
+#undef PS_TEA
     BDH_LAUNCH_CHECK();
     return 0;
 }
