@@ -210,7 +210,7 @@ struct bdh_system {
     long long ldx = 0;              // stride of drawn noise vectors: n, or n + 1 if n is odd
     int msplits = 0, tblocks = 0;
     bool ewald = false, tea = false;
-    double *Px = nullptr, *Pc = nullptr, *Pe = nullptr, *Feff = nullptr, *Cs = nullptr, *bt = nullptr;
+    double *Px = nullptr, *Pc = nullptr, *Pe = nullptr, *bt = nullptr;
     uint64_t* rng = nullptr;
     long long* rng_off = nullptr;
     int* rng_cnt = nullptr;
@@ -437,11 +437,16 @@ int matvec_dev(bdh_system* s, const double* xi = nullptr, bool tea = false, doub
 // The Geyer-Winter TEA displacement Rs (into s->Rs) from the Gaussians X, one pass over the
 // pairs (diff_rand.c:86-230), and with Rf_out also Rf = (dt / kT) D F from the same pass.
 // pos2: the sums of the mean tensor of the positions and pos2 (the IG-T corrector).
-int tea_parts(bdh_system* s, const double* X, double dt, double* Rf_out, const double4* pos2 = nullptr)
+// moved (with Rf_out): the positions may be moved by Rf + Rs in the same launch; says whether
+// they were.
+int tea_parts(bdh_system* s, const double* X, double dt, double* Rf_out, const double4* pos2 = nullptr,
+              bool* moved = nullptr)
 {
+    const int N = s->N;
+    const TeaSums sums{s->Pf, s->Px, s->Pc, s->Pe, s->msplits, pair_eparts(N, s->ewald)};
+    const double rf_scale = dt / (kB * s->cfg.T);
     if (s->perm) {
         // the same sums over the beads in the pair order, the results scattered back
-        const int N = s->N;
         const dim3 g(ceil_div(N, 256)), b(256);
         hipLaunchKernelGGL(pair_order_gather_kernel, g, b, 0, s->st, (const int*)s->perm, N, (const double4*)s->pos,
                            pos2, (const double*)s->F, X, s->pos_s, s->pos2_s, s->F_s, s->X_s);
@@ -454,29 +459,19 @@ int tea_parts(bdh_system* s, const double* X, double dt, double* Rf_out, const d
             : launch_pair_sums<double>(s->pos_s, s->F_s, s->X_s, N, s->preDii, s->preDij, dt, s->ewald, true,
                                        s->msplits, s->Pf, s->Px, s->Pc, s->Pe, s->st, p2);
         if (rc) return -1;
-        ReduceJobs jobs{};
-        int nj = 0;
-        if (Rf_out) jobs.job[nj++] = ReduceJob{s->Pf, s->Rf_s, s->n, s->msplits, 0, dt / (kB * s->cfg.T)};
-        jobs.job[nj++] = ReduceJob{s->Px, s->Feff, s->n, s->msplits, 0, 1.0};
-        jobs.job[nj++] = ReduceJob{s->Pc, s->Cs, s->n, s->msplits, 0, 1.0};
-        if (launch_reduce_partials(jobs, nj, s->n, s->st)) return -1;
-        if (launch_tea_close(s->pos_s, s->X_s, s->Feff, s->Cs, s->Pe, pair_eparts(N, s->ewald), N, s->preDii, dt, s->bt,
-                             s->Rs_s, s->st))
+        if (launch_tea_finish(sums, s->X_s, N, rf_scale, s->preDii, dt, s->bt, Rf_out ? s->Rf_s : nullptr, s->Rs_s,
+                              s->pos_s, false, 0, 0.0, s->st))
             return -1;
         hipLaunchKernelGGL(pair_order_scatter_kernel, g, b, 0, s->st, (const int*)s->perm, N,
                            (const double*)s->Rs_s, s->Rs, (const double*)(Rf_out ? s->Rf_s : nullptr), Rf_out);
         BDH_LAUNCH_CHECK();
+        if (moved) *moved = false;
         return 0;
     }
     if (matvec_dev(s, X, true, dt, pos2)) return -1;
-    ReduceJobs jobs{};
-    int nj = 0;
-    if (Rf_out) jobs.job[nj++] = ReduceJob{s->Pf, Rf_out, s->n, s->msplits, 0, dt / (kB * s->cfg.T)};
-    jobs.job[nj++] = ReduceJob{s->Px, s->Feff, s->n, s->msplits, 0, 1.0};
-    jobs.job[nj++] = ReduceJob{s->Pc, s->Cs, s->n, s->msplits, 0, 1.0};
-    if (launch_reduce_partials(jobs, nj, s->n, s->st)) return -1;
-    return launch_tea_close(s->pos, X, s->Feff, s->Cs, s->Pe, pair_eparts(s->N, s->ewald), s->N, s->preDii, dt, s->bt,
-                            s->Rs, s->st);
+    if (moved) *moved = true;
+    return launch_tea_finish(sums, X, N, rf_scale, s->preDii, dt, s->bt, Rf_out, s->Rs, s->pos, moved != nullptr,
+                             s->cfg.bc == 1, s->cfg.box, s->st);
 }
 
 int trmv_dev(bdh_system* s, const double* X, long long ldx, int m, const void* L = nullptr)
@@ -539,11 +534,14 @@ int one_step(bdh_system* s, const double* xi_dev, const double* Rs_dev, double d
     } else if (c.hydro == BDH_HYDRO_GEYER) {
         // TEA-HI: one pass over the pairs gives D.F, D.X, C and eps (diff_rand.c:86-230)
         REC_BEGIN(PH_MATVEC);
-        if (tea_parts(s, xi_dev, dt, s->Rf)) return -1;
+        bool moved = false;
+        if (tea_parts(s, xi_dev, dt, s->Rf, nullptr, s->flow ? nullptr : &moved)) return -1;
         REC_END(PH_MATVEC);
-        REC_BEGIN(PH_MOVE);
-        if (launch_em_update(s->pos, s->N, s->Rf, s->Rs, c.bc == 1, c.box, s->st, &fl)) return -1;
-        REC_END(PH_MOVE);
+        if (!moved) {
+            REC_BEGIN(PH_MOVE);
+            if (launch_em_update(s->pos, s->N, s->Rf, s->Rs, c.bc == 1, c.box, s->st, &fl)) return -1;
+            REC_END(PH_MOVE);
+        }
     } else {
         REC_BEGIN(PH_MOVE);
         if (s->flow) {
@@ -893,7 +891,7 @@ void bdh_destroy(bdh_system* s)
     dfree(s->A); dfree(s->Lbuf); dfree(s->xi); dfree(s->Pf); dfree(s->Pr); dfree(s->Rf); dfree(s->Rs);
     dfree(s->noise); dfree(s->RsB); dfree(s->pos_prev); dfree(s->F_prev); dfree(s->A2); dfree(s->Rf0); dfree(s->Rfs); dfree(s->FS); dfree(s->pos_star); dfree(s->perm); dfree(s->pos_s); dfree(s->pos2_s); dfree(s->F_s); dfree(s->X_s);
     dfree(s->Rf_s); dfree(s->Rs_s); dfree(s->rng); dfree(s->rng_off); dfree(s->rng_cnt); dfree(s->gwork); dfree(s->flags);
-    dfree(s->Px); dfree(s->Pc); dfree(s->Pe); dfree(s->Feff); dfree(s->Cs); dfree(s->bt);
+    dfree(s->Px); dfree(s->Pc); dfree(s->Pe); dfree(s->bt);
     dfree(s->cl.grid); dfree(s->cl.key); dfree(s->cl.count); dfree(s->cl.fill);
     dfree(s->cl.start); dfree(s->cl.list); dfree(s->cl.sorted); dfree(s->cl.pos);
     if (s->factor_exec) (void)hipGraphExecDestroy(s->factor_exec);
@@ -1055,8 +1053,6 @@ static int create_impl(const bdh_config* cfg, int N, const double* coord, const 
         if (dmalloc(&s->Px, sizeof(double) * s->n * s->msplits)) return -1;
         if (dmalloc(&s->Pc, sizeof(double) * s->n * s->msplits)) return -1;
         if (dmalloc(&s->Pe, sizeof(double) * pair_eparts(N, s->ewald))) return -1;
-        if (dmalloc(&s->Feff, sizeof(double) * s->n)) return -1;
-        if (dmalloc(&s->Cs, sizeof(double) * s->n)) return -1;
         if (dmalloc(&s->bt, sizeof(double) * 2)) return -1;
     }
     if (dmalloc(&s->Pr, sizeof(double) * s->n * s->tblocks * TRMV_MAX_RHS)) return -1;

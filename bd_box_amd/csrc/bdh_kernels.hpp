@@ -104,10 +104,16 @@ int launch_pair_sums_batch(const double4* d_pos, const double* d_F, double preDi
 template <typename T>
 int launch_ewald_assemble(const double4* d_pos, int N, double preDii, double preDij, T* d_A,
                           long long ld, hipStream_t st, const double4* d_pos2 = nullptr);
-// S = pair_eparts eps partials in d_Pe
-int launch_tea_close(const double4* d_pos, const double* d_xi, const double* d_Feff,
-                     const double* d_C, const double* d_Pe, int S, int N, double preDii, double dt,
-                     double* d_bt, double* d_Rs, hipStream_t st);
+// The partial sums of launch_pair_sums: `splits` rows of 3N in Pf, Px and Pc, `parts` values in Pe.
+struct TeaSums {
+    const double *Pf, *Px, *Pc, *Pe;
+    int splits, parts;
+};
+// beta and eps into d_bt, Rs, with d_Rf also Rf = rf_scale D F, and with `move` the positions moved
+// by both
+int launch_tea_finish(const TeaSums& sums, const double* d_xi, int N, double rf_scale, double preDii, double dt,
+                      double* d_bt, double* d_Rf, double* d_Rs, double4* d_pos, bool move, int pbc, double box,
+                      hipStream_t st);
 
 // ---- Cholesky and triangular products (bdh_chol.hip)
 constexpr int CHOL_NB = 64;   // panel width

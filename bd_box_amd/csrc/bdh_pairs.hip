@@ -551,14 +551,13 @@ int launch_ewald_assemble(const double4* d_pos, int N, double preDii, double pre
 }
 
 // ------------------------------------------------------------------ TEA closing
-// One block: eps from the per-workgroup partials of the pair sums (each unordered pair
-// counted twice, as from both rows), then beta; out[0] = beta, out[1] = eps.
-__global__ void __launch_bounds__(256)
-tea_beta_kernel(const double* __restrict__ Pe, int S, int N, double* __restrict__ out)
+// eps from the pair sums' partials Pe (each unordered pair counted twice, as from both rows), then
+// beta, by all 256 threads: out[0] = beta, out[1] = eps (LDS).
+__device__ __forceinline__ void tea_beta(const double* __restrict__ Pe, int parts, int N, double (&s)[256],
+                                         double (&out)[2])
 {
-    __shared__ double s[256];
     double a = 0.0;
-    for (int k = threadIdx.x; k < S; k += 256) a += Pe[k];
+    for (int k = threadIdx.x; k < parts; k += 256) a += Pe[k];
     s[threadIdx.x] = a;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
@@ -577,31 +576,109 @@ tea_beta_kernel(const double* __restrict__ Pe, int S, int N, double* __restrict_
         out[0] = beta;
         out[1] = eps;
     }
+    __syncthreads();
 }
 
-__global__ void tea_rs_kernel(const double4* __restrict__ pos, const double* __restrict__ xi,
-                              const double* __restrict__ Feff, const double* __restrict__ C,
-                              const double* __restrict__ bt, int N, double preDii, double dt,
-                              double* __restrict__ Rs)
+__global__ void __launch_bounds__(256)
+tea_beta_kernel(const double* __restrict__ Pe, int parts, int N, double* __restrict__ bt)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= 3 * N) return;
-    const double beta = bt[0];
-    const double dii = preDii / pos[r / 3].w;
+    __shared__ double s[256], out[2];
+    tea_beta(Pe, parts, N, s, out);
+    if (threadIdx.x < 2) bt[threadIdx.x] = out[threadIdx.x];
+}
+
+// Everything after the pair sums for 64 rows of the 3N-vectors per workgroup: the splits' partial
+// sums (in reduce_partials_kernel's order), Rf = rf_scale D F when asked for, beta, the TEA
+// displacement Rs and, with `move`, em_update_kernel's move of the row's coordinate, with Rf and Rs
+// as stored.  One launch of latency instead of four: N = 1777 16 -> 6 us.  BETA: from the partials
+// in every workgroup; otherwise bt holds it (TEA_OWN_BETA).
+template <bool BETA>
+__global__ void __launch_bounds__(256)
+tea_finish_kernel(TeaSums S, const double* __restrict__ xi, int N, double rf_scale, double preDii, double dt,
+                  double* __restrict__ bt, double* __restrict__ Rf, double* __restrict__ Rs,
+                  double* __restrict__ pos, int move, int pbc, double box)
+{
+    __shared__ double s_red[3][4][64];
+    __shared__ double s_tree[256], s_bt[2];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n = 3 * N, r = blockIdx.x * 64 + lane;
+    const double* const P[3] = {S.Pf, S.Px, S.Pc};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        double acc = 0.0;
+        if (r < n && (k > 0 || Rf)) {
+            const double* p = P[k] + r;
+            int x = wave;
+            for (; x + 12 <= S.splits - 1; x += 16) {
+                const double v0 = p[(long long)x * n];
+                const double v1 = p[(long long)(x + 4) * n];
+                const double v2 = p[(long long)(x + 8) * n];
+                const double v3 = p[(long long)(x + 12) * n];
+                acc += (v0 + v1) + (v2 + v3);
+            }
+            for (; x <= S.splits - 1; x += 4) acc += p[(long long)x * n];
+        }
+        s_red[k][wave][lane] = acc;
+    }
+    double beta;
+    if constexpr (BETA) {
+        tea_beta(S.Pe, S.parts, N, s_tree, s_bt);   // with barriers
+        beta = s_bt[0];
+        if (blockIdx.x == 0 && threadIdx.x < 2) bt[threadIdx.x] = s_bt[threadIdx.x];
+    } else {
+        __syncthreads();
+        beta = bt[0];
+    }
+    if (wave != 0 || r >= n) return;
+    double v[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        v[k] = (s_red[k][0][lane] + s_red[k][1][lane]) + (s_red[k][2][lane] + s_red[k][3][lane]);
+    double* q = pos + 4LL * (r / 3);
+    const double dii = preDii / q[3];
     const double X = xi[r] * sqrt(2.0 * dt / dii);
-    double c = C[r] * (beta * beta * (1.0 / dii));
+    double c = v[2] * (beta * beta * (1.0 / dii));
     c = sqrt(1.0 / (1.0 + c));
-    Rs[r] = c * (beta * Feff[r] + dii * X);
+    const double inner = beta * v[1] + dii * X;
+    double rf, rs;
+    {
+#pragma clang fp contract(off)
+        rf = rf_scale * v[0];
+        rs = c * inner;
+    }
+    if (Rf) Rf[r] = rf;
+    Rs[r] = rs;
+    if (move) {
+        q += r % 3;
+        double x = (rf + rs) + *q;
+        if (pbc) {
+            const double inv = 1.0 / box;
+            x -= box * floor(x * inv + 0.5);
+        }
+        *q = x;
+    }
 }
 
-int launch_tea_close(const double4* d_pos, const double* d_xi, const double* d_Feff,
-                     const double* d_C, const double* d_Pe, int S, int N, double preDii, double dt,
-                     double* d_bt, double* d_Rs, hipStream_t st)
+// Each workgroup sums up to this many partials for itself (4096: 32 kB from the L2, 1 us); a
+// launch of one workgroup does for more.
+constexpr int TEA_OWN_BETA = 4096;
+
+int launch_tea_finish(const TeaSums& sums, const double* d_xi, int N, double rf_scale, double preDii, double dt,
+                      double* d_bt, double* d_Rf, double* d_Rs, double4* d_pos, bool move, int pbc, double box,
+                      hipStream_t st)
 {
-    hipLaunchKernelGGL(tea_beta_kernel, dim3(1), dim3(256), 0, st, d_Pe, S, N, d_bt);
-    BDH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(tea_rs_kernel, dim3(ceil_div(3 * N, 256)), dim3(256), 0, st, d_pos, d_xi, d_Feff,
-                       d_C, d_bt, N, preDii, dt, d_Rs);
+    BDH_CHECK(!move || d_Rf, "tea_finish: a move needs Rf");
+    const dim3 grid(ceil_div(3 * N, 64));
+    double* pos = reinterpret_cast<double*>(d_pos);
+    if (sums.parts <= TEA_OWN_BETA) {
+        hipLaunchKernelGGL(tea_finish_kernel<true>, grid, dim3(256), 0, st, sums, d_xi, N, rf_scale, preDii, dt, d_bt,
+                           d_Rf, d_Rs, pos, (int)move, pbc, box);
+    } else {
+        hipLaunchKernelGGL(tea_beta_kernel, dim3(1), dim3(256), 0, st, sums.Pe, sums.parts, N, d_bt);
+        BDH_LAUNCH_CHECK();
+        hipLaunchKernelGGL(tea_finish_kernel<false>, grid, dim3(256), 0, st, sums, d_xi, N, rf_scale, preDii, dt,
+                           d_bt, d_Rf, d_Rs, pos, (int)move, pbc, box);
+    }
     BDH_LAUNCH_CHECK();
     return 0;
 }
