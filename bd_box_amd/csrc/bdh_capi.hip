@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -173,6 +174,13 @@ struct EventRecorder : PhaseRecorder {
 
 using namespace bdh;
 
+// Pinned memory for what goes back to the caller (fetch).
+constexpr size_t STAGE_MAX = 2u << 20;
+struct HostStage {
+    unsigned char* p = nullptr;
+    size_t cap = 0;
+};
+
 struct bdh_system {
     bdh_config cfg{};
     int N = 0, n = 0, n_pad = 0;
@@ -240,6 +248,7 @@ struct bdh_system {
     double4 *pos_s = nullptr, *pos2_s = nullptr;
     double *F_s = nullptr, *X_s = nullptr, *Rf_s = nullptr, *Rs_s = nullptr;
     long long order_step = 0;       // steps_done when perm was last computed
+    HostStage stage;
 };
 
 namespace {
@@ -259,11 +268,90 @@ void dfree(P*& p)
     p = nullptr;
 }
 
-int check_flags(bdh_system* s)
+// Device arrays to the caller's memory.  A copy to pageable memory waits for the stream and copies
+// through the runtime's own staging, 22 us for a few bytes, 42 us for 57 kB, 104 us for 256 kB; a
+// kernel that writes the object's pinned memory, one wait and a host copy take 11, 14 and 22 us
+// (the wait alone 9), 76 instead of 90 us at 1.3 MB.  Several arrays share the launch and the wait.
+struct Fetch {
+    void* dst;
+    const void* src;
+    size_t bytes;   // a multiple of 4
+};
+constexpr int FETCH_MAX = 6;
+
+struct FetchJobs {
+    const unsigned* src[FETCH_MAX];
+    unsigned* dst[FETCH_MAX];
+    int words[FETCH_MAX];
+};
+
+__global__ void __launch_bounds__(256) fetch_kernel(FetchJobs J)
+{
+    const unsigned* src = J.src[blockIdx.y];
+    unsigned* dst = J.dst[blockIdx.y];
+    const int n = J.words[blockIdx.y];
+    const int i0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+    if (n % 2 == 0 && (reinterpret_cast<uintptr_t>(src) & 7) == 0) {
+        for (int i = i0; i < n / 2; i += step) reinterpret_cast<uint2*>(dst)[i] = reinterpret_cast<const uint2*>(src)[i];
+    } else {
+        for (int i = i0; i < n; i += step) dst[i] = src[i];
+    }
+}
+
+// Pinned host memory of one object for fetches of up to `bytes` (at most STAGE_MAX) in all; a larger
+// one, or every one if the memory is refused, is copied by the runtime.
+void stage_alloc(HostStage& h, size_t bytes)
+{
+    bytes = std::min(bytes + 128 * FETCH_MAX, STAGE_MAX);
+    if (hipHostMalloc((void**)&h.p, bytes, hipHostMallocDefault) != hipSuccess) {
+        h.p = nullptr;
+        (void)hipGetLastError();
+        return;
+    }
+    h.cap = bytes;
+}
+
+int fetch(const HostStage& h, int device, hipStream_t st, const Fetch* f, int nf)
+{
+    FetchJobs J{};
+    size_t off[FETCH_MAX], used = 0, most = 0;
+    for (int k = 0; k < nf; ++k) {
+        off[k] = used;
+        used += (f[k].bytes + 127) / 128 * 128;
+        most = std::max(most, f[k].bytes);
+    }
+    if (nf > FETCH_MAX || used > h.cap) {
+        for (int k = 0; k < nf; ++k) BDH_HIP(hipMemcpyAsync(f[k].dst, f[k].src, f[k].bytes, hipMemcpyDeviceToHost, st));
+        BDH_HIP(hipStreamSynchronize(st));
+        return 0;
+    }
+    for (int k = 0; k < nf; ++k) {
+        J.src[k] = static_cast<const unsigned*>(f[k].src);
+        J.dst[k] = reinterpret_cast<unsigned*>(h.p + off[k]);
+        J.words[k] = (int)(f[k].bytes / 4);
+    }
+    BDH_HIP(hipSetDevice(device));
+    const int blocks = (int)std::min<size_t>(256, (most + 2047) / 2048);
+    hipLaunchKernelGGL(fetch_kernel, dim3(std::max(1, blocks), nf), dim3(256), 0, st, J);
+    BDH_LAUNCH_CHECK();
+    BDH_HIP(hipStreamSynchronize(st));
+    for (int k = 0; k < nf; ++k) std::memcpy(f[k].dst, h.p + off[k], f[k].bytes);
+    return 0;
+}
+
+int fetch(bdh_system* s, std::initializer_list<Fetch> f)
+{
+    return fetch(s->stage, s->device, s->st, f.begin(), (int)f.size());
+}
+
+// The flags of the work queued so far, with up to FETCH_MAX - 1 arrays in the same wait.
+int check_flags(bdh_system* s, const Fetch* more = nullptr, int nmore = 0)
 {
     int h[3];
-    BDH_HIP(hipMemcpyAsync(h, s->flags, sizeof(h), hipMemcpyDeviceToHost, s->st));
-    BDH_HIP(hipStreamSynchronize(s->st));
+    Fetch f[FETCH_MAX] = {{h, s->flags, sizeof(h)}};
+    BDH_CHECK(nmore < FETCH_MAX, "check_flags: too many arrays");
+    for (int k = 0; k < nmore; ++k) f[1 + k] = more[k];
+    if (fetch(s->stage, s->device, s->st, f, 1 + nmore)) return -1;
     if (h[1] < 0) {
         set_error("Cholesky decomposition error: a panel did not receive its diagonal block");
         return -3;
@@ -596,8 +684,7 @@ int step_with_retries(bdh_system* s, const double* xi_given, bool refactor)
         BDH_HIP(hipMemsetAsync(s->flags, 0, sizeof(int), s->st));
         if (one_step(s, X, chol ? s->RsB : nullptr, dt)) return -1;
         int fl = 0;
-        BDH_HIP(hipMemcpyAsync(&fl, s->flags, sizeof(int), hipMemcpyDeviceToHost, s->st));
-        BDH_HIP(hipStreamSynchronize(s->st));
+        if (fetch(s, {{&fl, s->flags, sizeof(int)}})) return -1;
         BDH_CHECK(!(fl & 2), "Overstretched bond");
         if (!(fl & 1)) break;
         if (s->cfg.algorithm == BDH_ERMAK_VAR && count < 16) dt /= 2;
@@ -647,8 +734,7 @@ int forces_flags(bdh_system* s, int& fl)
 {
     BDH_HIP(hipMemsetAsync(s->flags, 0, sizeof(int), s->st));
     if (compute_forces_dev(s)) return -1;
-    BDH_HIP(hipMemcpyAsync(&fl, s->flags, sizeof(int), hipMemcpyDeviceToHost, s->st));
-    BDH_HIP(hipStreamSynchronize(s->st));
+    if (fetch(s, {{&fl, s->flags, sizeof(int)}})) return -1;
     BDH_CHECK(!(fl & 2), "Overstretched bond");
     return 0;
 }
@@ -899,6 +985,7 @@ void bdh_destroy(bdh_system* s)
     dfree(s->fcache);
     dfree(s->bond_id);
     dfree(s->pgrad);
+    if (s->stage.p) (void)hipHostFree(s->stage.p);
     if (s->st) (void)hipStreamDestroy(s->st);
     delete s;
 }
@@ -1078,6 +1165,8 @@ static int create_impl(const bdh_config* cfg, int N, const double* coord, const 
     BDH_HIP(hipMemsetAsync(s->flags, 0, sizeof(int) * 4, s->st));
     BDH_HIP(hipMemsetAsync(s->Rf, 0, sizeof(double) * s->n, s->st));
     BDH_HIP(hipMemsetAsync(s->Rs, 0, sizeof(double) * s->n, s->st));
+    // coordinates, or what a reverse step returns
+    stage_alloc(s->stage, sizeof(double) * (N <= 4096 ? 8 * N : 4 * N));
     if (dmalloc(&s->rng, sizeof(uint64_t))) return -1;
     if (dmalloc(&s->rng_off, sizeof(long long))) return -1;
     if (dmalloc(&s->rng_cnt, sizeof(int) * (TRMV_MAX_RHS + 1))) return -1;
@@ -1258,10 +1347,11 @@ int bdh_compute_forces(bdh_system* s, double* F, double* E, int* repeat)
     BDH_HIP(hipMemsetAsync(s->flags, 0, sizeof(int), s->st));
     if (compute_forces_dev(s, E != nullptr)) return -1;
     int fl = 0;
-    if (F) BDH_HIP(hipMemcpyAsync(F, s->F, sizeof(double) * s->n, hipMemcpyDeviceToHost, s->st));
-    if (E) BDH_HIP(hipMemcpyAsync(E, s->E, sizeof(double) * 3, hipMemcpyDeviceToHost, s->st));
-    BDH_HIP(hipMemcpyAsync(&fl, s->flags, sizeof(int), hipMemcpyDeviceToHost, s->st));
-    BDH_HIP(hipStreamSynchronize(s->st));
+    Fetch f[3] = {{&fl, s->flags, sizeof(int)}};
+    int nf = 1;
+    if (F) f[nf++] = Fetch{F, s->F, sizeof(double) * s->n};
+    if (E) f[nf++] = Fetch{E, s->E, sizeof(double) * 3};
+    if (fetch(s->stage, s->device, s->st, f, nf)) return -1;
     if (repeat) *repeat = (fl & 1) ? 1 : 0;
     BDH_CHECK(!(fl & 2), "Overstretched bond");
     return 0;
@@ -1479,8 +1569,7 @@ int bdh_igt_phase(bdh_system* s, int phase, double dt, double* coord_out, int* r
     const FlowTerm cf = flow_term(s, FLOW_CORRECTOR, dt, s->FS);
     if (launch_em_update(s->pos, s->N, s->Rf0, Rs, s->cfg.bc == 1, s->cfg.box, s->st, &cf)) return -1;
     if (forces_flags(s, fl)) return -1;
-    BDH_HIP(hipMemcpyAsync(coord_out, s->pos, pb, hipMemcpyDeviceToHost, s->st));
-    BDH_HIP(hipStreamSynchronize(s->st));
+    if (fetch(s, {{coord_out, s->pos, pb}})) return -1;
     s->last_Rs = Rs;
     s->last_dt = dt;
     *result = (fl & 1) ? 2 : 0;
@@ -1560,9 +1649,7 @@ int bdh_set_forces(bdh_system* s, const double* F)
 int bdh_get_coords(bdh_system* s, double* coord)
 {
     BDH_CHECK(s && coord, "bdh_get_coords: bad arguments");
-    BDH_HIP(hipMemcpyAsync(coord, s->pos, sizeof(double) * 4 * s->N, hipMemcpyDeviceToHost, s->st));
-    BDH_HIP(hipStreamSynchronize(s->st));
-    return 0;
+    return fetch(s, {{coord, s->pos, sizeof(double) * 4 * s->N}});
 }
 
 int bdh_set_coords(bdh_system* s, const double* coord)
@@ -1723,7 +1810,8 @@ static int step_vjp_impl(bdh_system* s, int slot, const double* coord, const dou
     jobs.job[0] = ReduceJob{s->Pf, Dg, n, s->msplits, 0, 1.0};
     if (launch_reduce_partials(jobs, 1, n, s->st)) return -1;
     if (launch_adj_hvp(s->pos, s->Q, s->LJ, s->N, s->topo, s->fp, Dg, ctr, g_d, c, Y2, out, s->st)) return -1;
-    BDH_HIP(hipMemcpyAsync(rbar, out, sizeof(double) * n, hipMemcpyDeviceToHost, s->st));
+    Fetch back[FETCH_MAX - 1] = {{rbar, out, sizeof(double) * n}};
+    int nback = 1;
     if (pb) {
         // (c D g)^T dF/dtheta; the pair partials reuse Y2's storage, free again after the
         // Hessian-vector product (stream order)
@@ -1736,21 +1824,16 @@ static int step_vjp_impl(bdh_system* s, int slot, const double* coord, const dou
         double* outs[4] = {pb->eps, pb->R, pb->Q, pb->H};
         for (int q = 0; q < 4; ++q) {
             const size_t cnt = q < 3 ? (size_t)N : (size_t)s->nbonds;
-            if (outs[q] && cnt)
-                BDH_HIP(hipMemcpyAsync(outs[q], pe + (size_t)q * N, sizeof(double) * cnt, hipMemcpyDeviceToHost,
-                                       s->st));
+            if (outs[q] && cnt) back[nback++] = Fetch{outs[q], pe + (size_t)q * N, sizeof(double) * cnt};
         }
     }
-    BDH_HIP(hipStreamSynchronize(s->st));
-    return check_flags(s);
+    return check_flags(s, back, nback);
 }
 
 int bdh_get_forces(bdh_system* s, double* F)
 {
     BDH_CHECK(s && F, "bdh_get_forces: bad arguments");
-    BDH_HIP(hipMemcpyAsync(F, s->F, sizeof(double) * s->n, hipMemcpyDeviceToHost, s->st));
-    BDH_HIP(hipStreamSynchronize(s->st));
-    return 0;
+    return fetch(s, {{F, s->F, sizeof(double) * s->n}});
 }
 
 int bdh_last_dt(bdh_system* s, double* dt)
@@ -2055,6 +2138,7 @@ struct bdh_batch {
     EventRecorder* rec = nullptr;
     hipGraphExec_t factor_exec = nullptr;   // assembly + factorization of every chain, captured once
     hipGraphExec_t cycle_exec = nullptr;    // a whole refactor cycle of device-stream steps
+    HostStage stage;
 };
 
 namespace {
@@ -2063,9 +2147,8 @@ int batch_check(bdh_batch* b)
 {
     std::vector<int> st(b->B);
     int h[2];
-    BDH_HIP(hipMemcpyAsync(h, b->flags, sizeof(h), hipMemcpyDeviceToHost, b->st));
-    BDH_HIP(hipMemcpyAsync(st.data(), b->status, sizeof(int) * b->B, hipMemcpyDeviceToHost, b->st));
-    BDH_HIP(hipStreamSynchronize(b->st));
+    const Fetch f[2] = {{h, b->flags, sizeof(h)}, {st.data(), b->status, sizeof(int) * b->B}};
+    if (fetch(b->stage, b->device, b->st, f, 2)) return -1;
     for (int c = 0; c < b->B; ++c) {
         if (st[c] < 0) {
             set_error("Cholesky decomposition error in chain " + std::to_string(c) +
@@ -2541,6 +2624,9 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
                                 : launch_set_identity_pad<double>((double*)b->A + h.mat, h.n_pad, h.n, h.n_pad, b->st);
         if (rc) return -1;
     }
+    // coordinates if they fit, else the flags of every chain
+    const size_t coords = sizeof(double4) * b->Ntot, flags = sizeof(int) * b->B;
+    stage_alloc(b->stage, coords + 1024 <= STAGE_MAX ? std::max(coords, flags) : flags);
     if (dmalloc(&b->Lbuf, sizeof(double) * lb)) return -1;
     BDH_HIP(hipMemsetAsync(b->Lbuf, 0, sizeof(double) * lb, b->st));
 
@@ -2577,6 +2663,7 @@ void bdh_batch_destroy(bdh_batch* b)
 {
     if (!b) return;
     if (b->st) (void)hipStreamSynchronize(b->st);
+    if (b->stage.p) (void)hipHostFree(b->stage.p);
     dfree(b->d_ch); dfree(b->d_tab); dfree(b->d_tasks);
     dfree(b->pos); dfree(b->Q); dfree(b->LJ);
     dfree(b->conn_off); dfree(b->conn); dfree(b->bond_parm);
@@ -2674,17 +2761,15 @@ int bdh_batch_autotune(bdh_batch* b, int reps, int* cand, double* ms, int* ncand
 int bdh_batch_get_coords(bdh_batch* b, double* coord)
 {
     BDH_CHECK(b && coord, "bdh_batch_get_coords: bad arguments");
-    BDH_HIP(hipMemcpyAsync(coord, b->pos, sizeof(double4) * b->Ntot, hipMemcpyDeviceToHost, b->st));
-    BDH_HIP(hipStreamSynchronize(b->st));
-    return 0;
+    const Fetch f{coord, b->pos, sizeof(double4) * b->Ntot};
+    return fetch(b->stage, b->device, b->st, &f, 1);
 }
 
 int bdh_batch_get_forces(bdh_batch* b, double* F)
 {
     BDH_CHECK(b && F, "bdh_batch_get_forces: bad arguments");
-    BDH_HIP(hipMemcpyAsync(F, b->F, sizeof(double) * b->ntot, hipMemcpyDeviceToHost, b->st));
-    BDH_HIP(hipStreamSynchronize(b->st));
-    return 0;
+    const Fetch f{F, b->F, sizeof(double) * b->ntot};
+    return fetch(b->stage, b->device, b->st, &f, 1);
 }
 
 int bdh_batch_time_steps(bdh_batch* b, int steps, double* ms)
