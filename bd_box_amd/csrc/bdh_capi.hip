@@ -2520,10 +2520,11 @@ int batch_create_impl(const bdh_config* cfg, int B, const int* N, const double* 
         for (const auto& h : b->hc) orders.push_back(h.n_pad);
         const std::vector<FlowTask> tasks = chol_batch_tasks(orders);
         BDH_CHECK(tasks.size() <= (size_t)INT32_MAX, "bdh_batch_create: batch too large");
-        if (dmalloc(&b->d_tasks, sizeof(FlowTask) * tasks.size())) return -1;
+        if (dmalloc(&b->d_tasks, sizeof(FlowTask) * (tasks.size() + 1))) return -1;
         BDH_HIP(hipMemcpy(b->d_tasks, tasks.data(), sizeof(FlowTask) * tasks.size(), hipMemcpyHostToDevice));
         b->plan.tasks = b->d_tasks;
         b->plan.ntasks = (int)tasks.size();
+        b->plan.next = reinterpret_cast<int*>(b->d_tasks + tasks.size());
     }
 
     // forces (a single set of parameters; the pair-skip reach is the largest of any chain)

@@ -52,6 +52,18 @@ constexpr int SINV_P = 17;
 constexpr int SINV = 16 * SINV_P;
 constexpr int LB_STRIDE = CHOL_NB * CHOL_NB + 4 * SINV;
 
+// threadIdx.x; OPAQUE: as if unknown to the compiler, so that what depends on it is computed where it
+// is used.  Otherwise the FP64 tile functions keep addresses in registers that they then spill in
+// the chain (n = 768 205 us, 189 so; FP32 has the registers and is 1 % faster without), and in the
+// loop over tasks every address is taken out of the loop and spilled.
+template <bool OPAQUE>
+__device__ __forceinline__ int flow_tid()
+{
+    int t = threadIdx.x;
+    if constexpr (OPAQUE) asm volatile("" : "+v"(t));
+    return t;
+}
+
 // One wavefront: columns cw .. cw + 15 of the 64x64 block, lane = row, p[u] = column cw + u with
 // every earlier group's update made; finished columns go to L (LDS, column-major; what a lane
 // above the diagonal holds is not part of the factor).
@@ -305,7 +317,7 @@ __device__ __forceinline__ void quad_acc(const float* __restrict__ A, long long 
                                          floatx16 (&acc)[NQ])
 {
     constexpr int KC = 32 / NQ, NJ = KC / 2;
-    const int lane = threadIdx.x & 63, l32 = lane & 31, lh = lane >> 5;
+    const int lane = flow_tid<true>() & 63, l32 = lane & 31, lh = lane >> 5;
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
 #pragma unroll
@@ -346,7 +358,7 @@ template <int NQ>
 __device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long ld, int ra, int ca, int kb, int K,
                                          doublex4 (&acc)[NQ][2][2])
 {
-    const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+    const int lane = flow_tid<true>() & 63, l16 = lane & 15, lq = lane >> 4;
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
 #pragma unroll
@@ -409,11 +421,11 @@ __device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long
 // overlaps with everything else, since the workgroups of the following tile columns are
 // resident and accumulate what is already published.
 // Measured against one launch per 256-column outer panel (n_pad >= 1024) or per 64-column panel
-// (below), right-looking: n = 768 FP64 640 -> 205 us, n = 1353 FP32 720 -> 331 us, n = 3072 FP64
-// 1900 -> 840 us, n = 9000 FP32 5.95 -> 2.81 ms, FP64 11.3 -> 5.0 ms; the batch of 256 chains of
-// 64 .. 1024 beads FP32 6.9 -> 4.4 ms.  Beside another tile on its CU a tile takes 13.4 us for 128
+// (below), right-looking: n = 768 FP64 640 -> 190 us, n = 1353 FP32 720 -> 331 us, n = 3072 FP64
+// 1900 -> 787 us, n = 9000 FP32 5.95 -> 2.79 ms, FP64 11.3 -> 4.94 ms; the batch of 256 chains of
+// 64 .. 1024 beads FP32 6.9 -> 4.0 ms.  Beside another tile on its CU a tile takes 13.4 us for 128
 // columns in FP32 and 28.7 in FP64, MFMA issue at its peak; the rest at n = 9000 is the chain (31
-// us per tile column FP32, 36 FP64) and tiles that become resident too late to have caught up.
+// us per tile column FP32, 33 FP64) and tiles that become resident too late to have caught up.
 //
 // Visibility across XCDs, whose L2 caches are not coherent within a launch: what other
 // workgroups read is stored at agent scope (write-through), the flag that announces it is set
@@ -433,8 +445,10 @@ constexpr int FLOW_T = 128;
 constexpr int FLOW_COL = 2 * LB_STRIDE + CHOL_NB * CHOL_NB;
 constexpr int FLAG_STRIDE = 32;
 
-template <typename T>
+// LOOP: the kernel runs a loop over tasks.
+template <typename T, bool LOOP = false>
 struct FlowMat {
+    __device__ static int tid() { return flow_tid<LOOP || sizeof(T) == 8>(); }
     T* A;
     long long ld;
     int n, nt;   // order (without the identity padding), tile rows
@@ -509,7 +523,7 @@ struct FlowQuiet {
     }
     __device__ void add(int v)
     {
-        if (q && threadIdx.x == 0) __hip_atomic_fetch_add(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (q && flow_tid<true>() == 0) __hip_atomic_fetch_add(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __device__ int busy() const { return q ? __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0; }
     __device__ void pause() const
@@ -566,11 +580,11 @@ struct FlowAcc<double> {
 // array of HIP's own vector class, loaded under a condition, went through scratch memory and each
 // load was waited for at once), and the LDS reads of a product are issued before the MFMAs of the
 // one before: 22.6 -> 13.4 us per 128 columns FP32, 46.5 -> 28.7 FP64.
-template <bool SPLIT>
-__device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, int j, int K, FlowReady& rd,
+template <bool SPLIT, bool LOOP>
+__device__ __forceinline__ void flow_accumulate(const FlowMat<float, LOOP>& M, int i, int j, int K, FlowReady& rd,
                                                 const FlowQuiet& quiet, unsigned char* smem, FlowAcc<float>& acc)
 {
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = M.tid(), lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5;
     const float* C = M.tile(i, j) + 32 * w + l32;
@@ -704,11 +718,11 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<float>& M, int i, 
     }
 }
 
-template <bool SPLIT>
-__device__ __forceinline__ void flow_accumulate(const FlowMat<double>& M, int i, int j, int K, FlowReady& rd,
+template <bool SPLIT, bool LOOP>
+__device__ __forceinline__ void flow_accumulate(const FlowMat<double, LOOP>& M, int i, int j, int K, FlowReady& rd,
                                                 const FlowQuiet& quiet, unsigned char* smem, FlowAcc<double>& acc)
 {
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = M.tid(), lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, lq = lane >> 4;
     const double* C = M.tile(i, j) + 32 * w + lr;
@@ -847,11 +861,11 @@ __device__ __forceinline__ void flow_solve64(doublex4 (&z)[Z][G], int J0, const 
 // Blocks J0 .. J0 + 3 of z (X): their operand copy, published as panel 2 j + J0 / 4 of tile row i,
 // then the tile (i, j) itself, which nobody waits for (stored before the flag it cost the chain
 // 0.4 us a panel in FP64).
-template <typename T>
-__device__ __forceinline__ void flow_store(const FlowMat<T>& M, int i, int j, int J0, const doublex4 (&z)[8][2])
+template <typename T, bool LOOP>
+__device__ __forceinline__ void flow_store(const FlowMat<T, LOOP>& M, int i, int j, int J0, const doublex4 (&z)[8][2])
 {
-    const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
-    const int row = 32 * (threadIdx.x >> 6) + lr;
+    const int lane = M.tid() & 63, lr = lane & 15, lq = lane >> 4;
+    const int row = 32 * (M.tid() >> 6) + lr;
     T* o = const_cast<T*>(M.opnd(i, FLOW_T * j)) + row;   // columns of tile column j: ld apart, as in the tile
     T* t = M.tile(i, j) + row;
 #pragma unroll
@@ -873,12 +887,12 @@ __device__ __forceinline__ void flow_store(const FlowMat<T>& M, int i, int j, in
         }
 }
 
-template <typename T, bool SPLIT>
-__device__ __forceinline__ void flow_tile(const FlowMat<T>& M, int i, int j, unsigned char* smem)
+template <typename T, bool SPLIT, bool LOOP>
+__device__ __forceinline__ void flow_tile(const FlowMat<T, LOOP>& M, int i, int j, unsigned char* smem)
 {
     double* s0 = reinterpret_cast<double*>(smem);   // diagonal block
     double* s1 = s0 + LB_STRIDE;                    // L21
-    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    const int tid = M.tid(), lane = tid & 63, lr = lane & 15, lq = lane >> 4;
     doublex4 z[8][2];
     FlowQuiet quiet(i == j + 1 ? M.quiet : nullptr);
     {
@@ -901,7 +915,7 @@ __device__ __forceinline__ void flow_tile(const FlowMat<T>& M, int i, int j, uns
         for (int u = 0; u < N1; ++u) s1[tid + 256 * u] = v[u];
     }
     flow_solve64<2>(z, 0, s0, s0 + CHOL_NB * CHOL_NB);
-    flow_store<T>(M, i, j, 0, z);   // with a barrier: s1 is complete, s0 free
+    flow_store(M, i, j, 0, z);   // with a barrier: s1 is complete, s0 free
     // z_2 += L21 X_1^T
 #pragma unroll
     for (int K = 0; K < 4; ++K)
@@ -916,7 +930,7 @@ __device__ __forceinline__ void flow_tile(const FlowMat<T>& M, int i, int j, uns
     if (have < 2) flow_wait(M.dprog(j), 2, M.status);
     load_lkk(ws + LB_STRIDE + CHOL_NB * CHOL_NB, s0);
     flow_solve64<2>(z, 4, s0, s0 + CHOL_NB * CHOL_NB);
-    flow_store<T>(M, i, j, 4, z);
+    flow_store(M, i, j, 4, z);
     quiet.add(-1);
 }
 
@@ -1027,13 +1041,13 @@ struct FlowQuad<double> {
 // so that the update that precedes each diagonal block's factor, the last step of the chain, is
 // one block per wavefront: the last 64 columns are applied to the first diagonal block from the
 // LDS, to the others by wavefronts 1 .. 3 while wavefront 0 factors it.
-template <typename T>
-__device__ __forceinline__ void flow_diag(const FlowMat<T>& M, int j, unsigned char* smem)
+template <typename T, bool LOOP>
+__device__ __forceinline__ void flow_diag(const FlowMat<T, LOOP>& M, int j, unsigned char* smem)
 {
     constexpr int KC = sizeof(T) == 4 ? FLOW_KC32 : FLOW_KC64;
     constexpr int P = sizeof(T) == 4 ? FLOW_P32 : FLOW_P64;
     constexpr int V = 16 / sizeof(T);   // entries of one 16-byte access
-    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    const int tid = M.tid(), lane = tid & 63, lr = lane & 15, lq = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     double* s0 = reinterpret_cast<double*>(smem);
     double* s1 = s0 + LB_STRIDE;
@@ -1184,11 +1198,36 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T>& M, int j, unsigned c
     store_diag64<T>(s0, tl, M.ld, CHOL_NB);
 }
 
-template <typename T, bool SPLIT>
-__device__ __forceinline__ void flow_body(const FlowMat<T>& M, int i, int j)
+// The tasks of a batch in the order of their index.  With more of them than workgroups fit on the
+// chip, workgroups stay and take the next index from a counter: left to the dispatcher, which
+// places workgroups in order and waits for room in the shader engine whose turn it is, a sixth of
+// the places stood empty (256 chains of 64 .. 1024 beads FP32: 3.64 -> 3.39 ms).  Indexes are taken
+// in order by running workgroups, so what a workgroup waits for is still finished or running.  One
+// matrix keeps a workgroup per tile: its columns end together, and the loop's extra instructions
+// lie on its chain (n = 9000 FP32 2.79 ms, 2.98 with the loop, FP64 4.94 and 5.27).
+constexpr int FLOW_PLACES = 512;   // two workgroups on each of 256 CUs
+template <typename Body>
+__device__ __forceinline__ void flow_tasks(int* __restrict__ next, int count, Body&& body)
+{
+    __shared__ int s_task;
+    for (;;) {
+        int x = blockIdx.x;
+        if (next) {
+            if (threadIdx.x == 0) s_task = __hip_atomic_fetch_add(next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();   // and the LDS of the task before is free
+            x = __builtin_amdgcn_readfirstlane(s_task);
+        }
+        if (x >= count) break;
+        body(x);
+        if (!next) break;
+    }
+}
+
+template <typename T, bool SPLIT, bool LOOP>
+__device__ __forceinline__ void flow_body(const FlowMat<T, LOOP>& M, int i, int j)
 {
     __shared__ __align__(16) unsigned char smem[FLOW_SMEM];
-    if (i == j) flow_diag<T>(M, j, smem);
+    if (i == j) flow_diag(M, j, smem);
     else flow_tile<T, SPLIT>(M, i, j, smem);
 }
 
@@ -1414,24 +1453,29 @@ std::vector<FlowTask> chol_batch_tasks(const std::vector<int>& n_pad)
 }
 
 template <typename T>
-__device__ __forceinline__ FlowMat<T> flow_mat(T* A, double* Lbuf, const BatchChain& b, int* status)
+__device__ __forceinline__ FlowMat<T, true> flow_mat(T* A, double* Lbuf, const BatchChain& b, int* status)
 {
-    return FlowMat<T>{A + b.mat, b.n_pad, b.n, b.n_pad / FLOW_T, Lbuf + b.lb, status, nullptr};
+    return FlowMat<T, true>{A + b.mat, b.n_pad, b.n, b.n_pad / FLOW_T, Lbuf + b.lb, status, nullptr};
 }
 
 template <typename T, bool SPLIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 chol_flow_batch_kernel(T* __restrict__ A, double* __restrict__ Lbuf, const BatchChain* __restrict__ ch,
-                       const FlowTask* __restrict__ tasks, int* __restrict__ status)
+                       const FlowTask* __restrict__ tasks, int ntasks, int* __restrict__ next,
+                       int* __restrict__ status)
 {
-    const FlowTask t = tasks[blockIdx.x];
-    flow_body<T, SPLIT>(flow_mat(A, Lbuf, ch[t.c], status + t.c), t.i, t.j);
+    flow_tasks(next, ntasks, [&](int x) {
+        const FlowTask t = tasks[x];
+        flow_body<T, SPLIT>(flow_mat(A, Lbuf, ch[t.c], status + t.c), t.i, t.j);
+    });
 }
 
 template <typename T>
-__global__ void chol_flow_clear_batch_kernel(double* __restrict__ Lbuf, const BatchChain* __restrict__ ch)
+__global__ void chol_flow_clear_batch_kernel(double* __restrict__ Lbuf, const BatchChain* __restrict__ ch,
+                                             int* __restrict__ next)
 {
-    const FlowMat<T> M = flow_mat((T*)nullptr, Lbuf, ch[blockIdx.x], nullptr);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *next = 0;
+    const auto M = flow_mat((T*)nullptr, Lbuf, ch[blockIdx.x], nullptr);
     for (int x = threadIdx.x; x < 2 * M.nt * FLAG_STRIDE; x += blockDim.x) M.flags()[x] = 0;
 }
 
@@ -1442,17 +1486,19 @@ int chol_factor_batch(T* d_A, double* d_Lbuf, const BatchPlan& plan, int* d_stat
     BDH_CHECK(syrk_mode != SYRK_BF16X3 || sizeof(T) == 4, "chol_factor_batch: split SYRK needs FP32 storage");
     BDH_CHECK(sizeof(T) == 8 || syrk_mode != SYRK_F64, "chol_factor_batch: FP32 storage needs an FP32 SYRK");
     if (rec) rec->begin(PH_PANEL, st);
-    hipLaunchKernelGGL(chol_flow_clear_batch_kernel<T>, dim3(plan.nch), dim3(256), 0, st, d_Lbuf, plan.ch);
+    hipLaunchKernelGGL(chol_flow_clear_batch_kernel<T>, dim3(plan.nch), dim3(256), 0, st, d_Lbuf, plan.ch,
+                       plan.next);
     BDH_LAUNCH_CHECK();
     if (rec) rec->end(PH_PANEL, st);
     if (rec) rec->begin(PH_SYRK, st);
-    const dim3 grid(plan.ntasks);
+    int* next = plan.ntasks > FLOW_PLACES ? plan.next : nullptr;
+    const dim3 grid(std::min(plan.ntasks, FLOW_PLACES));
     if (sizeof(T) == 4 && syrk_mode == SYRK_BF16X3)
         hipLaunchKernelGGL((chol_flow_batch_kernel<T, sizeof(T) == 4>), grid, dim3(256), 0, st, d_A, d_Lbuf, plan.ch,
-                           plan.tasks, d_status);
+                           plan.tasks, plan.ntasks, next, d_status);
     else
         hipLaunchKernelGGL((chol_flow_batch_kernel<T, false>), grid, dim3(256), 0, st, d_A, d_Lbuf, plan.ch,
-                           plan.tasks, d_status);
+                           plan.tasks, plan.ntasks, next, d_status);
     BDH_LAUNCH_CHECK();
     if (rec) rec->end(PH_SYRK, st);
     return 0;

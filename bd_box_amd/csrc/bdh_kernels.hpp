@@ -59,6 +59,7 @@ struct BatchPlan {
     int asm_blocks = 0, pair_blocks = 0, force_blocks = 0, trmv_blocks = 0, rows_blocks = 0;
     const FlowTask* tasks = nullptr;   // the factorization's workgroups in index order
     int ntasks = 0;
+    int* next = nullptr;               // their counter
 };
 
 // ---- random stream (bdh_rng.hip)
