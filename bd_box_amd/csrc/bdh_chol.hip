@@ -1293,35 +1293,102 @@ size_t chol_lbuf_doubles(int n_pad)
 // X holds m right-hand sides (m <= M, X[k * ldx + c]): with L fixed between refactorizations,
 // the noise of a whole refactor cycle is one pass over L instead of one per step.
 // Tile: (64 lanes x V rows) x TRMV_COLS columns, V = 16 / sizeof(T) so each lane issues one
-// 16-byte load per column; the 4 waves split the tile's columns (unrolled for loads in
-// flight) and meet in LDS.  Entries above the diagonal are masked with a select after the
-// load (the storage there is finite but meaningless), so diagonal tiles take the same
-// vector path.  P[cb][k][r] receives row r's partial of right-hand side k over column
-// block cb (FP64 products and accumulation).
+// 16-byte load per column; the 4 waves split the tile's columns and meet in LDS.  Entries above
+// the diagonal are masked with a select after the load (the storage there is finite but
+// meaningless), so diagonal tiles take the same vector path.  P[cb][k][r] receives row r's
+// partial of right-hand side k over column block cb (FP64 products and accumulation).
+//
+// Bound: reading the lower triangle of L once.  The X values come four columns per scalar load
+// (an index clamped to m - 1 instead of a condition: the sums beyond m are not stored), and the
+// next columns of L are in flight during the sums.  With a condition around each X value, one
+// load and one branch per value, and without loads ahead, ten right-hand sides took at n = 9000
+// 70 us in FP32 and 89 in FP64; now 41 and 68 (162 and 324 MB: 3.9 and 4.7 TB/s).  One
+// right-hand side at n = 768 in FP64: 8.0 -> 5.9 us.
 constexpr int TRMV_COLS = 256;
 
-template <typename T, int M>
-__device__ __forceinline__ void trmv_accum(const T* __restrict__ col, int rbase, int c,
-                                           const double* __restrict__ xc, bool mask,
-                                           double (*acc)[M])
+template <typename T>
+using trmv_vec = T __attribute__((ext_vector_type(16 / sizeof(T))));
+
+// Column c's entries of a lane's V rows.  In a tile on the diagonal the lanes whose rows all
+// lie above it read the diagonal's own entry again instead of memory that the sum masks out.
+template <typename T, bool MASK>
+__device__ __forceinline__ trmv_vec<T> trmv_load(const T* __restrict__ col, int rbase, int c)
 {
     constexpr int V = 16 / sizeof(T);
-    double v[V];
-    if constexpr (V == 4) {
-        const float4 w = *reinterpret_cast<const float4*>(col + rbase);
-        v[0] = (!mask || rbase + 0 >= c) ? (double)w.x : 0.0;
-        v[1] = (!mask || rbase + 1 >= c) ? (double)w.y : 0.0;
-        v[2] = (!mask || rbase + 2 >= c) ? (double)w.z : 0.0;
-        v[3] = (!mask || rbase + 3 >= c) ? (double)w.w : 0.0;
-    } else {
-        const double2 w = *reinterpret_cast<const double2*>(col + rbase);
-        v[0] = (!mask || rbase + 0 >= c) ? w.x : 0.0;
-        v[1] = (!mask || rbase + 1 >= c) ? w.y : 0.0;
+    return *reinterpret_cast<const trmv_vec<T>*>(col + (MASK ? max(rbase, c & -V) : rbase));
+}
+
+template <typename T, int M, bool MASK>
+__device__ __forceinline__ void trmv_accum(trmv_vec<T> w, int rbase, int c,
+                                           const double* __restrict__ xc, double (*acc)[M])
+{
+    constexpr int V = 16 / sizeof(T);
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+        const double v = (!MASK || rbase + q >= c) ? (double)w[q] : 0.0;
+#pragma unroll
+        for (int k = 0; k < M; ++k) acc[q][k] += v * xc[k];
     }
+}
+
+// One wavefront's columns c .. c_hi - 1 of a tile, UNR at a time; the next UNR columns' loads
+// are in flight while these are summed.
+template <typename T, int M, bool MASK>
+__device__ __forceinline__ void trmv_columns(const T* __restrict__ L, long long ld, int rbase, int c,
+                                             int c_hi, const double* __restrict__ X, long long ldx,
+                                             int m, double (*acc)[M])
+{
+    constexpr int UNR = M >= 4 ? 4 : 8;
+    trmv_vec<T> w[UNR];
+    if (c + UNR <= c_hi) {
 #pragma unroll
-    for (int q = 0; q < V; ++q)
+        for (int u = 0; u < UNR; ++u)
+            w[u] = trmv_load<T, MASK>(L + (long long)(c + u) * ld, rbase, c + u);
+    }
+    for (; c + UNR <= c_hi; c += UNR) {
+        trmv_vec<T> wn[UNR];
+        // past the last whole group: this group's columns again, so the loads need no branch
+        const int cn = c + 2 * UNR <= c_hi ? c + UNR : c;
 #pragma unroll
-        for (int k = 0; k < M; ++k) acc[q][k] += v[q] * xc[k];
+        for (int u = 0; u < UNR; ++u)
+            wn[u] = trmv_load<T, MASK>(L + (long long)(cn + u) * ld, rbase, cn + u);
+        double xc[UNR][M];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u)
+#pragma unroll
+            for (int k = 0; k < M; ++k) xc[u][k] = X[min(k, m - 1) * ldx + c + u];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) trmv_accum<T, M, MASK>(w[u], rbase, c + u, xc[u], acc);
+        // without it the next group's loads are waited for before this group's sums
+        if constexpr (M >= 4) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) w[u] = wn[u];
+    }
+    for (; c < c_hi; ++c) {
+        double xc[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) xc[k] = X[min(k, m - 1) * ldx + c];
+        trmv_accum<T, M, MASK>(trmv_load<T, MASK>(L + (long long)c * ld, rbase, c), rbase, c, xc, acc);
+    }
+}
+
+// Right-hand sides K .. m - 1 of a tile: the four wavefronts' sums meet in alternate halves of
+// s_red, one barrier each (every thread that passes it has read the half written next).  A
+// recursion, since with k a variable the sums would have to be indexed at run time.
+template <int K, int V, int M>
+__device__ __forceinline__ void trmv_store(double (*acc)[M], int m, double (*s_red)[4][64 * V], int wave,
+                                           int lane, double* __restrict__ P, int n, int r0)
+{
+    if constexpr (K < M) {
+        if (K >= m) return;
+        double(*red)[64 * V] = s_red[K & 1];
+#pragma unroll
+        for (int q = 0; q < V; ++q) red[wave][lane * V + q] = acc[q][K];
+        __syncthreads();
+        for (int rr = threadIdx.x; rr < 64 * V && r0 + rr < n; rr += 256)
+            P[(long long)K * n + r0 + rr] = (red[0][rr] + red[1][rr]) + (red[2][rr] + red[3][rr]);
+        trmv_store<K + 1, V, M>(acc, m, s_red, wave, lane, P, n, r0);
+    }
 }
 
 template <typename T, int M>
@@ -1331,10 +1398,9 @@ __device__ __forceinline__ void trmv_partial_body(const T* __restrict__ L, long 
 {
     constexpr int V = 16 / sizeof(T);
     constexpr int ROWS = 64 * V;
-    constexpr int UNR = M >= 8 ? 4 : (M >= 4 ? 4 : 8);
     const int r0 = rb * ROWS, cbeg = cb * TRMV_COLS;
     if (cbeg > r0 + ROWS - 1 || cbeg >= n) return;  // tile entirely above the diagonal
-    __shared__ double s_red[4][ROWS];
+    __shared__ double s_red[2][4][ROWS];
     // the wavefront index is uniform: its columns, and so the X values, come through the
     // scalar cache into SGPRs instead of one vector load per lane
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1344,47 +1410,18 @@ __device__ __forceinline__ void trmv_partial_body(const T* __restrict__ L, long 
     for (int q = 0; q < V; ++q)
 #pragma unroll
         for (int k = 0; k < M; ++k) acc[q][k] = 0.0;
-    const int cend = min(n, cbeg + TRMV_COLS);
     const int wcols = TRMV_COLS / 4;
+    // columns beyond the tile's last row hold nothing of the lower triangle
+    const int cend = min(min(n, cbeg + TRMV_COLS), r0 + ROWS);
     const int c_lo = cbeg + wave * wcols, c_hi = min(cend, c_lo + wcols);
     // the whole tile is below the diagonal when its last column precedes its first row
-    const bool mask = (cbeg + TRMV_COLS - 1) > r0;
     if (rbase < n) {
-        int c = c_lo;
-        for (; c + UNR <= c_hi; c += UNR) {
-            double xc[UNR][M];
-#pragma unroll
-            for (int u = 0; u < UNR; ++u)
-#pragma unroll
-                for (int k = 0; k < M; ++k) xc[u][k] = (k < m) ? X[k * ldx + c + u] : 0.0;
-#pragma unroll
-            for (int u = 0; u < UNR; ++u)
-                trmv_accum<T, M>(L + (long long)(c + u) * ld, rbase, c + u, xc[u], mask, acc);
-        }
-        for (; c < c_hi; ++c) {
-            double xc[M];
-#pragma unroll
-            for (int k = 0; k < M; ++k) xc[k] = (k < m) ? X[k * ldx + c] : 0.0;
-            trmv_accum<T, M>(L + (long long)c * ld, rbase, c, xc, mask, acc);
-        }
+        if (cbeg + TRMV_COLS - 1 > r0)
+            trmv_columns<T, M, true>(L, ld, rbase, c_lo, c_hi, X, ldx, m, acc);
+        else
+            trmv_columns<T, M, false>(L, ld, rbase, c_lo, c_hi, X, ldx, m, acc);
     }
-    for (int k = 0; k < m; ++k) {
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < V; ++q) {
-            double a = 0.0;
-#pragma unroll
-            for (int kk = 0; kk < M; ++kk) a = (kk == k) ? acc[q][kk] : a;
-            s_red[wave][lane * V + q] = a;
-        }
-        __syncthreads();
-        for (int rr = tid; rr < ROWS; rr += 256) {
-            const int row = r0 + rr;
-            if (row < n)
-                P[((long long)cb * m + k) * n + row] =
-                    (s_red[0][rr] + s_red[1][rr]) + (s_red[2][rr] + s_red[3][rr]);
-        }
-    }
+    trmv_store<0, V, M>(acc, m, s_red, wave, lane, P + (long long)cb * m * n, n, r0);
 }
 
 template <typename T, int M>
@@ -1504,8 +1541,13 @@ int chol_factor_batch(T* d_A, double* d_Lbuf, const BatchPlan& plan, int* d_stat
     return 0;
 }
 
+// At least four wavefronts a SIMD for up to ten right-hand sides (128 registers, five of them
+// spilled in FP32): a batch has tiles for many rounds of workgroups, and their number in flight
+// hides the tiles' starts and ends.  256 chains of 64 .. 1024 beads, ten sides, FP32: 278 us
+// with the 133 registers the compiler takes by itself, 255 with 128; the launch of one matrix is
+// a single round and measured 41 -> 46 us at n = 9000, so it keeps its registers.
 template <typename T, int M>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, M <= 10 ? 4 : 2)
 trmv_batch_kernel(const T* __restrict__ A, const double* __restrict__ X, long long x_stride, int m,
                   const BatchChain* __restrict__ ch, const int* __restrict__ prefix, int nch,
                   double* __restrict__ Pt)
