@@ -457,7 +457,7 @@ int assemble_and_factor_launches(bdh_system* s, void* Abuf, const double4* pos2)
 
 // D at the current positions (with pos2: the mean of the tensors at both sets of positions)
 // into Abuf (default: the system's matrix), factored in place.  The refactor of the system's
-// own matrix (the same ~150 launches with the same arguments every time) is captured into a
+// own matrix (the same few launches with the same arguments every time) is captured into a
 // HIP graph on first use and replayed afterwards; phase timing runs the launches directly.
 int assemble_and_factor(bdh_system* s, void* Abuf = nullptr, const double4* pos2 = nullptr)
 {
@@ -2188,7 +2188,7 @@ int batch_forces(bdh_batch* b)
 
 int batch_factor_launches(bdh_batch* b);
 
-// The refactor of every chain (the same ~50 launches with the same arguments each time) is
+// The refactor of every chain (the same few launches with the same arguments each time) is
 // captured into a HIP graph on first use and replayed; phase timing runs the launches.
 int batch_factor(bdh_batch* b)
 {
@@ -2225,9 +2225,8 @@ int batch_set_tiles(bdh_batch* b, int left_max, int outer)
 
 int batch_set_schedule(bdh_batch* b, int left_max) { return batch_set_tiles(b, left_max, b->outer); }
 
-// Candidate schedules: all right-looking (0), then left-looking for the chains up to each
-// of at most BDH_TUNE_MAX - 1 of the batch's distinct padded sizes (evenly spaced in sorted
-// order, the largest always included, which makes every chain left-looking).
+// Candidate left_max values: 0, then at most BDH_TUNE_MAX - 1 of the batch's distinct padded
+// sizes (evenly spaced in sorted order, the largest always included).
 std::vector<int> batch_tune_candidates(const bdh_batch* b)
 {
     std::vector<int> sizes;
@@ -2240,10 +2239,10 @@ std::vector<int> batch_tune_candidates(const bdh_batch* b)
     return cand;
 }
 
-// Each candidate (left_max, outer): one refactor to capture its graph, then `reps` timed
-// replays (HIP events on the batch's stream); its time is the fastest replay.  Every replay
-// recomputes the same matrices from the unchanged positions, so the candidates see identical
-// work.  The fastest candidate is kept.
+// Each candidate (left_max, outer): one refactor, then `reps` timed ones (HIP events on the
+// batch's stream); its time is the fastest.  Every one recomputes the same matrices from the
+// unchanged positions with the same launches, so the times differ by noise only; the fastest
+// candidate is kept.
 int batch_tune(bdh_batch* b, int reps, const std::vector<std::pair<int, int>>& cand, int* ib_out,
                std::vector<double>& t)
 {
@@ -2295,7 +2294,7 @@ int batch_autotune(bdh_batch* b, int reps, int* cand_out, double* ms_out, int* n
     return 0;
 }
 
-// The schedules of batch_tune_candidates under each outer panel width 256, 512 and 1024
+// The values of batch_tune_candidates under each outer panel width 256, 512 and 1024
 // (widths no wider than the largest chain's padded order).
 int batch_autotune_tiles(bdh_batch* b, int reps, int* cand_left, int* cand_outer, double* ms_out,
                          int* ncand, int* best)
@@ -2382,7 +2381,7 @@ int batch_cycle(bdh_batch* b, int m, bool refactor, const double* X, long long x
 }
 
 // Steps of every chain.  A whole refactor cycle on the device streams is one graph launch:
-// its ~(50 + 5 R) launches (the chains' Gaussians, assembly and factorization, L.xi of the
+// its launches, about five a step (the chains' Gaussians, assembly and factorization, L.xi of the
 // cycle, then per step D.F, move and forces) are captured on first use and replayed; every
 // argument (pointers, grid sizes, the stream counters kept in device memory) is the same from
 // one cycle to the next.  Partial cycles, given Gaussians and phase timing run the launches.

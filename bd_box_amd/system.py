@@ -401,8 +401,8 @@ class BDBatch:
         return {p: (float(ms[i]), int(cnt[i])) for i, p in enumerate(BDSystem.PHASES)}
 
     def set_schedule(self, left_max: int):
-        """Chains with padded size n_pad <= left_max factor with left-looking updates inside
-        each outer panel, the others right-looking; -1 restores the single-system choice."""
+        """Keeps left_max for schedule(); the factorization has one schedule, so the launches
+        and the results are the same for every value."""
         _lib.check(_lib.load().bdh_batch_set_schedule(self._h, int(left_max)), "set_schedule")
 
     def schedule(self) -> int:

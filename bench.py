@@ -80,19 +80,8 @@ def batch_workload(count, seed):
 
 
 # ----------------------------------------------------------------------------- roofline
-def syrk_flops_per_factor(n, n_pad, nb=64):
-    """Algorithmic flops of the trailing updates of one factorization (lower triangle
-    only, unpadded size): sum over 64-column panels of nb * m (m + 1), m = rows below the
-    panel.  The two-level schedule applies exactly these updates, grouped differently."""
-    f = 0
-    for c0 in range(0, n_pad, nb):
-        m = max(0, n - (c0 + nb))
-        f += nb * m * (m + 1)
-    return f
-
-
 def measured_traffic(kernel, path=TRAFFIC_FILE):
-    """HBM bytes per launch of `kernel` (the kernel's symbol, e.g. "syrk_f32_kernel<false>")
+    """HBM bytes per launch of `kernel` (the kernel's symbol, e.g. "chol_flow_kernel<float, false>")
     from the committed rocprofv3 counter summary, with the counter run's command."""
     try:
         with open(path) as f:
@@ -125,7 +114,7 @@ def _counter_rows(d):
 
 
 def _short_kernel(name):
-    """'void bdh::chol_epoch_f32_kernel<false>(float*, ...)' -> 'chol_epoch_f32_kernel<false>'."""
+    """'void bdh::chol_flow_kernel<float, false>(...)' -> 'chol_flow_kernel<float, false>'."""
     name = name.strip().replace("(anonymous namespace)::", "")
     if name.startswith("void "):
         name = name[5:]
@@ -181,47 +170,8 @@ def summarize_traffic(fetch_dir, write_dir, out_path, command):
     print(json.dumps({k: round(v["hbm_bytes_per_launch"]) for k, v in kernels.items()}))
 
 
-def update_steps(n_pad, nb=64, outer=256, left_max=4096):
-    """(kb, K, t0, t1) of each update launch of one factorization: inside an outer panel
-    the next panel's columns (n_pad <= left_max: left-looking, all of the outer panel's
-    panels so far) or the outer panel's remaining columns (one panel); at its end the whole
-    trailing matrix with the outer panel."""
-    out = []
-    k = 0
-    while True:
-        c0 = k * nb
-        t0 = c0 + nb
-        if t0 >= n_pad:
-            return out
-        P0 = c0 // outer * outer
-        P1 = min(n_pad, P0 + outer)
-        if t0 < P1 and n_pad <= left_max:
-            out.append((P0, c0 + nb - P0, t0, t0 + nb))
-        elif t0 < P1:
-            out.append((c0, nb, t0, P1))
-        else:
-            out.append((P0, P1 - P0, t0, n_pad))
-        k += 1
-
-
-def update_bytes_per_factor(n_pad, word=4, left_max=4096, outer=256):
-    """Algorithmic HBM bytes of one factorization's update launches: every updated C entry
-    (rows t0..n_pad, columns t0..t1, lower part) read and written once, and the operand rows
-    t0..n_pad x K read once per launch."""
-    b = 0
-    for kb, K, t0, t1 in update_steps(n_pad, outer=outer, left_max=left_max):
-        rows = n_pad - t0
-        w = t1 - t0
-        c_entries = w * rows - w * (w - 1) // 2
-        b += 2 * word * c_entries + word * rows * K
-    return b
-
-
-SYRK_KERNEL = {"fp64": "syrk_f64_kernel", "f32": "syrk_f32_kernel<false>",
-               "split": "syrk_f32_kernel<true>"}
-EPOCH_KERNEL = {"fp64": "chol_epoch_f64_kernel", "f32": "chol_epoch_f32_kernel<false>",
-                "split": "chol_epoch_f32_kernel<true>"}
-CHOL_EPOCH_MIN = 1024   # n_pad from which the factorization runs as one launch per outer panel
+CHOL_KERNEL = {"fp64": "chol_flow_kernel<double, false>", "f32": "chol_flow_kernel<float, false>",
+               "split": "chol_flow_kernel<float, true>"}
 
 
 def chol_flops(n):
@@ -231,7 +181,6 @@ def chol_flops(n):
 
 def roofline(phases, n, mode, refactors):
     """Roofline of the phase with the largest share of the timed run."""
-    n_pad = -(-n // 128) * 128
     s = 8 if mode == "fp64" else 4
     dom = max(phases, key=lambda k: phases[k][0])
     ms, cnt = phases[dom]
@@ -241,19 +190,12 @@ def roofline(phases, n, mode, refactors):
         # three products per FP32 product (split: the ceiling is a third of the bf16 peak)
         peak = {"fp64": PEAK_TFLOPS["f64_mfma"], "f32": PEAK_TFLOPS["f32_mfma"],
                 "split": PEAK_TFLOPS["bf16_mfma"] / 3.0}[mode]
-        if n_pad >= CHOL_EPOCH_MIN:
-            # one launch per 256-column outer panel does the whole factorization (diagonal
-            # blocks, panel solves, trailing updates)
-            kern = EPOCH_KERNEL[mode]
-            fl = chol_flops(n) * refactors
-            basis = (f"n={n}: n^3/3 + n^2/2 + n/6 flops per factorization (every flop of the "
-                     f"factorization runs in these launches), {refactors} factorizations / "
-                     f"{cnt} launches of {kern}")
-        else:
-            kern = SYRK_KERNEL[mode]
-            fl = syrk_flops_per_factor(n, n_pad) * refactors
-            basis = (f"n={n}: sum over 64-wide panels of 64 m (m+1) flops (lower-triangle "
-                     f"trailing updates), {refactors} factorizations / {cnt} launches of {kern}")
+        # one launch does the whole factorization
+        kern = CHOL_KERNEL[mode]
+        fl = chol_flops(n) * refactors
+        basis = (f"n={n}: n^3/3 + n^2/2 + n/6 flops per factorization (every flop of the "
+                 f"factorization runs in these launches), {refactors} factorizations / "
+                 f"{cnt} launches of {kern}")
         achieved = fl / (ms * 1e-3) / 1e12
         out["kernel_symbol"] = kern
         if mode == "split":
@@ -443,8 +385,8 @@ def main():
     ap.add_argument("--traffic-command", default="",
                     help="with --summarize-traffic: the commands that made the counter runs")
     ap.add_argument("--no-autotune", dest="autotune", action="store_false",
-                    help="batch workload: keep the single-system update schedule instead of "
-                         "timing the candidates before the run")
+                    help="batch workload: do not time the candidates of update schedule and panel "
+                         "width before the run (they give the same launches and results)")
     args = ap.parse_args()
     if args.summarize_traffic:
         return summarize_traffic(*args.summarize_traffic, args.traffic_command)
@@ -762,7 +704,7 @@ def bench_batch(args):
     """Steps/s of a batch of independent chains (every chain advances one step per step),
     mixed (FP32 MFMA trailing updates, FP64 diagonal blocks) beside FP64 and split-bf16,
     each phase one launch over all chains and every full refactor cycle one graph launch;
-    tile shapes (update schedule, outer panel width) chosen by the autotuner per precision."""
+    the autotuner's candidates (update schedule, outer panel width) timed per precision."""
     import torch
     from bd_box_amd.system import BDBatch, FP64, MIXED, MIXED_SPLIT
     systems, prm, P, seeds = batch_workload(args.chains, args.seed)
@@ -813,19 +755,15 @@ def bench_batch(args):
     ph = out["mixed"][1]
     cyc = 2 * R
     ms, cnt = ph["syrk"]
-    fl = sum(syrk_flops_per_factor(3 * N, -(-3 * N // 128) * 128) for N in sizes) * 2
-    lm = sched["mixed"]["left_max"] if "mixed" in sched else 4096
-    ow = sched["mixed"]["outer"] if "mixed" in sched else 256
-    by = sum(update_bytes_per_factor(-(-3 * N // 128) * 128, left_max=lm, outer=ow) for N in sizes) * 2
-    ach = by / (ms * 1e-3) / 1e9
-    tr, _ = measured_traffic("syrk_f32_batch_kernel<false>", TRAFFIC_FILE_BATCH)
-    roof = {"kernel": "syrk", "launches": cnt, "avg_ms": ms / max(cnt, 1), "bound": "hbm",
-            "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
-            "traffic": tr, "mfma_tflops": fl / (ms * 1e-3) / 1e12,
-            "mfma_frac": fl / (ms * 1e-3) / 1e12 / PEAK_TFLOPS["f32_mfma"],
-            "basis": "sum over chains and update launches of the updated lower-trapezoid C "
-                     "entries read and written (FP32) plus the K-column operand rows read once, "
-                     "2 factorizations; traffic = measured HBM bytes per launch"}
+    fl = sum(chol_flops(3 * N) for N in sizes) * 2
+    ach = fl / (ms * 1e-3) / 1e12
+    tr, _ = measured_traffic("chol_flow_batch_kernel<float, false>", TRAFFIC_FILE_BATCH)
+    roof = {"kernel": "syrk", "launches": cnt, "avg_ms": ms / max(cnt, 1), "bound": "mfma",
+            "achieved": ach, "peak": PEAK_TFLOPS["f32_mfma"], "unit": "TFLOP/s",
+            "frac": ach / PEAK_TFLOPS["f32_mfma"], "traffic": tr,
+            "kernel_symbol": "chol_flow_batch_kernel<float, false>",
+            "basis": "n^3/3 + n^2/2 + n/6 flops of every chain's factorization (one launch does "
+                     "them all), 2 factorizations; traffic = measured HBM bytes per launch"}
     value = out["mixed"][0]
     line = {
         "metric": f"BD steps/s, batch of {len(sizes)} chains N~logU[64,1024] RPY+Cholesky",
@@ -837,7 +775,7 @@ def bench_batch(args):
                                f"refactored every {R} steps, FP32 MFMA trailing updates, FP64 "
                                f"diagonal blocks, each refactor cycle one graph launch",
                    "chains": len(sizes), "beads": Ntot, "refactor_every": R,
-                   "update_schedule": sched or "single-system default (left_max 4096)",
+                   "update_schedule": sched or "one schedule, not timed",
                    "parallelism": "1 GPU"},
         "chain_steps_per_s": value * len(sizes),
         "bead_steps_per_s": value * Ntot,
