@@ -562,7 +562,12 @@ static_assert(2 * 2 * FLOW_KC32 * FLOW_P32 * 4 <= FLOW_SMEM && 2 * 2 * FLOW_KC64
 // 128 columns, transposed (the MFMA row index runs over the tile's columns): FP32 four 32x32 blocks,
 // FP64 8 x 2 16x16 blocks.  FP32 keeps C - sum in m and adds a partial sum of at most FLOW_FLUSH
 // columns to it at a time, so a partial sum's rounding is relative to that part alone (the
-// rounding of a C updated once per 256 columns); FP64 accumulates on -C.
+// rounding of a C updated once per 256 columns); FP64 accumulates on -C: one register set, and a
+// rounding of what remains of C per 4 columns.  Measured for the chains' tensors against sums in
+// extended precision: rms residual of an entry below the diagonal up to 5e-17 of the tensor's
+// largest entry (n = 768), ||(L - L_LAPACK) x|| / ||L x|| 1.2e-15 at n = 768 and 5.6e-15 at n = 9000 (with
+// C updated in memory once per 256 columns 3e-16 and 7e-16; that fold inside this loop costs
+// 190 -> 205 us and 5.05 -> 6.09 ms, every 1024 columns 5.19 ms for half of the difference).
 constexpr int FLOW_FLUSH = 256;
 template <typename T>
 struct FlowAcc;
