@@ -259,23 +259,24 @@ __device__ __forceinline__ void recip_sum(const EwaldTables& E, double rx, doubl
 // Real-space images r + L (h, f, g) with h^2 + f^2 + g^2 <= RR, h, then f, then g ascending, within
 // sqrt(rc2) of the pair: image(x, y, z, r2) for each.  A column (h, f) that lies beyond the cutoff
 // for every pair of the wavefront is skipped whole.
+// Every coordinate is formed from its index with one rounding.  A coordinate stepped by L from r - R L
+// carries the rounding at R L: the pair (i, i) then misses its central image's zero for most boxes
+// that are not exact in a few bits, and near images lose bits in all of them.
 template <typename T, typename F>
 __device__ __forceinline__ void each_image(const double box, const int RR, const T rc2, double rx, double ry,
                                            double rz, F&& image)
 {
     const int R = isqrt_small(RR);
-    double dx = rx - box * R;
-    for (int h = -R; h <= R; ++h, dx += box) {
-        const T x = (T)dx;
+    for (int h = -R; h <= R; ++h) {
+        const T x = (T)__builtin_fma(box, (double)h, rx);
         const int nf = isqrt_small(RR - h * h);
-        double dy = ry - box * nf;
-        for (int f = -nf; f <= nf; ++f, dy += box) {
-            const T y = (T)dy, rho = x * x + y * y;
+        for (int f = -nf; f <= nf; ++f) {
+            const T y = (T)__builtin_fma(box, (double)f, ry), rho = x * x + y * y;
             if (!__any(rho <= rc2)) continue;
             const int ng = isqrt_small(RR - h * h - f * f);
-            double dz = rz - box * ng;
-            for (int g = -ng; g <= ng; ++g, dz += box) {
-                const T z = (T)dz, r2 = rho + z * z;
+            double gd = -ng;
+            for (int g = -ng; g <= ng; ++g, gd += 1.0) {
+                const T z = (T)__builtin_fma(box, gd, rz), r2 = rho + z * z;
                 if (r2 != (T)0 && r2 <= rc2) image(x, y, z, r2);
             }
         }

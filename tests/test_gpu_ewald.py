@@ -144,3 +144,26 @@ def test_pair_sums_vs_tensor(api, N, method):
         err = np.linalg.norm(b.compute_Rf() - ref) / np.linalg.norm(ref)
         assert err <= tol, (prec, err)
         b.close()
+
+
+@pytest.mark.parametrize("box", [1000.1, 999.9, 850.3, 640.0])
+@pytest.mark.parametrize("R,ext", [(2, None), (3, None), (4, None), (5, None), (2, (1.25, 3, 3, 0.0)),
+                                   (2, (0.8, 4, 2, 0.0)), (2, (1.0, 5, 1, 2.1))])
+def test_ewald_tensor_any_box(api, box, R, ext):
+    """Box edges with no short binary form (a .prm file's are rounded to 24 bits, a caller's own are
+    not), where R L is inexact: a bead's own central image is left out all the same.  The bounds
+    of test_ewald_tensor_vs_numpy."""
+    s, P = _spheres(40, 0.05, 5, "beenakker", R)
+    s.coord[:, :3] *= box / P.box
+    P.box = box
+    if ext:
+        ext = ext[:3] + (ext[3] * box,)
+    ref = _plain(s, P, ext)
+    print("ewald tensor", box, R, ext, flush=True)
+    for prec, tol in ((api.FP64, 2e-13), (api.MIXED, 1e-6)):
+        b = api.BDSystem(s, P, precision=prec)
+        if ext:
+            b.set_ewald_split(ext[0], ext[1], ext[2], r_cut=ext[3])
+        err = np.abs(b.compute_D() - ref).max() / np.abs(ref).max()
+        assert err <= tol, (prec, err)
+        b.close()
