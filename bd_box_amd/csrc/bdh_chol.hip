@@ -421,8 +421,8 @@ __device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long
 // overlaps with everything else, since the workgroups of the following tile columns are
 // resident and accumulate what is already published.
 // Measured against one launch per 256-column outer panel (n_pad >= 1024) or per 64-column panel
-// (below), right-looking: n = 768 FP64 640 -> 190 us, n = 1353 FP32 720 -> 331 us, n = 3072 FP64
-// 1900 -> 787 us, n = 9000 FP32 5.95 -> 2.79 ms, FP64 11.3 -> 4.94 ms; the batch of 256 chains of
+// (below), right-looking: n = 768 FP64 640 -> 202 us, n = 1353 FP32 720 -> 331 us, n = 3072 FP64
+// 1900 -> 840 us, n = 9000 FP32 5.95 -> 2.82 ms, FP64 11.3 -> 5.7 ms; the batch of 256 chains of
 // 64 .. 1024 beads FP32 6.9 -> 4.0 ms.  Beside another tile on its CU a tile takes 13.4 us for 128
 // columns in FP32 and 28.7 in FP64, MFMA issue at its peak; the rest at n = 9000 is the chain (31
 // us per tile column FP32, 33 FP64) and tiles that become resident too late to have caught up.
@@ -560,14 +560,17 @@ static_assert(2 * 2 * FLOW_KC32 * FLOW_P32 * 4 <= FLOW_SMEM && 2 * 2 * FLOW_KC64
 
 // The accumulated sums of a tile, per wavefront w rows 32 w .. 32 w + 31 of tile row i and all
 // 128 columns, transposed (the MFMA row index runs over the tile's columns): FP32 four 32x32 blocks,
-// FP64 8 x 2 16x16 blocks.  FP32 keeps C - sum in m and adds a partial sum of at most FLOW_FLUSH
-// columns to it at a time, so a partial sum's rounding is relative to that part alone (the
-// rounding of a C updated once per 256 columns); FP64 accumulates on -C: one register set, and a
-// rounding of what remains of C per 4 columns.  Measured for the chains' tensors against sums in
-// extended precision: rms residual of an entry below the diagonal up to 5e-17 of the tensor's
-// largest entry (n = 768), ||(L - L_LAPACK) x|| / ||L x|| 1.2e-15 at n = 768 and 5.6e-15 at n = 9000 (with
-// C updated in memory once per 256 columns 3e-16 and 7e-16; that fold inside this loop costs
-// 190 -> 205 us and 5.05 -> 6.09 ms, every 1024 columns 5.19 ms for half of the difference).
+// FP64 8 x 2 16x16 blocks.  A partial sum of at most FLOW_FLUSH columns starts from zero and is
+// then taken from C as a whole, so that its rounding is relative to that part alone: FP32 keeps
+// C - sum in m; FP64 has registers for one set, and C - sum stays in the tile's own entries of A.
+// Errors ||(A - L L^T) x|| / ||A x|| in extended precision, tensors of chains and of periodic
+// suspensions, N = 60 .. 3000: 1.9e-16 .. 2.9e-16 and 2.2e-16 .. 4.3e-16; with C updated by a launch
+// per 256 columns 2.0e-16 .. 3.2e-16 and 2.4e-16 .. 4.4e-16.  Accumulating on -C, without a pass over
+// C in memory: 7.2e-16 at n = 768, 2.9e-15 at n = 9000.  From zero, but with no pass in between: 4.6e-16
+// at n = 9000; with one every 512 columns 4.2e-16 at n = 2100, periodic (3.0e-16 as here).
+// FP64 us on -C / as here: n = 768 196 / 202, 1353 361 / 371, 3072 812 / 840, 4500 1270 / 1350, 9000
+// 5050 / 5680; the batch of 256 chains 6.4 / 6.9 ms.  A pass moves 256 kB a tile every 57 us; one
+// block at a time beside the stages' products it spills (n = 9000 7.1 ms), as FP64 atomics 5.8 ms.
 constexpr int FLOW_FLUSH = 256;
 template <typename T>
 struct FlowAcc;
@@ -578,6 +581,24 @@ struct FlowAcc<float> {
 template <>
 struct FlowAcc<double> {
     doublex4 a[8][2];
+};
+
+// Lane l's entries of FP64 tiles: (column c, row r) of a tile at t is entry (c + l / 16, r + l % 16).
+// One 32-bit offset a lane beside addresses that are the same for all lanes, all of them formed where
+// they are used: taken out of the loop they would spill.
+struct FlowLane {
+    unsigned off;
+    long long ld;
+    __device__ explicit FlowLane(long long ld_) : ld(ld_)
+    {
+        asm volatile("" : "+s"(ld));
+        const int l = flow_tid<true>() & 63;
+        off = ((unsigned)(l >> 4) * (unsigned)ld + (l & 15)) * (unsigned)sizeof(double);
+    }
+    __device__ double* operator()(double* t, int c, int r) const
+    {
+        return reinterpret_cast<double*>(reinterpret_cast<char*>(t + c * ld) + off) + r;
+    }
 };
 
 // Sums over the K columns 0 .. K - 1 (K a multiple of 128) of tile (i, j) into acc.  The next
@@ -730,15 +751,57 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<double, LOOP>& M, 
     const int tid = M.tid(), lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, lq = lane >> 4;
-    const double* C = M.tile(i, j) + 32 * w + lr;
+    double* C = M.tile(i, j) + 32 * w;
+    const int nc = K / FLOW_KC64;
 #pragma unroll
     for (int J = 0; J < 8; ++J)
 #pragma unroll
-        for (int g = 0; g < 2; ++g)
+        for (int g = 0; g < 2; ++g) acc.a[J][g] = doublex4{0.0, 0.0, 0.0, 0.0};
+    // acc -= C, the loads of four blocks in flight together
+    auto less_c = [&] {
+        const FlowLane at(M.ld);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc.a[J][g][r] = -C[(long long)(16 * J + 4 * r + lq) * M.ld + 16 * g];
-    const int nc = K / FLOW_KC64;
-    if (nc == 0) return;
+        for (int J0 = 0; J0 < 8; J0 += 4) {
+            double v[4][4][2];
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) v[x][r][g] = *at(C, 16 * (J0 + x) + 4 * r, 16 * g);
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) acc.a[J0 + x][g][r] -= v[x][r][g];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // C -= acc, two blocks at a time (more of them spill); acc starts anew
+    auto fold = [&] {
+        const FlowLane at(M.ld);
+#pragma unroll
+        for (int J = 0; J < 8; ++J) {
+            double v[4][2];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) v[r][g] = *at(C, 16 * J + 4 * r, 16 * g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    *at(C, 16 * J + 4 * r, 16 * g) = v[r][g] - acc.a[J][g][r];
+                    acc.a[J][g][r] = 0.0;
+                }
+            if (J & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (nc == 0) {
+        less_c();
+        return;
+    }
     auto need = [](int c) { return c * FLOW_KC64 / CHOL_NB + 1; };
     double (*st)[2][FLOW_KC64][FLOW_P64] = reinterpret_cast<double (*)[2][FLOW_KC64][FLOW_P64]>(smem);
     constexpr int NV = FLOW_KC64 * FLOW_T / 2 / 256;
@@ -788,6 +851,7 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<double, LOOP>& M, 
                 for (int g = 0; g < 2; ++g) acc.a[J][g] = mfma_f64_16x16x4(a[s & 1][J], b[s & 1][g], acc.a[J][g]);
             __builtin_amdgcn_sched_barrier(0);
         }
+        if (more && (c + 1) % (FLOW_FLUSH / FLOW_KC64) == 0) fold();
         if (busy) quiet.pause();
         if (more) {
             if (!pre) {
@@ -798,6 +862,7 @@ __device__ __forceinline__ void flow_accumulate(const FlowMat<double, LOOP>& M, 
         }
         __syncthreads();
     }
+    less_c();
 }
 
 // z = sum - C in FP64, z[J][g][r] = column 16 J + 4 r + l/16, row 16 g + l%16 of the wavefront's 32
@@ -921,17 +986,30 @@ __device__ __forceinline__ void flow_tile(const FlowMat<T, LOOP>& M, int i, int 
     }
     flow_solve64<2>(z, 0, s0, s0 + CHOL_NB * CHOL_NB);
     flow_store(M, i, j, 0, z);   // with a barrier: s1 is complete, s0 free
-    // z_2 += L21 X_1^T
+    // z_2 += L21 X_1^T; FP64 as a sum of its own, like the partial sums before
+    constexpr int NJ = sizeof(T) == 8 ? 2 : 4;
 #pragma unroll
-    for (int K = 0; K < 4; ++K)
+    for (int J0 = 4; J0 < 8; J0 += NJ) {
+        doublex4 y[NJ][2];
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4)
+        for (int J = 0; J < NJ; ++J)
 #pragma unroll
-            for (int J = 0; J < 4; ++J) {
-                const double a = s1[(16 * K + 4 * s4 + lq) * CHOL_NB + 16 * J + lr];
+            for (int g = 0; g < 2; ++g) y[J][g] = sizeof(T) == 8 ? doublex4{0.0, 0.0, 0.0, 0.0} : z[J0 + J][g];
 #pragma unroll
-                for (int g = 0; g < 2; ++g) z[4 + J][g] = mfma_f64_16x16x4(a, z[K][g][s4], z[4 + J][g]);
-            }
+        for (int K = 0; K < 4; ++K)
+#pragma unroll
+            for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+                for (int J = 0; J < NJ; ++J) {
+                    const double a = s1[(16 * K + 4 * s4 + lq) * CHOL_NB + 16 * (J0 - 4 + J) + lr];
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) y[J][g] = mfma_f64_16x16x4(a, z[K][g][s4], y[J][g]);
+                }
+#pragma unroll
+        for (int J = 0; J < NJ; ++J)
+#pragma unroll
+            for (int g = 0; g < 2; ++g) z[J0 + J][g] = sizeof(T) == 8 ? z[J0 + J][g] + y[J][g] : y[J][g];
+    }
     if (have < 2) flow_wait(M.dprog(j), 2, M.status);
     load_lkk(ws + LB_STRIDE + CHOL_NB * CHOL_NB, s0);
     flow_solve64<2>(z, 4, s0, s0 + CHOL_NB * CHOL_NB);
@@ -940,7 +1018,8 @@ __device__ __forceinline__ void flow_tile(const FlowMat<T, LOOP>& M, int i, int 
 }
 
 // One 32x32 block of a diagonal tile on one wavefront, transposed as in FlowAcc: columns 32 mb ..,
-// rows 32 nb .. of the tile.
+// rows 32 nb .. of the tile at t.  a is the partial sum; C - sum is in m, in FP64 from hold() on and
+// in the tile's entries before (three blocks a wavefront have no registers for both).
 template <typename T>
 struct FlowQuad;
 template <>
@@ -955,7 +1034,8 @@ struct FlowQuad<float> {
             a[r] = 0.f;
         }
     }
-    __device__ void flush()
+    __device__ void hold(const float*, long long, int, int) {}
+    __device__ void flush(float*, long long, int, int)
     {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -988,19 +1068,40 @@ struct FlowQuad<float> {
 };
 template <>
 struct FlowQuad<double> {
-    doublex4 a[2][2];
-    __device__ void init(const double* t, long long ld, int mb, int nb, int lane)
+    doublex4 a[2][2], m[2][2];
+    __device__ void init(const double*, long long, int, int, int)
     {
-        const double* C = t + 32 * nb + (lane & 15);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) a[x][y] = doublex4{0.0, 0.0, 0.0, 0.0};
+    }
+    __device__ void hold(double* t, long long ld, int mb, int nb)
+    {
+        const FlowLane at(ld);
+        t += 32 * mb * ld + 32 * nb;
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
             for (int y = 0; y < 2; ++y)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    a[x][y][r] = -C[(long long)(32 * mb + 16 * x + 4 * r + (lane >> 4)) * ld + 16 * y];
+                for (int r = 0; r < 4; ++r) m[x][y][r] = *at(t, 16 * x + 4 * r, 16 * y);
     }
-    __device__ void flush() {}
+    __device__ void flush(double* t, long long ld, int mb, int nb)
+    {
+        hold(t, ld, mb, nb);
+        const FlowLane at(ld);
+        t += 32 * mb * ld + 32 * nb;
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) *at(t, 16 * x + 4 * r, 16 * y) = m[x][y][r] - a[x][y][r];
+                a[x][y] = doublex4{0.0, 0.0, 0.0, 0.0};
+            }
+        __builtin_amdgcn_sched_barrier(0);
+    }
     template <int KC, typename S>
     __device__ void mac(const S* s, int P, int mb, int nb, int lane)
     {
@@ -1036,7 +1137,7 @@ struct FlowQuad<double> {
 #pragma unroll
             for (int y = 0; y < 2; ++y)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) f(16 * x + 4 * r + (lane >> 4), 16 * y + (lane & 15), -a[x][y][r]);
+                for (int r = 0; r < 4; ++r) f(16 * x + 4 * r + (lane >> 4), 16 * y + (lane & 15), m[x][y][r] - a[x][y][r]);
     }
 };
 
@@ -1114,17 +1215,19 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T, LOOP>& M, int j, unsi
                 }
                 store((c + 1) & 1);
             }
-            if ((c + 1) % (FLOW_FLUSH / KC) == 0 || !more) {
-                q0.flush();
+            // (the last part stays apart in FP64, where it costs a pass over memory)
+            if ((c + 1) % (FLOW_FLUSH / KC) == 0 ? more || sizeof(T) == 4 : !more && sizeof(T) == 4) {
+                q0.flush(tl, M.ld, m0, n0);
                 if (w) {
-                    q1.flush();
-                    q2.flush();
+                    q1.flush(tl, M.ld, m1, n1);
+                    q2.flush(tl, M.ld, m2, n2);
                 }
             }
             __syncthreads();
         }
         // the last 64 columns of rows 0 .. 63 through s1
         quiet.add(1);   // tile (j, j - 1) has published its first panel
+        q0.hold(tl, M.ld, m0, n0);
         rd.wait(2 * j);
         constexpr int NL = CHOL_NB * CHOL_NB / V / 256;
         vec x[NL];
@@ -1142,6 +1245,8 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T, LOOP>& M, int j, unsi
         }
         __syncthreads();
         if (w < 3) q0.template mac<CHOL_NB>(sl, CHOL_NB, m0, n0, lane);
+    } else {
+        q0.hold(tl, M.ld, m0, n0);
     }
     auto to_block = [&](FlowQuad<T>& q, int mb, int nb) {
         q.each(lane, [&](int c, int r, double v) { s0[(32 * nb + r) * DG_LD + 32 * mb + c] = v; });
@@ -1152,14 +1257,27 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T, LOOP>& M, int j, unsi
     if (w < 3) to_block(q0, m0, n0);
     factor_diag64(s0, c0, M.status, [&] {   // begins with a barrier
         if (!second) return;
-        if (j > 0) {
-            const T* p = M.opnd(j, FLOW_T * j - CHOL_NB);
-            if (w == 3) q0.mac_global(p, M.ld, m0, n0);
-            q1.mac_global(p, M.ld, m1, n1);
-            q2.mac_global(p, M.ld, m2, n2);
+        const T* p = j > 0 ? M.opnd(j, FLOW_T * j - CHOL_NB) : nullptr;
+        if constexpr (sizeof(T) == 8) {
+            // one block at a time: together their operands spill
+            if (w == 3) {
+                if (p) q0.mac_global(p, M.ld, m0, n0);
+                to_lower(q0, m0, n0);
+            }
+            if (p) q1.mac_global(p, M.ld, m1, n1);
+            q1.hold(tl, M.ld, m1, n1);
+            if (p) q2.mac_global(p, M.ld, m2, n2);
+            to_lower(q1, m1, n1);
+        } else {
+            // all of the loads ahead of the sums: one block at a time n = 768 takes 197 us instead of 187
+            if (p) {
+                if (w == 3) q0.mac_global(p, M.ld, m0, n0);
+                q1.mac_global(p, M.ld, m1, n1);
+                q2.mac_global(p, M.ld, m2, n2);
+            }
+            if (w == 3) to_lower(q0, m0, n0);
+            to_lower(q1, m1, n1);
         }
-        if (w == 3) to_lower(q0, m0, n0);
-        to_lower(q1, m1, n1);
     });
     store_lkk(s0, ws);
     if (!second) {
@@ -1185,7 +1303,8 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T, LOOP>& M, int j, unsi
         }
     __syncthreads();   // L21 in s1; s0 is free
     if (w) {
-        q2.flush();
+        if constexpr (sizeof(T) == 4) q2.flush(tl, M.ld, m2, n2);
+        q2.hold(tl, M.ld, m2, n2);
         q2.template mac<CHOL_NB>(s1, CHOL_NB, m2 - 2, n2 - 2, lane);
         to_block(q2, m2 - 2, n2 - 2);
     }

@@ -70,3 +70,23 @@ def test_factor_reports_first_bad_pivot(api, row):
         M = np.asfortranarray(A).copy(order="F")
         rc = _lib.load().bdh_dpotrf(b"L", M.ctypes.data_as(C.POINTER(C.c_double)), 300, 300, prec)
         assert rc == row + 1, (prec, rc)
+
+
+@pytest.mark.parametrize("N", [256, 451, 1000])
+def test_factor_rounding_of_chains(api, N):
+    """FP64 factor of a chain's tensor in extended precision: an entry of A - L L^T collects a rounding
+    of what remains of A's entry per 256 columns, and those of a partial sum of 256 columns, which
+    are relative to that sum: as 16 of the former.  Random signs, 2^-53 each."""
+    from bd_box_amd import workloads as wl
+    from oracle import pyoracle as po
+    s = wl.chain(N, seed=1)
+    A = po.compute_D(s.coord, po.params_from(wl.parse_params(wl.chain_params())))
+    A = np.tril(A) + np.tril(A, -1).T
+    print(f"factor rounding N={N}", flush=True)
+    L, info = api.dpotrf(A, "L", api.FP64)
+    assert info == 0
+    A, L = A.astype(np.longdouble), np.tril(L).astype(np.longdouble)
+    x = np.random.default_rng(N).normal(size=3 * N).astype(np.longdouble)
+    y = A @ x
+    err = np.sqrt((((y - L @ (L.T @ x)) ** 2).sum() / (y ** 2).sum()))
+    assert err <= 2.0 ** -53 * np.sqrt(16 + 3 * N / 256), float(err)
