@@ -412,9 +412,13 @@ __device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long
 // its tile and publishes it.
 //   i > j  (flow_tile)  z = A_ij - sum, solved with L_jj and stored: the rows 128 i .. of panel j.
 //   i = j  (flow_diag)  z factored: the two 64x64 diagonal blocks and the block below the first.
-// Workgroups take the tiles column by column in the order of their index, so every tile a
-// workgroup waits for belongs to a lower index: it is finished or resident, and the waits end
-// whatever the number of resident workgroups.  The waits are bounded anyway (flow_wait).
+// A workgroup takes its tile from a counter when it starts (flow_task), column by column, so every
+// tile it waits for was taken before by a workgroup that is finished or running, and the waits end
+// whatever the number of resident workgroups, the order in which they start, and what else runs.
+// With the workgroup's index in place of the counter they would not have to: workgroups go to the
+// XCDs by index and wait there for room, and two factorizations on two streams could each hold all
+// places of the XCD on which the other's lowest unfinished tile waits for one.
+// The waits are bounded anyway (flow_wait).
 // What bounds it: for small matrices the chain diagonal block -> solve of the next block row ->
 // its update -> next diagonal block; for large ones MFMA issue of the accumulation, which no
 // longer reads and writes C once per outer panel and whose operands are shared in L2.  The chain
@@ -1322,25 +1326,29 @@ __device__ __forceinline__ void flow_diag(const FlowMat<T, LOOP>& M, int j, unsi
     store_diag64<T>(s0, tl, M.ld, CHOL_NB);
 }
 
-// The tasks of a batch in the order of their index.  With more of them than workgroups fit on the
-// chip, workgroups stay and take the next index from a counter: left to the dispatcher, which
-// places workgroups in order and waits for room in the shader engine whose turn it is, a sixth of
-// the places stood empty (256 chains of 64 .. 1024 beads FP32: 3.64 -> 3.39 ms).  Indexes are taken
-// in order by running workgroups, so what a workgroup waits for is still finished or running.  One
-// matrix keeps a workgroup per tile: its columns end together, and the loop's extra instructions
-// lie on its chain (n = 9000 FP32 2.79 ms, 2.98 with the loop, FP64 4.94 and 5.27).
+// The next index of the counter, for the workgroup.
+__device__ __forceinline__ int flow_task(int* __restrict__ next)
+{
+    __shared__ int s_task;
+    if (threadIdx.x == 0) s_task = __hip_atomic_fetch_add(next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();   // and the LDS of the task before is free
+    return __builtin_amdgcn_readfirstlane(s_task);
+}
+
+// The tasks of a batch in the order of the counter.  With more of them than workgroups fit on the
+// chip, workgroups stay and take another: left to the dispatcher, which places workgroups in order
+// and waits for room in the shader engine whose turn it is, a sixth of the places stood empty (256
+// chains of 64 .. 1024 beads FP32: 3.64 -> 3.39 ms).  One matrix keeps a workgroup per tile: its
+// columns end together, and the loop's extra instructions lie on its chain (n = 9000 FP32 2.79 ms,
+// 2.98 with the loop, FP64 4.94 and 5.27).
 constexpr int FLOW_PLACES = 512;   // two workgroups on each of 256 CUs
+constexpr int FLOW_STEP = 10;      // 100 ns (in 100 MHz ticks), in which the counter serves eight workgroups
+// A null counter: one task, no loop (with a loop in every case the compiler spills 30 to 50 registers).
 template <typename Body>
 __device__ __forceinline__ void flow_tasks(int* __restrict__ next, int count, Body&& body)
 {
-    __shared__ int s_task;
     for (;;) {
-        int x = blockIdx.x;
-        if (next) {
-            if (threadIdx.x == 0) s_task = __hip_atomic_fetch_add(next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __syncthreads();   // and the LDS of the task before is free
-            x = __builtin_amdgcn_readfirstlane(s_task);
-        }
+        const int x = next ? flow_task(next) : 0;
         if (x >= count) break;
         body(x);
         if (!next) break;
@@ -1357,10 +1365,17 @@ __device__ __forceinline__ void flow_body(const FlowMat<T, LOOP>& M, int i, int 
 
 template <typename T, bool SPLIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-chol_flow_kernel(FlowMat<T> M)
+chol_flow_kernel(FlowMat<T> M, int* __restrict__ next)
 {
+    // The first workgroups ask in the order of their index, one of each XCD at a time: all at once, the
+    // counter serves one XCD after the other, and neighbouring tiles share an XCD and its CUs (FP64
+    // n = 4500 1350 -> 1650 us).
+    if (threadIdx.x == 0 && blockIdx.x < FLOW_PLACES) {
+        const long long t0 = wall_clock64(), wait = (long long)(blockIdx.x / 8) * FLOW_STEP;
+        while (wall_clock64() - t0 < wait) __builtin_amdgcn_s_sleep(1);
+    }
     // tile column by column
-    int x = blockIdx.x, j = 0;
+    int x = flow_task(next), j = 0;
     while (x >= M.nt - j) {
         x -= M.nt - j;
         ++j;
@@ -1388,6 +1403,8 @@ int chol_factor(T* d_A, long long ld, int n, int n_pad, double* d_Lbuf, int* d_s
     const bool shared = tiles > QUIET_TILES;
     FlowMat<T> M{d_A, ld, n, nt, d_Lbuf, d_status, shared ? d_flags + nflags : nullptr};
     if (shared) nflags += FLOW_CUS;
+    int* next = d_flags + nflags;
+    nflags += 1;
     if (rec) rec->begin(PH_PANEL, st);
     hipLaunchKernelGGL(chol_flow_clear_kernel, dim3(ceil_div(nflags, 256)), dim3(256), 0, st, d_flags, nflags);
     BDH_LAUNCH_CHECK();
@@ -1396,11 +1413,11 @@ int chol_factor(T* d_A, long long ld, int n, int n_pad, double* d_Lbuf, int* d_s
     const dim3 grid(tiles);
     if constexpr (sizeof(T) == 4) {
         if (syrk_mode == SYRK_BF16X3)
-            hipLaunchKernelGGL((chol_flow_kernel<T, true>), grid, dim3(256), 0, st, M);
+            hipLaunchKernelGGL((chol_flow_kernel<T, true>), grid, dim3(256), 0, st, M, next);
         else
-            hipLaunchKernelGGL((chol_flow_kernel<T, false>), grid, dim3(256), 0, st, M);
+            hipLaunchKernelGGL((chol_flow_kernel<T, false>), grid, dim3(256), 0, st, M, next);
     } else {
-        hipLaunchKernelGGL((chol_flow_kernel<T, false>), grid, dim3(256), 0, st, M);
+        hipLaunchKernelGGL((chol_flow_kernel<T, false>), grid, dim3(256), 0, st, M, next);
     }
     BDH_LAUNCH_CHECK();
     if (rec) rec->end(PH_SYRK, st);
@@ -1410,7 +1427,7 @@ int chol_factor(T* d_A, long long ld, int n, int n_pad, double* d_Lbuf, int* d_s
 size_t chol_lbuf_doubles(int n_pad)
 {
     const size_t nt = n_pad / FLOW_T;
-    return nt * FLOW_COL + (2 * nt * FLAG_STRIDE + FLOW_CUS) / 2;
+    return nt * FLOW_COL + (2 * nt * FLAG_STRIDE + FLOW_CUS + FLAG_STRIDE) / 2;   // flags, quiet counters, task counter
 }
 
 // ------------------------------------------------------------------ Y = L X (partials)
@@ -1652,7 +1669,7 @@ int chol_factor_batch(T* d_A, double* d_Lbuf, const BatchPlan& plan, int* d_stat
     BDH_LAUNCH_CHECK();
     if (rec) rec->end(PH_PANEL, st);
     if (rec) rec->begin(PH_SYRK, st);
-    int* next = plan.ntasks > FLOW_PLACES ? plan.next : nullptr;
+    int* next = plan.ntasks > 1 ? plan.next : nullptr;
     const dim3 grid(std::min(plan.ntasks, FLOW_PLACES));
     if (sizeof(T) == 4 && syrk_mode == SYRK_BF16X3)
         hipLaunchKernelGGL((chol_flow_batch_kernel<T, sizeof(T) == 4>), grid, dim3(256), 0, st, d_A, d_Lbuf, plan.ch,

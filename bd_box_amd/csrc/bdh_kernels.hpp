@@ -44,7 +44,7 @@ __device__ __forceinline__ int batch_find(const int* __restrict__ prefix, int nc
     return lo;
 }
 
-// One workgroup of the batch's factorization: tile (i, j) of chain c's lower triangle.
+// One task of the batch's factorization: tile (i, j) of chain c's lower triangle.
 struct FlowTask {
     int c;
     short i, j;
@@ -57,7 +57,7 @@ struct BatchPlan {
     const int *asm_pre = nullptr, *pair_pre = nullptr, *force_pre = nullptr, *trmv_pre = nullptr;
     const int *rows_pre = nullptr;
     int asm_blocks = 0, pair_blocks = 0, force_blocks = 0, trmv_blocks = 0, rows_blocks = 0;
-    const FlowTask* tasks = nullptr;   // the factorization's workgroups in index order
+    const FlowTask* tasks = nullptr;   // the factorization's tiles in the order they are taken in
     int ntasks = 0;
     int* next = nullptr;               // their counter
 };
@@ -133,7 +133,7 @@ template <typename T>
 int launch_trmv_partials(const T* d_L, long long ld, int n, const double* d_X, long long ldx, int m,
                          double* d_P, hipStream_t st);
 int trmv_blk_cols();   // columns per partial of the L.x kernel
-// Workgroups of the factorization of a batch with the given padded orders, in index order.
+// Tiles of the factorization of a batch with the given padded orders, in the order they are taken in.
 std::vector<FlowTask> chol_batch_tasks(const std::vector<int>& n_pad);
 template <typename T>
 int trmv_blocks(int n);                           // row x column blocks of the L.x partials
