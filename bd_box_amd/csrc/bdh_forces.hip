@@ -114,12 +114,17 @@ constexpr int FT_MAX_N = 16384;   // tile-pair partials: 3N x ceil(N / 64) doubl
 // k on wavefront k mod 4.  W wavefronts take FT_GROUPS / W groups each, one after the other; the groups'
 // sums meet in one binary tree, so the forces do not depend on W.
 // Partners in tile J are known from a bit mask made once: looking them up in the topology for
-// every pair cost a chain of global loads per shift.  A first pass over the separations finds the
-// shifts that have a pair in reach anywhere in the wavefront; most tile pairs of a large system
-// have none and end there.
+// every pair cost a chain of global loads per shift.  A first pass over the separations ends most
+// tile pairs of a large system, which have no pair in reach; with W = 4, where the chip is full, it
+// ends at the first shift that has one, and the shifts from there on are tested as they come.
 // Bound by the serial pair terms of the tile pairs near the diagonal where N is small, by VALU
-// issue where it is large.  One wavefront's 16 shifts with the partner look-up, five divisions and
-// the bond energies' logarithms: N = 256 FP64 21.5 us; now 8.7, the batch of 256 chains 102 -> 80.
+// issue and the number of wavefronts in flight where it is large: the groups' sums wait in LDS and
+// energies are a kernel of their own, so that seven wavefronts a SIMD fit in FP32 and five in FP64.
+// One wavefront's 16 shifts with the partner look-up, five divisions and the bond energies'
+// logarithms: N = 256 FP64 21.5 us; now 8.7, the batch of 256 chains 102 -> 83 (FP32).  Spheres in
+// random order, where nearly every tile pair has some pairs in reach, N = 16000 FP32 with 32 in reach
+// of each 162 us a step -> 172 (245 with every shift tested twice and five wavefronts a SIMD), with
+// 590 502 -> 444 (575).
 constexpr int FT_GROUPS = 16;
 constexpr int FT_BATCH_W = 4;   // a batch fills the chip
 
@@ -128,13 +133,13 @@ struct TilesShared {
     double4 pos[FT_TILE];
     double q[FT_TILE];
     double2 lj[FT_TILE];
-    double col[W][3][FT_TILE];
-    double row[W][3][FT_TILE];
-    double bond[4][3][FT_TILE];
+    double col[W][3][FT_TILE];    // column sums of a wavefront's current group
+    double row[W][3][FT_TILE];    // row sums
+    double tot[W][3][FT_TILE];    // column sums; on the diagonal the bonds, four wavefronts'
     double e[W][3];
 };
 
-template <typename T, int W>
+template <typename T, int W, bool ENERGY>
 __device__ __forceinline__ void forces_tiles_body(const double4* __restrict__ pos, const double* __restrict__ Q,
                                                   const double2* __restrict__ LJ, int N, const Topology& topo,
                                                   const ForceParams& fp, double* __restrict__ PF,
@@ -146,7 +151,7 @@ __device__ __forceinline__ void forces_tiles_body(const double4* __restrict__ po
     auto& s_lj = sm.lj;
     auto& s_col = sm.col;
     auto& s_row = sm.row;
-    auto& s_bond = sm.bond;
+    auto& s_tot = sm.tot;
     auto& s_e = sm.e;
     static_assert(FT_GROUPS == 16 && (W == 4 || W == 8 || W == 16), "groups are summed by a binary tree");
     const int t = threadIdx.x, w = threadIdx.y, tid = w * FT_TILE + t;
@@ -167,19 +172,25 @@ __device__ __forceinline__ void forces_tiles_body(const double4* __restrict__ po
     const double4 pi = iv ? pos[i] : make_double4(0, 0, 0, 1);
     const double qi = iv ? Q[i] : 0.0;
     const double2 lji = iv ? LJ[i] : make_double2(0, 0);
-    double e[3] = {0.0, 0.0, 0.0}, one[6], two[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    double e[3] = {0.0, 0.0, 0.0}, one[6];
     int rep = 0;
     __syncthreads();
     // shift 16 y + x of group g(x) near anywhere in the wavefront: bit y + 4 x
     constexpr int PER = FT_TILE / FT_GROUPS, GW = FT_GROUPS / W;
     unsigned near = 0;
-#pragma unroll 2
+#pragma unroll 4
     for (int u = 0; u < GW * PER; ++u) {
         const int sh = w * GW + u / PER + FT_GROUPS * (u % PER);
         const int jl = (t + sh) & (FT_TILE - 1);
         double dx = s_pos[jl].x - pi.x, dy = s_pos[jl].y - pi.y, dz = s_pos[jl].z - pi.z;
         const bool far = !iv || j0 + jl >= N || (diag && sh == 0) || pair_r2(dx, dy, dz, fp.pbc, fp.box) > fp.far_r2;
-        if (__ballot(!far)) near |= 1u << u;
+        if (__ballot(!far)) {
+            near |= 1u << u;
+            if constexpr (W == 4) {
+                near = ~0u << u;
+                break;
+            }
+        }
     }
     unsigned long long partners = 0;
     if (near && iv && fp.use_conn)
@@ -190,60 +201,82 @@ __device__ __forceinline__ void forces_tiles_body(const double4* __restrict__ po
 #pragma unroll 1
     for (int x = 0; x < (near ? GW : 0); ++x) {
         const int g = w * GW + x;
-        const bool any = (near >> (PER * x)) & ((1 << PER) - 1);
         PairAcc a{0, 0, 0, 0, 0, 0};
-        if (any) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) s_col[w][k][t] = 0.0;
+        bool any = false;   // a pair in reach so far, anywhere in the wavefront
 #pragma unroll 1
-            for (int y = 0; y < PER; ++y) {
-                if (!((near >> (PER * x + y)) & 1)) continue;
-                const int sh = g + FT_GROUPS * y;
-                const int jl = (t + sh) & (FT_TILE - 1);
-                if (!iv || j0 + jl >= N || (diag && sh == 0)) continue;
-                double dx = s_pos[jl].x - pi.x, dy = s_pos[jl].y - pi.y, dz = s_pos[jl].z - pi.z;
-                const double r2 = pair_r2(dx, dy, dz, fp.pbc, fp.box);
-                if (r2 > fp.far_r2) continue;
-                PairAcc p{0, 0, 0, 0, 0, 0};
-                pair_term<T>(dx, dy, dz, r2, qi, s_q[jl], lji, s_lj[jl], (partners >> jl) & 1, fp, p, PE != nullptr);
-                a.fx += p.fx;
-                a.fy += p.fy;
-                a.fz += p.fz;
+        for (int y = 0; y < PER; ++y) {
+            if (!((near >> (PER * x + y)) & 1)) continue;
+            const int sh = g + FT_GROUPS * y;
+            const int jl = (t + sh) & (FT_TILE - 1);
+            double dx = s_pos[jl].x - pi.x, dy = s_pos[jl].y - pi.y, dz = s_pos[jl].z - pi.z;
+            const double r2 = pair_r2(dx, dy, dz, fp.pbc, fp.box);
+            const bool far = !iv || j0 + jl >= N || (diag && sh == 0) || r2 > fp.far_r2;
+            if (!__ballot(!far)) continue;
+            if (!any) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) s_col[w][k][t] = 0.0;
+                any = true;
+                // another lane of this wavefront, which owns the row, adds to it next
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+            if (far) continue;
+            PairAcc p{0, 0, 0, 0, 0, 0};
+            pair_term<T>(dx, dy, dz, r2, qi, s_q[jl], lji, s_lj[jl], (partners >> jl) & 1, fp, p, ENERGY);
+            a.fx += p.fx;
+            a.fy += p.fy;
+            a.fz += p.fz;
+            if constexpr (ENERGY) {
                 e[0] += p.e_lj;
                 e[1] += p.e_c;
-                rep |= p.rep;
-                if (!diag) {
-                    s_col[w][0][jl] -= p.fx;
-                    s_col[w][1][jl] -= p.fy;
-                    s_col[w][2][jl] -= p.fz;
-                }
+            }
+            rep |= p.rep;
+            if (!diag) {
+                s_col[w][0][jl] -= p.fx;
+                s_col[w][1][jl] -= p.fy;
+                s_col[w][2][jl] -= p.fz;
             }
         }
-        double v[6] = {a.fx, a.fy, a.fz, 0.0, 0.0, 0.0};
-        if (any)
+        // a group without a pair in reach adds nothing
+        if (any) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            double v[6] = {a.fx, a.fy, a.fz, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int k = 0; k < 3; ++k) v[3 + k] = s_col[w][k][t];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            one[k] = x & 1 ? one[k] + v[k] : v[k];
-            if (W == 16 || x == 1) two[k] = one[k];
-            else if (x == 3) two[k] += one[k];
+            for (int k = 0; k < 6; ++k) one[k] = x & 1 ? one[k] + v[k] : v[k];
+        } else if (!(x & 1)) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) one[k] = 0.0;
         }
+        if (W == 16 || x == 1) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                s_row[w][k][t] = one[k];
+                s_tot[w][k][t] = one[3 + k];
+            }
+        } else if (x == 3) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                s_row[w][k][t] += one[k];
+                s_tot[w][k][t] += one[3 + k];
+            }
+        }
+    }
+    if (!near) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s_row[w][k][t] = s_tot[w][k][t] = 0.0;
     }
     if (diag && w < 4) {
         PairAcc a{0, 0, 0, 0, 0, 0};
-        if (iv) e[2] = bond_terms(pos, i, pi, topo, fp, a, PE != nullptr, w, 4);
+        if (iv) e[2] = bond_terms(pos, i, pi, topo, fp, a, ENERGY, w, 4);
         rep |= a.rep;
-        s_bond[w][0][t] = a.fx;
-        s_bond[w][1][t] = a.fy;
-        s_bond[w][2][t] = a.fz;
+        s_tot[w][0][t] = a.fx;
+        s_tot[w][1][t] = a.fy;
+        s_tot[w][2][t] = a.fz;
     }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        s_row[w][k][t] = two[k];
-        s_col[w][k][t] = two[3 + k];
-    }
-    if (PE) {
+    if constexpr (ENERGY) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
 #pragma unroll
@@ -268,15 +301,15 @@ __device__ __forceinline__ void forces_tiles_body(const double4* __restrict__ po
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             out[k] = sum(s_row, k);
-            if (diag) out[k] += (s_bond[0][k][t] + s_bond[1][k][t]) + (s_bond[2][k][t] + s_bond[3][k][t]);
+            if (diag) out[k] += (s_tot[0][k][t] + s_tot[1][k][t]) + (s_tot[2][k][t] + s_tot[3][k][t]);
         }
     }
     if (w == 1 && !diag && j0 + t < N) {
         double* out = PF + (long long)I * 3 * N + 3 * (j0 + t);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) out[k] = sum(s_col, k);
+        for (int k = 0; k < 3; ++k) out[k] = sum(s_tot, k);
     }
-    if (PE && w == 2 && t < 3) {
+    if (ENERGY && w == 2 && t < 3) {
         // pairs of a diagonal tile are seen from both ends; bonds from both of theirs
         double v = 0.0;
         for (int y = 0; y < W; ++y) v += s_e[y][t];
@@ -286,14 +319,14 @@ __device__ __forceinline__ void forces_tiles_body(const double4* __restrict__ po
     if (rep & 2) atomicOr(flags, 2);
 }
 
-template <typename T, int W>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 && sizeof(T) == 4 ? 5 : 4)))
+template <typename T, int W, bool ENERGY>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 4 ? (sizeof(T) == 4 ? 7 : 5) : 4)))
 forces_tiles_kernel(const double4* __restrict__ pos, const double* __restrict__ Q,
                     const double2* __restrict__ LJ, int N, Topology topo, ForceParams fp,
                     double* __restrict__ PF, double* __restrict__ PE, int* __restrict__ flags)
 {
     __shared__ TilesShared<W> sm;
-    forces_tiles_body<T, W>(pos, Q, LJ, N, topo, fp, PF, PE, flags, blockIdx.x, blockIdx.x, sm);
+    forces_tiles_body<T, W, ENERGY>(pos, Q, LJ, N, topo, fp, PF, PE, flags, blockIdx.x, blockIdx.x, sm);
 }
 
 template <typename T>
@@ -326,7 +359,7 @@ forces_batch_kernel(const double4* __restrict__ pos, const double* __restrict__ 
     t.conn_off += b.bead0 + c;
     t.bond_off += b.bead0 + c;
     if (b.N <= FT_MAX_N) {
-        forces_tiles_body<T, FT_BATCH_W>(pos + b.bead0, Q + b.bead0, LJ + b.bead0, b.N, t, fp, Pf + b.pf, nullptr, flags,
+        forces_tiles_body<T, FT_BATCH_W, false>(pos + b.bead0, Q + b.bead0, LJ + b.bead0, b.N, t, fp, Pf + b.pf, nullptr, flags,
                              x, 0, sm.tiles);
     } else {
         const int gx = (b.N + FR_ROWS - 1) / FR_ROWS;
@@ -373,19 +406,22 @@ int launch_forces(const double4* d_pos, const double* d_Q, const double2* d_LJ, 
     if (N <= FT_MAX_N) {
         BDH_CHECK(splits == ceil_div(N, FT_TILE), "forces: tile-pair partials expect one split per tile");
         // Few tile pairs: the time is one workgroup's serial shifts, so more wavefronts take them;
-        // many: the chip is full and wide workgroups only add prologues.  A step without
-        // hydrodynamics, us, W = 4 / 8 / 16, FP32 and FP64: N = 1000 (136 pairs) 23.5 / 16.3 / 16.1,
-        // 24.2 / 18.0 / 17.2; 1500 (300) 23.9 / 17.1 / 16.6, 24.5 / 18.5 / 18.0; 2000 (528) 23.8 / 17.8
-        // / 19.9, 24.6 / 19.1 / 20.6; 3000 (1128) 26.9 / 24.0 / 27.1, 28.8 / 25.6 / 27.3; 5000 (3160)
-        // 36.6 / 38.1 / 47.3, 38.9 / 39.8 / 46.5; 10000 74.3 / 95.2 / 138, 81.1 / 96.2 / 132.
+        // many: the chip is full and wide workgroups only add prologues.  A step without hydrodynamics,
+        // us, W = 4 / 8 / 16, FP32 and FP64.  Chains: N = 256 20.1 / 15.6 / 13.5, 21.1 / 16.9 / 15.0; 1000
+        // (136 pairs) 20.8 / 16.6 / 14.6, 21.8 / 18.2 / 15.8; 2000 (528) 22.9 / 21.0 / 18.7, 25.7 / 24.1 /
+        // 19.5; 3000 (1128) 24.5 / 23.9 / 23.2, 26.7 / 26.1 / 25.6; 4000 (2016) 27.8 / 29.2 / 29.3, 29.2 /
+        // 30.3 / 34.4; 10000 63.9 / 89.8 / 98.3, 72.3 / 93.9 / 124.  Spheres in random order: 1500 (300)
+        // 14.8 / 13.2 / 13.0, 14.3 / 13.1 / 14.6; 2000 15.3 / 14.5 / 14.7, 14.6 / 14.4 / 16.0; 3000 17.6
+        // / 20.0 / 20.3, 17.6 / 19.5 / 21.8.
         const int blocks = force_blocks(N);
         auto launch = [&](auto w) {
             constexpr int W = decltype(w)::value;
-            hipLaunchKernelGGL((forces_tiles_kernel<T, W>), dim3(blocks), dim3(FT_TILE, W), 0, st, d_pos, d_Q,
-                               d_LJ, N, topo, fp, d_PF, d_PE, d_flags);
+            auto* kernel = d_PE ? forces_tiles_kernel<T, W, true> : forces_tiles_kernel<T, W, false>;
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(FT_TILE, W), 0, st, d_pos, d_Q, d_LJ, N, topo, fp, d_PF,
+                               d_PE, d_flags);
         };
         if (blocks <= 320) launch(std::integral_constant<int, 16>{});
-        else if (blocks <= 2048) launch(std::integral_constant<int, 8>{});
+        else if (blocks <= 1400) launch(std::integral_constant<int, 8>{});
         else launch(std::integral_constant<int, 4>{});
         BDH_LAUNCH_CHECK();
         return 0;
