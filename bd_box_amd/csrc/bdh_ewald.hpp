@@ -321,7 +321,7 @@ __device__ __forceinline__ Blk6 beenakker_block(double rx, double ry, double rz,
     // exponent factor: FP64 -alpha^2; FP32 -alpha^2 log2(e), high and low part
     const double nlg = sizeof(T) == 8 ? -E.alpha2 : -E.alpha2 * 1.4426950408889634074;
     const T nl = (T)nlg, nl_lo = (T)(nlg - (double)nl);
-    T Ot[7] = {0, 0, 0, 0, 0, 0, 0};   // xx yy zz xy xz yz of c2 e e^T, and c1
+    T Ot[7] = {0, 0, 0, 0, 0, 0, 0};   // xx yy zz xy xz yz of c2 e e^T, and c1 (FP32)
     each_image<T>(E.box, E.RR_real, (T)E.rc2, rx, ry, rz, [&](T x, T y, T z, T rr) {
         const T inv_r = inv_dist(rr), ir2 = inv_r * inv_r;
         const T X = erfcx_image(rr * inv_r * al) * inv_r;
@@ -329,13 +329,21 @@ __device__ __forceinline__ Blk6 beenakker_block(double rx, double ry, double rz,
         const T c1 = ex * (X * ((T)0.75 + sg1 * ir2) + (p0 + as * ir2 + rr * (p1 + p2 * rr)));
         const T w = ex * ir2 * (X * ((T)0.75 + sg2 * ir2) + (q0 + as3 * ir2 + rr * (q1 - p2 * rr)));
         const T wx = w * x, wy = w * y, wz = w * z;
-        Ot[0] += wx * x;
-        Ot[1] += wy * y;
-        Ot[2] += wz * z;
+        // FP64: c1 and c2 e e^T, of opposite signs, meet before the sum over the images rounds them;
+        // FP32's error is the terms' own
+        if constexpr (sizeof(T) == 8) {
+            Ot[0] += wx * x + c1;
+            Ot[1] += wy * y + c1;
+            Ot[2] += wz * z + c1;
+        } else {
+            Ot[0] += wx * x;
+            Ot[1] += wy * y;
+            Ot[2] += wz * z;
+            Ot[6] += c1;
+        }
         Ot[3] += wx * y;
         Ot[4] += wx * z;
         Ot[5] += wy * z;
-        Ot[6] += c1;
     });
     // reciprocal space (FP64); none when every factor is zero (the reference's split, whose
     // factors underflow)

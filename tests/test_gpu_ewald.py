@@ -167,3 +167,44 @@ def test_ewald_tensor_any_box(api, box, R, ext):
         err = np.abs(b.compute_D() - ref).max() / np.abs(ref).max()
         assert err <= tol, (prec, err)
         b.close()
+
+
+def _beenakker_long(s, P, R):
+    """Off-diagonal blocks of the reference's split (no reciprocal terms) in extended precision."""
+    LD = np.longdouble
+    sp, kt = LD("1.77245385090551602729816748334114518"), LD(KB6 * P.T / (P.visc * P.vfactor))
+    al, sg = LD(SP / P.box), (s.coord[:, None, 3] ** 2 + s.coord[None, :, 3] ** 2).astype(LD) / 2
+    d = s.coord[None, :, :3].astype(LD) - s.coord[:, None, :3]
+    B = np.zeros((s.N, s.N, 3, 3), LD)
+    off = ~np.eye(s.N, dtype=bool)
+    for hfg in _sphere(R):
+        x = d + LD(P.box) * np.array(hfg, LD)
+        r2 = np.where(off, (x * x).sum(-1), 1)
+        r = np.sqrt(r2)
+        y = al * r
+        eg = np.exp(-y * y) / sp
+        term, erf = y, y   # erf y = 2 exp(-y^2) / sqrt(pi) sum (2 y^2)^n y / (2 n + 1)!!
+        for n in range(1, 260):
+            term = term * (2 * y * y) / (2 * n + 1)
+            erf = erf + term
+        ec = 1 - 2 * eg * erf
+        c1 = eg * (al * sg / r2 + 14 * al ** 3 * sg - LD(4.5) * al - 20 * al ** 5 * sg * r2 + 3 * al ** 3 * r2 +
+                   4 * al ** 7 * sg * r2 * r2) + ec * (LD(0.75) / r + LD(0.5) * sg / (r * r2))
+        c2 = eg * (-3 * al * sg / r2 - 2 * al ** 3 * sg + LD(1.5) * al + 16 * al ** 5 * sg * r2 - 3 * al ** 3 * r2 -
+                   4 * al ** 7 * sg * r2 * r2) + ec * (LD(0.75) / r - LD(1.5) * sg / (r * r2))
+        B += c1[..., None, None] * np.eye(3, dtype=LD) + (c2 / r2)[..., None, None] * x[..., :, None] * x[..., None, :]
+    return kt * B, off
+
+
+@pytest.mark.parametrize("seed", [3, 4])
+def test_ewald_rounding(api, seed):
+    """515 images in FP64 against extended precision: an entry's own rounding and as much again from
+    the sum, each uniform in half the largest entry's unit 2^-52: rms 2^-53 sqrt(2 / 3)."""
+    s, P = _spheres(50, 0.15, seed, "beenakker", 5)
+    ref, off = _beenakker_long(s, P, 5)
+    print("ewald rounding", seed, flush=True)
+    b = api.BDSystem(s, P, precision=api.FP64)
+    D = b.compute_D()
+    b.close()
+    err = np.abs(D.reshape(50, 3, 50, 3).transpose(0, 2, 1, 3) - ref)[off].max((1, 2)) / np.abs(D).max()
+    assert np.sqrt((err ** 2).mean()) <= 2.0 ** -53 * np.sqrt(2 / 3), float(np.sqrt((err ** 2).mean()))
