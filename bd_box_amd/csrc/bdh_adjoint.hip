@@ -101,10 +101,12 @@ adj_diag_inv_kernel(const double* __restrict__ L, long long ld, int np, double* 
 //          i in the second
 //   MUL_M  M(i, q) = -sum_k M(i, k) T(k, q), k in the second block
 //   MUL_Z  Z(r, c) = sum_j G(j, r) M(j, c), r <= c
+// Every stage's partial sum starts from zero and is added as a whole: Z's terms cancel, and with sums
+// over all of n the reverse step of 300 beads was 2.4e-15 off (of its norm, extended precision),
+// where the two triangular solves these products replace had 8.8e-16; so 8.4e-16, for 2 % of the time.
 // Tiles with the longest sums come first.  Bound by MFMA issue in the large levels and MUL_Z and
-// by one tile's length in the small ones: n = 3072 the inverse 0.36 ms in 12 launches, Z 0.19 ms (51
-// TFLOP/s), against 2.25 ms for the two triangular solves they replace; with four wavefronts 0.44
-// and 0.20 ms.
+// by one tile's length in the small ones: n = 3072 the inverse 0.38 ms in 12 launches, Z 0.20 ms,
+// against 2.25 ms for the triangular solves; with four wavefronts 0.44 and 0.20 ms.
 enum { MUL_T, MUL_M, MUL_Z };
 constexpr int ADJ_KC = 32, ADJ_PN = ADJ_NB + 16, ADJ_PT = ADJ_KC + 2;
 
@@ -166,7 +168,7 @@ adj_mul_kernel(const double* A, long long lda, const double* B, int np, int sb, 
         }
     };
     const int r0 = 32 * (wave & 1), c0 = 16 * (wave >> 1), lr = lane & 15, lk = lane >> 4;
-    doublex4 acc[2] = {doublex4{0.0, 0.0, 0.0, 0.0}, doublex4{0.0, 0.0, 0.0, 0.0}};
+    doublex4 sum[2] = {doublex4{0.0, 0.0, 0.0, 0.0}, doublex4{0.0, 0.0, 0.0, 0.0}};
     // transposed: accumulator r of lane l is column 4 r + l / 16, row l % 16
     const int kb = k0 * ADJ_NB, ke = k1 * ADJ_NB;
     auto stage = [&](int k, int buf) {   // stage k is in LDS half buf, the next in registers buf ^ 1, two on to buf
@@ -182,6 +184,7 @@ adj_mul_kernel(const double* A, long long lda, const double* B, int np, int sb, 
             for (int x = 0; x < 2; ++x)
                 av[s & 1][x] = AN ? sa[kk * ADJ_PN + r0 + 16 * x + lr] : sa[(r0 + 16 * x + lr) * ADJ_PT + kk];
         };
+        doublex4 acc[2] = {doublex4{0.0, 0.0, 0.0, 0.0}, doublex4{0.0, 0.0, 0.0, 0.0}};
         fetch(0);
 #pragma unroll
         for (int s = 0; s < ADJ_KC / 4; ++s) {
@@ -190,6 +193,8 @@ adj_mul_kernel(const double* A, long long lda, const double* B, int np, int sb, 
             for (int x = 0; x < 2; ++x) acc[x] = mfma_f64_16x16x4(bv[s & 1], av[s & 1][x], acc[x]);
             __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int x = 0; x < 2; ++x) sum[x] += acc[x];
         if (k + ADJ_KC < ke) store(buf ^ 1, buf ^ 1);
     };
     static_assert(ADJ_NB % (2 * ADJ_KC) == 0, "whole pairs of stages");
@@ -204,7 +209,7 @@ adj_mul_kernel(const double* A, long long lda, const double* B, int np, int sb, 
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int x = 0; x < 2; ++x) out[(long long)4 * r * np + 16 * x] = MODE == MUL_M ? -acc[x][r] : acc[x][r];
+        for (int x = 0; x < 2; ++x) out[(long long)4 * r * np + 16 * x] = MODE == MUL_M ? -sum[x][r] : sum[x][r];
 }
 
 // Column r of G (workgroup r) from the start of r's 64-block, zero above the diagonal.  Thread t

@@ -27,3 +27,38 @@ def test_step_vjp_sizes(N):
     rbar = s.step_vjp(sysm.coord, xi, g)
     ref = ad.step_vjp(sysm, po.params_from(P), sysm.coord, xi, g)
     assert np.linalg.norm(rbar - ref) < 1e-9 * np.linalg.norm(ref)
+
+
+def test_step_vjp_rounding():
+    """The noise term's rounding at 300 beads (Gaussians 1e5 times their size, so that it is all that
+    counts), against a factor and an inverse in extended precision: two products whose partial sums
+    have 32 terms, sqrt(32) 2^-53 each, and as much again for the factor, its inverse and L^T g:
+    12 2^-53."""
+    from bd_box_amd import system as S
+    from oracle import adjoint as ad
+    from oracle import pyoracle as po
+    N, LD = 300, np.longdouble
+    n = 3 * N
+    sysm = wl.chain(N, seed=900 + N)
+    P = wl.parse_params(wl.chain_params())
+    p = po.params_from(P)
+    rng = np.random.default_rng(N)
+    xi, g = 1e5 * rng.normal(size=n), rng.normal(size=n)
+    D = po.compute_D(sysm.coord, p).astype(LD)
+    L, M = np.zeros((n, n), LD), np.zeros((n, n), LD)
+    for j in range(n):
+        v = D[j:, j] - L[j:, :j] @ L[j, :j]
+        L[j:, j] = v / np.sqrt(v[0])
+    for i in range(n):
+        M[i] = -(L[i, :i] @ M[:i]) / L[i, i]
+        M[i, i] = 1 / L[i, i]
+    Phi = np.tril(np.outer(L.T @ g.astype(LD), xi.astype(LD))) * np.sqrt(2 * LD(P.dt))
+    Phi -= np.diag(np.diag(Phi)) / 2
+    Z = M.T @ Phi @ M
+    F, _, _ = po.forces(sysm, p)
+    c = P.dt / (ad.KB * P.T)
+    U = (((Z + Z.T) / 2).astype(float) + c * 0.5 * (np.outer(g, F) + np.outer(F, g)))
+    ref = g + ad.rpy_contract_grad(sysm.coord, U, p) - c * ad.hessian_vec(sysm, p, sysm.coord, D.astype(float) @ g)
+    print(f"step vjp rounding N={N}", flush=True)
+    rbar = S.BDSystem(sysm, P, precision=S.FP64, refactor_every=1).step_vjp(sysm.coord, xi, g)
+    assert np.linalg.norm(rbar - ref) <= 12 * 2.0 ** -53 * np.linalg.norm(ref)
