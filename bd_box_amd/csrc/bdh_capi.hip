@@ -179,6 +179,7 @@ constexpr size_t STAGE_MAX = 2u << 20;
 struct HostStage {
     unsigned char* p = nullptr;
     size_t cap = 0;
+    std::mutex use;   // a fetch's from its launch to its host copy: any thread may read an object
 };
 
 struct bdh_system {
@@ -311,8 +312,9 @@ void stage_alloc(HostStage& h, size_t bytes)
     h.cap = bytes;
 }
 
-int fetch(const HostStage& h, int device, hipStream_t st, const Fetch* f, int nf)
+int fetch(HostStage& h, int device, hipStream_t st, const Fetch* f, int nf)
 {
+    BDH_CHECK(nf <= FETCH_MAX, "fetch: too many arrays");
     FetchJobs J{};
     size_t off[FETCH_MAX], used = 0, most = 0;
     for (int k = 0; k < nf; ++k) {
@@ -320,17 +322,18 @@ int fetch(const HostStage& h, int device, hipStream_t st, const Fetch* f, int nf
         used += (f[k].bytes + 127) / 128 * 128;
         most = std::max(most, f[k].bytes);
     }
-    if (nf > FETCH_MAX || used > h.cap) {
+    if (used > h.cap) {
         for (int k = 0; k < nf; ++k) BDH_HIP(hipMemcpyAsync(f[k].dst, f[k].src, f[k].bytes, hipMemcpyDeviceToHost, st));
         BDH_HIP(hipStreamSynchronize(st));
         return 0;
     }
+    BDH_HIP(hipSetDevice(device));
+    std::lock_guard<std::mutex> lock(h.use);
     for (int k = 0; k < nf; ++k) {
         J.src[k] = static_cast<const unsigned*>(f[k].src);
         J.dst[k] = reinterpret_cast<unsigned*>(h.p + off[k]);
         J.words[k] = (int)(f[k].bytes / 4);
     }
-    BDH_HIP(hipSetDevice(device));
     const int blocks = (int)std::min<size_t>(256, (most + 2047) / 2048);
     hipLaunchKernelGGL(fetch_kernel, dim3(std::max(1, blocks), nf), dim3(256), 0, st, J);
     BDH_LAUNCH_CHECK();

@@ -33,3 +33,28 @@ def test_round_trip(N):
     F, E, _ = s.compute_forces()
     assert np.array_equal(s.forces(), F) and np.isfinite(E).all()
     assert N == 1 or np.any(F != 0.0)
+
+
+@pytest.mark.parametrize("N", [40, 3000])
+def test_readers_in_threads(N):
+    """Positions and forces of one system read by four threads at once, 200 times each: every reader
+    gets its own array, whole."""
+    from bd_box_amd import system as S
+    sysm = wl.chain(N, seed=N)
+    s = S.BDSystem(sysm, wl.parse_params(wl.chain_params(hydro="none")), precision=S.FP64)
+    s.compute_hydro(1)
+    xyz, F = s.coords(), s.forces()
+    wrong = []
+
+    def read(get, want):
+        for _ in range(200):
+            if not np.array_equal(get(), want):
+                wrong.append(get)
+
+    print(f"readers in threads N={N}", flush=True)
+    threads = [threading.Thread(target=read, args=a) for a in 2 * [(s.coords, xyz), (s.forces, F)]]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
