@@ -312,6 +312,24 @@ void stage_alloc(HostStage& h, size_t bytes)
     h.cap = bytes;
 }
 
+// The object's device for a launch, then the calling thread's own again.
+struct DeviceScope {
+    int before = -1;
+    int enter(int device)
+    {
+        int now = 0;
+        BDH_HIP(hipGetDevice(&now));
+        if (now == device) return 0;
+        BDH_HIP(hipSetDevice(device));
+        before = now;
+        return 0;
+    }
+    ~DeviceScope()
+    {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+
 int fetch(HostStage& h, int device, hipStream_t st, const Fetch* f, int nf)
 {
     BDH_CHECK(nf <= FETCH_MAX, "fetch: too many arrays");
@@ -327,7 +345,8 @@ int fetch(HostStage& h, int device, hipStream_t st, const Fetch* f, int nf)
         BDH_HIP(hipStreamSynchronize(st));
         return 0;
     }
-    BDH_HIP(hipSetDevice(device));
+    DeviceScope scope;
+    if (scope.enter(device)) return -1;
     std::lock_guard<std::mutex> lock(h.use);
     for (int k = 0; k < nf; ++k) {
         J.src[k] = static_cast<const unsigned*>(f[k].src);

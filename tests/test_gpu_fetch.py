@@ -58,3 +58,21 @@ def test_readers_in_threads(N):
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_reading_leaves_the_device():
+    """A system of one GPU read by a thread whose current device is another: it still is afterwards."""
+    import torch
+
+    from bd_box_amd import system as S
+    if torch.cuda.device_count() < 2:
+        pytest.skip("needs two GPUs")
+    s = S.BDSystem(wl.chain(20, seed=1), wl.parse_params(wl.chain_params()), precision=S.FP64, device=0)
+    s.compute_hydro(1)
+    torch.cuda.set_device(1)
+    print("reading leaves the device", flush=True)
+    try:
+        s.coords(), s.forces()
+        assert torch.cuda.current_device() == 1
+    finally:
+        torch.cuda.set_device(0)
