@@ -2261,42 +2261,34 @@ std::vector<int> batch_tune_candidates(const bdh_batch* b)
     return cand;
 }
 
-// Each candidate (left_max, outer): one refactor, then `reps` timed ones (HIP events on the
-// batch's stream); its time is the fastest.  Every one recomputes the same matrices from the
-// unchanged positions with the same launches, so the times differ by noise only; the fastest
-// candidate is kept.
-int batch_tune(bdh_batch* b, int reps, const std::vector<std::pair<int, int>>& cand, int* ib_out,
-               std::vector<double>& t)
+// The time of one refactor (one untimed, then the fastest of `reps`, by HIP events on the batch's
+// stream) for each of the candidates (left_max, outer): they are the same launches, so one of them is
+// timed for all and the first is kept.
+int batch_tune(bdh_batch* b, int reps, const std::vector<std::pair<int, int>>& cand, std::vector<double>& t)
 {
     hipEvent_t e0, e1;
     BDH_HIP(hipEventCreate(&e0));
     BDH_HIP(hipEventCreate(&e1));
-    int rc = 0, ib = 0;
-    t.assign(cand.size(), 0.0);
-    for (size_t i = 0; i < cand.size() && !rc; ++i) {
-        rc = batch_set_tiles(b, cand[i].first, cand[i].second) || batch_factor(b) || batch_check(b) ? -1 : 0;
-        double tmin = 1e30;
-        for (int r = 0; r < reps && !rc; ++r) {
-            float ms = 0.f;
-            const bool ok = hipEventRecord(e0, b->st) == hipSuccess && batch_factor(b) == 0 &&
-                            hipEventRecord(e1, b->st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
-                            hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
-            if (!ok) {
-                set_error("bdh_batch_autotune: a timed refactor failed");
-                rc = -1;
-            }
-            tmin = std::min(tmin, (double)ms);
+    int rc = batch_factor(b) || batch_check(b) ? -1 : 0;
+    double tmin = 1e30;
+    for (int r = 0; r < reps && !rc; ++r) {
+        float ms = 0.f;
+        const bool ok = hipEventRecord(e0, b->st) == hipSuccess && batch_factor(b) == 0 &&
+                        hipEventRecord(e1, b->st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
+                        hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
+        if (!ok) {
+            set_error("bdh_batch_autotune: a timed refactor failed");
+            rc = -1;
         }
-        if (!rc) rc = batch_check(b);
-        t[i] = tmin;
-        if (t[i] < t[ib]) ib = (int)i;
+        tmin = std::min(tmin, (double)ms);
     }
+    if (!rc) rc = batch_check(b);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    if (batch_set_tiles(b, cand[ib].first, cand[ib].second)) return -1;
+    t.assign(cand.size(), tmin);
+    if (batch_set_tiles(b, cand[0].first, cand[0].second)) return -1;
     b->have_L = false;
-    *ib_out = ib;
     return 0;
 }
 
@@ -2305,10 +2297,9 @@ int batch_autotune(bdh_batch* b, int reps, int* cand_out, double* ms_out, int* n
     std::vector<std::pair<int, int>> cand;
     for (int l : batch_tune_candidates(b)) cand.emplace_back(l, b->outer);
     std::vector<double> t;
-    int ib = 0;
-    if (batch_tune(b, reps, cand, &ib, t)) return -1;
+    if (batch_tune(b, reps, cand, t)) return -1;
     *ncand = (int)cand.size();
-    *best = cand[ib].first;
+    *best = cand[0].first;
     for (size_t i = 0; i < cand.size(); ++i) {
         if (cand_out) cand_out[i] = cand[i].first;
         if (ms_out) ms_out[i] = t[i];
@@ -2330,10 +2321,9 @@ int batch_autotune_tiles(bdh_batch* b, int reps, int* cand_left, int* cand_outer
     }
     BDH_CHECK((int)cand.size() <= BDH_TUNE_TILES_MAX, "bdh_batch_autotune_tiles: too many candidates");
     std::vector<double> t;
-    int ib = 0;
-    if (batch_tune(b, reps, cand, &ib, t)) return -1;
+    if (batch_tune(b, reps, cand, t)) return -1;
     *ncand = (int)cand.size();
-    *best = ib;
+    *best = 0;
     for (size_t i = 0; i < cand.size(); ++i) {
         if (cand_left) cand_left[i] = cand[i].first;
         if (cand_outer) cand_outer[i] = cand[i].second;

@@ -411,8 +411,8 @@ class BDBatch:
         return v.value
 
     def autotune(self, reps: int = 3):
-        """Times the refactor under each candidate schedule and keeps the fastest (before the
-        first step).  Returns (chosen left_max, {left_max: ms})."""
+        """Times the refactor (before the first step).  Returns (left_max kept, {left_max: ms}):
+        there is one schedule, so one time for every candidate, and the first is kept."""
         cand = (C.c_int * 8)()
         ms = np.zeros(8)
         n, best = C.c_int(), C.c_int()
@@ -429,9 +429,8 @@ class BDBatch:
         return lm.value, ou.value
 
     def autotune_tiles(self, reps: int = 3):
-        """Times the refactor under every (schedule, outer panel width) candidate and keeps
-        the fastest (before the first step).  Returns ((left_max, outer), {(left_max, outer):
-        ms})."""
+        """autotune over (schedule, outer panel width): ((left_max, outer) kept, {(left_max,
+        outer): ms}), one time for every candidate."""
         M = 24
         cl, co = (C.c_int * M)(), (C.c_int * M)()
         ms = np.zeros(M)

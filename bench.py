@@ -385,8 +385,7 @@ def main():
     ap.add_argument("--traffic-command", default="",
                     help="with --summarize-traffic: the commands that made the counter runs")
     ap.add_argument("--no-autotune", dest="autotune", action="store_false",
-                    help="batch workload: do not time the candidates of update schedule and panel "
-                         "width before the run (they give the same launches and results)")
+                    help="accepted and without effect: the batch's factorization has one schedule")
     args = ap.parse_args()
     if args.summarize_traffic:
         return summarize_traffic(*args.summarize_traffic, args.traffic_command)
@@ -703,8 +702,7 @@ def bench_periodic(args):
 def bench_batch(args):
     """Steps/s of a batch of independent chains (every chain advances one step per step),
     mixed (FP32 MFMA trailing updates, FP64 diagonal blocks) beside FP64 and split-bf16,
-    each phase one launch over all chains and every full refactor cycle one graph launch;
-    the autotuner's candidates (update schedule, outer panel width) timed per precision."""
+    each phase one launch over all chains and every full refactor cycle one graph launch."""
     import torch
     from bd_box_amd.system import BDBatch, FP64, MIXED, MIXED_SPLIT
     systems, prm, P, seeds = batch_workload(args.chains, args.seed)
@@ -715,14 +713,9 @@ def bench_batch(args):
     warm = min(args.warmup, R)
     log(f"batch workload: {len(sizes)} chains, {Ntot} beads (N {min(sizes)}..{max(sizes)}), "
         f"{steps} timed steps")
-    out, sched = {}, {}
+    out = {}
     for name, prec in (("mixed", MIXED), ("fp64", FP64), ("split", MIXED_SPLIT)):
         b = BDBatch(systems, P, seeds, precision=prec, refactor_every=R)
-        if args.autotune:
-            best, times = b.autotune_tiles(reps=3)
-            sched[name] = {"left_max": best[0], "outer": best[1],
-                           "refactor_ms": {f"{k[0]}/{k[1]}": v for k, v in times.items()}}
-            log(f"{name}: autotuned tiles left_max={best[0]} outer={best[1]} (refactor ms {times})")
         b.compute_hydro(warm)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -740,8 +733,6 @@ def bench_batch(args):
     disp = {}
     for name, prec in (("mixed", MIXED), ("fp64", FP64)):
         b = BDBatch(systems, P, seeds, precision=prec, refactor_every=R)
-        if name in sched:
-            b.set_tiles(sched[name]["left_max"], sched[name]["outer"])
         b.compute_hydro(R)
         disp[name] = b.coords()[:, :3]
         b.close()
@@ -775,7 +766,6 @@ def bench_batch(args):
                                f"refactored every {R} steps, FP32 MFMA trailing updates, FP64 "
                                f"diagonal blocks, each refactor cycle one graph launch",
                    "chains": len(sizes), "beads": Ntot, "refactor_every": R,
-                   "update_schedule": sched or "one schedule, not timed",
                    "parallelism": "1 GPU"},
         "chain_steps_per_s": value * len(sizes),
         "bead_steps_per_s": value * Ntot,

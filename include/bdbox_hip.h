@@ -308,10 +308,10 @@ int bdh_batch_phase_times(bdh_batch* batch, double* ms, long long* counts);
  * launches and the same results; the value is kept for bdh_batch_get_schedule. */
 int bdh_batch_set_schedule(bdh_batch* batch, int left_max);
 int bdh_batch_get_schedule(bdh_batch* batch, int* left_max);
-/* Times the refactor of every chain (assembly + factorization, graph replays, fastest of
- * `reps`) under each candidate left_max -- 0, then up to BDH_TUNE_MAX - 1 of the batch's padded
- * sizes, the largest included -- and keeps the fastest.  cand / ms (BDH_TUNE_MAX entries each,
- * may be NULL) receive the candidates and their times, *ncand their count, *best the choice.
+/* Times the refactor of every chain (assembly + factorization, graph replays, fastest of `reps`).
+ * There is one schedule, so it is timed once: cand / ms (BDH_TUNE_MAX entries each, may be NULL)
+ * receive the values of left_max -- 0, then up to BDH_TUNE_MAX - 1 of the batch's padded sizes, the
+ * largest included -- each with that time, *ncand their count, *best the first, which is kept.
  * Call it before the first step; the first step then refactors as usual. */
 #define BDH_TUNE_MAX 8
 int bdh_batch_autotune(bdh_batch* batch, int reps, int* cand, double* ms, int* ncand, int* best);
@@ -323,7 +323,7 @@ int bdh_batch_get_tiles(bdh_batch* batch, int* left_max, int* outer);
 /* bdh_batch_autotune over tile shapes: every schedule candidate of bdh_batch_autotune under
  * each outer panel width (256, then 512 and 1024 where the largest chain reaches them), at
  * most BDH_TUNE_TILES_MAX candidates.  cand_left / cand_outer / ms (may be NULL) receive
- * the candidates and their refactor times, *ncand their count, *best the index kept. */
+ * the candidates, each with the one time, *ncand their count, *best the index kept (0). */
 #define BDH_TUNE_TILES_MAX 24
 int bdh_batch_autotune_tiles(bdh_batch* batch, int reps, int* cand_left, int* cand_outer, double* ms,
                              int* ncand, int* best);

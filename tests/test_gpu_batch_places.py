@@ -24,3 +24,16 @@ def test_batch_equals_systems(chains):
             s = S.BDSystem(systems[c], p, precision=prec)
             s.compute_hydro(2)
             assert np.array_equal(b.chain_coords(c), s.coords()), (prec, c)
+
+
+def test_tuner_times_one_schedule():
+    """Candidates that are the same launches get one time and the first is kept."""
+    from bd_box_amd import system as S
+    b = S.BDBatch([wl.chain(N, seed=N) for N in (60, 200, 700)], wl.parse_params(wl.chain_params()), [1, 2, 3],
+                  precision=S.MIXED)
+    print("tuner", flush=True)
+    for tune, first in ((b.autotune, 0), (b.autotune_tiles, (0, 256))):
+        best, times = tune(reps=2)
+        assert best == first and len(times) > 1
+        assert len(set(times.values())) == 1 and times[best] > 0.0
+    b.close()
