@@ -256,13 +256,14 @@ __device__ __forceinline__ void recip_sum(const EwaldTables& E, double rx, doubl
     Q[5] = -o2;
 }
 
-// Real-space images r + L (h, f, g) with h^2 + f^2 + g^2 <= RR, h, then f, then g ascending, within
-// sqrt(rc2) of the pair: image(x, y, z, r2) for each.  A column (h, f) that lies beyond the cutoff
-// for every pair of the wavefront is skipped whole.
+// Real-space images r + L (h, f, g) with h^2 + f^2 + g^2 <= RR, h, then f, then g ascending, with CUT
+// within sqrt(rc2) of the pair: image(x, y, z, r2) for each.  A column (h, f) that lies beyond the
+// cutoff for every pair of the wavefront is skipped whole.  Without CUT a coordinate that is not a
+// number reaches the image term and the tensor.
 // Every coordinate is formed from its index with one rounding.  A coordinate stepped by L from r - R L
 // carries the rounding at R L: the pair (i, i) then misses its central image's zero for most boxes
 // that are not exact in a few bits, and near images lose bits in all of them.
-template <typename T, typename F>
+template <typename T, bool CUT, typename F>
 __device__ __forceinline__ void each_image(const double box, const int RR, const T rc2, double rx, double ry,
                                            double rz, F&& image)
 {
@@ -272,12 +273,12 @@ __device__ __forceinline__ void each_image(const double box, const int RR, const
         const int nf = isqrt_small(RR - h * h);
         for (int f = -nf; f <= nf; ++f) {
             const T y = (T)__builtin_fma(box, (double)f, ry), rho = x * x + y * y;
-            if (!__any(rho <= rc2)) continue;
+            if (CUT && !__any(rho <= rc2)) continue;
             const int ng = isqrt_small(RR - h * h - f * f);
             double gd = -ng;
             for (int g = -ng; g <= ng; ++g, gd += 1.0) {
                 const T z = (T)__builtin_fma(box, gd, rz), r2 = rho + z * z;
-                if (r2 != (T)0 && r2 <= rc2) image(x, y, z, r2);
+                if (r2 != (T)0 && (!CUT || r2 <= rc2)) image(x, y, z, r2);
             }
         }
     }
@@ -322,7 +323,7 @@ __device__ __forceinline__ Blk6 beenakker_block(double rx, double ry, double rz,
     const double nlg = sizeof(T) == 8 ? -E.alpha2 : -E.alpha2 * 1.4426950408889634074;
     const T nl = (T)nlg, nl_lo = (T)(nlg - (double)nl);
     T Ot[7] = {0, 0, 0, 0, 0, 0, 0};   // xx yy zz xy xz yz of c2 e e^T, and c1 (FP32)
-    each_image<T>(E.box, E.RR_real, (T)E.rc2, rx, ry, rz, [&](T x, T y, T z, T rr) {
+    each_image<T, true>(E.box, E.RR_real, (T)E.rc2, rx, ry, rz, [&](T x, T y, T z, T rr) {
         const T inv_r = inv_dist(rr), ir2 = inv_r * inv_r;
         const T X = erfcx_image(rr * inv_r * al) * inv_r;
         const T ex = exp_image(rr, nl, nl_lo);
@@ -394,7 +395,7 @@ __device__ __forceinline__ Blk6 smith_block(double rx, double ry, double rz, dou
     const T fo = (T)E.preO, fq = (T)preQ;
     const double nlg = sizeof(T) == 8 ? -E.alpha2 : -E.alpha2 * 1.4426950408889634074;
     const T nl = (T)nlg, nl_lo = (T)(nlg - (double)nl);
-    each_image<T>(1.0, E.RR_real, (T)E.rc2, rx * E.inv_L, ry * E.inv_L, rz * E.inv_L, [&](T x, T y, T z, T rr) {
+    each_image<T, false>(1.0, E.RR_real, (T)0, rx * E.inv_L, ry * E.inv_L, rz * E.inv_L, [&](T x, T y, T z, T rr) {
         const T inv_r = inv_dist(rr), ir2 = inv_r * inv_r, rn = rr * inv_r;
         const T eg = exp_image(rr, nl, nl_lo);
         const T ec = erfcx_image(rn * al) * eg;

@@ -208,3 +208,22 @@ def test_ewald_rounding(api, seed):
     b.close()
     err = np.abs(D.reshape(50, 3, 50, 3).transpose(0, 2, 1, 3) - ref)[off].max((1, 2)) / np.abs(D).max()
     assert np.sqrt((err ** 2).mean()) <= 2.0 ** -53 * np.sqrt(2 / 3), float(np.sqrt((err ** 2).mean()))
+
+
+@pytest.mark.parametrize("R", [0, 2])
+def test_smith_tensor_shows_nan(api, R):
+    """A coordinate that is not a number is one in every Smith block of its bead, also where no
+    reciprocal vector carries it; the other beads' blocks are as without it."""
+    s, P = _spheres(20, 0.05, 7, "smith", R)
+    print("smith nan", R, flush=True)
+    for prec in (api.FP64, api.MIXED):
+        b = api.BDSystem(s, P, precision=prec)
+        ref = b.compute_D()
+        c = s.coord.copy()
+        c[4, 1] = np.nan
+        b.set_coords(c)
+        D = b.compute_D().reshape(20, 3, 20, 3)
+        b.close()
+        rest = [k for k in range(20) if k != 4]
+        assert np.isnan(D[4][:, rest]).all() and np.isnan(D[rest][:, :, 4]).all()
+        assert np.array_equal(D[np.ix_(rest, range(3), rest, range(3))], ref.reshape(20, 3, 20, 3)[np.ix_(rest, range(3), rest, range(3))])
