@@ -25,3 +25,30 @@ def test_tea_step_vs_oracle(N):
         s.compute_hydro(1, xi)
         d = s.coords()[:, :3] - sysm.coord[:, :3]
         assert np.linalg.norm(d - d_ref) <= tol * np.linalg.norm(d_ref), prec
+
+
+@pytest.mark.parametrize("hydro", ["cholesky", "geyer"])
+def test_pair_sums_of_a_lost_bead(hydro):
+    """A bead so far away that its squared distance is beyond FP64's range (and its blocks with the
+    others zero) moves by its own mobility, and the others as without it: 1e-14, a few roundings."""
+    from bd_box_amd import system as S
+    N = 70
+    sysm = wl.chain(N, seed=3)
+    sysm = wl.System(sysm.coord, sysm.Q, sysm.LJ, sysm.bonds[:0], sysm.bond_parms[:0])
+    sysm.coord[9, :3] = [1e160, -2e160, 3e160]
+    P = wl.parse_params(wl.chain_params(hydro=hydro))
+    print("lost bead", hydro, flush=True)
+    F = np.random.default_rng(1).normal(size=(N, 3))
+    s = S.BDSystem(sysm, P, precision=S.FP64)
+    s.set_forces(F)
+    Rf = s.compute_Rf().reshape(N, 3)
+    rest = np.arange(N) != 9
+    less = wl.System(sysm.coord[rest], sysm.Q[rest], sysm.LJ[rest], sysm.bonds[:0], sysm.bond_parms[:0])
+    r = S.BDSystem(less, P, precision=S.FP64)
+    r.set_forces(F[rest])
+    ref = r.compute_Rf().reshape(-1, 3)
+    assert np.abs(Rf[rest] - ref).max() <= 1e-14 * np.abs(ref).max()
+    one = S.BDSystem(wl.System(sysm.coord[9:10], sysm.Q[:1], sysm.LJ[:1], sysm.bonds[:0], sysm.bond_parms[:0]), P,
+                     precision=S.FP64)
+    one.set_forces(F[9:10])
+    assert np.array_equal(Rf[9], one.compute_Rf())
