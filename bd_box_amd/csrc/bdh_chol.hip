@@ -31,17 +31,6 @@ __device__ __forceinline__ double readlane_f64(double v, int src)
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// 1/sqrt(x): hardware estimate (relative error about 2^-23) refined by one third-order step,
-// y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2, whose truncation (5/16 e^3) is below 2^-68.  Four
-// dependent operations where two Newton steps take eight; the diagonal factor's pivot chain
-// runs through it once per column.
-__device__ __forceinline__ double rsqrt_f64(double x)
-{
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = __builtin_fma(-(x * y), y, 1.0);
-    return __builtin_fma(__builtin_fma(e, 0.375, 0.5), y * e, y);
-}
-
 // Per diagonal block, the workspace Lb holds (FP64):
 //   Lb[0 .. 4095]      L_kk column-major, zeros above the diagonal
 //   Lb[4096 + SINV J]  inverse of its J-th 16x16 diagonal sub-block, column-major with pitch
@@ -68,7 +57,9 @@ __device__ __forceinline__ int flow_tid()
 // every earlier group's update made; finished columns go to L (LDS, column-major; what a lane
 // above the diagonal holds is not part of the factor).
 // Per column t the pivot chain is: reciprocal square root, l_{t+1,t}, the next pivot
-// a_{t+1,t+1} - l_{t+1,t}^2.  Column t + 1 takes column t's update from a broadcast (v_readlane) of
+// a_{t+1,t+1} - l_{t+1,t}^2.  The root is the hardware's estimate (relative error about 2^-23) refined
+// by one third-order step, y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2, whose truncation (5/16 e^3) is
+// below 2^-68: four dependent operations where two Newton steps take eight.  Column t + 1 takes column t's update from a broadcast (v_readlane) of
 // its entry before it is scaled, so it does not wait for the LDS; the later ones take it one
 // column late from LDS broadcasts of the stored column, two at a time between the dependent
 // operations of the next pivot (fill), which are 12 cycles apart where an FP64 FMA issues in 4.
@@ -233,11 +224,6 @@ __device__ __forceinline__ void factor_diag64(double* __restrict__ sD, int c0, i
     __syncthreads();   // L and the inverses complete in LDS
 }
 
-__device__ __forceinline__ void factor_diag64(double* __restrict__ sD, int c0, int* __restrict__ status)
-{
-    factor_diag64(sD, c0, status, [] {});
-}
-
 // Agent-scope store: written through to memory, so it is visible to every workgroup once it has
 // completed.
 __device__ __forceinline__ void st_agent(double* p, double v)
@@ -307,99 +293,82 @@ __device__ __forceinline__ void split_bf16(float x, unsigned& hi, unsigned& lo)
     lo = bf16_bits(x - __builtin_bit_cast(float, hi << 16));
 }
 
-// acc[q] = sum_k A[ra + i][kb + k] A[ca + 32 q + j][kb + k] over NQ 32 x 32 quadrants side by side
-// (rows ra .., columns ca + 32 q ..), K a multiple of 32, on one wavefront's MFMA with operands
-// loaded straight from A (no LDS), KC = 32 / NQ k at a time with the next KC in flight.
-// v_mfma_f32_32x32x2_f32: lane l feeds row l % 32, k = l / 32; acc[q][r] holds row
-// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of quadrant q.
-template <int NQ>
-__device__ __forceinline__ void quad_acc(const float* __restrict__ A, long long ld, int ra, int ca, int kb, int K,
-                                         floatx16 (&acc)[NQ])
+// acc = sum_k A[ra + i][k] A[ca + j][k], k < K (a multiple of 32), of a 32 x 32 block on one
+// wavefront's MFMA with operands loaded straight from A (no LDS), 32 k at a time with the next 32 in
+// flight.  v_mfma_f32_32x32x2_f32: lane l feeds row l % 32, k = l / 32; acc[r] holds row
+// 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
+__device__ __forceinline__ void quad_acc(const float* __restrict__ A, long long ld, int ra, int ca, int K,
+                                         floatx16& acc)
 {
-    constexpr int KC = 32 / NQ, NJ = KC / 2;
+    constexpr int KC = 32, NJ = KC / 2;
     const int lane = flow_tid<true>() & 63, l32 = lane & 31, lh = lane >> 5;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
-    float av[NJ], bv[NQ][NJ];
-    auto load = [&](int k0, float (&a)[NJ], float (&bq)[NQ][NJ]) {
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    float av[NJ], bv[NJ];
+    auto load = [&](int k0, float (&a)[NJ], float (&b)[NJ]) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const float* col = A + (long long)(kb + k0 + 2 * j + lh) * ld;
+            const float* col = A + (long long)(k0 + 2 * j + lh) * ld;
             a[j] = col[ra + l32];
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) bq[q][j] = col[ca + 32 * q + l32];
+            b[j] = col[ca + l32];
         }
     };
     load(0, av, bv);
     for (int k0 = 0; k0 < K; k0 += KC) {
-        float an[NJ], bn[NQ][NJ];
+        float an[NJ], bn[NJ];
         if (k0 + KC < K) load(k0 + KC, an, bn);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) acc[q] = mfma_f32_32x32x2(av[j], bv[q][j], acc[q]);
+        for (int j = 0; j < NJ; ++j) acc = mfma_f32_32x32x2(av[j], bv[j], acc);
         if (k0 + KC < K) {
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
                 av[j] = an[j];
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) bv[q][j] = bn[q][j];
+                bv[j] = bn[j];
             }
         }
     }
 }
 
-// The same in FP64, K a multiple of 16: v_mfma_f64_16x16x4_f64 on the 2 x 2 tiles of each
-// quadrant, lane l feeds row l % 16, k = l / 16; acc[q][i][j][r] holds row 16 i + 4 r + l / 16,
-// column 16 j + l % 16 of quadrant q.  16 k at a time with the next 16 in flight.
-template <int NQ>
-__device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long ld, int ra, int ca, int kb, int K,
-                                         doublex4 (&acc)[NQ][2][2])
+// The same in FP64, K a multiple of 16: v_mfma_f64_16x16x4_f64 on the 2 x 2 tiles of the block,
+// lane l feeds row l % 16, k = l / 16; acc[i][j][r] holds row 16 i + 4 r + l / 16, column
+// 16 j + l % 16.  16 k at a time with the next 16 in flight.
+__device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long ld, int ra, int ca, int K,
+                                         doublex4 (&acc)[2][2])
 {
     const int lane = flow_tid<true>() & 63, l16 = lane & 15, lq = lane >> 4;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[q][i][j] = doublex4{0.0, 0.0, 0.0, 0.0};
-    double av[4][2], bv[NQ][4][2];
-    auto load = [&](int k0, double (&a)[4][2], double (&bq)[NQ][4][2]) {
+        for (int j = 0; j < 2; ++j) acc[i][j] = doublex4{0.0, 0.0, 0.0, 0.0};
+    double av[4][2], bv[4][2];
+    auto load = [&](int k0, double (&a)[4][2], double (&b)[4][2]) {
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
-            const double* col = A + (long long)(kb + k0 + 4 * s4 + lq) * ld;
-            a[s4][0] = col[ra + l16];
-            a[s4][1] = col[ra + 16 + l16];
+            const double* col = A + (long long)(k0 + 4 * s4 + lq) * ld;
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                bq[q][s4][0] = col[ca + 32 * q + l16];
-                bq[q][s4][1] = col[ca + 32 * q + 16 + l16];
+            for (int i = 0; i < 2; ++i) {
+                a[s4][i] = col[ra + 16 * i + l16];
+                b[s4][i] = col[ca + 16 * i + l16];
             }
         }
     };
     load(0, av, bv);
     for (int k0 = 0; k0 < K; k0 += 16) {
-        double an[4][2], bn[NQ][4][2];
+        double an[4][2], bn[4][2];
         if (k0 + 16 < K) load(k0 + 16, an, bn);
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4)
 #pragma unroll
-            for (int q = 0; q < NQ; ++q)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[q][i][j] = mfma_f64_16x16x4(av[s4][i], bv[q][s4][j], acc[q][i][j]);
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma_f64_16x16x4(av[s4][i], bv[s4][j], acc[i][j]);
         if (k0 + 16 < K) {
 #pragma unroll
             for (int s4 = 0; s4 < 4; ++s4)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     av[s4][i] = an[s4][i];
-#pragma unroll
-                    for (int q = 0; q < NQ; ++q) bv[q][s4][i] = bn[q][s4][i];
+                    bv[s4][i] = bn[s4][i];
                 }
         }
     }
@@ -1059,9 +1028,9 @@ struct FlowQuad<float> {
     // K = 64 columns straight from memory
     __device__ void mac_global(const float* p, long long ld, int mb, int nb)
     {
-        floatx16 t[1];
-        quad_acc<1>(p, ld, 32 * mb, 32 * nb, 0, CHOL_NB, t);
-        a += t[0];
+        floatx16 t;
+        quad_acc(p, ld, 32 * mb, 32 * nb, CHOL_NB, t);
+        a += t;
     }
     template <typename F>
     __device__ void each(int lane, F&& f)
@@ -1126,12 +1095,12 @@ struct FlowQuad<double> {
     }
     __device__ void mac_global(const double* p, long long ld, int mb, int nb)
     {
-        doublex4 t[1][2][2];
-        quad_acc<1>(p, ld, 32 * mb, 32 * nb, 0, CHOL_NB, t);
+        doublex4 t[2][2];
+        quad_acc(p, ld, 32 * mb, 32 * nb, CHOL_NB, t);
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
-            for (int y = 0; y < 2; ++y) a[x][y] += t[0][x][y];
+            for (int y = 0; y < 2; ++y) a[x][y] += t[x][y];
     }
     template <typename F>
     __device__ void each(int lane, F&& f)
