@@ -59,8 +59,9 @@ __device__ __forceinline__ int flow_tid()
 // Per column t the pivot chain is: reciprocal square root, l_{t+1,t}, the next pivot
 // a_{t+1,t+1} - l_{t+1,t}^2.  The root is the hardware's estimate (relative error about 2^-23) refined
 // by one third-order step, y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2, whose truncation (5/16 e^3) is
-// below 2^-68: four dependent operations where two Newton steps take eight.  Column t + 1 takes column t's update from a broadcast (v_readlane) of
-// its entry before it is scaled, so it does not wait for the LDS; the later ones take it one
+// below 2^-68: four dependent operations where two Newton steps take eight.  Column t + 1 takes
+// column t's update from a broadcast (v_readlane) of its entry before it is scaled, so it does not
+// wait for the LDS; the later ones take it one
 // column late from LDS broadcasts of the stored column, two at a time between the dependent
 // operations of the next pivot (fill), which are 12 cycles apart where an FP64 FMA issues in 4.
 // step(t): work of the caller's for the same gaps.
@@ -139,7 +140,10 @@ __device__ __forceinline__ void factor_group16(double (&p)[16], double (&y)[16],
 // trailing 16x16 tiles stay in MFMA accumulators from the start, transposed (accumulator r of
 // lane l: column 4 r + l/16 of the tile, row l%16), so the next group's tiles reach the
 // lane = row form with one conflict-free pass through the LDS columns they will be factored in.
-// What bounds it: the chain of 64 pivots, each about 80 cycles of dependent FP64 operations.
+// What bounds it: one wavefront's serial work.  Of 19000 cycles (7.9 us) on an idle GPU the 64
+// pivots take 62 %, 160 to 215 cycles each: about 80 of dependent operations, then the issue of the
+// column's updates and the LDS reads of its broadcasts.  The inverses' stores, the updates between
+// the groups and the tiles' way through the LDS take 36 %.
 // 64x64 block on an idle GPU: 11.2 us as a pipeline of the four wavefronts over the column
 // groups, 8.2 us as here.
 // A non-positive (or NaN) pivot records row c0 + j + 1 in *status (the first one wins) and the
@@ -389,16 +393,17 @@ __device__ __forceinline__ void quad_acc(const double* __restrict__ A, long long
 // places of the XCD on which the other's lowest unfinished tile waits for one.
 // The waits are bounded anyway (flow_wait).
 // What bounds it: for small matrices the chain diagonal block -> solve of the next block row ->
-// its update -> next diagonal block; for large ones MFMA issue of the accumulation, which no
-// longer reads and writes C once per outer panel and whose operands are shared in L2.  The chain
+// its update -> next diagonal block; for large ones MFMA issue of the accumulation, whose operands
+// are shared in L2 (C is read and written once in FP32, once per 256 columns in FP64).  The chain
 // overlaps with everything else, since the workgroups of the following tile columns are
 // resident and accumulate what is already published.
 // Measured against one launch per 256-column outer panel (n_pad >= 1024) or per 64-column panel
 // (below), right-looking: n = 768 FP64 640 -> 202 us, n = 1353 FP32 720 -> 331 us, n = 3072 FP64
 // 1900 -> 840 us, n = 9000 FP32 5.95 -> 2.82 ms, FP64 11.3 -> 5.7 ms; the batch of 256 chains of
 // 64 .. 1024 beads FP32 6.9 -> 4.0 ms.  Beside another tile on its CU a tile takes 13.4 us for 128
-// columns in FP32 and 28.7 in FP64, MFMA issue at its peak; the rest at n = 9000 is the chain (31
-// us per tile column FP32, 33 FP64) and tiles that become resident too late to have caught up.
+// columns in FP32 and 28.7 in FP64 (without the passes over C), MFMA issue at its peak; the rest at
+// n = 9000 is the chain (31 us per tile column FP32, 33 FP64) and tiles that become resident too
+// late to have caught up.
 //
 // Visibility across XCDs, whose L2 caches are not coherent within a launch: what other
 // workgroups read is stored at agent scope (write-through), the flag that announces it is set
@@ -1309,7 +1314,7 @@ __device__ __forceinline__ int flow_task(int* __restrict__ next)
 // and waits for room in the shader engine whose turn it is, a sixth of the places stood empty (256
 // chains of 64 .. 1024 beads FP32: 3.64 -> 3.39 ms).  One matrix keeps a workgroup per tile: its
 // columns end together, and the loop's extra instructions lie on its chain (n = 9000 FP32 2.79 ms,
-// 2.98 with the loop, FP64 4.94 and 5.27).
+// 2.98 with the loop, FP64 4.94 and 5.27, both before FP64 took its sums in parts).
 constexpr int FLOW_PLACES = 512;   // two workgroups on each of 256 CUs
 constexpr int FLOW_STEP = 10;      // 100 ns (in 100 MHz ticks), in which the counter serves eight workgroups
 // A null counter: one task, no loop (with a loop in every case the compiler spills 30 to 50 registers).

@@ -104,8 +104,9 @@ constexpr ImageCoef IMAGE_COEF = {
 
 // exp(-u) for the squared distance r2 with u = alpha^2 r2.  FP32: the hardware's base-2 exponential
 // of the product with -alpha^2 log2(e) in two parts (nl, nl_lo), so the argument is rounded once.
-// FP64 (nl = -alpha^2): 2^n exp(r) with |r| <= ln(2)/2 and the Taylor polynomial of degree 13, even
-// and odd powers in chains of their own; arguments of any size (the result goes to zero).
+// FP64 (nl = -alpha^2): 2^n exp(r) with |r| <= ln(2)/2, n ln(2) taken off in two parts (Cody and
+// Waite, Software Manual for the Elementary Functions, 1980), and the Taylor polynomial of degree
+// 13, even and odd powers in chains of their own; arguments of any size (the result goes to zero).
 __device__ __forceinline__ double exp_image(double r2, double nl, double)
 {
     const double x = nl * r2;
@@ -128,8 +129,9 @@ __device__ __forceinline__ float exp_image(float r2, float nl, float nl_lo)
 
 // exp(x^2) erfc(x) for x >= 0.  FP32 (the mixed step's real-space images): the form of Abramowitz &
 // Stegun 7.1.26, t (a1 + t (a2 + ...)), t = 1 / (1 + p x), with one term more and p and the
-// coefficients fitted to the smallest largest error of erfc: 8e-9 (7.1.26: 1.4e-7), so FP32
-// rounding is what is left; the reciprocal is the hardware's with one Newton step.  FP64: the expansion of Shepherd and
+// coefficients fitted to the smallest largest error of erfc, which with the coefficients as rounded
+// here is 4.5e-8, at x = 0 (7.1.26: 1.4e-7); with the sum in FP32 too it is 3.8e-7 (7.1.26: 5.6e-7).
+// The reciprocal is the hardware's with one Newton step.  FP64: the expansion of Shepherd and
 // Laframboise (Math. Comp. 36 (1981) 249), (1 + 2 x) exp(x^2) erfc(x) as a polynomial in t = (x -
 // 3.75) / (x + 3.75), degree 22, coefficients fitted in 60-digit arithmetic: relative error <=
 // 3.2e-16 over 0 <= x <= 30; even and odd powers in chains of their own.  The exponential is the
@@ -287,9 +289,9 @@ __device__ __forceinline__ void each_image(const double box, const int RR, const
 // Beenakker block for the pair (i, j): r = r_j - r_i (no minimum image, dist_vec), radii
 // ai, aj; self = (i == j) adds the self term and clears the off-diagonal entries.
 // What bounds it: VALU issue (93 % of the cycles of the N = 8192 TEA sums), per image about 40
-// operations in FP32 and 100 in FP64 after the pair's constants are taken out of the loop, where
+// instructions in FP32 and 100 in FP64 after the pair's constants are taken out of the loop, where
 // the term as written in the reference took 78 in FP32 with its divisions and exponentials
-// (converged split at N = 8192, mixed: 6.2 -> 3.9 ms for all pairs).
+// (converged split at N = 8192, mixed: 6.2 -> 4.0 ms for all pairs).
 template <typename T>
 __device__ __forceinline__ Blk6 beenakker_block(double rx, double ry, double rz, double ai,
                                                 double aj, bool self, double preDii,
