@@ -3,6 +3,9 @@ import sys
 
 import numpy as np
 import pytest
+# Before libbdbox_hip.so: a process that loads the library first runs on the system's HIP runtime;
+# torch then brings its own beside it and finds no GPU, and tests that ask torch for one are skipped.
+import torch  # noqa: F401
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 if ROOT not in sys.path:
